@@ -196,6 +196,7 @@ struct egs_problem_s {
     double *d_dscr = nullptr;   // ts * ts scratch of the diagonal-tile factorization
     double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr, *d_partials = nullptr;
     int *d_info = nullptr;
+    double *d_tab = nullptr;    // Matern tables of the last covariance parameters (kTabSlots of them)
 
     std::vector<int64_t> h_off;
     std::vector<uint8_t> h_store;
@@ -217,7 +218,7 @@ struct egs_problem_s {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     egs::MaternParams *d_prm = nullptr;
-    egs::MaternParams h_prm;
+    egs::MaternParams h_prm{};
 
     egs::TileMap map() const {
         egs::TileMap m;
@@ -260,6 +261,25 @@ constexpr double kMaxNu = 100.0;
 
 bool valid_nu(double nu) { return nu > 0.0 && nu <= kMaxNu; }
 
+// Table slots of the orders without a closed form (see matern_table_eval);
+// parameters far outside any data's scale are evaluated directly.
+void assign_tables(egs::MaternParams &prm) {
+    prm.inv_range2 = 1.0 / (prm.range * prm.range);
+    prm.ntab = 0;
+    for (int q = 0; q < 4; ++q) {
+        prm.tab[q] = -1;
+        const double nu = prm.nu[q], con = std::fabs(prm.con[q]);
+        if (nu == 0.5 || nu == 1.5 || nu == 2.5 || nu > egs::kTabMaxNu) continue;
+        if (!(prm.range > 1e-100 && prm.range < 1e100 && con > 1e-100 && con < 1e100)) continue;
+        for (int r = 0; r < q && prm.tab[q] < 0; ++r)
+            if (prm.tab[r] >= 0 && prm.nu[r] == nu && prm.con[r] == prm.con[q]) prm.tab[q] = prm.tab[r];
+        if (prm.tab[q] < 0) {
+            prm.tab_pair[prm.ntab] = q;
+            prm.tab[q] = prm.ntab++;
+        }
+    }
+}
+
 int make_params(int kernel, int metric, const double *th, egs::MaternParams &prm) {
     if (!th) return fail(EGS_ERR_INVALID_ARG, "theta is null");
     const int nth = kernel == EGS_KERNEL_BIVARIATE_MATERN_PARSIMONIOUS ? 6 : 3;
@@ -280,6 +300,7 @@ int make_params(int kernel, int metric, const double *th, egs::MaternParams &prm
             prm.nu[q] = nu;
             prm.con[q] = sigma2 * (1.0 / (std::pow(2.0, nu - 1) * std::tgamma(nu)));
         }
+        assign_tables(prm);
         return EGS_SUCCESS;
     }
     if (kernel == EGS_KERNEL_BIVARIATE_MATERN_PARSIMONIOUS) {
@@ -302,6 +323,7 @@ int make_params(int kernel, int metric, const double *th, egs::MaternParams &prm
         prm.con[0] = con1;
         prm.con[1] = prm.con[2] = con12;
         prm.con[3] = con2;
+        assign_tables(prm);
         return EGS_SUCCESS;
     }
     return fail(EGS_ERR_INVALID_ARG, "unknown kernel %d", kernel);
@@ -352,6 +374,7 @@ void free_problem_buffers(egs_problem_s *p) {
     pfree(p, p->d_aux);
     pfree(p, p->d_partials);
     pfree(p, p->d_info);
+    pfree(p, p->d_tab);
     for (auto &q : p->d_pairs_cls) {
         pfree(p, q);
         q = nullptr;
@@ -403,6 +426,7 @@ void free_problem_buffers(egs_problem_s *p) {
     p->d_pairs = nullptr;
     p->d_winv = p->d_dscr = p->d_obs = p->d_work = p->d_aux = p->d_partials = nullptr;
     p->d_info = nullptr;
+    p->d_tab = nullptr;
     for (auto &e : p->ev) e = nullptr;
 }
 
@@ -576,7 +600,8 @@ int run_covariance(egs_problem_s *p, const double *theta) {
     if (st) return st;
     const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
     const int pi = prof_begin(p, EGS_PROFILE_COVARIANCE, 0.0);
-    egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm, p->d_x, p->d_y, dz, p->n,
+    egs::launch_matern_tables(p->d_tab, prm, nullptr, p->ctx->stream);
+    egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm, p->d_x, p->d_y, dz, p->n, p->d_tab,
                              is_mixed(p) ? p->d_sig64 : nullptr, p->ctx->stream);
     prof_end(p, pi);
     EGS_HIP(hipGetLastError());
@@ -1055,7 +1080,8 @@ int64_t footprint(const egs_problem_s &q) {
     const int64_t nb = (int64_t) sizeof(double) * q.n_loc, vb = (int64_t) sizeof(double) * npad;
     int64_t b = dev_class_bytes(nb) * (q.dim == 3 ? 3 : 2) + dev_class_bytes(8 * nt * nt) + dev_class_bytes(nt * nt) +
                 dev_class_bytes(8 * ntiles) + dev_class_bytes(8 * nt * q.nsb * egs::kBlk * egs::kBlk) +
-                dev_class_bytes(8 * ts * ts) + 3 * dev_class_bytes(vb) + dev_class_bytes(16 * nt) + dev_class_bytes(4);
+                dev_class_bytes(8 * ts * ts) + 3 * dev_class_bytes(vb) + dev_class_bytes(16 * nt) + dev_class_bytes(4) +
+                dev_class_bytes(8 * egs::kTabSlots * egs::kTabDoubles);
     int64_t arena = 0;
     for (int j = 0; j < q.nt; ++j)
         for (int i = j; i < q.nt; ++i) {
@@ -1224,7 +1250,8 @@ int egs_problem_create(egs_context_t ctx, int kernel, int64_t n_loc, const doubl
               pmalloc(p, &p->d_obs, vb) == hipSuccess && pmalloc(p, &p->d_work, vb) == hipSuccess &&
               pmalloc(p, &p->d_aux, vb) == hipSuccess &&
               pmalloc(p, &p->d_partials, sizeof(double) * 2 * (size_t) nt) == hipSuccess &&
-              pmalloc(p, &p->d_info, sizeof(int)) == hipSuccess;
+              pmalloc(p, &p->d_info, sizeof(int)) == hipSuccess &&
+              pmalloc(p, &p->d_tab, sizeof(double) * egs::kTabSlots * egs::kTabDoubles) == hipSuccess;
     if (!ok) return cleanup(fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the problem's device buffers"));
     for (auto &e : p->ev)
         if (hipEventCreate(&e) != hipSuccess) return cleanup(fail(EGS_ERR_HIP, "hipEventCreate failed"));
@@ -1470,8 +1497,11 @@ int enqueue_fp64_eval(egs_problem_s *p) {
     hipStream_t s = p->ctx->stream;
     egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
     const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
+    p->h_prm.kernel = p->kernel;   // the launches are shaped by the kernel and the metric alone
+    p->h_prm.metric = p->metric;
+    egs::launch_matern_tables(p->d_tab, p->h_prm, p->d_prm, s);
     egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), p->h_prm, p->d_x, p->d_y, dz, p->n,
-                             nullptr, s, p->d_prm);
+                             p->d_tab, nullptr, s, p->d_prm);
     const int st = run_potrf(p);
     if (st) return st;
     run_forward(p);
@@ -1678,8 +1708,9 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             egs_problem_s *p = problems[b];
             egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
             const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
+            egs::launch_matern_tables(p->d_tab, prm[b], nullptr, s);
             egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm[b], p->d_x, p->d_y, dz, p->n,
-                                     nullptr, s);
+                                     p->d_tab, nullptr, s);
             egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_info), 1, s);
             p->has_cov = false;
             p->factored = false;
@@ -2003,8 +2034,9 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
     if (e == hipSuccess) e = hipMemcpyAsync(dym, ym, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess && three_d) e = hipMemcpyAsync(dzm, zm, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
+        egs::launch_matern_tables(p->d_tab, prm, nullptr, s);
         egs::launch_cov_gemv(d_out, rows, p->n, prm, dxm, dym, three_d ? dzm : nullptr, p->d_x, p->d_y,
-                             three_d ? p->d_z : nullptr, weights, s);
+                             three_d ? p->d_z : nullptr, weights, p->d_tab, s);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(zmiss, d_out, sizeof(double) * (size_t) rows, hipMemcpyDeviceToHost, s);

@@ -2,17 +2,113 @@
 // Kernel<T>::GenerateCovarianceMatrix (Kernel.hpp:93-97) for every lower tile of
 // Sigma at once (the reference submits one dcmg task per tile,
 // dcmg-codelet.cpp:47-74, and evaluates GSL's K_nu per element on CPU threads).
-//
-// One workgroup writes one 64 x 64 block of one tile.  The 64 row locations and
-// 64 column locations are staged in LDS; each wave then writes whole 64-element
-// column segments of the column-major tile (512 contiguous bytes per store
-// instruction in FP64).  Arithmetic is FP64 throughout; the store converts to
-// the tile's storage precision.
+// Arithmetic is FP64 throughout; the store converts to the tile's storage
+// precision.  Orders without a closed form go through the tables of
+// matern_table_eval.
+#include <algorithm>
+
 #include "egs_common.hpp"
 #include "egs_kernels.hpp"
 #include "egs_matern.hpp"
 
 namespace egs {
+
+// ------------------------------------------------------------------------
+// Matern tables (see matern_table_eval): one wave per row, each lane
+// evaluating K_nu at one Chebyshev node; grid (row groups, slots).  The sums
+// over the nodes are compensated and a_0 is kept to twice the precision: a
+// row's own error is common to all entries it serves, so that the jumps
+// between rows, unlike rounding noise, add up in z'Sigma^-1 z (at 40,000
+// locations and nu = 1, 16 nodes and one double for a_0 put 1.3e-11 into the
+// log-likelihood).  Bound: the latency of one K_nu, 20 us whatever the size.
+// ------------------------------------------------------------------------
+constexpr int kNodes = 64;
+constexpr int kDegree = kTabDegree;
+constexpr int kRowsPerGroup = kThreads / kNodes;
+
+// Powers of t in T_k(t): kCheb[k][m].
+__constant__ const double kCheb[kDegree + 1][kDegree + 1] = {
+    {1}, {0, 1}, {-1, 0, 2}, {0, -3, 0, 4}, {1, 0, -8, 0, 8}, {0, 5, 0, -20, 0, 16}, {-1, 0, 18, 0, -48, 0, 32},
+    {0, -7, 0, 56, 0, -112, 0, 64}, {1, 0, -32, 0, 160, 0, -256, 0, 128}, {0, 9, 0, -120, 0, 432, 0, -576, 0, 256},
+    {-1, 0, 50, 0, -400, 0, 1120, 0, -1280, 0, 512}};
+
+// d where row r begins: 8 log2(d) + 2 d + 80 = r.  Newton in log(d) (convex,
+// increasing; FP32 is enough, the rows' fits overlap).
+__device__ __forceinline__ float table_edge(float r) {
+    float x = fminf((r - 80.0f) * 0.0866434f, 5.0f);   // log(d) without the 2 d term: from above
+    for (int it = 0; it < 12; ++it) {
+        const float d = expf(x);
+        x -= (11.5415603f * x + 2.0f * d + 80.0f - r) / (11.5415603f + 2.0f * d);
+    }
+    return expf(x);
+}
+
+// sum += a * b with the rounding errors in err (two-product, two-sum)
+__device__ __forceinline__ void add_product(double &sum, double &err, double a, double b) {
+#pragma clang fp contract(off)
+    const double p = a * b;
+    const double pe = fma(a, b, -p);
+    const double t = sum + p;
+    const double z = t - sum;
+    err += ((sum - (t - z)) + (p - z)) + pe;
+    sum = t;
+}
+
+__global__ void __launch_bounds__(kThreads) matern_table_kernel(double *tabs, MaternParams prm_host,
+                                                                const MaternParams *prm_dev) {
+    __shared__ double s_cos[4 * kNodes];   // cos(pi m / (2 kNodes))
+    __shared__ double s_f[kRowsPerGroup][kNodes];
+    __shared__ double s_c[kRowsPerGroup][kDegree + 1], s_e[kRowsPerGroup][kDegree + 1];
+    const MaternParams prm = prm_dev ? *prm_dev : prm_host;
+    const int slot = blockIdx.y;
+    if (slot >= prm.ntab) return;
+    const int pair = prm.tab_pair[slot];
+    const int g = threadIdx.x / kNodes, j = threadIdx.x % kNodes;
+    const int row = blockIdx.x * kRowsPerGroup + g;
+    s_cos[threadIdx.x] = cospi((double) threadIdx.x / (2.0 * kNodes));
+    const double d0 = table_edge((float) row), d1 = table_edge((float) row + 1.0f);
+    const double pad = 2e-3 * (d1 * d1 - d0 * d0);
+    const double lo = d0 * d0 - pad, hi = d1 * d1 + pad;
+    const double mid = (float) (0.5 * (lo + hi)), half = 0.5 * (hi - lo);
+    __syncthreads();
+    const double d = sqrt(fma(half, s_cos[2 * j + 1], mid));
+    s_f[g][j] = prm.con[pair] * pow(d, prm.nu[pair]) * bessel_knu(prm.nu[pair], d);
+    __syncthreads();
+    if (j <= kDegree) {
+        double c = 0.0, e = 0.0;
+        for (int q = 0; q < kNodes; ++q) add_product(c, e, s_f[g][q], s_cos[(j * (2 * q + 1)) % (4 * kNodes)]);
+        s_c[g][j] = c * (j == 0 ? 1.0 / kNodes : 2.0 / kNodes);   // powers of two: exact
+        s_e[g][j] = e * (j == 0 ? 1.0 / kNodes : 2.0 / kNodes);
+    }
+    __syncthreads();
+    if (row >= kTabRows) return;
+    double *tab = tabs + (int64_t) slot * kTabDoubles;
+    double *out = tab + row * kTabWidth;
+    if (j <= kDegree) {
+        double a = 0.0, e = 0.0;
+        for (int k = kDegree; k >= j; --k) {
+            add_product(a, e, s_c[g][k], kCheb[k][j]);
+            e += s_e[g][k] * kCheb[k][j];
+        }
+        if (j == 0) {
+            out[0] = a + e;
+            out[1] = (a - (a + e)) + e;
+        } else {
+            a += e;
+            for (int m = 0; m < j; ++m) a /= half;
+            out[1 + j] = a;
+        }
+    } else if (j == kDegree + 1) {
+        reinterpret_cast<float *>(tab + kTabRows * kTabWidth)[row] = (float) mid;
+    }
+}
+
+void launch_matern_tables(double *tabs, const MaternParams &prm, const MaternParams *prm_dev, hipStream_t s) {
+    const int slots = prm_dev ? (prm.kernel == 1 ? kTabSlots : 1) : prm.ntab;
+    if (slots == 0) return;
+    hipLaunchKernelGGL(matern_table_kernel, dim3((kTabRows + kRowsPerGroup - 1) / kRowsPerGroup, slots),
+                       dim3(kThreads), 0, s, tabs, prm, prm_dev);
+}
 
 struct CovTilesArgs {
     TileMap map;
@@ -21,70 +117,137 @@ struct CovTilesArgs {
     Locs loc;
     int64_t n;              // true matrix dimension; rows/cols >= n are identity padding
     int three_d;
+    int cols;               // columns per workgroup, a multiple of 64
+    const double *tabs;     // Matern tables of prm
     double *sig64;          // optional FP64 copy of every lower tile (tile i*(i+1)/2 + j, ts*ts each)
     const MaternParams *prm_dev;   // optional: read the parameters here instead of prm
 };
 
-// One workgroup per 64-row strip of a tile (all ts columns): the strip's row
-// locations and the tile's column locations (3 ts doubles of dynamic LDS) are
-// staged once, then each wave writes 64 consecutive rows (512 bytes in FP64)
-// of one column at a time.
-
-__global__ void __launch_bounds__(kThreads) covgen_tiles_kernel(CovTilesArgs a) {
-    __shared__ double s_rx[kBlk], s_ry[kBlk], s_rz[kBlk];
-    extern __shared__ double s_cols[];
+// One workgroup per 64-row strip and `cols` columns of a tile: the strip's row
+// locations and the tables sit in LDS, the columns' locations pass through it
+// 256 at a time; each wave writes 64 consecutive rows (512 bytes in FP64) of
+// one column at a time.
+//
+// Bound: FP64 VALU and, for orders without a closed form, the table's LDS
+// reads (96 bytes per entry, 64 neighbouring rows share few table rows).
+// Measured with K_nu per entry -> with the table: 10,007 locations, nu 0.83,
+// ts 384: 6.14 -> 0.13 ms (plus 0.02 ms for the table); 45,001, nu 0.55, ts
+// 960 with the FP64 copy: 69 -> 2.6 ms.  24 regions of 500-3,000 in turn:
+// 1.08 ms -> 16 us each (one strip of 64 x ts per workgroup left most of the
+// GPU idle there; see the split in launch_covgen_tiles).
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kThreads, 4) covgen_tiles_kernel(CovTilesArgs a) {
+    constexpr int kStageCols = 256;
+    __shared__ double s_cx[kStageCols], s_cy[kStageCols], s_cz[kStageCols];
+    __shared__ __align__(16) double s_tab[kTabs > 0 ? kTabs * kTabDoubles : 1];
     // parameters from device memory when given (a captured graph replays with new theta)
     const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
     const int ts = a.map.ts;
-    double *s_cx = s_cols, *s_cy = s_cols + ts, *s_cz = s_cols + 2 * ts;
     const int2 ij = a.pairs[blockIdx.y];
     const int sbr = blockIdx.x;
     const int64_t r0 = (int64_t) ij.x * ts + sbr * kBlk;
-    const int64_t c0 = (int64_t) ij.y * ts;
+    const int c_beg = blockIdx.z * a.cols, c_end = min(ts, c_beg + a.cols);
     const int t = threadIdx.x;
     const bool three_d = a.three_d != 0;
-    const int shift = prm.kernel == 1 ? 1 : 0;
-
-    // Stage the locations of this strip's rows and of the tile's columns.
-    if (t < kBlk) {
-        const int64_t li = (r0 + t) >> shift;
-        const bool ok = (r0 + t) < a.n;
-        s_rx[t] = ok ? a.loc.x[li] : 0.0;
-        s_ry[t] = ok ? a.loc.y[li] : 0.0;
-        s_rz[t] = (ok && three_d) ? a.loc.z[li] : 0.0;
-    }
-    for (int u = t; u < ts; u += kThreads) {
-        const int64_t lj = (c0 + u) >> shift;
-        const bool ok = (c0 + u) < a.n;
-        s_cx[u] = ok ? a.loc.x[lj] : 0.0;
-        s_cy[u] = ok ? a.loc.y[lj] : 0.0;
-        s_cz[u] = (ok && three_d) ? a.loc.z[lj] : 0.0;
-    }
-    __syncthreads();
+    if (kTabs > 0 && prm.ntab > 0)
+        for (int e = t; e < kTabs * kTabDoubles; e += kThreads) s_tab[e] = a.tabs[e];
 
     const int r = t % kBlk;
     const int64_t gr = r0 + r;
     const bool row_pad = gr >= a.n;
-    const double rx = s_rx[r], ry = s_ry[r], rz = s_rz[r];
-    const int rvar = (int) (gr & 1);
+    StagedLoc row{0.0, 0.0, 0.0};
+    if (!row_pad) row = stage_location<kSphere>(a.loc.x[gr], a.loc.y[gr], three_d ? a.loc.z[gr] : 0.0);
     const uint8_t store = a.map.store[ij.x * a.map.nt + ij.y];
     char *tile = a.map.base + a.map.off[ij.x * a.map.nt + ij.y];
     const int64_t sig_base = ((int64_t) ij.x * (ij.x + 1) / 2 + ij.y) * ts * ts;
-    for (int cc = t / kBlk; cc < ts; cc += kThreads / kBlk) {
-        const int64_t gc = c0 + cc;
-        double v;
-        if (row_pad || gc >= a.n) {
-            v = (gr == gc) ? 1.0 : 0.0;
-        } else {
-            const int pair = shift ? (rvar * 2 + (int) (gc & 1)) : 0;
-            const double dist = distance(rx, ry, rz, s_cx[cc], s_cy[cc], s_cz[cc], prm.metric, three_d);
-            const double d = dist / prm.range;
-            v = (d == 0.0) ? prm.sig[pair] : matern_scaled(d, prm.con[pair], prm.sig[pair], prm.nu[pair]);
+    for (int cb = c_beg; cb < c_end; cb += kStageCols) {
+        const int64_t gc0 = (int64_t) ij.y * ts + cb;
+        const int ncol = min(kStageCols, c_end - cb);
+        __syncthreads();   // the tables are staged; the columns before are done
+        if (t < ncol && gc0 + t < a.n) {
+            const StagedLoc col = stage_location<kSphere>(a.loc.x[gc0 + t], a.loc.y[gc0 + t],
+                                                 three_d ? a.loc.z[gc0 + t] : 0.0);
+            s_cx[t] = col.x;
+            s_cy[t] = col.y;
+            s_cz[t] = col.z;
         }
-        const int64_t idx = (int64_t) (sbr * kBlk + r) + (int64_t) cc * ts;
-        if (store == kStoreF64) reinterpret_cast<double *>(tile)[idx] = v;
-        else reinterpret_cast<float *>(tile)[idx] = (float) v;
-        if (a.sig64) a.sig64[sig_base + idx] = v;
+        __syncthreads();
+#pragma unroll 1
+        for (int cc = t / kBlk; cc < ncol; cc += kThreads / kBlk) {
+            const int64_t gc = gc0 + cc;
+            double v;
+            if (row_pad || gc >= a.n) {
+                v = (gr == gc) ? 1.0 : 0.0;
+            } else {
+                const StagedLoc col{s_cx[cc], s_cy[cc], s_cz[cc]};
+                v = staged_covariance<(kTabs > 0), kSphere>(prm, 0, staged_separation<kSphere>(row, col, three_d), s_tab);
+            }
+            const int64_t idx = (int64_t) (sbr * kBlk + r) + (int64_t) (cb + cc) * ts;
+            if (store == kStoreF64) reinterpret_cast<double *>(tile)[idx] = v;
+            else reinterpret_cast<float *>(tile)[idx] = (float) v;
+            if (a.sig64) a.sig64[sig_base + idx] = v;
+        }
+    }
+}
+
+// The bivariate kernel: a thread takes a pair of locations, whose distance
+// serves the 2 x 2 covariances of their variables (the two cross terms are
+// equal); 32 row locations, 16 column locations at a time.  9,001 locations on
+// the sphere, orders 0.5 and 1: 14.3 ms with a distance and K_nu per entry,
+// 0.67 ms so.
+constexpr int kBivThreads = 512;
+
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kBivThreads, kTabs < 3 ? 4 : 2) covgen_tiles_biv_kernel(CovTilesArgs a) {
+    constexpr int kRowLocs = kBlk / 2, kColStep = kBivThreads / kRowLocs;
+    __shared__ __align__(16) double s_tab[kTabs > 0 ? kTabs * kTabDoubles : 1];
+    const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
+    const int ts = a.map.ts;
+    const int2 ij = a.pairs[blockIdx.y];
+    const int sbr = blockIdx.x;
+    const int64_t r0 = (int64_t) ij.x * ts + sbr * kBlk, c0 = (int64_t) ij.y * ts;
+    const int c_beg = blockIdx.z * a.cols, c_end = min(ts, c_beg + a.cols);
+    const int t = threadIdx.x;
+    if (kTabs > 0 && prm.ntab > 0) {
+        for (int e = t; e < kTabs * kTabDoubles; e += kBivThreads) s_tab[e] = a.tabs[e];
+        __syncthreads();
+    }
+    const int r = t % kRowLocs;
+    const int64_t gr = r0 + 2 * r;       // n is even: a location's two rows are both real or both padding
+    const bool row_pad = gr >= a.n;
+    StagedLoc row{0.0, 0.0, 0.0};
+    if (!row_pad) row = stage_location<kSphere>(a.loc.x[gr >> 1], a.loc.y[gr >> 1], 0.0);
+    const uint8_t store = a.map.store[ij.x * a.map.nt + ij.y];
+    char *tile = a.map.base + a.map.off[ij.x * a.map.nt + ij.y];
+    const int64_t sig_base = ((int64_t) ij.x * (ij.x + 1) / 2 + ij.y) * ts * ts;
+#pragma unroll 1
+    for (int cc = c_beg + 2 * (t / kRowLocs); cc < c_end; cc += 2 * kColStep) {
+        const int64_t gc = c0 + cc;
+        double v00, v01, v11;
+        if (row_pad || gc >= a.n) {
+            v00 = v11 = (gr == gc) ? 1.0 : 0.0;
+            v01 = 0.0;
+        } else {
+            const StagedLoc col = stage_location<kSphere>(a.loc.x[gc >> 1], a.loc.y[gc >> 1], 0.0);
+            const double q = staged_separation<kSphere>(row, col, false);
+            v00 = staged_covariance<(kTabs > 0), kSphere>(prm, 0, q, s_tab);
+            v01 = staged_covariance<(kTabs > 0), kSphere>(prm, 1, q, s_tab);
+            v11 = staged_covariance<(kTabs > 0), kSphere>(prm, 3, q, s_tab);
+        }
+        const int64_t idx = (int64_t) (sbr * kBlk + 2 * r) + (int64_t) cc * ts;   // even: ts and cc are
+        const f64x2 left{v00, v01}, right{v01, v11};
+        if (store == kStoreF64) {
+            *reinterpret_cast<f64x2 *>(reinterpret_cast<double *>(tile) + idx) = left;
+            *reinterpret_cast<f64x2 *>(reinterpret_cast<double *>(tile) + idx + ts) = right;
+        } else {
+            typedef float f32x2 __attribute__((ext_vector_type(2)));
+            *reinterpret_cast<f32x2 *>(reinterpret_cast<float *>(tile) + idx) = f32x2{(float) v00, (float) v01};
+            *reinterpret_cast<f32x2 *>(reinterpret_cast<float *>(tile) + idx + ts) = f32x2{(float) v01, (float) v11};
+        }
+        if (a.sig64) {
+            *reinterpret_cast<f64x2 *>(a.sig64 + sig_base + idx) = left;
+            *reinterpret_cast<f64x2 *>(a.sig64 + sig_base + idx + ts) = right;
+        }
     }
 }
 
@@ -110,8 +273,8 @@ __global__ void __launch_bounds__(kThreads) covgen_rect_kernel(CovRectArgs a) {
 }
 
 void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, const MaternParams &prm,
-                         const double *x, const double *y, const double *z, int64_t n, double *sig64, hipStream_t s,
-                         const MaternParams *prm_dev) {
+                         const double *x, const double *y, const double *z, int64_t n, const double *tabs,
+                         double *sig64, hipStream_t s, const MaternParams *prm_dev) {
     if (npairs <= 0) return;
     CovTilesArgs a;
     a.map = map;
@@ -120,11 +283,32 @@ void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, cons
     a.loc = Locs{x, y, z};
     a.n = n;
     a.three_d = z != nullptr;
+    a.tabs = tabs;
     a.sig64 = sig64;
     a.prm_dev = prm_dev;
+    // a strip's columns are split over workgroups until these fill the GPU
+    // (kFill: eight per CU); whole strips stage the tables once each
+    constexpr int kFill = 2048;
     const int nsb = map.ts / kBlk;
-    dim3 grid(nsb, npairs);
-    hipLaunchKernelGGL(covgen_tiles_kernel, grid, dim3(kThreads), 3 * sizeof(double) * (size_t) map.ts, s, a);
+    const int want = (int) std::min<int64_t>(nsb, (kFill + (int64_t) nsb * npairs - 1) / ((int64_t) nsb * npairs));
+    const int per = (nsb + want - 1) / want;
+    a.cols = per * kBlk;
+    const dim3 grid(nsb, npairs, (nsb + per - 1) / per);
+    // a captured launch serves every theta: as many tables as the kernel may need
+    const int tables = prm_dev ? (prm.kernel == 1 ? kTabSlots : 1) : prm.ntab;
+    using Kernel = void (*)(CovTilesArgs);
+    static const Kernel univariate[2][2] = {{covgen_tiles_kernel<0, false>, covgen_tiles_kernel<1, false>},
+                                            {covgen_tiles_kernel<0, true>, covgen_tiles_kernel<1, true>}};
+    static const Kernel bivariate[2][kTabSlots + 1] = {
+        {covgen_tiles_biv_kernel<0, false>, covgen_tiles_biv_kernel<1, false>, covgen_tiles_biv_kernel<2, false>,
+         covgen_tiles_biv_kernel<3, false>},
+        {covgen_tiles_biv_kernel<0, true>, covgen_tiles_biv_kernel<1, true>, covgen_tiles_biv_kernel<2, true>,
+         covgen_tiles_biv_kernel<3, true>}};
+    const bool sphere = prm.metric == 1;
+    if (prm.kernel == 1)
+        hipLaunchKernelGGL(bivariate[sphere][tables], grid, dim3(kBivThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL(univariate[sphere][tables], grid, dim3(kThreads), 0, s, a);
 }
 
 void launch_covgen_rect(double *out, int rows, int cols, int64_t row_off, int64_t col_off, const MaternParams &prm,

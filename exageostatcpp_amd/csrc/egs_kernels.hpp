@@ -28,13 +28,17 @@ struct BatchJob {
 };
 
 // ---- covariance generation (egs_covgen.hip)
+// Tables of the orders prm marks (MaternParams::tab) into tabs, kTabSlots of
+// kTabDoubles; prm_dev as in launch_covgen_tiles.
+void launch_matern_tables(double *tabs, const MaternParams &prm, const MaternParams *prm_dev, hipStream_t s);
+// tabs: the tables of prm (launch_matern_tables, earlier on the same stream).
 // sig64 (may be null): also writes every generated tile in FP64 to
 // sig64 + (i*(i+1)/2 + j) * ts * ts, column-major.
 // prm_dev, when given, holds the parameters in device memory (read instead of
 // prm, so that a captured launch can be replayed for another theta).
 void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, const MaternParams &prm,
-                         const double *x, const double *y, const double *z, int64_t n, double *sig64, hipStream_t s,
-                         const MaternParams *prm_dev = nullptr);
+                         const double *x, const double *y, const double *z, int64_t n, const double *tabs, double *sig64,
+                         hipStream_t s, const MaternParams *prm_dev = nullptr);
 void launch_covgen_rect(double *out, int rows, int cols, int64_t row_off, int64_t col_off, const MaternParams &prm,
                         const double *x1, const double *y1, const double *z1, const double *x2, const double *y2,
                         const double *z2, hipStream_t s);
@@ -74,7 +78,7 @@ void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s
 // out[r] = sum_c Sigma(l1_r, l2_c) x[c] for r < rows, c < cols (kriging mean).
 void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams &prm, const double *x1,
                      const double *y1, const double *z1, const double *x2, const double *y2, const double *z2,
-                     const double *xv, hipStream_t s);
+                     const double *xv, const double *tabs, hipStream_t s);
 // partial[cb * npad + r] = sum over column chunk cb of Sigma(r, c) v[c] (FP64,
 // regenerated from the locations); matvec_chunks(n) chunks.
 void launch_cov_matvec(double *partial, const double *v, int64_t n, int64_t npad, const MaternParams &prm,

@@ -152,6 +152,55 @@ __device__ inline double matern_scaled(double d, double con, double sigma2, doub
     return con * pow(d, nu) * bessel_knu(nu, d);
 }
 
+// ------------------------------------------------------------------------
+// K_nu of general order through a table.  For one theta the Matern function
+// con d^nu K_nu(d) depends on d alone, so its K_nu (a series or a continued
+// fraction of some hundred to thousand instructions, divergent within a wave)
+// is evaluated only at the nodes of a piecewise polynomial in s = d^2, built
+// on the device once per evaluation (matern_table_kernel):
+//   * row = floor(4 log2(s) + 2 sqrt(s) + 80): intervals of constant ratio
+//     where the d^(2 nu) singularity at 0 rules, of constant width in d (1/2)
+//     where exp(-d) does; the row of an s is found in FP32, each row's fit is
+//     wide enough (0.2% beyond its ends) for that rounding;
+//   * degree 10, from 64 Chebyshev nodes: the truncation error is below 4e-17
+//     relative for 0.05 <= nu <= 20, and the fit averages the nodes' rounding;
+//   * row layout: a_0 in two parts and a_1 .. a_10, coefficients in powers of
+//     s - center (96 bytes: six 16-byte LDS reads); after the rows, the
+//     centers in FP32 (exact).
+// Outside [kTabMin, kTabMax) (d < 2^-10 or d >= 90.5) and for orders or
+// parameters the host does not mark (MaternParams::tab) the direct evaluation
+// is used.
+constexpr int kTabRows = 316;
+constexpr int kTabDegree = 10;
+constexpr int kTabWidth = kTabDegree + 2;
+constexpr int kTabDoubles = kTabRows * kTabWidth + kTabRows / 2;   // the rows and their centers
+constexpr int kTabSlots = 3;               // distinct orders of a kernel (bivariate: 3)
+constexpr double kTabMin = 0x1p-20, kTabMax = 8192.0;
+constexpr double kTabMaxNu = 20.0;         // larger orders overflow K_nu inside the table's range
+
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+// The table's value at s in [kTabMin, kTabMax); tab 16-byte aligned.
+__device__ __forceinline__ double matern_table_eval(const double *tab, double s) {
+    const float sf = (float) s;
+    int row = (int) fmaf(4.0f, __builtin_amdgcn_logf(sf), fmaf(2.0f, __builtin_amdgcn_sqrtf(sf), 80.0f));
+    row = min(max(row, 0), kTabRows - 1);
+    const double u = s - (double) reinterpret_cast<const float *>(tab + kTabRows * kTabWidth)[row];
+    const f64x2 *c = reinterpret_cast<const f64x2 *>(tab + row * kTabWidth);
+    const f64x2 c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3], c4 = c[4], c5 = c[5];
+    double v = c5[1];
+    v = fma(v, u, c5[0]);
+    v = fma(v, u, c4[1]);
+    v = fma(v, u, c4[0]);
+    v = fma(v, u, c3[1]);
+    v = fma(v, u, c3[0]);
+    v = fma(v, u, c2[1]);
+    v = fma(v, u, c2[0]);
+    v = fma(v, u, c1[1]);
+    v = fma(v, u, c1[0]);
+    return c0[0] + fma(v, u, c0[1]);
+}
+
 // Great-circle distance in km with x = latitude, y = longitude in degrees
 // (DistanceCalculationHelpers.cpp:27-36; earth radius 6371 km).
 __device__ inline double distance_earth(double lat1, double lon1, double lat2, double lon2) {
@@ -160,6 +209,22 @@ __device__ inline double distance_earth(double lat1, double lon1, double lat2, d
     const double u = sin((l2 - l1) * 0.5);
     const double v = sin((lon2 * deg - lon1 * deg) * 0.5);
     return 2.0 * 6371.0 * asin(sqrt(u * u + cos(l1) * cos(l2) * v * v));
+}
+
+// A location as the tile kernels stage it: x, y, z, or for great-circle
+// distances latitude and longitude in radians and cos(latitude), so that a
+// pair costs no conversion and no cosine.
+struct StagedLoc {
+    double x, y, z;
+};
+template <bool kSphere>
+__device__ __forceinline__ StagedLoc stage_location(double x, double y, double z) {
+// no contraction: a fused (y deg) - y' would make equal locations differ
+#pragma clang fp contract(off)
+    if constexpr (!kSphere) return StagedLoc{x, y, z};
+    const double deg = 3.141592653589793 / 180.0;
+    const double l = x * deg;
+    return StagedLoc{l, y * deg, cos(l)};
 }
 
 // Locations as structure of arrays; z == nullptr for 2D.
@@ -189,10 +254,42 @@ struct MaternParams {
     int kernel;
     int metric;
     double range;
+    double inv_range2;   // 1 / range^2
+    int tab[4];          // table slot of each pair's order, -1: evaluated directly
+    int ntab;            // slots in use
+    int tab_pair[kTabSlots];   // the pair whose function a slot holds
     double sig[4];   // [a*2+b]
     double nu[4];
     double con[4];
 };
+
+// Separation of two staged locations: the squared Euclidean distance (the
+// table's argument needs no square root), or the great-circle distance.
+template <bool kSphere>
+__device__ __forceinline__ double staged_separation(const StagedLoc &a, const StagedLoc &b, bool three_d) {
+    if constexpr (kSphere) {
+        const double u = sin((b.x - a.x) * 0.5);
+        const double v = sin((b.y - a.y) * 0.5);
+        return 2.0 * 6371.0 * asin(sqrt(u * u + a.z * b.z * v * v));
+    } else {
+        const double dx = b.x - a.x, dy = b.y - a.y;
+        if (!three_d) return dx * dx + dy * dy;
+        const double dz = b.z - a.z;
+        return dx * dx + dy * dy + dz * dz;
+    }
+}
+
+// Covariance of a pair of variables at separation q (staged_separation).
+template <bool kTable, bool kSphere>
+__device__ __forceinline__ double staged_covariance(const MaternParams &p, int pair, double q, const double *tabs) {
+    if constexpr (kTable) {
+        const double s = (kSphere ? q * q : q) * p.inv_range2;
+        const int slot = p.tab[pair];
+        if (slot >= 0 && s >= kTabMin && s < kTabMax) return matern_table_eval(tabs + slot * kTabDoubles, s);
+    }
+    const double d = (kSphere ? q : sqrt(q)) / p.range;
+    return d == 0.0 ? p.sig[pair] : matern_scaled(d, p.con[pair], p.sig[pair], p.nu[pair]);
+}
 
 // Covariance between matrix rows r and c (indices into the n-dimensional
 // matrix; for the bivariate kernel, row r is variable r%2 at location r/2).

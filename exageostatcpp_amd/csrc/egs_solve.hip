@@ -242,22 +242,37 @@ __global__ void __launch_bounds__(kThreads) trmv_kernel(TileMap map, const doubl
     if (t < kBlk) out[gblk * kBlk + t] = ((sp[0][t] + sp[1][t]) + sp[2][t]) + sp[3][t];
 }
 
-// Kriging mean: out[r] = sum_c Sigma(l1_r, l2_c) x[c].
+// Kriging mean: out[r] = sum_c Sigma(l1_r, l2_c) x[c], one workgroup per row;
+// the tables of the row's orders (see matern_table_eval) are staged in LDS.
 struct CovGemvArgs {
     double *out;
     int64_t rows, cols;
     MaternParams prm;
     Locs l1, l2;
     const double *x;
+    const double *tabs;
     int three_d;
 };
 
-__global__ void __launch_bounds__(kThreads) cov_gemv_kernel(CovGemvArgs a) {
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kThreads, kTabs < 2 ? 4 : 4 - kTabs) cov_gemv_kernel(CovGemvArgs a) {
     __shared__ double red[kThreads];
+    __shared__ __align__(16) double s_tab[kTabs > 0 ? kTabs * kTabDoubles : 1];
+    for (int e = threadIdx.x; e < kTabs * kTabDoubles; e += kThreads) s_tab[e] = a.tabs[e];
+    __syncthreads();
     const int64_t r = blockIdx.x;
+    const bool three_d = a.three_d != 0;
+    const int shift = a.prm.kernel == 1 ? 1 : 0;
+    const int64_t i = r >> shift;
+    const StagedLoc row = stage_location<kSphere>(a.l1.x[i], a.l1.y[i], three_d ? a.l1.z[i] : 0.0);
     double s = 0.0;
-    for (int64_t c = threadIdx.x; c < a.cols; c += kThreads)
-        s += covariance_entry(a.prm, a.l1, a.l2, r, c, a.three_d != 0) * a.x[c];
+#pragma unroll 1
+    for (int64_t c = threadIdx.x; c < a.cols; c += kThreads) {
+        const int64_t j = c >> shift;
+        const StagedLoc col = stage_location<kSphere>(a.l2.x[j], a.l2.y[j], three_d ? a.l2.z[j] : 0.0);
+        const int pair = shift ? (int) ((r & 1) * 2 + (c & 1)) : 0;
+        s += staged_covariance<(kTabs > 0), kSphere>(a.prm, pair, staged_separation<kSphere>(row, col, three_d), s_tab) * a.x[c];
+    }
     s = wg_sum(s, red);
     if (threadIdx.x == 0) a.out[r] = s;
 }
@@ -438,7 +453,7 @@ void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s
 
 void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams &prm, const double *x1,
                      const double *y1, const double *z1, const double *x2, const double *y2, const double *z2,
-                     const double *xv, hipStream_t s) {
+                     const double *xv, const double *tabs, hipStream_t s) {
     if (rows <= 0) return;
     CovGemvArgs a;
     a.out = out;
@@ -448,8 +463,12 @@ void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams
     a.l1 = Locs{x1, y1, z1};
     a.l2 = Locs{x2, y2, z2};
     a.x = xv;
+    a.tabs = tabs;
     a.three_d = (z1 != nullptr && z2 != nullptr);
-    hipLaunchKernelGGL(cov_gemv_kernel, dim3((unsigned) rows), dim3(kThreads), 0, s, a);
+    static void (*const kernels[2][kTabSlots + 1])(CovGemvArgs) = {
+        {cov_gemv_kernel<0, false>, cov_gemv_kernel<1, false>, cov_gemv_kernel<2, false>, cov_gemv_kernel<3, false>},
+        {cov_gemv_kernel<0, true>, cov_gemv_kernel<1, true>, cov_gemv_kernel<2, true>, cov_gemv_kernel<3, true>}};
+    hipLaunchKernelGGL(kernels[prm.metric == 1][prm.ntab], dim3((unsigned) rows), dim3(kThreads), 0, s, a);
 }
 
 void launch_dlarnv_normal(double *e, int64_t n, uint64_t seed48, hipStream_t s) {
