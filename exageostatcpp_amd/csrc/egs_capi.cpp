@@ -193,7 +193,7 @@ struct egs_problem_s {
     uint8_t *d_store = nullptr;
     int2 *d_pairs = nullptr;
     double *d_winv = nullptr;
-    double *d_dscr = nullptr;   // ts * ts scratch of the diagonal-tile factorization
+    int *d_sync = nullptr;      // tickets and flags of the tile columns' factorization (launch_tile_column)
     double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr, *d_partials = nullptr;
     int *d_info = nullptr;
     double *d_tab = nullptr;    // Matern tables of the last covariance parameters (kTabSlots of them)
@@ -230,6 +230,8 @@ struct egs_problem_s {
         return m;
     }
     int ntheta() const { return kernel == 1 ? 6 : 3; }
+    int64_t sync_ints() const { return (int64_t) nt * egs::tile_column_sync_ints(ts); }
+    int *sync(int k) const { return d_sync + (int64_t) k * egs::tile_column_sync_ints(ts); }
     double *winv(int k) const { return d_winv + (int64_t) k * nsb * egs::kBlk * egs::kBlk; }
 };
 
@@ -368,7 +370,7 @@ void free_problem_buffers(egs_problem_s *p) {
     pfree(p, p->d_store);
     pfree(p, p->d_pairs);
     pfree(p, p->d_winv);
-    pfree(p, p->d_dscr);
+    pfree(p, p->d_sync);
     pfree(p, p->d_obs);
     pfree(p, p->d_work);
     pfree(p, p->d_aux);
@@ -424,7 +426,8 @@ void free_problem_buffers(egs_problem_s *p) {
     p->d_off = nullptr;
     p->d_store = nullptr;
     p->d_pairs = nullptr;
-    p->d_winv = p->d_dscr = p->d_obs = p->d_work = p->d_aux = p->d_partials = nullptr;
+    p->d_sync = nullptr;
+    p->d_winv = p->d_obs = p->d_work = p->d_aux = p->d_partials = nullptr;
     p->d_info = nullptr;
     p->d_tab = nullptr;
     for (auto &e : p->ev) e = nullptr;
@@ -623,7 +626,7 @@ double update_flops(const egs_problem_s *p, int j0, int j1) {
     return f;
 }
 
-// Diagonal tile k: 64 x 64 blocks left-looking, then the panel below it.
+// Diagonal tile k and the panel below it.
 void factor_panel(egs_problem_s *p, int k) {
     hipStream_t s = p->ctx->stream;
     const egs::TileMap m = p->map();
@@ -631,28 +634,27 @@ void factor_panel(egs_problem_s *p, int k) {
     const double ts = (double) p->ts;
     double *wk = p->winv(k);
     const double kb = real_rows(p, k);
+    // rows within band64 of the diagonal are FP64 tiles, the rest FP32
+    const int rows64 = is_mixed(p) ? std::min(nt - 1 - k, p->band64) : nt - 1 - k;
+    const int rows32 = nt - 1 - k - rows64;
+    // the FP64 rows go with the diagonal tile when they are few; the FP32 rows
+    // of a bivariate plan are solved together with the FP64 ones (both on FP64
+    // MFMA)
+    const bool fused = rows64 > 0 && egs::tile_column_solves_rows(p->ts, rows64) &&
+                       (rows32 == 0 || p->f32_panel_solve);
     int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0);
-    egs::launch_factor_diag(m, k, wk, p->d_dscr, p->d_info, p->n, s);
+    egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info, p->n, fused ? rows64 : 0, s);
     prof_end(p, pi);
     if (k + 1 < nt) {
         double rows_below = 0.0;
-        for (int i = k + 1; i < nt; ++i) rows_below += real_rows(p, i);
+        for (int i = k + 1 + (fused ? rows64 : 0); i < nt; ++i) rows_below += real_rows(p, i);
         pi = prof_begin(p, EGS_PROFILE_PANEL_TRSM, rows_below * ts * ts);
-        if (!is_mixed(p)) {
-            egs::launch_trsm_rows(m, k, (int64_t) (k + 1) * nsb, (nt - k - 1) * nsb, 0, nsb, wk, s);
+        const int64_t g64 = (int64_t) (k + 1) * nsb, g32 = g64 + (int64_t) rows64 * nsb;
+        if (rows32 > 0 && !p->f32_panel_solve) {
+            egs::launch_trsm_rows_mixed(m, k, g64, rows64 * nsb, rows32 * nsb, wk, s);
         } else {
-            // rows within band64 of the diagonal are FP64 tiles, the rest FP32;
-            // both in one launch when both are solved on FP64 MFMA
-            const int last64 = std::min(nt - 1, k + p->band64);
-            const int rows32 = std::max(0, nt - 1 - last64);
-            if (!p->f32_panel_solve) {
-                egs::launch_trsm_rows_mixed(m, k, (int64_t) (k + 1) * nsb, (last64 - k) * nsb, rows32 * nsb, wk, s);
-            } else {
-                if (last64 >= k + 1)
-                    egs::launch_trsm_rows(m, k, (int64_t) (k + 1) * nsb, (last64 - k) * nsb, 0, nsb, wk, s, false);
-                egs::launch_trsm_rows(m, k, (int64_t) (last64 + 1) * nsb, rows32 * nsb, 0, nsb, wk, s, true,
-                                      p->f32_panel_solve);
-            }
+            if (!fused) egs::launch_trsm_rows(m, k, g64, rows64 * nsb, 0, nsb, wk, s);
+            egs::launch_trsm_rows(m, k, g32, rows32 * nsb, 0, nsb, wk, s, true, p->f32_panel_solve);
         }
         prof_end(p, pi);
         if (is_mixed(p)) {
@@ -745,6 +747,7 @@ int run_potrf(egs_problem_s *p) {
     }
     // a fill kernel, not a memset: this sequence is captured into a graph
     egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_info), 1, s);
+    egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_sync), (int) p->sync_ints(), s);
     if (p->mode == EGS_PRECISION_MIXED) {
         egs::launch_zero_u32(p->d_pmax, nt, s);
         egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_counts), 6, s);
@@ -1080,7 +1083,7 @@ int64_t footprint(const egs_problem_s &q) {
     const int64_t nb = (int64_t) sizeof(double) * q.n_loc, vb = (int64_t) sizeof(double) * npad;
     int64_t b = dev_class_bytes(nb) * (q.dim == 3 ? 3 : 2) + dev_class_bytes(8 * nt * nt) + dev_class_bytes(nt * nt) +
                 dev_class_bytes(8 * ntiles) + dev_class_bytes(8 * nt * q.nsb * egs::kBlk * egs::kBlk) +
-                dev_class_bytes(8 * ts * ts) + 3 * dev_class_bytes(vb) + dev_class_bytes(16 * nt) + dev_class_bytes(4) +
+                dev_class_bytes(4 * q.sync_ints()) + 3 * dev_class_bytes(vb) + dev_class_bytes(16 * nt) + dev_class_bytes(4) +
                 dev_class_bytes(8 * egs::kTabSlots * egs::kTabDoubles);
     int64_t arena = 0;
     for (int j = 0; j < q.nt; ++j)
@@ -1246,7 +1249,7 @@ int egs_problem_create(egs_context_t ctx, int kernel, int64_t n_loc, const doubl
               pmalloc(p, &p->d_store, (size_t) nt * nt) == hipSuccess &&
               pmalloc(p, &p->d_pairs, sizeof(int2) * p->h_pairs.size()) == hipSuccess &&
               pmalloc(p, &p->d_winv, sizeof(double) * (size_t) nt * p->nsb * egs::kBlk * egs::kBlk) == hipSuccess &&
-              pmalloc(p, &p->d_dscr, sizeof(double) * (size_t) p->ts * p->ts) == hipSuccess &&
+              pmalloc(p, &p->d_sync, sizeof(int) * (size_t) p->sync_ints()) == hipSuccess &&
               pmalloc(p, &p->d_obs, vb) == hipSuccess && pmalloc(p, &p->d_work, vb) == hipSuccess &&
               pmalloc(p, &p->d_aux, vb) == hipSuccess &&
               pmalloc(p, &p->d_partials, sizeof(double) * 2 * (size_t) nt) == hipSuccess &&
@@ -1682,7 +1685,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             J.k = k;
             J.pairs = p->d_pairs;
             J.winv_k = p->winv(k);
-            J.scratch = p->d_dscr;
+            J.sync = p->sync(k);
             J.info = p->d_info;
             J.n = p->n;
             J.z = p->d_work;
@@ -1712,6 +1715,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm[b], p->d_x, p->d_y, dz, p->n,
                                      p->d_tab, nullptr, s);
             egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_info), 1, s);
+            egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_sync), (int) p->sync_ints(), s);
             p->has_cov = false;
             p->factored = false;
             invalidate_graph(p);
@@ -1719,8 +1723,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
         // lockstep right-looking factorization: one launch per kernel and step for all problems
         for (int k = 0; k < max_nt; ++k) {
             const egs::BatchJob *J = ctx->d_jobs + first[k];
-            egs::launch_factor_diag_batch(J, active[k], ts, s);
-            egs::launch_panel_update_batch(J, active[k + 1], ts, max_nt - k - 1, s);
+            egs::launch_step_batch(J, active[k], ts, max_nt - k - 1, active[k + 1], s);
         }
         for (int k = 0; k < max_nt; ++k)
             egs::launch_forward_batch(ctx->d_jobs + first[k], active[k], ts, max_nt - k - 1, s);

@@ -3,12 +3,12 @@
 // tile, TRSM of the panel below it, SYRK/GEMM of the trailing tiles).
 //
 // Step k of the factorization:
-//   * the diagonal tile is factored right-looking in 64 x 64 blocks
-//     (diag_step_kernel, diag_copy_kernel below), which also leaves the
-//     64 x 64 inverses of its diagonal blocks;
-//   * the panel below the diagonal tile is solved by one workgroup per 64-row
-//     block, marching over the 64-column blocks of L_kk and applying the
-//     64 x 64 inverses (trsm_rows_kernel);
+//   * the diagonal tile is factored in 64 x 64 blocks, which also leaves the
+//     64 x 64 inverses of its diagonal blocks, and a short panel below it is
+//     solved by the same launch (tile_column_kernel);
+//   * a longer panel is solved by one workgroup per 64-row block, marching over
+//     the 64-column blocks of L_kk and applying the 64 x 64 inverses
+//     (trsm_rows_kernel);
 //   * the trailing tiles are updated with FP64 MFMA: update192 (egs_update.hip)
 //     when ts is a multiple of 192, else update_kernel here, one workgroup per
 //     64 x 64 output block with K = ts.
@@ -731,240 +731,417 @@ void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream
 }
 
 // ------------------------------------------------------------------------
-// Diagonal tile, right-looking in 64 x 64 blocks, one launch per block
-// column (diag_step_kernel).  Launch jb:
-//   workgroup 0         applies column jb - 1 to block (jb, jb), then factors
-//                       that block and inverts it (potrf64_body);
-//   workgroups 1 ..     apply column jb - 1 to the other blocks (r, c),
-//                       jb <= c <= r (diag_update_body): form
-//                       L_r = A_r,jb-1 W_jb-1^T and L_c = A_c,jb-1 W_jb-1^T and
-//                       apply A_rc -= L_r L_c^T; the diagonal blocks (r, r)
-//                       also write L_r to a scratch copy of the tile (the
-//                       tile's own block (r, jb - 1) is still being read by
-//                       other workgroups);
-//   diag_copy_kernel    at the end moves the solved blocks below the diagonal
-//                       from the scratch copy into the tile.
-// Block (jb, jb) needs only column jb - 1's update before it is factored, so
-// the rest of that update runs beside the factorization instead of before it.
+// Cholesky and inverse of one 64 x 64 block, held in LDS (row stride kPv
+// doubles).  On entry the lower part of sD is the block A (its upper part is
+// never used) and sE is anything; on return the lower part of sD holds L with
+// column c still to be multiplied by s_rs[c], and the upper part of sE holds
+// L^{-T} with column c still to be multiplied by s_rs[c].  The identity is
+// stacked under A and takes the same column operations: A L^{-T} = L turns I
+// into L^{-T}.
+//
+// Four panels of 16 columns.  Waves 0 and 1 factor a panel in registers, one
+// row per lane: wave 0 the rows of A from the panel's diagonal down and, in the
+// lanes above, the identity's rows that are no longer zero; wave 1 the
+// identity's 16 rows of the panel.  Both keep the 16 diagonal rows in every
+// 16-lane row as well, so that a column step y_c -= (y_j / piv) a_cj is one
+// v_fmac_f64_dpp per register, the a_cj broadcast inside the 16 lanes (lane
+// reads into scalar registers cost three times the issue slots).  The next
+// pivot a_j+1,j+1 - a_j+1,j^2 / piv and its reciprocal (hardware estimate and
+// one third-order step) are formed ahead of the update, so that no step waits
+// for it.  The other columns are updated with FP64 MFMA: after panel p the 16
+// columns of panel p + 1 (one 16 x 16 tile per wave), the rest by waves 2 and
+// 3 while waves 0 and 1 factor panel p + 1.
+//
+// Bound: the issue of wave 0 (64 column steps of about 160 cycles); 7.8 us per
+// block from LDS to LDS.  The form before (the block over four waves, one LDS
+// exchange and one barrier per column) took 26 us.
 // ------------------------------------------------------------------------
-namespace {
-// value of v in lane l (l uniform across the wave)
-__device__ __forceinline__ double readlane_f64(double v, int l) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
+constexpr int kPan = 16;
+constexpr int kPv = kLdsPad;
+
+// 1 / sqrt(x): the hardware estimate and two Newton steps (each doubles the
+// correct bits)
+__device__ __forceinline__ double rsqrt_f64(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    const double h = 0.5 * x;
+    r = fma(r, fma(-h * r, r, 0.5), r);
+    return fma(r, fma(-h * r, r, 0.5), r);
 }
-}  // namespace
 
-// Block (jb, jb) of diagonal tile k: L = chol(A) in place and W = L^{-1} into
-// winv_k, both lower (zeros above the diagonal).  The block lives in registers:
-// thread (w, i) = (threadIdx.x / 64, lane) holds row i of columns c = w + kW q,
-// q < 64 / kW, in y[q]: column c of A until step c, then column c of X, which
-// becomes L^{-1}.  Column step j (64 steps, one barrier each) is the
-// right-looking Cholesky step A_ic -= L_ij L_cj (c > j) fused with the
-// column-oriented inversion X_jc /= L_jj, X_ic -= L_ij X_jc (i > j, c <= j).
-// X is kept with its rows unscaled (row j of X times L_jj); the rows are
-// scaled once at the end.  Both updates are then y_ic -= r_i g_c with
-// r_i = A_ij / A_jj (i > j, else 0) and g_c the uniform operand: A_cj from LDS
-// (column j, published by its owner wave at the end of step j - 1, double
-// buffered) for c > j, the unscaled X_jc read from lane j for c <= j.  At step
-// j the owner wave of column j stores L's column j and restarts its register
-// as column j of X.
-// kW = 4 waves, one per SIMD: the block size of the update workgroups it
-// launches with (8 waves, two per SIMD, factor a block 2.5% faster alone).
-constexpr int kPotrfWaves = kThreads / 64;
+// yc += z_j[lane C of the 16-lane row] * my, zc likewise with mz
+template <int C>
+__device__ __forceinline__ void fmac2_bcast(double &yc, double &zc, double zj, double my, double mz) {
+    asm("v_fmac_f64_dpp %0, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+        : "+v"(yc), "+v"(zc)
+        : "v"(zj), "v"(my), "v"(mz), "n"(C));
+}
 
-__device__ __forceinline__ void potrf64_body(const TileMap &map, int k, int jb, double *winv_k, int *info, int64_t n) {
-    constexpr int kW = kPotrfWaves;
-    constexpr int kCols = kBlk / kW;   // columns per thread
-    __shared__ double s_col[2][kBlk];
-    __shared__ double s_rs[kBlk];     // 1 / L_jj
-    const int ts = map.ts;
-    const int t = threadIdx.x;
-    const int i = t & 63;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);   // wave index, held in a scalar register
-    double *Ajj = tile_f64(map, k, k) + (int64_t) jb * kBlk + (int64_t) jb * kBlk * ts;
-    double y[kCols];
+// a and b of lane N of the 16-lane row (after two wait states, which a DPP
+// read of a register that a vector instruction has just written needs)
+template <int N>
+__device__ __forceinline__ void bcast2(double a, double b, double &oa, double &ob) {
+    asm("s_nop 1\n\t"
+        "v_mov_b64_dpp %0, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b64_dpp %1, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
+        : "=&v"(oa), "=&v"(ob)
+        : "v"(a), "v"(b), "n"(N));
+}
+
+// Columns J + 2 .. 15 of column step J: the G-th third of them, column J + 2
+// (the next step's pivot column) first.
+template <int J, int G, int C = J + 2>
+__device__ __forceinline__ void panel_group(double (&y)[kPan], double (&z)[kPan], double my, double mz) {
+    if constexpr (C < kPan) {
+        constexpr int rest = kPan - 3 - J;
+        constexpr int g = C == J + 2 ? 0 : (C - J - 3) * 3 / rest;
+        if constexpr (g == G) fmac2_bcast<C>(y[C], z[C], z[J], my, mz);
+        panel_group<J, G, C + 1>(y, z, my, mz);
+    }
+}
+
+// Column steps J .. 15 of a panel: piv is pivot J, r its reciprocal; both go
+// to s_piv (the same from every lane).  The scheduling fences keep the
+// reciprocal's dependent steps apart, with the update's FMAs between them.
+template <int J>
+__device__ __forceinline__ void panel_steps(double (&y)[kPan], double (&z)[kPan], double piv, double r,
+                                            double *s_piv) {
+    s_piv[2 * J] = r;
+    s_piv[2 * J + 1] = piv;
+    if constexpr (J + 1 < kPan) {
+        const double my = -y[J] * r, mz = -z[J] * r;
+        double zb, zd;
+        bcast2<J + 1>(z[J], z[J + 1], zb, zd);
+        const double next = fma(-(zb * r), zb, zd);   // rounded as the update below rounds it
+        double q = __builtin_amdgcn_rcp(next);
+        fmac2_bcast<J + 1>(y[J + 1], z[J + 1], z[J], my, mz);
+        __builtin_amdgcn_sched_barrier(0);
+        panel_group<J, 0>(y, z, my, mz);
+        __builtin_amdgcn_sched_barrier(0);
+        double e = fma(-next, q, 1.0);
+        __builtin_amdgcn_sched_barrier(0);
+        panel_group<J, 1>(y, z, my, mz);
+        __builtin_amdgcn_sched_barrier(0);
+        e = fma(e, e, e);
+        __builtin_amdgcn_sched_barrier(0);
+        panel_group<J, 2>(y, z, my, mz);
+        __builtin_amdgcn_sched_barrier(0);
+        q = fma(e, q, q);
+        panel_steps<J + 1>(y, z, next, q, s_piv);
+    }
+}
+
+// Tile (rb, cb) of 16 x 16 minus panel p's product: rows of A (rb > p) or of
+// the identity (rb <= p; still zero at rb == p).
+__device__ __forceinline__ void panel_tile(double *sD, double *sE, const double *s_piv, int p, int rb, int cb) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    double *S = rb <= p ? sE : sD;
+    f64x4 acc;
 #pragma unroll
-    for (int q = 0; q < kCols; ++q) y[q] = Ajj[i + (int64_t) (w + kW * q) * ts];
-    if (w == 0) s_col[0][i] = y[0];
-    __syncthreads();
-    // j = kW p + jj: with p unrolled, column c = w + kW q is known to lie
-    // before column j for q < p and after it for q > p; only q = p compares
-    // the wave index with jj
+    for (int v = 0; v < 4; ++v) acc[v] = rb == p ? 0.0 : S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr];
 #pragma unroll
-    for (int p = 0; p < kCols; ++p) {
+    for (int kk = 0; kk < kPan; kk += 4) {
+        const int c = kPan * p + kk + lk;
+        acc = mfma_f64(-S[(kPan * rb + lr) * kPv + c] * s_piv[2 * c], sD[(kPan * cb + lr) * kPv + c], acc);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr] = acc[v];
+}
+
+// s_piv: 2 * 64 + 2 * 16 doubles.  Thread 0 gets the first column without a
+// positive pivot (-1: none).
+__device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv, double *s_rs) {
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave index, held in a scalar register
+    const int lr = lane & 15;
+    constexpr int kPanels = kBlk / kPan;
 #pragma unroll 1
-        for (int jj = 0; jj < kW; ++jj) {
-            const int j = kW * p + jj;
-            const int buf = jj & 1;
-            // every LDS operand of the step is read here, ahead of the pivot's
-            // arithmetic, so that the step waits on LDS once
-            const double piv = s_col[buf][j];
-            const double aij = s_col[buf][i];
-            double gl[kCols];
+    for (int p = 0; p < kPanels; ++p) {
+        const int c0 = kPan * p;
+        if (w < 2) {
+            double *row = w == 1 ? sE + (c0 + lr) * kPv + c0 : (lane >= c0 ? sD : sE) + lane * kPv + c0;
+            const double *dia = sD + (c0 + lr) * kPv + c0;
+            double y[kPan], z[kPan];
 #pragma unroll
-            for (int q = p; q < kCols; ++q) gl[q] = s_col[buf][w + kW * q];
-            if (t == 0 && !(piv > 0.0)) {
-                const int64_t col = (int64_t) k * ts + (int64_t) jb * kBlk + j;
-                if (col < n) atomicCAS(info, 0, (int) (col + 1));
-            }
-            // 1 / sqrt(piv): the hardware estimate and two Newton steps (each
-            // doubles the correct bits; the chain is 7 dependent operations
-            // instead of a correctly rounded square root followed by a division)
-            double rs = __builtin_amdgcn_rsq(piv);
-            const double hp = 0.5 * piv;
-            rs = fma(rs, fma(-hp * rs, rs, 0.5), rs);
-            rs = fma(rs, fma(-hp * rs, rs, 0.5), rs);
-            const double sq = piv * rs;
-            if (t == 0) s_rs[j] = rs;
-            const double lo = i > j ? aij * rs : 0.0;   // L_ij below the diagonal
-            const double r = lo * rs;
-            // column j of the unscaled X after its own step
-            const double xj0 = i == j ? 1.0 : -r;
+            for (int q = 0; q < kPan; ++q) z[q] = dia[q];
 #pragma unroll
-            for (int q = 0; q < kCols; ++q) {
-                if (q < p) {
-                    // c < j: X's column, operand X_jc from lane j
-                    y[q] = fma(-r, readlane_f64(y[q], j), y[q]);
-                } else if (q > p) {
-                    // c > j: A's column, operand A_cj from LDS
-                    y[q] = fma(-r, gl[q], y[q]);
-                    if (q == p + 1 && w == 0 && jj == kW - 1) s_col[buf ^ 1][i] = y[q];
-                } else {
-                    // c = w + kW p against j = kW p + jj: selects rather than
-                    // branches, so that y does not pass through branch joins
-                    const double g = w < jj ? readlane_f64(y[q], j) : gl[q];
-                    const double upd = fma(-r, g, y[q]);
-                    if (w == jj) Ajj[i + (int64_t) j * ts] = i > j ? lo : (i == j ? sq : 0.0);
-                    if (w == jj + 1) s_col[buf ^ 1][i] = upd;
-                    y[q] = w == jj ? xj0 : upd;   // c == j: L's column stored, X's column starts
-                }
+            for (int q = 0; q < kPan; ++q) y[q] = w == 0 ? row[q] : (lr == q ? 1.0 : 0.0);
+            __syncthreads();   // both waves have read the diagonal rows
+            double piv, unused;
+            bcast2<0>(z[0], z[0], piv, unused);
+            double r = __builtin_amdgcn_rcp(piv);
+            const double e = fma(-piv, r, 1.0);
+            r = fma(fma(e, e, e), r, r);
+            panel_steps<0>(y, z, piv, r, w == 0 ? s_piv + 2 * c0 : s_piv + 2 * kBlk);
+            if (w == 0 || lane < kPan) {
+#pragma unroll
+                for (int q = 0; q < kPan; ++q) row[q] = y[q];
             }
+        } else {
+            __syncthreads();
+            // the columns beyond panel p, minus panel p - 1
+            int idx = 0;
+            if (p > 0)
+                for (int cb = p + 1; cb < kPanels; ++cb)
+                    for (int rb = 0; rb < kPanels; ++rb)
+                        if ((rb < p || rb >= cb) && (idx++ & 1) == (w & 1)) panel_tile(sD, sE, s_piv, p - 1, rb, cb);
+        }
+        __syncthreads();
+        if (p + 1 < kPanels) {
+            panel_tile(sD, sE, s_piv, p, w, p + 1);
             __syncthreads();
         }
     }
-    double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-    const double rsi = s_rs[i];
-#pragma unroll
-    for (int q = 0; q < kCols; ++q) {
-        const int c = w + kW * q;
-        W[i + c * kBlk] = i >= c ? y[q] * rsi : 0.0;
+    int bad = -1;
+    if (w == 0) {
+        const double piv = s_piv[2 * lane + 1];
+        const unsigned long long m = __ballot(!(piv > 0.0));
+        if (m) bad = __ffsll((long long) m) - 1;
+        s_rs[lane] = rsqrt_f64(piv);
     }
-}
-
-// acc = X (64 x 64, column-major, ldx) W^T, W the 64 x 64 lower inverse (ld 64).
-__device__ __forceinline__ void times_wt(Acc64 &acc, const double *X, int64_t ldx, const double *W, GemmSmem &sm) {
-    acc_zero(acc);
-    wg_gemm_nt(acc, X, ldx, W, kBlk, kBlk, sm);
-}
-
-__device__ __forceinline__ void diag_update_body(const TileMap &map, int k, int jb, const double *winv_k,
-                                                 double *scratch, int bx) {
-    // 66.5 KB of LDS: L_r and L_c stay in registers until both GEMMs are done,
-    // then go through sm (sm.a and sm.b), so that a workgroup fits beside one
-    // workgroup of the trailing update
-    __shared__ GemmSmem sm;
-    static_assert(sizeof(GemmSmem::a) >= sizeof(double) * kBlk * kLdsPad, "L_r must fit in the staging buffer");
-    static_assert(sizeof(GemmSmem::b) >= sizeof(double) * kBlk * kLdsPad, "L_c must fit in the staging buffer");
-    double (*sLr)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.a[0][0][0]);
-    double (*sLc)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.b[0][0][0]);
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    // bx enumerates the pairs jb < c <= r < nsb column by column
-    int idx = bx, c = jb + 1;
-    while (idx >= nsb - c) {
-        idx -= nsb - c;
-        ++c;
-    }
-    const int r = c + idx;
-    double *T = tile_f64(map, k, k);
-    const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int mq = wv & 1, nq = wv >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    Acc64 acc_r, acc_c;
-    times_wt(acc_r, T + r * kBlk + (int64_t) jb * kBlk * ts, ts, W, sm);
-    if (c != r) times_wt(acc_c, T + c * kBlk + (int64_t) jb * kBlk * ts, ts, W, sm);
-    // the GEMMs end with a barrier: sm is free
-    acc_foreach(acc_r, [&](int rr, int cc, double v) { sLr[rr][cc] = v; });
-    if (c != r) acc_foreach(acc_c, [&](int rr, int cc, double v) { sLc[rr][cc] = v; });
     __syncthreads();
-    const double (*Lc)[kLdsPad] = (c != r) ? sLc : sLr;
-    // A_rc -= L_r L_c^T
-    Acc64 upd;
-    acc_zero(upd);
+    return bad;
+}
+
+// ------------------------------------------------------------------------
+// Tile column k in one launch: the Cholesky of its diagonal tile in 64 x 64
+// blocks, the inverses of the diagonal blocks (winv_k), and the panel solve of
+// `halves` blocks of 32 rows below it.
+//
+// Workgroups take a ticket each and run the task of that number; a task waits
+// only for blocks of lower tickets, so the workgroups that run can always
+// finish, however few of them the GPU holds.  Tasks, with L_rc the solved block
+// (r, c) of the diagonal tile:
+//   per block column c:  the diagonal task c (blocks (c, c - 1) and (c, c)),
+//                        then the tasks (r, c), r >= c + 2 (one block each);
+//   after them           the 32-row blocks below the tile, all block columns.
+// A task adds up its blocks' products with the earlier block columns as those
+// are published (flags in `sync`, one per block, zero at the launch), so that
+// a diagonal task has only X = T W^T, D -= X X^T and the factorization left
+// when the inverse before it arrives.  Bound: that chain, 20 us per 64 columns
+// alone (7.8 us of it the factorization, the rest two 64 x 64 x 64 products, the
+// loads and the flag).  One launch per block column (each waiting anew for room
+// beside the trailing update), a copy, and the panel solve after the whole tile
+// took 36 us per 64 columns alone, 90 to 140 us beside the trailing update, plus
+// 40 (ts 320) to 440 us (ts 960) for the panel.  One evaluation: 400 locations
+// 0.54 -> 0.34 ms, 1,600 1.41 -> 0.83 ms, 10,007 14.8 -> 13.2 ms.
+// ------------------------------------------------------------------------
+namespace {
+
+struct PanelSmem {
+    double a[kBlk * kPv];   // operand columns: element (row, col) at col * kPv + row
+    double b[kBlk * kPv];
+    double piv[2 * kBlk + 2 * kPan];
+    double rs[kBlk];
+};
+static_assert(sizeof(GemmSmem) <= sizeof(PanelSmem), "the row blocks stage through the same LDS");
+
+// Waits until another workgroup of the launch has published the block.
+__device__ __forceinline__ void wait_block(const int *flag) {
+    if (threadIdx.x == 0) {
+        while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+}
+
+// Publishes what the workgroup has stored.
+__device__ __forceinline__ void publish_block(int *flag) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A 64 x 64 block of a column-major matrix into LDS, in flight as 16 loads per
+// thread.
+__device__ __forceinline__ void load_block(double (&v)[16], const double *src, int64_t ld) {
+    const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = src[row + (int64_t) (w + 4 * q) * ld];
+}
+__device__ __forceinline__ void put_block(double *s, const double (&v)[16]) {
+    const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) s[(w + 4 * q) * kPv + row] = v[q];
+}
+
+// acc += A B^T, or acc -= A B^T, for 64 x 64 operands in LDS.
+template <bool kSubtract>
+__device__ __forceinline__ void mma_block(Acc64 &acc, const double *a, const double *b) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int mq = w & 1, nq = w >> 1;
+    const int lr = lane & 15, lk = lane >> 4;
 #pragma unroll 4
     for (int kk = 0; kk < kBlk; kk += 4) {
-        const double a0 = sLr[mq * 32 + lr][kk + lk];
-        const double a1 = sLr[mq * 32 + 16 + lr][kk + lk];
-        const double b0 = Lc[nq * 32 + lr][kk + lk];
-        const double b1 = Lc[nq * 32 + 16 + lr][kk + lk];
-        upd.v[0][0] = mfma_f64(b0, a0, upd.v[0][0]);
-        upd.v[0][1] = mfma_f64(b0, a1, upd.v[0][1]);
-        upd.v[1][0] = mfma_f64(b1, a0, upd.v[1][0]);
-        upd.v[1][1] = mfma_f64(b1, a1, upd.v[1][1]);
-    }
-    double *C = T + r * kBlk + (int64_t) c * kBlk * ts;
-    double cv[16];
-    int q = 0;
-    acc_foreach(upd, [&](int rr, int cc, double) { cv[q++] = C[rr + (int64_t) cc * ts]; });
-    q = 0;
-    acc_foreach(upd, [&](int rr, int cc, double v) { C[rr + (int64_t) cc * ts] = cv[q++] - v; });
-    if (c == r) {
-        double *S = scratch + r * kBlk + (int64_t) jb * kBlk * ts;
-        for (int e = threadIdx.x; e < kBlk * kBlk; e += kThreads) {
-            const int rr = e & 63, cc = e >> 6;
-            S[rr + (int64_t) cc * ts] = sLr[rr][cc];
+        double a0 = a[(kk + lk) * kPv + mq * 32 + lr];
+        double a1 = a[(kk + lk) * kPv + mq * 32 + 16 + lr];
+        if (kSubtract) {
+            a0 = -a0;
+            a1 = -a1;
         }
+        const double b0 = b[(kk + lk) * kPv + nq * 32 + lr];
+        const double b1 = b[(kk + lk) * kPv + nq * 32 + 16 + lr];
+        acc.v[0][0] = mfma_f64(b0, a0, acc.v[0][0]);
+        acc.v[0][1] = mfma_f64(b0, a1, acc.v[0][1]);
+        acc.v[1][0] = mfma_f64(b1, a0, acc.v[1][0]);
+        acc.v[1][1] = mfma_f64(b1, a1, acc.v[1][1]);
     }
 }
 
-// Launch jb of the diagonal tile (see above); rem (rem + 1) / 2 workgroups
-// for jb > 0, rem = nsb - jb, and one for jb = 0.
-__device__ __forceinline__ void diag_step_body(const TileMap &map, int k, int jb, double *winv_k, double *scratch,
-                                               int *info, int64_t n, int bx) {
-    if (jb > 0) {
-        // workgroup 0 takes the first pair, (jb, jb)
-        diag_update_body(map, k, jb - 1, winv_k, scratch, bx);
-        if (bx != 0) return;
-        __syncthreads();   // block (jb, jb) updated by every thread
+// The accumulators hold the block C (column-major, ld).
+__device__ __forceinline__ void acc_load(Acc64 &acc, const double *C, int64_t ld) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = (w & 1) * 32 + (lane & 15), c = (w >> 1) * 32 + (lane >> 4);
+#pragma unroll
+    for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc.v[ni][mi][v] = C[r + mi * 16 + (int64_t) (c + ni * 16 + 4 * v) * ld];
+}
+
+// Block (r, c) of the tile T (ld ts), r > c: solved in place and published;
+// its columns stay in sm.a.  With acc_d, acc_d -= L_rb L_rb^T for every b <= c.
+// The products are subtracted from the block itself, one MFMA after another:
+// the residual shrinks as they go, and with it the rounding (summing them
+// first rounds at the size of the block).
+__device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, int c, const double *winv_k, int *flags,
+                                            PanelSmem &sm, Acc64 *acc_d) {
+    double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
+    double va[16], vb[16];
+    Acc64 acc;
+    acc_load(acc, X, ts);
+    for (int b = 0; b < c; ++b) {
+        wait_block(flags + r * nsb + b);
+        wait_block(flags + c * nsb + b);
+        load_block(va, T + r * kBlk + (int64_t) b * kBlk * ts, ts);
+        load_block(vb, T + c * kBlk + (int64_t) b * kBlk * ts, ts);
+        put_block(sm.a, va);
+        put_block(sm.b, vb);
+        __syncthreads();
+        mma_block<true>(acc, sm.a, sm.b);
+        if (acc_d) mma_block<true>(*acc_d, sm.a, sm.a);
+        __syncthreads();
     }
-    potrf64_body(map, k, jb, winv_k, info, n);
+    acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
+    wait_block(flags + c * nsb + c);
+    load_block(vb, winv_k + (int64_t) c * kBlk * kBlk, kBlk);
+    put_block(sm.b, vb);
+    __syncthreads();
+    acc_zero(acc);
+    mma_block<false>(acc, sm.a, sm.b);
+    __syncthreads();
+    acc_foreach(acc, [&](int i, int j, double v) {
+        X[i + (int64_t) j * ts] = v;
+        sm.a[j * kPv + i] = v;
+    });
+    if (acc_d) {
+        __syncthreads();
+        mma_block<true>(*acc_d, sm.a, sm.a);
+    }
+    publish_block(flags + r * nsb + c);
 }
 
-__global__ void __launch_bounds__(kThreads) diag_step_kernel(TileMap map, int k, int jb, double *winv_k,
-                                                             double *scratch, int *info, int64_t n) {
-    diag_step_body(map, k, jb, winv_k, scratch, info, n, blockIdx.x);
+// Diagonal task r: block (r, r - 1), then block (r, r) factored and inverted.
+__device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r, double *winv_k, int *flags, int *info,
+                                              int64_t col0, int64_t n, PanelSmem &sm) {
+    double *D = T + r * kBlk + (int64_t) r * kBlk * ts;
+    Acc64 acc_d;
+    acc_load(acc_d, D, ts);
+    if (r > 0) solve_block(T, ts, nsb, r, r - 1, winv_k, flags, sm, &acc_d);
+    acc_foreach(acc_d, [&](int i, int j, double v) { sm.a[i * kPv + j] = v; });
+    __syncthreads();
+    const int bad = potrf64_lds(sm.a, sm.b, sm.piv, sm.rs);
+    if (threadIdx.x == 0 && bad >= 0 && col0 + r * kBlk + bad < n) atomicCAS(info, 0, (int) (col0 + r * kBlk + bad + 1));
+    double *W = winv_k + (int64_t) r * kBlk * kBlk;
+    const int i = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double rsi = sm.rs[i];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int j = w + 4 * q;
+        W[i + j * kBlk] = i >= j ? sm.b[j * kPv + i] * rsi : 0.0;
+        D[i + (int64_t) j * ts] = i > j ? sm.a[i * kPv + j] * sm.rs[j] : i == j ? sm.piv[2 * j + 1] * rsi : 0.0;
+    }
+    publish_block(flags + r * nsb + r);
 }
 
-namespace {
-unsigned diag_step_blocks(int nsb, int jb) {
-    const int rem = nsb - jb;
-    return jb == 0 ? 1u : (unsigned) (rem * (rem + 1) / 2);
+// 32 rows X of the panel below the tile, all block columns.
+__device__ __forceinline__ void rows_task(const double *T, int ts, int nsb, double *X, const double *winv_k,
+                                          const int *flags, GemmSmem &sm) {
+    double (*sT)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.a[0][0][0]);
+    const int lane = threadIdx.x & 63;
+    const int w = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    for (int jb = 0; jb < nsb; ++jb) {
+        AccHalf acc;
+        acc_zero(acc);
+        if (jb > 0) {
+            // the diagonal task has waited for the row's earlier blocks
+            wait_block(flags + jb * nsb + jb - 1);
+            wg_gemm_nt_half(acc, X, ts, T + jb * kBlk, ts, jb * kBlk, sm);
+        }
+        double *Xj = X + (int64_t) jb * kBlk * ts;
+        acc_foreach(acc, [&](int r, int c, double v) { sT[r][c] = Xj[r + (int64_t) c * ts] - v; });
+        wait_block(flags + jb * nsb + jb);
+        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
+        AccHalf acc2;
+        acc_zero(acc2);
+#pragma unroll 4
+        for (int kk = 0; kk < kBlk; kk += 4) {
+            const double a0 = sT[lr][kk + lk];
+            const double a1 = sT[16 + lr][kk + lk];
+            const double b0 = W[(w * 16 + lr) + (kk + lk) * kBlk];
+            acc2.v[0] = mfma_f64(b0, a0, acc2.v[0]);
+            acc2.v[1] = mfma_f64(b0, a1, acc2.v[1]);
+        }
+        acc_foreach(acc2, [&](int r, int c, double v) { Xj[r + (int64_t) c * ts] = v; });
+        __syncthreads();
+    }
 }
+
+// Tasks of the diagonal tile, and the task of a ticket: r < 0 for rows.
+__host__ __device__ inline int tile_tasks(int nsb) { return nsb + (nsb - 1) * (nsb - 2) / 2; }
+
 }  // namespace
 
-// Blocks (r, c), r > c, of the scratch copy back into diagonal tile k.
-__device__ __forceinline__ void diag_copy_body(const TileMap &map, int k, const double *scratch, int bx) {
+// One task of tile column k; sync: the column's ticket (unused here) and flags.
+__device__ __forceinline__ void tile_column_task(const TileMap &map, int k, double *winv_k, int *sync, int *info,
+                                                 int64_t n, int halves, int task, PanelSmem &sm) {
     const int ts = map.ts;
     const int nsb = ts / kBlk;
-    int idx = bx, c = 0;
-    while (idx >= nsb - 1 - c) {
-        idx -= nsb - 1 - c;
+    int *flags = sync + 1;
+    double *T = tile_f64(map, k, k);
+    if (task >= tile_tasks(nsb)) {
+        const int h = task - tile_tasks(nsb);
+        if (h >= halves) return;
+        const int per = ts / kHalf;
+        double *X = tile_f64(map, k + 1 + h / per, k) + (h % per) * kHalf;
+        rows_task(T, ts, nsb, X, winv_k, flags, *reinterpret_cast<GemmSmem *>(&sm));
+        return;
+    }
+    // block column c holds the diagonal task and nsb - 2 - c others
+    int c = 0, idx = task;
+    while (idx > max(0, nsb - 2 - c)) {
+        idx -= 1 + max(0, nsb - 2 - c);
         ++c;
     }
-    const int r = c + 1 + idx;
-    double *T = tile_f64(map, k, k);
-    const int64_t base = r * kBlk + (int64_t) c * kBlk * ts;
-    for (int e = threadIdx.x; e < kBlk * kBlk; e += kThreads) {
-        const int rr = e & 63, cc = e >> 6;
-        T[base + rr + (int64_t) cc * ts] = scratch[base + rr + (int64_t) cc * ts];
-    }
+    if (idx == 0)
+        diagonal_task(T, ts, nsb, c, winv_k, flags, info, (int64_t) k * ts, n, sm);
+    else
+        solve_block(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, nullptr);
 }
 
-__global__ void __launch_bounds__(kThreads) diag_copy_kernel(TileMap map, int k, const double *scratch) {
-    diag_copy_body(map, k, scratch, blockIdx.x);
+__device__ __forceinline__ int take_ticket(int *counter) {
+    __shared__ int s_ticket;
+    if (threadIdx.x == 0) s_ticket = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    return s_ticket;
+}
+
+__global__ void __launch_bounds__(kThreads) tile_column_kernel(TileMap map, int k, double *winv_k, int *sync, int *info,
+                                                               int64_t n, int halves) {
+    __shared__ PanelSmem sm;
+    tile_column_task(map, k, winv_k, sync, info, n, halves, take_ticket(sync), sm);
 }
 
 // ------------------------------------------------------------------------
@@ -972,14 +1149,13 @@ __global__ void __launch_bounds__(kThreads) diag_copy_kernel(TileMap map, int k,
 // same tile size, problem b described by jobs[b] (blockIdx.y, or blockIdx.z
 // for the update); workgroups beyond a problem's extent exit at once.
 // ------------------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) diag_step_batch_kernel(const BatchJob *jobs, int jb) {
-    const BatchJob &J = jobs[blockIdx.y];
-    diag_step_body(J.map, J.k, jb, J.winv_k, J.scratch, J.info, J.n, blockIdx.x);
-}
-
-__global__ void __launch_bounds__(kThreads) diag_copy_batch_kernel(const BatchJob *jobs) {
-    const BatchJob &J = jobs[blockIdx.y];
-    diag_copy_body(J.map, J.k, J.scratch, blockIdx.x);
+// Tickets interleave the problems: task t / njobs of problem t % njobs.
+__global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const BatchJob *jobs, int njobs, int with_rows) {
+    __shared__ PanelSmem sm;
+    const int t = take_ticket(jobs[0].sync);
+    const BatchJob &J = jobs[t % njobs];
+    const int halves = with_rows ? (J.map.nt - J.k - 1) * (J.map.ts / kHalf) : 0;
+    tile_column_task(J.map, J.k, J.winv_k, J.sync, J.info, J.n, halves, t / njobs, sm);
 }
 
 __global__ void __launch_bounds__(kThreads) trsm_rows_batch_kernel(const BatchJob *jobs) {
@@ -1005,38 +1181,38 @@ __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *
     update_body(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y);
 }
 
-void launch_factor_diag_batch(const BatchJob *jobs, int njobs, int ts, hipStream_t s) {
+// Panels of at most this many 64-row blocks are solved by the launch that
+// factors the diagonal tile; a longer one by its own launch after it (its
+// workgroups would hold the GPU's slots while they wait for the diagonal tile,
+// and 64-row blocks load L_kk half as often per flop).
+constexpr int kFusedRows = 128;
+
+void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nrest, hipStream_t s) {
     if (njobs <= 0) return;
     const int nsb = ts / kBlk;
-    for (int jb = 0; jb < nsb; ++jb)
-        hipLaunchKernelGGL(diag_step_batch_kernel, dim3(diag_step_blocks(nsb, jb), njobs), dim3(kThreads), 0, s, jobs,
-                           jb);
-    if (nsb > 1)
-        hipLaunchKernelGGL(diag_copy_batch_kernel, dim3((unsigned) (nsb * (nsb - 1) / 2), njobs), dim3(kThreads), 0, s,
+    const bool fused = rest * nsb * nrest <= kFusedRows;
+    const int tasks = tile_tasks(nsb) + (fused ? rest * (ts / kHalf) : 0);
+    hipLaunchKernelGGL(tile_column_batch_kernel, dim3((unsigned) (tasks * njobs)), dim3(kThreads), 0, s, jobs, njobs,
+                       fused ? 1 : 0);
+    if (rest <= 0 || nrest <= 0) return;
+    if (!fused && rest * nsb * nrest < kHalfRowsBelow)
+        hipLaunchKernelGGL(trsm_rows_half_batch_kernel, dim3((unsigned) (2 * rest * nsb), nrest), dim3(kThreads), 0, s,
                            jobs);
-}
-
-void launch_panel_update_batch(const BatchJob *jobs, int njobs, int ts, int rest, hipStream_t s) {
-    if (njobs <= 0 || rest <= 0) return;
-    const int nsb = ts / kBlk;
-    if (rest * nsb * njobs < kHalfRowsBelow)
-        hipLaunchKernelGGL(trsm_rows_half_batch_kernel, dim3((unsigned) (2 * rest * nsb), njobs), dim3(kThreads), 0, s,
-                           jobs);
-    else
-        hipLaunchKernelGGL(trsm_rows_batch_kernel, dim3((unsigned) (rest * nsb), njobs), dim3(kThreads), 0, s, jobs);
-    hipLaunchKernelGGL(update_batch_kernel, dim3((unsigned) (nsb * nsb), (unsigned) (rest * (rest + 1) / 2), njobs),
+    else if (!fused)
+        hipLaunchKernelGGL(trsm_rows_batch_kernel, dim3((unsigned) (rest * nsb), nrest), dim3(kThreads), 0, s, jobs);
+    hipLaunchKernelGGL(update_batch_kernel, dim3((unsigned) (nsb * nsb), (unsigned) (rest * (rest + 1) / 2), nrest),
                        dim3(kThreads), 0, s, jobs);
 }
 
-void launch_factor_diag(const TileMap &map, int k, double *winv_k, double *scratch, int *info, int64_t n,
+int tile_column_sync_ints(int ts) { return 1 + (ts / kBlk) * (ts / kBlk); }
+
+bool tile_column_solves_rows(int ts, int rows) { return (int64_t) rows * (ts / kBlk) <= kFusedRows; }
+
+void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int rows,
                         hipStream_t s) {
-    const int nsb = map.ts / kBlk;
-    for (int jb = 0; jb < nsb; ++jb)
-        hipLaunchKernelGGL(diag_step_kernel, dim3(diag_step_blocks(nsb, jb)), dim3(kThreads), 0, s, map, k, jb, winv_k,
-                           scratch, info, n);
-    if (nsb > 1)
-        hipLaunchKernelGGL(diag_copy_kernel, dim3((unsigned) (nsb * (nsb - 1) / 2)), dim3(kThreads), 0, s, map, k,
-                           scratch);
+    const int halves = rows * (map.ts / kHalf);
+    hipLaunchKernelGGL(tile_column_kernel, dim3((unsigned) (tile_tasks(map.ts / kBlk) + halves)), dim3(kThreads), 0, s,
+                       map, k, winv_k, sync, info, n, halves);
 }
 
 }  // namespace egs

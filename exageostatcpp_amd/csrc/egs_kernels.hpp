@@ -13,14 +13,15 @@ namespace egs {
 
 // One problem's share of a batched step (FP64 plan): step k of the tiled
 // Cholesky or of the forward solve on the tiles of `map`, with that problem's
-// update order (pairs), diagonal-block inverses of tile k, diagonal scratch,
-// not-SPD flag (n: its real dimension) and solve vector with its partials.
+// update order (pairs), diagonal-block inverses of tile k, the tile column's
+// ticket and flags (launch_tile_column), not-SPD flag (n: its real dimension)
+// and solve vector with its partials.
 struct BatchJob {
     TileMap map;
     int k;
     const int2 *pairs;
     double *winv_k;
-    double *scratch;
+    int *sync;
     int *info;
     int64_t n;
     double *z;
@@ -84,17 +85,22 @@ void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams
 void launch_cov_matvec(double *partial, const double *v, int64_t n, int64_t npad, const MaternParams &prm,
                        const double *x, const double *y, const double *z, hipStream_t s);
 int matvec_chunks(int64_t n);
-// Cholesky of diagonal tile k in place, right-looking in 64 x 64 blocks, with
-// the inverses of its diagonal blocks in winv_k; scratch holds ts * ts doubles.
-void launch_factor_diag(const TileMap &map, int k, double *winv_k, double *scratch, int *info, int64_t n,
+// Cholesky of diagonal tile k in place, in 64 x 64 blocks, with the inverses of
+// its diagonal blocks in winv_k, and the panel solve of the `rows` FP64 tiles
+// below it (tile_column_solves_rows: whether that many should be; the others
+// take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
+// tile_column_sync_ints(ts) ints, zero before the launch.
+int tile_column_sync_ints(int ts);
+bool tile_column_solves_rows(int ts, int rows);
+void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int rows,
                         hipStream_t s);
-// Batched steps over njobs problems of tile size ts (jobs in device memory):
-// factor diagonal tile k of each; then solve panel k and apply it to tile
-// columns k+1 .. of each (rest = the largest nt - k - 1 among the jobs; jobs
-// with fewer tiles exit early); forward-solve tile row k with its partials
-// and subtract it from the rows below.
-void launch_factor_diag_batch(const BatchJob *jobs, int njobs, int ts, hipStream_t s);
-void launch_panel_update_batch(const BatchJob *jobs, int njobs, int ts, int rest, hipStream_t s);
+// Batched steps over problems of tile size ts (jobs in device memory, those
+// with most tiles first): factor tile column k of each of njobs, then apply
+// panel k to tile columns k+1 .. of the first nrest, the ones that have them
+// (rest = the largest nt - k - 1; jobs with fewer tiles exit early);
+// forward-solve tile row k with its partials and subtract it from the rows
+// below.
+void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nrest, hipStream_t s);
 void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int rest, hipStream_t s);
 // X_k = L_kk^{-T} for every diagonal tile k (tinv: nt * ts * ts doubles).
 void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream_t s);

@@ -1,0 +1,74 @@
+"""The Cholesky of a tile column (diagonal tile, inverses and panel solve in one
+launch) against LAPACK, at the edges of its task lists: one 64 x 64 block, two
+(no block task), the largest tile, panels below and beyond the rows that the
+launch takes, ragged last tiles; and batches on both sides of that rule.
+
+Tolerance: n eps times a small constant on the factor's backward error
+(Higham's bound for Cholesky), 64 n eps relative to the largest entry.
+"""
+import numpy as np
+import pytest
+
+import exageostatcpp_amd as egs
+from exageostatcpp_amd import capi
+from oracle import orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = egs.Context(0)
+    yield c
+    c.close()
+
+
+def locations(n, seed):
+    return tuple(np.random.default_rng(seed).random((2, n)))
+
+
+@pytest.mark.parametrize("n,dts", [(40, 64), (64, 64), (65, 64), (128, 128), (500, 128), (700, 192), (1000, 320),
+                                   (2048, 2048), (2100, 2048), (1500, 64),
+                                   (8256, 64), (8320, 64), (8400, 64)])   # 128, 129 and 131 row blocks below
+def test_factor_backward_error(ctx, n, dts):
+    x, y = locations(n, n)
+    p = egs.Problem(ctx, 0, x, y, dts=dts)
+    p.covariance([1.0, 0.1, 0.5])
+    a = p.get_matrix()
+    p.potrf()
+    low = p.get_matrix()
+    p.close()
+    a = a + np.tril(a, -1).T
+    err = np.max(np.abs(low @ low.T - a))
+    assert err < 64 * n * np.finfo(float).eps
+    assert np.all(np.diag(low) > 0)
+
+
+@pytest.mark.parametrize("sizes,dts", [([50, 64, 65], 64), ([900, 700, 500, 200], 128), ([3000, 700, 650, 64], 64),
+                                       ([500, 1100, 2900, 1500, 700, 640, 385, 384], 384)])
+def test_batch_of_uneven_problems(ctx, sizes, dts):
+    th = [1.0, 0.1, 0.5]
+    probs, want = [], []
+    for i, n in enumerate(sizes):
+        x, y = locations(n, 100 + i)
+        z = np.random.default_rng(i).standard_normal(n)
+        p = egs.Problem(ctx, 0, x, y, dts=dts)
+        p.set_observations(z)
+        want.append(p.loglik(th))
+        probs.append(p)
+    for (llh, ld, q), (l0, d0, q0) in zip(capi.loglik_batch(probs, [th] * len(probs)), want):
+        assert abs(llh - l0) <= 1e-11 * abs(l0) and abs(ld - d0) <= 1e-11 * abs(d0) and abs(q - q0) <= 1e-11 * abs(q0)
+    for p in probs:
+        p.close()
+
+
+@pytest.mark.parametrize("dts", [64, 128, 320])
+@pytest.mark.parametrize("kernel,theta,minor", [(0, [-1.0, 0.1, 0.5], 1),
+                                                (1, [1.0, 1.0, 0.1, 0.5, 0.5, 1.5], 2)])   # correlation above 1
+def test_first_failing_minor_is_reported(ctx, dts, kernel, theta, minor):
+    x, y = locations(300, 3)
+    p = egs.Problem(ctx, kernel, x, y, dts=dts)
+    p.set_observations(np.ones(p.n))
+    with pytest.raises(egs.NotPositiveDefinite, match=r"leading minor %d\)" % minor):
+        p.loglik(theta)
+    p.close()
