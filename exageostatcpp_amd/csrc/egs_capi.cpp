@@ -209,7 +209,7 @@ struct egs_problem_s {
     double factored_theta[6] = {0, 0, 0, 0, 0, 0};
     double cov_theta[6] = {0, 0, 0, 0, 0, 0};
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    std::vector<hipEvent_t> ev_panel, ev_bulk;   // per step: panel solved / bulk update done
+    std::vector<hipEvent_t> ev_column, ev_bulk;   // per step k: column k+1 updated / column k+2 updated
     double t_cov = 0, t_fact = 0, t_solve = 0;
     Profiler prof;
     // FP64 evaluations replayed from a captured graph (egs_problem_set_graph):
@@ -414,11 +414,11 @@ void free_problem_buffers(egs_problem_s *p) {
     for (auto &e : p->prof.ev)
         if (e) hipEventDestroy(e);
     p->prof.ev.clear();
-    for (auto &e : p->ev_panel)
+    for (auto &e : p->ev_column)
         if (e) hipEventDestroy(e);
     for (auto &e : p->ev_bulk)
         if (e) hipEventDestroy(e);
-    p->ev_panel.clear();
+    p->ev_column.clear();
     p->ev_bulk.clear();
     p->prof.pending.clear();
     p->d_x = p->d_y = p->d_z = nullptr;
@@ -683,10 +683,6 @@ double update_flops_cls(const egs_problem_s *p, int c, int j0, int j1) {
     return f;
 }
 
-// FP64 updates of at most this many tiles on the critical stream use 64 x 64
-// workgroups: 225 per tile, each done in a ninth of the time of a 192 x 192 one.
-constexpr int kShortUpdate = 8;
-
 // Updates of step k under a mixed plan for tile columns [j0, nt) restricted to
 // the column range encoded by the class prefix counts: entries [lo_c, hi_c) of
 // each class list.  critical: the launches are on the critical path.
@@ -702,9 +698,7 @@ void launch_mixed_update(egs_problem_s *p, int k, int jcol_lo, int jcol_hi, hipS
         const int pi = prof_begin(p, prof_id[c], update_flops_cls(p, c, jcol_lo, jcol_hi), st);
         const int2 *pr = p->d_pairs_cls[c] + beg;
         const int slot = k % kPanelSlots;
-        if (c == 0 && critical && end - beg <= kShortUpdate)
-            egs::launch_update64(m, p->d_p64[slot], pr, end - beg, k, st);
-        else if (c == 0) egs::launch_update192_panel(m, p->d_p64[slot], pr, end - beg, k, st);
+        if (c == 0) egs::launch_update(m, p->d_p64[slot], pr, end - beg, k, critical, st);
         else if (c == 1) egs::launch_update192_f32(m, p->d_p32[slot], pr, end - beg, k, st);
         else {
             const bool all_single = std::isinf(p->tau_single);
@@ -738,11 +732,11 @@ int run_potrf(egs_problem_s *p) {
     const egs::TileMap m = p->map();
     const int nt = p->nt;
     p->has_cov = false;   // the factorization overwrites the tiles
-    for (int k = (int) p->ev_panel.size(); k < nt; ++k) {
+    for (int k = (int) p->ev_column.size(); k < nt; ++k) {
         hipEvent_t e1 = nullptr, e2 = nullptr;
         EGS_HIP(hipEventCreateWithFlags(&e1, hipEventDisableTiming));
         EGS_HIP(hipEventCreateWithFlags(&e2, hipEventDisableTiming));
-        p->ev_panel.push_back(e1);
+        p->ev_column.push_back(e1);
         p->ev_bulk.push_back(e2);
     }
     // a fill kernel, not a memset: this sequence is captured into a graph
@@ -753,21 +747,33 @@ int run_potrf(egs_problem_s *p) {
         egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_counts), 6, s);
     }
     factor_panel(p, 0);
-    EGS_HIP(hipEventRecord(p->ev_panel[0], s));
     for (int k = 0; k + 1 < nt; ++k) {
         const int beyond = nt - k - 2;                 // tile columns k+2 .. nt-1
         const int n_beyond = beyond * (beyond + 1) / 2;
         const int n_next = nt - k - 1;                 // tiles (i, k+1), i >= k+1
+        // Tile column k+1 first, and alone but for what is left of bulk step
+        // k-1: beside bulk step k it would take twice as long, and with it
+        // everything after it.  Then its factorization beside bulk step k.
+        if (k > 0) EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[k - 1], 0));
+        if (is_mixed(p)) {
+            launch_mixed_update(p, k, k + 1, k + 2, s, true);
+        } else {
+            const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 1, k + 2), s);
+            egs::launch_update(m, nullptr, p->d_pairs + n_beyond, n_next, k, true, s);
+            prof_end(p, pi, s);
+        }
+        EGS_HIP(hipEventRecord(p->ev_column[k], s));
+        factor_panel(p, k + 1);
         // Bulk step k: column k+2 first, then ev_bulk[k], then columns k+3 ..:
         // the critical stream's step k+1 needs only column k+2, so it overlaps
         // the rest of this step.  (The list holds columns in descending order:
         // column k+2 is the last beyond - 1 ... entries of the prefix.)
-        EGS_HIP(hipStreamWaitEvent(b, p->ev_panel[k], 0));
+        EGS_HIP(hipStreamWaitEvent(b, p->ev_column[k], 0));
         if (is_mixed(p)) {
             if (k + 2 < nt) launch_mixed_update(p, k, k + 2, k + 3, b);
         } else if (n_beyond > 0) {
             const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 2, k + 3), b);
-            egs::launch_update(m, p->d_pairs + (n_beyond - beyond), beyond, k, b);
+            egs::launch_update(m, nullptr, p->d_pairs + (n_beyond - beyond), beyond, k, false, b);
             prof_end(p, pi, b);
         }
         EGS_HIP(hipEventRecord(p->ev_bulk[k], b));
@@ -775,20 +781,9 @@ int run_potrf(egs_problem_s *p) {
             if (k + 3 < nt) launch_mixed_update(p, k, k + 3, nt, b);
         } else if (n_beyond > beyond) {
             const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 3, nt), b);
-            egs::launch_update(m, p->d_pairs, n_beyond - beyond, k, b);
+            egs::launch_update(m, nullptr, p->d_pairs, n_beyond - beyond, k, false, b);
             prof_end(p, pi, b);
         }
-        if (k > 0) EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[k - 1], 0));
-        if (is_mixed(p)) {
-            launch_mixed_update(p, k, k + 1, k + 2, s, true);
-        } else {
-            const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 1, k + 2), s);
-            if (n_next <= kShortUpdate) egs::launch_update64(m, nullptr, p->d_pairs + n_beyond, n_next, k, s);
-            else egs::launch_update(m, p->d_pairs + n_beyond, n_next, k, s);
-            prof_end(p, pi, s);
-        }
-        factor_panel(p, k + 1);
-        EGS_HIP(hipEventRecord(p->ev_panel[k + 1], s));
     }
     // ev_bulk[nt - 1] (unused by the steps) marks the end of the bulk stream;
     // a one-tile matrix never uses it (and a capture must not wait on an event

@@ -10,8 +10,8 @@
 //     the 64-column blocks of L_kk and applying the 64 x 64 inverses
 //     (trsm_rows_kernel);
 //   * the trailing tiles are updated with FP64 MFMA: update192 (egs_update.hip)
-//     when ts is a multiple of 192, else update_kernel here, one workgroup per
-//     64 x 64 output block with K = ts.
+//     when ts is a multiple of 192 and the tiles are many, else update_kernel
+//     here, one workgroup per 64 x 64 output block with K = ts.
 // Every contraction uses v_mfma_f64_16x16x4f64 through wg_gemm_nt: four waves
 // each own a 32 x 32 quadrant of the 64 x 64 output; K is staged through LDS in
 // chunks of 32 columns, double buffered, with the next chunk's global loads
@@ -657,18 +657,24 @@ void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, 
                            g0, count64, winv_k);
 }
 
-void launch_update(const TileMap &map, const int2 *pairs, int npairs, int k, hipStream_t s) {
-    if (npairs <= 0) return;
-    if (update192_supported(map.ts)) {
-        launch_update192(map, pairs, npairs, k, s);
-        return;
-    }
-    launch_update64(map, nullptr, pairs, npairs, k, s);
-}
+// Up to this many 64 x 64 blocks (three per CU) are updated one workgroup each:
+// they run at once, and end sooner than the 96 x 192 blocks of update192, of
+// which a few tiles have too few (measured: 8 tiles of 384 44 against 68 us,
+// 20 75 / 79, 40 119 / 122, 160 407 / 334; 2 tiles of 960 94 / 154, 4 184 /
+// 166; 64 tiles of 192 39 / 46).  On the critical path, where the update shares
+// the GPU with the one before, the shorter workgroups pay up to twice as many
+// (6,001 locations, tiles of 960: 5.2 against 5.4 ms).
+constexpr int kSmallBlocks = 768, kSmallBlocksCritical = 1800;
 
-void launch_update64(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s) {
+void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, bool critical,
+                   hipStream_t s) {
     if (npairs <= 0) return;
     const int nsb = map.ts / kBlk;
+    if (update192_supported(map.ts) &&
+        (int64_t) npairs * nsb * nsb > (critical ? kSmallBlocksCritical : kSmallBlocks)) {
+        launch_update192(map, p64, pairs, npairs, k, s);
+        return;
+    }
     hipLaunchKernelGGL(update_kernel, dim3(nsb * nsb, npairs), dim3(kThreads), 0, s, map, p64, pairs, k);
 }
 

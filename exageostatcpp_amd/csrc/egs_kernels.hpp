@@ -54,16 +54,15 @@ void launch_trsm_rows(const TileMap &map, int k, int64_t g0, int count, int jb0,
 // row blocks from g0 on, then count32 FP32 ones.
 void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, int count32, const double *winv_k,
                             hipStream_t s);
-// Trailing update C_ij -= L_ik L_jk^T for the first npairs lower tiles of the
-// update order (all (i, j) with i >= j > k).
-void launch_update(const TileMap &map, const int2 *pairs, int npairs, int k, hipStream_t s);
-// The 64 x 64-block update whatever ts (more, shorter workgroups than the
-// 192 x 192 form: lower latency for a few tiles); p64 as launch_update192_panel
-// when given, else panel k is read from the tiles.
-void launch_update64(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s);
-// 192 x 192-block variant of the update (egs_update.hip), used when ts % 192 == 0.
+// Trailing update C_ij -= L_ik L_jk^T for npairs lower tiles with i >= j > k;
+// p64 (may be null): read panel k from its contiguous FP64 copy (tile i at
+// p64 + (i-k-1) ts^2) instead of from the tiles.  critical: the next panel waits
+// for these tiles.
+void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, bool critical,
+                   hipStream_t s);
+// Its 96 x 192-block form (egs_update.hip), for ts % 192 == 0.
 bool update192_supported(int ts);
-void launch_update192(const TileMap &map, const int2 *pairs, int npairs, int k, hipStream_t s);
+void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s);
 
 // ---- triangular solves and reductions (egs_solve.hip)
 // Forward solve of tile row k: y_k = L_kk^{-1} z_k in place, with per-tile
@@ -164,9 +163,6 @@ void launch_update192_16(const TileMap &map, const uint16_t *p16h, const uint16_
                          const float *bmax, const unsigned *pmax, float tau, const uint8_t *p8, float tau8,
                          const int2 *pairs, int npairs, int k, Operands op, unsigned long long *counts,
                          hipStream_t s);
-// FP64 update reading panel k from a contiguous FP64 copy (tile i at p64 + (i-k-1) ts^2).
-void launch_update192_panel(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k,
-                            hipStream_t s);
 // e = LAPACK dlarnv(3, iseed) N(0,1) values (48-bit LCG stream, Box-Muller).
 void launch_dlarnv_normal(double *e, int64_t n, uint64_t seed48, hipStream_t s);
 // dst = src (n doubles), padding [n, npad) with zeros.
