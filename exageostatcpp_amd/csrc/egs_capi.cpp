@@ -653,8 +653,8 @@ void factor_panel(egs_problem_s *p, int k) {
         if (rows32 > 0 && !p->f32_panel_solve) {
             egs::launch_trsm_rows_mixed(m, k, g64, rows64 * nsb, rows32 * nsb, wk, s);
         } else {
-            if (!fused) egs::launch_trsm_rows(m, k, g64, rows64 * nsb, 0, nsb, wk, s);
-            egs::launch_trsm_rows(m, k, g32, rows32 * nsb, 0, nsb, wk, s, true, p->f32_panel_solve);
+            if (!fused) egs::launch_trsm_rows(m, k, g64, rows64 * nsb, wk, s);
+            egs::launch_trsm_rows(m, k, g32, rows32 * nsb, wk, s, true, p->f32_panel_solve);
         }
         prof_end(p, pi);
         if (is_mixed(p)) {

@@ -23,568 +23,226 @@
 namespace egs {
 
 constexpr int kKc = 32;          // K chunk staged in LDS
-constexpr int kLdsPad = 65;      // LDS row stride (doubles) for 64-wide panels
-constexpr int kStage = kBlk * kKc / kThreads;   // elements of A (and of B) per thread per chunk
+constexpr int kLdsPad = 65;      // LDS row stride for 64-wide panels
 
-struct GemmSmem {
-    double a[2][kKc][kLdsPad];
-    double b[2][kKc][kLdsPad];
+// Staging buffers of the contractions, in the compute type.
+template <typename CT>
+struct Smem {
+    CT a[2][kKc][kLdsPad];
+    CT b[2][kKc][kLdsPad];
+};
+using GemmSmem = Smem<double>;
+
+// The 16 x 16 x 4 MFMA of a compute type: element v of lane l's result holds
+// column col(l / 16, v) of the second operand's 16 and row l % 16 of the first.
+template <typename CT>
+struct Mfma;
+template <>
+struct Mfma<double> {
+    typedef f64x4 vec;
+    static __device__ __forceinline__ vec mul(double b, double a, vec c) { return mfma_f64(b, a, c); }
+    static __device__ __forceinline__ int col(int lk, int v) { return lk + 4 * v; }
+};
+template <>
+struct Mfma<float> {
+    typedef f32x4 vec;
+    static __device__ __forceinline__ vec mul(float b, float a, vec c) { return mfma_f32(b, a, c); }
+    static __device__ __forceinline__ int col(int lk, int v) { return 4 * lk + v; }
 };
 
-// acc[ni][mi][v] holds C[mq*32 + mi*16 + lane%16][nq*32 + ni*16 + lane/16 + 4*v]
-// for wave w = threadIdx.x / 64, mq = w & 1, nq = w >> 1.
-struct Acc64 {
-    f64x4 v[2][2];
+// A kRows x 64 block over the workgroup's four waves: with 64 rows wave w holds
+// the 32 x 32 quadrant (w & 1, w >> 1), with 32 rows columns 16 w .. +15;
+// v[ni][mi] are its 16 x 16 tiles.
+template <typename CT, int kRows>
+struct Acc {
+    static constexpr int kNi = kRows / 32;
+    typename Mfma<CT>::vec v[kNi][2];
+    static __device__ __forceinline__ int row0() { return kRows == 64 ? ((threadIdx.x >> 6) & 1) * 32 : 0; }
+    static __device__ __forceinline__ int col0() {
+        return kRows == 64 ? (threadIdx.x >> 7) * 32 : (threadIdx.x >> 6) * 16;
+    }
 };
+using Acc64 = Acc<double, 64>;
 
-__device__ __forceinline__ void acc_zero(Acc64 &acc) {
+template <typename CT, int kRows>
+__device__ __forceinline__ void acc_zero(Acc<CT, kRows> &acc) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < Acc<CT, kRows>::kNi; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc.v[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-}
-
-// acc += A (64 x K, column-major, lda) * B (64 x K, column-major, ldb)^T.
-// K must be a multiple of kKc.
-template <typename TA>
-__device__ void wg_gemm_nt(Acc64 &acc, const TA *__restrict__ A, int64_t lda, const double *__restrict__ B,
-                           int64_t ldb, int K, GemmSmem &sm) {
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int w = t >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    // element e = t + q * 256 of a 64 x kKc chunk: row e % 64, column e / 64
-    const int srow = t & 63;
-    double ra[kStage], rb[kStage];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) {
-        const int col = (t >> 6) + q * (kThreads / kBlk);
-        ra[q] = (double) A[srow + (int64_t) col * lda];
-        rb[q] = B[srow + (int64_t) col * ldb];
-    }
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) {
-        const int col = (t >> 6) + q * (kThreads / kBlk);
-        sm.a[0][col][srow] = ra[q];
-        sm.b[0][col][srow] = rb[q];
-    }
-    __syncthreads();
-    const int nch = K / kKc;
-    for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        const bool more = c + 1 < nch;
-        if (more) {
-            const int64_t k0 = (int64_t) (c + 1) * kKc;
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int col = (t >> 6) + q * (kThreads / kBlk);
-                ra[q] = (double) A[srow + (k0 + col) * lda];
-                rb[q] = B[srow + (k0 + col) * ldb];
-            }
-        }
-#pragma unroll
-        for (int kk = 0; kk < kKc; kk += 4) {
-            const double a0 = sm.a[buf][kk + lk][mq * 32 + lr];
-            const double a1 = sm.a[buf][kk + lk][mq * 32 + 16 + lr];
-            const double b0 = sm.b[buf][kk + lk][nq * 32 + lr];
-            const double b1 = sm.b[buf][kk + lk][nq * 32 + 16 + lr];
-            acc.v[0][0] = mfma_f64(b0, a0, acc.v[0][0]);
-            acc.v[0][1] = mfma_f64(b0, a1, acc.v[0][1]);
-            acc.v[1][0] = mfma_f64(b1, a0, acc.v[1][0]);
-            acc.v[1][1] = mfma_f64(b1, a1, acc.v[1][1]);
-        }
-        if (more) {
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int col = (t >> 6) + q * (kThreads / kBlk);
-                sm.a[buf ^ 1][col][srow] = ra[q];
-                sm.b[buf ^ 1][col][srow] = rb[q];
-            }
-        }
-        __syncthreads();
-    }
+        for (int j = 0; j < 2; ++j) acc.v[i][j] = typename Mfma<CT>::vec{0, 0, 0, 0};
 }
 
 // Visit every (row, col, value) of the accumulator.
-template <typename F>
-__device__ __forceinline__ void acc_foreach(const Acc64 &acc, F f) {
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
+template <typename CT, int kRows, typename F>
+__device__ __forceinline__ void acc_foreach(const Acc<CT, kRows> &acc, F f) {
+    using A = Acc<CT, kRows>;
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
 #pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = mq * 32 + mi * 16 + (lane & 15);
-                const int c = nq * 32 + ni * 16 + (lane >> 4) + 4 * v;
-                f(r, c, acc.v[ni][mi][v]);
-            }
-}
-
-// ------------------------------------------------------------------------
-// Row-block triangular solve against L_kk, column blocks [jb0, jb1).
-// ------------------------------------------------------------------------
-// 66.5 KB of LDS (sm): T is formed after each GEMM through sm (it reuses
-// sm.a), so that a workgroup fits beside one workgroup of the trailing update.
-template <typename TX>
-__device__ __forceinline__ void trsm_rows_body(const TileMap &map, int k, int64_t g0, int jb0, int jb1,
-                                               const double *winv_k, int bx, GemmSmem &sm) {
-    static_assert(sizeof(GemmSmem::a) >= sizeof(double) * kBlk * kLdsPad, "T must fit in the staging buffer");
-    double (*sT)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.a[0][0][0]);
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    const int64_t g = g0 + bx;
-    const int i = (int) (g / nsb);
-    const int rb = (int) (g % nsb);
-    TX *X = reinterpret_cast<TX *>(map.base + map.off[i * map.nt + k]) + rb * kBlk;
-    const double *L = tile_f64(map, k, k);
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
-
-    for (int jb = jb0; jb < jb1; ++jb) {
-        Acc64 acc;
-        acc_zero(acc);
-        if (jb > 0) wg_gemm_nt(acc, X, ts, L + jb * kBlk, ts, jb * kBlk, sm);
-        TX *Xj = X + (int64_t) jb * kBlk * ts;
-        acc_foreach(acc, [&](int r, int c, double v) { sT[r][c] = (double) Xj[r + (int64_t) c * ts] - v; });
-        __syncthreads();
-        // X_j = T W_j^T :  acc2[r][c] = sum_l T[r][l] W[c][l]
-        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        Acc64 acc2;
-        acc_zero(acc2);
-#pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const double a0 = sT[mq * 32 + lr][kk + lk];
-            const double a1 = sT[mq * 32 + 16 + lr][kk + lk];
-            const double b0 = W[(nq * 32 + lr) + (kk + lk) * kBlk];
-            const double b1 = W[(nq * 32 + 16 + lr) + (kk + lk) * kBlk];
-            acc2.v[0][0] = mfma_f64(b0, a0, acc2.v[0][0]);
-            acc2.v[0][1] = mfma_f64(b0, a1, acc2.v[0][1]);
-            acc2.v[1][0] = mfma_f64(b1, a0, acc2.v[1][0]);
-            acc2.v[1][1] = mfma_f64(b1, a1, acc2.v[1][1]);
-        }
-        acc_foreach(acc2, [&](int r, int c, double v) { Xj[r + (int64_t) c * ts] = (TX) v; });
-        __syncthreads();
-    }
-}
-
-template <typename TX>
-__global__ void __launch_bounds__(kThreads) trsm_rows_kernel(TileMap map, int k, int64_t g0, int jb0, int jb1,
-                                                             const double *winv_k) {
-    __shared__ GemmSmem sm;
-    trsm_rows_body<TX>(map, k, g0, jb0, jb1, winv_k, blockIdx.x, sm);
-}
-
-// ------------------------------------------------------------------------
-// The same solve in 32-row blocks.  A row block's solve is a chain of ts / 64
-// dependent steps bound by its CU's FP64 MFMA rate; in 32-row blocks a short
-// panel (the end of a factorization, small problems) spreads over twice the
-// CUs, each with half the MFMA work (and the same loads of L_kk).
-// ------------------------------------------------------------------------
-namespace {
-constexpr int kHalf = 32;   // rows per block
-
-// acc.v[mi] holds C[mi*16 + lane%16][w*16 + lane/16 + 4*v], w = threadIdx.x / 64.
-struct AccHalf {
-    f64x4 v[2];
-};
-
-__device__ __forceinline__ void acc_zero(AccHalf &acc) {
-    acc.v[0] = f64x4{0.0, 0.0, 0.0, 0.0};
-    acc.v[1] = f64x4{0.0, 0.0, 0.0, 0.0};
-}
-
-template <typename F>
-__device__ __forceinline__ void acc_foreach(const AccHalf &acc, F f) {
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) f(mi * 16 + (lane & 15), w * 16 + (lane >> 4) + 4 * v, acc.v[mi][v]);
-}
-
-// acc += A (32 x K, column-major, lda) * B (64 x K, column-major, ldb)^T,
-// staged like wg_gemm_nt (A in the first 32 rows of sm.a).  K must be a
-// multiple of kKc.
-template <typename TA>
-__device__ void wg_gemm_nt_half(AccHalf &acc, const TA *__restrict__ A, int64_t lda, const double *__restrict__ B,
-                                int64_t ldb, int K, GemmSmem &sm) {
-    constexpr int kStageA = kHalf * kKc / kThreads;   // 4
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int w = t >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    // A chunk element (row t % 32, column t / 32 + 8 q); B chunk element
-    // (row t % 64, column t / 64 + 4 q)
-    const int arow = t & (kHalf - 1), acol = t / kHalf;
-    const int brow = t & 63, bcol = t >> 6;
-    double ra[kStageA], rb[kStage];
-#pragma unroll
-    for (int q = 0; q < kStageA; ++q) ra[q] = (double) A[arow + (int64_t) (acol + q * (kThreads / kHalf)) * lda];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) rb[q] = B[brow + (int64_t) (bcol + q * (kThreads / kBlk)) * ldb];
-#pragma unroll
-    for (int q = 0; q < kStageA; ++q) sm.a[0][acol + q * (kThreads / kHalf)][arow] = ra[q];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) sm.b[0][bcol + q * (kThreads / kBlk)][brow] = rb[q];
-    __syncthreads();
-    const int nch = K / kKc;
-    for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        const bool more = c + 1 < nch;
-        if (more) {
-            const int64_t k0 = (int64_t) (c + 1) * kKc;
-#pragma unroll
-            for (int q = 0; q < kStageA; ++q) ra[q] = (double) A[arow + (k0 + acol + q * (kThreads / kHalf)) * lda];
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) rb[q] = B[brow + (k0 + bcol + q * (kThreads / kBlk)) * ldb];
-        }
-#pragma unroll
-        for (int kk = 0; kk < kKc; kk += 4) {
-            const double a0 = sm.a[buf][kk + lk][lr];
-            const double a1 = sm.a[buf][kk + lk][16 + lr];
-            const double b0 = sm.b[buf][kk + lk][w * 16 + lr];
-            acc.v[0] = mfma_f64(b0, a0, acc.v[0]);
-            acc.v[1] = mfma_f64(b0, a1, acc.v[1]);
-        }
-        if (more) {
-#pragma unroll
-            for (int q = 0; q < kStageA; ++q) sm.a[buf ^ 1][acol + q * (kThreads / kHalf)][arow] = ra[q];
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) sm.b[buf ^ 1][bcol + q * (kThreads / kBlk)][brow] = rb[q];
-        }
-        __syncthreads();
-    }
-}
-}  // namespace
-
-// Row block g0 + bx of 32 rows (ts / 32 per tile row), all column blocks.
-template <typename TX>
-__device__ __forceinline__ void trsm_rows_half_body(const TileMap &map, int k, int64_t g0, const double *winv_k,
-                                                    int bx, GemmSmem &sm) {
-    double (*sT)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.a[0][0][0]);
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    const int nrb = ts / kHalf;
-    const int64_t g = g0 + bx;
-    const int i = (int) (g / nrb);
-    const int rb = (int) (g % nrb);
-    TX *X = reinterpret_cast<TX *>(map.base + map.off[i * map.nt + k]) + rb * kHalf;
-    const double *L = tile_f64(map, k, k);
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-
-    for (int jb = 0; jb < nsb; ++jb) {
-        AccHalf acc;
-        acc_zero(acc);
-        if (jb > 0) wg_gemm_nt_half(acc, X, ts, L + jb * kBlk, ts, jb * kBlk, sm);
-        TX *Xj = X + (int64_t) jb * kBlk * ts;
-        acc_foreach(acc, [&](int r, int c, double v) { sT[r][c] = (double) Xj[r + (int64_t) c * ts] - v; });
-        __syncthreads();
-        // X_j = T W_j^T
-        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        AccHalf acc2;
-        acc_zero(acc2);
-#pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const double a0 = sT[lr][kk + lk];
-            const double a1 = sT[16 + lr][kk + lk];
-            const double b0 = W[(w * 16 + lr) + (kk + lk) * kBlk];
-            acc2.v[0] = mfma_f64(b0, a0, acc2.v[0]);
-            acc2.v[1] = mfma_f64(b0, a1, acc2.v[1]);
-        }
-        acc_foreach(acc2, [&](int r, int c, double v) { Xj[r + (int64_t) c * ts] = (TX) v; });
-        __syncthreads();
-    }
-}
-
-template <typename TX>
-__global__ void __launch_bounds__(kThreads) trsm_rows_half_kernel(TileMap map, int k, int64_t g0,
-                                                                  const double *winv_k) {
-    __shared__ GemmSmem sm;
-    trsm_rows_half_body<TX>(map, k, g0, winv_k, blockIdx.x, sm);
-}
-
-// ------------------------------------------------------------------------
-// The same solve for FP32 panel rows with v_mfma_f32_16x16x4f32 (FP32
-// accumulation; L and W converted to FP32 as they are staged, 50 KB of LDS):
-// 1.8x the rate of the FP64 form, for the univariate kernel's mixed plans
-// (the bivariate field's error grew 3-14x with it).  FP32 result element v of
-// lane l is D[4 (l / 16) + v][l % 16].
-// ------------------------------------------------------------------------
-struct GemmSmem32 {
-    float a[2][kKc][kLdsPad];
-    float b[2][kKc][kLdsPad];
-};
-struct Acc32 {
-    f32x4 v[2][2];
-};
-
-__device__ void wg_gemm_nt_f32(Acc32 &acc, const float *__restrict__ A, int64_t lda, const double *__restrict__ B,
-                               int64_t ldb, int K, GemmSmem32 &sm) {
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int w = t >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    const int srow = t & 63;
-    float ra[kStage], rb[kStage];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) {
-        const int col = (t >> 6) + q * (kThreads / kBlk);
-        ra[q] = A[srow + (int64_t) col * lda];
-        rb[q] = (float) B[srow + (int64_t) col * ldb];
-    }
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) {
-        const int col = (t >> 6) + q * (kThreads / kBlk);
-        sm.a[0][col][srow] = ra[q];
-        sm.b[0][col][srow] = rb[q];
-    }
-    __syncthreads();
-    const int nch = K / kKc;
-    for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        const bool more = c + 1 < nch;
-        if (more) {
-            const int64_t k0 = (int64_t) (c + 1) * kKc;
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int col = (t >> 6) + q * (kThreads / kBlk);
-                ra[q] = A[srow + (k0 + col) * lda];
-                rb[q] = (float) B[srow + (k0 + col) * ldb];
-            }
-        }
-#pragma unroll
-        for (int kk = 0; kk < kKc; kk += 4) {
-            const float a0 = sm.a[buf][kk + lk][mq * 32 + lr];
-            const float a1 = sm.a[buf][kk + lk][mq * 32 + 16 + lr];
-            const float b0 = sm.b[buf][kk + lk][nq * 32 + lr];
-            const float b1 = sm.b[buf][kk + lk][nq * 32 + 16 + lr];
-            acc.v[0][0] = mfma_f32(b0, a0, acc.v[0][0]);
-            acc.v[0][1] = mfma_f32(b0, a1, acc.v[0][1]);
-            acc.v[1][0] = mfma_f32(b1, a0, acc.v[1][0]);
-            acc.v[1][1] = mfma_f32(b1, a1, acc.v[1][1]);
-        }
-        if (more) {
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) {
-                const int col = (t >> 6) + q * (kThreads / kBlk);
-                sm.a[buf ^ 1][col][srow] = ra[q];
-                sm.b[buf ^ 1][col][srow] = rb[q];
-            }
-        }
-        __syncthreads();
-    }
-}
-
-template <typename F>
-__device__ __forceinline__ void acc32_foreach(const Acc32 &acc, F f) {
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni)
+    for (int ni = 0; ni < A::kNi; ++ni)
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = mq * 32 + mi * 16 + (lane & 15);
-                const int c = nq * 32 + ni * 16 + 4 * (lane >> 4) + v;
-                f(r, c, acc.v[ni][mi][v]);
-            }
+            for (int v = 0; v < 4; ++v)
+                f(A::row0() + mi * 16 + lr, A::col0() + ni * 16 + Mfma<CT>::col(lk, v), acc.v[ni][mi][v]);
 }
 
-__global__ void __launch_bounds__(kThreads) trsm_rows_f32mfma_kernel(TileMap map, int k, int64_t g0, int jb0,
-                                                                     int jb1, const double *winv_k) {
-    __shared__ GemmSmem32 sm;
-    __shared__ float sW[kBlk][kLdsPad];
-    static_assert(sizeof(GemmSmem32::a) >= sizeof(float) * kBlk * kLdsPad, "T must fit in the staging buffer");
-    float (*sT)[kLdsPad] = reinterpret_cast<float (*)[kLdsPad]>(&sm.a[0][0][0]);
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    const int64_t g = g0 + blockIdx.x;
-    const int i = (int) (g / nsb);
-    const int rb = (int) (g % nsb);
-    float *X = reinterpret_cast<float *>(map.base + map.off[i * map.nt + k]) + rb * kBlk;
-    const double *L = tile_f64(map, k, k);
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    for (int jb = jb0; jb < jb1; ++jb) {
-        Acc32 acc;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc.v[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (jb > 0) wg_gemm_nt_f32(acc, X, ts, L + jb * kBlk, ts, jb * kBlk, sm);
-        float *Xj = X + (int64_t) jb * kBlk * ts;
-        acc32_foreach(acc, [&](int r, int c, float v) { sT[r][c] = Xj[r + (int64_t) c * ts] - v; });
-        // W_jb (64 x 64 lower inverse, ld 64) as FP32 in LDS: sW[c][l] = W[c][l]
-        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        for (int e = threadIdx.x; e < kBlk * kBlk; e += kThreads) sW[e & 63][e >> 6] = (float) W[e];
-        __syncthreads();
-        Acc32 acc2;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc2.v[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+// acc += the product of K columns of a (rows) and b (columns), element (row,
+// k) at k * kLdsPad + row.
+template <typename CT, int kRows, int K>
+__device__ __forceinline__ void lds_product(Acc<CT, kRows> &acc, const CT *a, const CT *b) {
+    using A = Acc<CT, kRows>;
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
 #pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const float a0 = sT[mq * 32 + lr][kk + lk];
-            const float a1 = sT[mq * 32 + 16 + lr][kk + lk];
-            const float b0 = sW[nq * 32 + lr][kk + lk];
-            const float b1 = sW[nq * 32 + 16 + lr][kk + lk];
-            acc2.v[0][0] = mfma_f32(b0, a0, acc2.v[0][0]);
-            acc2.v[0][1] = mfma_f32(b0, a1, acc2.v[0][1]);
-            acc2.v[1][0] = mfma_f32(b1, a0, acc2.v[1][0]);
-            acc2.v[1][1] = mfma_f32(b1, a1, acc2.v[1][1]);
-        }
-        acc32_foreach(acc2, [&](int r, int c, float v) { Xj[r + (int64_t) c * ts] = v; });
-        __syncthreads();
+    for (int kk = 0; kk < K; kk += 4) {
+        CT x[2], y[A::kNi];
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) x[mi] = a[(kk + lk) * kLdsPad + A::row0() + mi * 16 + lr];
+#pragma unroll
+        for (int ni = 0; ni < A::kNi; ++ni) y[ni] = b[(kk + lk) * kLdsPad + A::col0() + ni * 16 + lr];
+#pragma unroll
+        for (int ni = 0; ni < A::kNi; ++ni)
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi) acc.v[ni][mi] = Mfma<CT>::mul(y[ni], x[mi], acc.v[ni][mi]);
     }
 }
 
-// The FP32-MFMA solve in 32-row blocks (as trsm_rows_half_body): wave w
-// holds rows 0-31 and columns 16 w .. 16 w + 15; acc.v[mi] element v of lane
-// l is C[mi*16 + l%16][16 w + 4 (l/16) + v].
-struct AccHalf32 {
-    f32x4 v[2];
+// acc += A (kRows x K, column-major, lda) * B (64 x K, column-major, ldb)^T; K a
+// multiple of 64.  K chunks of 32 columns go through LDS, double buffered; two
+// chunks' loads are in flight in registers while one is multiplied (these
+// kernels run on few workgroups, so each has to hide its own memory latency).
+// Against one chunk in flight, and with C, B_j and W_j loaded ahead of the
+// products (below): the panel solve of 60 row blocks of 960 columns 268 -> 246
+// us, one evaluation of 1,600 locations 0.85 -> 0.79 ms, of 20,000 55.4 ->
+// 53.8 ms.
+template <typename CT, int kRows, typename TA>
+__device__ void wg_gemm_nt(Acc<CT, kRows> &acc, const TA *__restrict__ A, int64_t lda, const double *__restrict__ B,
+                           int64_t ldb, int K, Smem<CT> &sm) {
+    constexpr int kA = kRows * kKc / kThreads, kB = kBlk * kKc / kThreads;   // elements per thread and chunk
+    const int t = threadIdx.x;
+    const int arow = t % kRows, acol = t / kRows;
+    const int brow = t % kBlk, bcol = t / kBlk;
+    const TA *Ap = A + arow + (int64_t) acol * lda;
+    const double *Bp = B + brow + (int64_t) bcol * ldb;
+    TA ra[2][kA];
+    double rb[2][kB];
+    auto issue = [&](int set, int c) {
+        const int64_t k0 = (int64_t) c * kKc;
+#pragma unroll
+        for (int q = 0; q < kA; ++q) ra[set][q] = Ap[(k0 + q * (kThreads / kRows)) * lda];
+#pragma unroll
+        for (int q = 0; q < kB; ++q) rb[set][q] = Bp[(k0 + q * (kThreads / kBlk)) * ldb];
+    };
+    auto stage = [&](int set) {
+#pragma unroll
+        for (int q = 0; q < kA; ++q) sm.a[set][acol + q * (kThreads / kRows)][arow] = (CT) ra[set][q];
+#pragma unroll
+        for (int q = 0; q < kB; ++q) sm.b[set][bcol + q * (kThreads / kBlk)][brow] = (CT) rb[set][q];
+    };
+    const int nch = K / kKc;   // even
+    issue(0, 0);
+    issue(1, 1);
+    stage(0);
+    __syncthreads();
+    for (int c0 = 0; c0 < nch; c0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int c = c0 + u;
+            if (c + 2 < nch) issue(u, c + 2);
+            lds_product<CT, kRows, kKc>(acc, &sm.a[u][0][0], &sm.b[u][0][0]);
+            if (c + 1 < nch) stage(u ^ 1);
+            __syncthreads();
+        }
+    }
+}
+
+// ------------------------------------------------------------------------
+// Panel solve X L_kk^T = B of kRows rows: marching over the 64-column blocks of
+// L_kk, X_j = (B_j - X_0..j-1 L_j,0..j-1^T) W_j^T with the 64 x 64 inverses W.
+// CT is the compute type (FP32 for FP32 rows of univariate mixed plans: 1.8x
+// the rate; the bivariate field's error grew 3-14x with it).  B_j and W_j are
+// loaded ahead of the product they wait for.  `wait` blocks until row block j
+// of L_kk's earlier columns (row) and W_j (inverse) are there; kAhead: they are
+// from the start.  T goes through the product's LDS (sm), so that a workgroup
+// fits beside the trailing update's.
+// ------------------------------------------------------------------------
+struct NoWait {
+    static constexpr bool kAhead = true;
+    __device__ __forceinline__ void row(int) const {}
+    __device__ __forceinline__ void inverse(int) const {}
 };
 
-__device__ void wg_gemm_nt_f32_half(AccHalf32 &acc, const float *__restrict__ A, int64_t lda,
-                                    const double *__restrict__ B, int64_t ldb, int K, GemmSmem32 &sm) {
-    constexpr int kStageA = kHalf * kKc / kThreads;   // 4
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int w = t >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    const int arow = t & (kHalf - 1), acol = t / kHalf;
-    const int brow = t & 63, bcol = t >> 6;
-    float ra[kStageA], rb[kStage];
-#pragma unroll
-    for (int q = 0; q < kStageA; ++q) ra[q] = A[arow + (int64_t) (acol + q * (kThreads / kHalf)) * lda];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) rb[q] = (float) B[brow + (int64_t) (bcol + q * (kThreads / kBlk)) * ldb];
-#pragma unroll
-    for (int q = 0; q < kStageA; ++q) sm.a[0][acol + q * (kThreads / kHalf)][arow] = ra[q];
-#pragma unroll
-    for (int q = 0; q < kStage; ++q) sm.b[0][bcol + q * (kThreads / kBlk)][brow] = rb[q];
-    __syncthreads();
-    const int nch = K / kKc;
-    for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        const bool more = c + 1 < nch;
-        if (more) {
-            const int64_t k0 = (int64_t) (c + 1) * kKc;
-#pragma unroll
-            for (int q = 0; q < kStageA; ++q) ra[q] = A[arow + (k0 + acol + q * (kThreads / kHalf)) * lda];
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) rb[q] = (float) B[brow + (k0 + bcol + q * (kThreads / kBlk)) * ldb];
-        }
-#pragma unroll
-        for (int kk = 0; kk < kKc; kk += 4) {
-            const float a0 = sm.a[buf][kk + lk][lr];
-            const float a1 = sm.a[buf][kk + lk][16 + lr];
-            const float b0 = sm.b[buf][kk + lk][w * 16 + lr];
-            acc.v[0] = mfma_f32(b0, a0, acc.v[0]);
-            acc.v[1] = mfma_f32(b0, a1, acc.v[1]);
-        }
-        if (more) {
-#pragma unroll
-            for (int q = 0; q < kStageA; ++q) sm.a[buf ^ 1][acol + q * (kThreads / kHalf)][arow] = ra[q];
-#pragma unroll
-            for (int q = 0; q < kStage; ++q) sm.b[buf ^ 1][bcol + q * (kThreads / kBlk)][brow] = rb[q];
-        }
-        __syncthreads();
-    }
-}
-
-template <typename F>
-__device__ __forceinline__ void acc32_foreach(const AccHalf32 &acc, F f) {
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) f(mi * 16 + (lane & 15), w * 16 + 4 * (lane >> 4) + v, acc.v[mi][v]);
-}
-
-// g0 in 32-row blocks; all column blocks.
-__global__ void __launch_bounds__(kThreads) trsm_rows_f32mfma_half_kernel(TileMap map, int k, int64_t g0,
-                                                                          const double *winv_k) {
-    __shared__ GemmSmem32 sm;
-    __shared__ float sW[kBlk][kLdsPad];
-    float (*sT)[kLdsPad] = reinterpret_cast<float (*)[kLdsPad]>(&sm.a[0][0][0]);
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    const int nrb = ts / kHalf;
-    const int64_t g = g0 + blockIdx.x;
-    const int i = (int) (g / nrb);
-    const int rb = (int) (g % nrb);
-    float *X = reinterpret_cast<float *>(map.base + map.off[i * map.nt + k]) + rb * kHalf;
-    const double *L = tile_f64(map, k, k);
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
+template <typename CT, int kRows, typename TX, typename Wait>
+__device__ __forceinline__ void solve_rows(const double *T, int ts, int nsb, TX *X, const double *winv_k, Smem<CT> &sm,
+                                           const Wait &wait) {
+    using A = Acc<CT, kRows>;
+    const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
+    CT *sT = &sm.a[0][0][0], *sW = &sm.b[0][0][0];
     for (int jb = 0; jb < nsb; ++jb) {
-        AccHalf32 acc;
-        acc.v[0] = f32x4{0.f, 0.f, 0.f, 0.f};
-        acc.v[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (jb > 0) wg_gemm_nt_f32_half(acc, X, ts, L + jb * kBlk, ts, jb * kBlk, sm);
-        float *Xj = X + (int64_t) jb * kBlk * ts;
-        acc32_foreach(acc, [&](int r, int c, float v) { sT[r][c] = Xj[r + (int64_t) c * ts] - v; });
+        TX *Xj = X + (int64_t) jb * kBlk * ts;
         const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        for (int e = threadIdx.x; e < kBlk * kBlk; e += kThreads) sW[e & 63][e >> 6] = (float) W[e];
-        __syncthreads();
-        AccHalf32 acc2;
-        acc2.v[0] = f32x4{0.f, 0.f, 0.f, 0.f};
-        acc2.v[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const float a0 = sT[lr][kk + lk];
-            const float a1 = sT[16 + lr][kk + lk];
-            const float b0 = sW[w * 16 + lr][kk + lk];
-            acc2.v[0] = mfma_f32(b0, a0, acc2.v[0]);
-            acc2.v[1] = mfma_f32(b0, a1, acc2.v[1]);
+        double wv[16];
+        TX xv[A::kNi * 8];
+        int e = 0;
+        A acc;
+        acc_zero(acc);
+        acc_foreach(acc, [&](int r, int c, CT) { xv[e++] = Xj[r + (int64_t) c * ts]; });
+        if (Wait::kAhead)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) wv[q] = W[row + (w + 4 * q) * kBlk];
+        if (jb > 0) {
+            wait.row(jb);
+            wg_gemm_nt<CT, kRows>(acc, X, ts, T + jb * kBlk, ts, jb * kBlk, sm);
         }
-        acc32_foreach(acc2, [&](int r, int c, float v) { Xj[r + (int64_t) c * ts] = v; });
+        e = 0;
+        acc_foreach(acc, [&](int r, int c, CT v) { sT[c * kLdsPad + r] = (CT) xv[e++] - v; });
+        if (!Wait::kAhead) {
+            wait.inverse(jb);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) wv[q] = W[row + (w + 4 * q) * kBlk];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) sW[(w + 4 * q) * kLdsPad + row] = (CT) wv[q];
+        __syncthreads();
+        acc_zero(acc);
+        lds_product<CT, kRows, kBlk>(acc, sT, sW);
+        acc_foreach(acc, [&](int r, int c, CT v) { Xj[r + (int64_t) c * ts] = (TX) v; });
         __syncthreads();
     }
+}
+
+// Row block g of kRows rows of the tile column's panel.
+template <typename CT, int kRows, typename TX>
+__device__ __forceinline__ void solve_row_block(const TileMap &map, int k, int64_t g, const double *winv_k,
+                                                Smem<CT> &sm) {
+    const int per = map.ts / kRows;
+    TX *X = reinterpret_cast<TX *>(map.base + map.off[(g / per) * map.nt + k]) + (g % per) * kRows;
+    solve_rows<CT, kRows>(tile_f64(map, k, k), map.ts, map.ts / kBlk, X, winv_k, sm, NoWait());
+}
+
+// Row blocks of kRows rows from g0 on, one workgroup each.  A row block's solve
+// is a chain of ts / 64 dependent steps bound by its CU's MFMA rate; in 32-row
+// blocks a short panel spreads over twice the CUs, each with half the MFMA work
+// (and the same loads of L_kk).
+template <typename CT, int kRows, typename TX>
+__global__ void __launch_bounds__(kThreads) trsm_rows_kernel(TileMap map, int k, int64_t g0, const double *winv_k) {
+    __shared__ Smem<CT> sm;
+    solve_row_block<CT, kRows, TX>(map, k, g0 + blockIdx.x, winv_k, sm);
 }
 
 // FP64 rows [g0, g0 + count64) and FP32 rows after them in one launch, both
 // on FP64 MFMA, so that the two panel solves of a mixed plan run side by side
 // rather than one after the other (each is a chain of ts / 64 dependent steps
 // per workgroup).  Plans whose FP32 rows are solved on FP32 MFMA keep two
-// launches: that kernel's lighter workgroups (50 KB of LDS) would otherwise
+// launches: that kernel's lighter workgroups (33 KB of LDS) would otherwise
 // carry the FP64 body's LDS and registers.
+template <int kRows>
 __global__ void __launch_bounds__(kThreads) trsm_rows_mixed_kernel(TileMap map, int k, int64_t g0, int count64,
                                                                    const double *winv_k) {
     __shared__ GemmSmem sm;
-    const int nsb = map.ts / kBlk;
     if ((int) blockIdx.x < count64)
-        trsm_rows_body<double>(map, k, g0, 0, nsb, winv_k, blockIdx.x, sm);
+        solve_row_block<double, kRows, double>(map, k, g0 + blockIdx.x, winv_k, sm);
     else
-        trsm_rows_body<float>(map, k, g0, 0, nsb, winv_k, blockIdx.x, sm);
-}
-
-// The same in 32-row blocks (g0 and count64 in 32-row blocks).
-__global__ void __launch_bounds__(kThreads) trsm_rows_half_mixed_kernel(TileMap map, int k, int64_t g0, int count64,
-                                                                        const double *winv_k) {
-    __shared__ GemmSmem sm;
-    if ((int) blockIdx.x < count64)
-        trsm_rows_half_body<double>(map, k, g0, winv_k, blockIdx.x, sm);
-    else
-        trsm_rows_half_body<float>(map, k, g0, winv_k, blockIdx.x, sm);
+        solve_row_block<double, kRows, float>(map, k, g0 + blockIdx.x, winv_k, sm);
 }
 
 // ------------------------------------------------------------------------
@@ -605,13 +263,13 @@ __device__ __forceinline__ void update_body(const TileMap &map, const double *p6
     const int64_t tt = (int64_t) ts * ts;
     const double *A = (p64 ? p64 + (ij.x - k - 1) * tt : tile_f64(map, ij.x, k)) + sbm * kBlk;
     const double *B = (p64 ? p64 + (ij.y - k - 1) * tt : tile_f64(map, ij.y, k)) + sbn * kBlk;
+    // C's 16 values are loaded ahead of the product, whose loads follow in flight
     Acc64 acc;
     acc_zero(acc);
-    wg_gemm_nt(acc, A, ts, B, ts, ts, sm);
-    // read all 16 values of C first: one memory round trip for the read-modify-write
     double cv[16];
     int q = 0;
     acc_foreach(acc, [&](int r, int c, double) { cv[q++] = C[r + (int64_t) c * ts]; });
+    wg_gemm_nt(acc, A, ts, B, ts, ts, sm);
     q = 0;
     acc_foreach(acc, [&](int r, int c, double v) { C[r + (int64_t) c * ts] = cv[q++] - v; });
 }
@@ -625,36 +283,26 @@ __global__ void __launch_bounds__(kThreads) update_kernel(TileMap map, const dou
 // as often per flop).
 constexpr int kHalfRowsBelow = 256;
 
-void launch_trsm_rows(const TileMap &map, int k, int64_t g0, int count, int jb0, int jb1, const double *winv_k,
-                      hipStream_t s, bool x_f32, bool f32mfma) {
-    if (count <= 0 || jb1 <= jb0) return;
-    const bool halves = count < kHalfRowsBelow && jb0 == 0 && jb1 == map.ts / kBlk;
-    if (halves && x_f32 && f32mfma)
-        hipLaunchKernelGGL(trsm_rows_f32mfma_half_kernel, dim3(2 * count), dim3(kThreads), 0, s, map, k, 2 * g0,
-                           winv_k);
-    else if (x_f32 && f32mfma)
-        hipLaunchKernelGGL(trsm_rows_f32mfma_kernel, dim3(count), dim3(kThreads), 0, s, map, k, g0, jb0, jb1, winv_k);
-    else if (halves && x_f32)
-        hipLaunchKernelGGL(trsm_rows_half_kernel<float>, dim3(2 * count), dim3(kThreads), 0, s, map, k, 2 * g0,
-                           winv_k);
-    else if (halves)
-        hipLaunchKernelGGL(trsm_rows_half_kernel<double>, dim3(2 * count), dim3(kThreads), 0, s, map, k, 2 * g0,
-                           winv_k);
-    else if (x_f32)
-        hipLaunchKernelGGL(trsm_rows_kernel<float>, dim3(count), dim3(kThreads), 0, s, map, k, g0, jb0, jb1, winv_k);
-    else
-        hipLaunchKernelGGL(trsm_rows_kernel<double>, dim3(count), dim3(kThreads), 0, s, map, k, g0, jb0, jb1, winv_k);
+void launch_trsm_rows(const TileMap &map, int k, int64_t g0, int count, const double *winv_k, hipStream_t s, bool x_f32,
+                      bool f32mfma) {
+    if (count <= 0) return;
+    using Kernel = void (*)(TileMap, int, int64_t, const double *);
+    static const Kernel kernels[3][2] = {
+        {trsm_rows_kernel<double, 64, double>, trsm_rows_kernel<double, 32, double>},
+        {trsm_rows_kernel<double, 64, float>, trsm_rows_kernel<double, 32, float>},
+        {trsm_rows_kernel<float, 64, float>, trsm_rows_kernel<float, 32, float>}};
+    const int half = count < kHalfRowsBelow;
+    hipLaunchKernelGGL(kernels[x_f32 ? (f32mfma ? 2 : 1) : 0][half], dim3((unsigned) (count << half)), dim3(kThreads),
+                       0, s, map, k, g0 << half, winv_k);
 }
 
 void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, int count32, const double *winv_k,
                             hipStream_t s) {
     if (count64 + count32 <= 0) return;
-    if (count64 + count32 < kHalfRowsBelow)
-        hipLaunchKernelGGL(trsm_rows_half_mixed_kernel, dim3((unsigned) (2 * (count64 + count32))), dim3(kThreads), 0,
-                           s, map, k, 2 * g0, 2 * count64, winv_k);
-    else
-        hipLaunchKernelGGL(trsm_rows_mixed_kernel, dim3((unsigned) (count64 + count32)), dim3(kThreads), 0, s, map, k,
-                           g0, count64, winv_k);
+    const int half = count64 + count32 < kHalfRowsBelow;
+    hipLaunchKernelGGL(half ? trsm_rows_mixed_kernel<32> : trsm_rows_mixed_kernel<64>,
+                       dim3((unsigned) ((count64 + count32) << half)), dim3(kThreads), 0, s, map, k, g0 << half,
+                       count64 << half, winv_k);
 }
 
 // Up to this many 64 x 64 blocks (three per CU) are updated one workgroup each:
@@ -687,48 +335,19 @@ void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int
 // ------------------------------------------------------------------------
 __global__ void __launch_bounds__(kThreads) tinv_kernel(TileMap map, const double *winv, double *tinv) {
     __shared__ GemmSmem sm;
-    __shared__ double sT[kBlk][kLdsPad];
     const int ts = map.ts;
     const int nsb = ts / kBlk;
     const int rb = blockIdx.x, k = blockIdx.y;
     double *X = tinv + (int64_t) k * ts * ts + rb * kBlk;
-    const double *L = tile_f64(map, k, k);
-    const double *winv_k = winv + (int64_t) k * nsb * kBlk * kBlk;
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
     for (int e = threadIdx.x; e < kBlk * ts; e += kThreads) {
         const int r = e & 63, c = e >> 6;
         X[r + (int64_t) c * ts] = (c == rb * kBlk + r) ? 1.0 : 0.0;
     }
     __syncthreads();
-    for (int jb = rb; jb < nsb; ++jb) {
-        Acc64 acc;
-        acc_zero(acc);
-        if (jb > rb)
-            wg_gemm_nt(acc, X + (int64_t) rb * kBlk * ts, ts, L + jb * kBlk + (int64_t) rb * kBlk * ts, ts,
-                       (jb - rb) * kBlk, sm);
-        double *Xj = X + (int64_t) jb * kBlk * ts;
-        acc_foreach(acc, [&](int r, int c, double v) { sT[r][c] = Xj[r + (int64_t) c * ts] - v; });
-        __syncthreads();
-        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        Acc64 acc2;
-        acc_zero(acc2);
-#pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const double a0 = sT[mq * 32 + lr][kk + lk];
-            const double a1 = sT[mq * 32 + 16 + lr][kk + lk];
-            const double b0 = W[(nq * 32 + lr) + (kk + lk) * kBlk];
-            const double b1 = W[(nq * 32 + 16 + lr) + (kk + lk) * kBlk];
-            acc2.v[0][0] = mfma_f64(b0, a0, acc2.v[0][0]);
-            acc2.v[0][1] = mfma_f64(b0, a1, acc2.v[0][1]);
-            acc2.v[1][0] = mfma_f64(b1, a0, acc2.v[1][0]);
-            acc2.v[1][1] = mfma_f64(b1, a1, acc2.v[1][1]);
-        }
-        acc_foreach(acc2, [&](int r, int c, double v) { Xj[r + (int64_t) c * ts] = v; });
-        __syncthreads();
-    }
+    // from block column rb on: the solve of the tile's trailing part
+    const int64_t skip = (int64_t) rb * kBlk;
+    solve_rows<double, 64>(tile_f64(map, k, k) + skip + skip * ts, ts, nsb - rb, X + skip * ts,
+                           winv + ((int64_t) k * nsb + rb) * kBlk * kBlk, sm, NoWait());
 }
 
 void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream_t s) {
@@ -762,6 +381,7 @@ void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream
 // block from LDS to LDS.  The form before (the block over four waves, one LDS
 // exchange and one barrier per column) took 26 us.
 // ------------------------------------------------------------------------
+constexpr int kHalf = 32;         // rows of a panel block solved beside the diagonal tile
 constexpr int kPan = 16;
 constexpr int kPv = kLdsPad;
 
@@ -971,22 +591,13 @@ __device__ __forceinline__ void put_block(double *s, const double (&v)[16]) {
     for (int q = 0; q < 16; ++q) s[(w + 4 * q) * kPv + row] = v[q];
 }
 
-// acc += A B^T, or acc -= A B^T, for 64 x 64 operands in LDS.
-template <bool kSubtract>
-__device__ __forceinline__ void mma_block(Acc64 &acc, const double *a, const double *b) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int mq = w & 1, nq = w >> 1;
-    const int lr = lane & 15, lk = lane >> 4;
+// acc -= A B^T for 64 x 64 operands in LDS.
+__device__ __forceinline__ void subtract_block(Acc64 &acc, const double *a, const double *b) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
 #pragma unroll 4
     for (int kk = 0; kk < kBlk; kk += 4) {
-        double a0 = a[(kk + lk) * kPv + mq * 32 + lr];
-        double a1 = a[(kk + lk) * kPv + mq * 32 + 16 + lr];
-        if (kSubtract) {
-            a0 = -a0;
-            a1 = -a1;
-        }
-        const double b0 = b[(kk + lk) * kPv + nq * 32 + lr];
-        const double b1 = b[(kk + lk) * kPv + nq * 32 + 16 + lr];
+        const double *x = a + (kk + lk) * kPv + Acc64::row0() + lr, *y = b + (kk + lk) * kPv + Acc64::col0() + lr;
+        const double a0 = -x[0], a1 = -x[16], b0 = y[0], b1 = y[16];
         acc.v[0][0] = mfma_f64(b0, a0, acc.v[0][0]);
         acc.v[0][1] = mfma_f64(b0, a1, acc.v[0][1]);
         acc.v[1][0] = mfma_f64(b1, a0, acc.v[1][0]);
@@ -1025,8 +636,8 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
         put_block(sm.a, va);
         put_block(sm.b, vb);
         __syncthreads();
-        mma_block<true>(acc, sm.a, sm.b);
-        if (acc_d) mma_block<true>(*acc_d, sm.a, sm.a);
+        subtract_block(acc, sm.a, sm.b);
+        if (acc_d) subtract_block(*acc_d, sm.a, sm.a);
         __syncthreads();
     }
     acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
@@ -1035,7 +646,7 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
     put_block(sm.b, vb);
     __syncthreads();
     acc_zero(acc);
-    mma_block<false>(acc, sm.a, sm.b);
+    lds_product<double, 64, kBlk>(acc, sm.a, sm.b);
     __syncthreads();
     acc_foreach(acc, [&](int i, int j, double v) {
         X[i + (int64_t) j * ts] = v;
@@ -1043,7 +654,7 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
     });
     if (acc_d) {
         __syncthreads();
-        mma_block<true>(*acc_d, sm.a, sm.a);
+        subtract_block(*acc_d, sm.a, sm.a);
     }
     publish_block(flags + r * nsb + c);
 }
@@ -1071,39 +682,15 @@ __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r,
     publish_block(flags + r * nsb + r);
 }
 
-// 32 rows X of the panel below the tile, all block columns.
-__device__ __forceinline__ void rows_task(const double *T, int ts, int nsb, double *X, const double *winv_k,
-                                          const int *flags, GemmSmem &sm) {
-    double (*sT)[kLdsPad] = reinterpret_cast<double (*)[kLdsPad]>(&sm.a[0][0][0]);
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    for (int jb = 0; jb < nsb; ++jb) {
-        AccHalf acc;
-        acc_zero(acc);
-        if (jb > 0) {
-            // the diagonal task has waited for the row's earlier blocks
-            wait_block(flags + jb * nsb + jb - 1);
-            wg_gemm_nt_half(acc, X, ts, T + jb * kBlk, ts, jb * kBlk, sm);
-        }
-        double *Xj = X + (int64_t) jb * kBlk * ts;
-        acc_foreach(acc, [&](int r, int c, double v) { sT[r][c] = Xj[r + (int64_t) c * ts] - v; });
-        wait_block(flags + jb * nsb + jb);
-        const double *W = winv_k + (int64_t) jb * kBlk * kBlk;
-        AccHalf acc2;
-        acc_zero(acc2);
-#pragma unroll 4
-        for (int kk = 0; kk < kBlk; kk += 4) {
-            const double a0 = sT[lr][kk + lk];
-            const double a1 = sT[16 + lr][kk + lk];
-            const double b0 = W[(w * 16 + lr) + (kk + lk) * kBlk];
-            acc2.v[0] = mfma_f64(b0, a0, acc2.v[0]);
-            acc2.v[1] = mfma_f64(b0, a1, acc2.v[1]);
-        }
-        acc_foreach(acc2, [&](int r, int c, double v) { Xj[r + (int64_t) c * ts] = v; });
-        __syncthreads();
-    }
-}
+// What a row block below the tile waits for (the diagonal task of block column
+// j has itself waited for the row's earlier blocks).
+struct BlockWait {
+    static constexpr bool kAhead = false;
+    const int *flags;
+    int nsb;
+    __device__ __forceinline__ void row(int j) const { wait_block(flags + j * nsb + j - 1); }
+    __device__ __forceinline__ void inverse(int j) const { wait_block(flags + j * nsb + j); }
+};
 
 // Tasks of the diagonal tile, and the task of a ticket: r < 0 for rows.
 __host__ __device__ inline int tile_tasks(int nsb) { return nsb + (nsb - 1) * (nsb - 2) / 2; }
@@ -1122,7 +709,7 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
         if (h >= halves) return;
         const int per = ts / kHalf;
         double *X = tile_f64(map, k + 1 + h / per, k) + (h % per) * kHalf;
-        rows_task(T, ts, nsb, X, winv_k, flags, *reinterpret_cast<GemmSmem *>(&sm));
+        solve_rows<double, kHalf>(T, ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm), BlockWait{flags, nsb});
         return;
     }
     // block column c holds the diagonal task and nsb - 2 - c others
@@ -1164,20 +751,13 @@ __global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const Batch
     tile_column_task(J.map, J.k, J.winv_k, J.sync, J.info, J.n, halves, t / njobs, sm);
 }
 
+template <int kRows>
 __global__ void __launch_bounds__(kThreads) trsm_rows_batch_kernel(const BatchJob *jobs) {
     const BatchJob &J = jobs[blockIdx.y];
-    const int nsb = J.map.ts / kBlk;
-    if ((int) blockIdx.x >= (J.map.nt - J.k - 1) * nsb) return;
+    const int per = J.map.ts / kRows;
+    if ((int) blockIdx.x >= (J.map.nt - J.k - 1) * per) return;
     __shared__ GemmSmem sm;
-    trsm_rows_body<double>(J.map, J.k, (int64_t) (J.k + 1) * nsb, 0, nsb, J.winv_k, blockIdx.x, sm);
-}
-
-__global__ void __launch_bounds__(kThreads) trsm_rows_half_batch_kernel(const BatchJob *jobs) {
-    const BatchJob &J = jobs[blockIdx.y];
-    const int nrb = J.map.ts / kHalf;
-    if ((int) blockIdx.x >= (J.map.nt - J.k - 1) * nrb) return;
-    __shared__ GemmSmem sm;
-    trsm_rows_half_body<double>(J.map, J.k, (int64_t) (J.k + 1) * nrb, J.winv_k, blockIdx.x, sm);
+    solve_row_block<double, kRows, double>(J.map, J.k, (int64_t) (J.k + 1) * per + blockIdx.x, J.winv_k, sm);
 }
 
 __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *jobs) {
@@ -1201,11 +781,11 @@ void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nr
     hipLaunchKernelGGL(tile_column_batch_kernel, dim3((unsigned) (tasks * njobs)), dim3(kThreads), 0, s, jobs, njobs,
                        fused ? 1 : 0);
     if (rest <= 0 || nrest <= 0) return;
-    if (!fused && rest * nsb * nrest < kHalfRowsBelow)
-        hipLaunchKernelGGL(trsm_rows_half_batch_kernel, dim3((unsigned) (2 * rest * nsb), nrest), dim3(kThreads), 0, s,
-                           jobs);
-    else if (!fused)
-        hipLaunchKernelGGL(trsm_rows_batch_kernel, dim3((unsigned) (rest * nsb), nrest), dim3(kThreads), 0, s, jobs);
+    if (!fused) {
+        const int half = rest * nsb * nrest < kHalfRowsBelow;
+        hipLaunchKernelGGL(half ? trsm_rows_batch_kernel<32> : trsm_rows_batch_kernel<64>,
+                           dim3((unsigned) ((rest * nsb) << half), nrest), dim3(kThreads), 0, s, jobs);
+    }
     hipLaunchKernelGGL(update_batch_kernel, dim3((unsigned) (nsb * nsb), (unsigned) (rest * (rest + 1) / 2), nrest),
                        dim3(kThreads), 0, s, jobs);
 }

@@ -46,10 +46,9 @@ void launch_covgen_rect(double *out, int rows, int cols, int64_t row_off, int64_
 
 // ---- tiled Cholesky (egs_chol.hip)
 // Triangular solve X L_kk^T = B for row blocks [g0, g0 + count) of tile column k
-// (global 64-row block g lives in tile g / nsb at row (g % nsb) * 64), column
-// blocks [jb0, jb1).
-void launch_trsm_rows(const TileMap &map, int k, int64_t g0, int count, int jb0, int jb1, const double *winv_k,
-                      hipStream_t s, bool x_f32 = false, bool f32mfma = false);
+// (global 64-row block g lives in tile g / nsb at row (g % nsb) * 64).
+void launch_trsm_rows(const TileMap &map, int k, int64_t g0, int count, const double *winv_k, hipStream_t s,
+                      bool x_f32 = false, bool f32mfma = false);
 // Both panel solves of a mixed plan in one launch on FP64 MFMA: count64 FP64
 // row blocks from g0 on, then count32 FP32 ones.
 void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, int count32, const double *winv_k,
