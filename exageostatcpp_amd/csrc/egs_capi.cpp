@@ -163,9 +163,6 @@ struct egs_problem_s {
     // generation of a mixed plan (the refinement's Sigma v reads it), and the
     // per-tile partials of that product; null when the copy does not fit
     double *d_sig64 = nullptr, *d_prow = nullptr, *d_pcol = nullptr;
-    // inverses X_k = L_kk^{-T} of the diagonal tiles (preconditioner solves)
-    // and the solve's output vector
-    double *d_tinv = nullptr, *d_ybuf = nullptr;
     double *d_mv = nullptr;                  // matrix-vector chunk partials
     double *d_dot = nullptr;                 // dot-product block partials
     double *d_pred = nullptr;                // prediction targets and outputs, pred_cap doubles
@@ -338,12 +335,6 @@ void free_sigma_copy(egs_problem_s *p) {
     p->d_sig64 = p->d_prow = p->d_pcol = nullptr;
 }
 
-void free_tile_inverses(egs_problem_s *p) {
-    pfree(p, p->d_tinv);
-    pfree(p, p->d_ybuf);
-    p->d_tinv = p->d_ybuf = nullptr;
-}
-
 // Drop the captured evaluation graph (the launch sequence it recorded no
 // longer matches the problem's plan or buffers).
 void invalidate_graph(egs_problem_s *p) {
@@ -408,7 +399,6 @@ void free_problem_buffers(egs_problem_s *p) {
     p->d_pred = nullptr;
     p->pred_cap = 0;
     free_sigma_copy(p);
-    free_tile_inverses(p);
     for (auto &e : p->ev)
         if (e) hipEventDestroy(e);
     for (auto &e : p->prof.ev)
@@ -541,13 +531,6 @@ int setup_mixed(egs_problem_s *p) {
             pmalloc(p, &p->d_mv, sizeof(double) * (size_t) egs::matvec_chunks(p->n) * p->npad) != hipSuccess ||
             pmalloc(p, &p->d_dot, sizeof(double) * egs::dot_blocks()) != hipSuccess)
             return fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the mixed-precision work buffers");
-    }
-    if (!p->d_tinv) {
-        if (pmalloc(p, &p->d_tinv, sizeof(double) * (size_t) p->nt * p->ts * p->ts) != hipSuccess ||
-            pmalloc(p, &p->d_ybuf, sizeof(double) * (size_t) p->npad) != hipSuccess) {
-            free_tile_inverses(p);
-            return fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the diagonal-tile inverses");
-        }
     }
     if (!p->d_sig64) {
         // Optional: without it Sigma v regenerates the covariance on the fly.
@@ -792,7 +775,6 @@ int run_potrf(egs_problem_s *p) {
         EGS_HIP(hipEventRecord(p->ev_bulk[nt - 1], b));
         EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[nt - 1], 0));
     }
-    if (is_mixed(p)) egs::launch_tinv(m, p->d_winv, p->d_tinv, s);
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;
 }
@@ -808,70 +790,30 @@ int read_info(egs_problem_s *p) {
     return EGS_SUCCESS;
 }
 
-// Forward solve of d_work in place; per-tile log-det / dot partials go to
-// `partials` (d_partials unless given).
-void run_forward(egs_problem_s *p, double *partials = nullptr) {
+// d_work = L^{-1} src (src null: of d_work itself); the log-det and dot partials
+// of its 64-row blocks go to `partials` (may be null).
+void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partials) {
     hipStream_t s = p->ctx->stream;
-    const egs::TileMap m = p->map();
-    if (!partials) partials = p->d_partials;
     const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
-    for (int k = 0; k < p->nt; ++k) {
-        egs::launch_trsv_diag(m, k, p->winv(k), p->d_work, partials, s);
-        egs::launch_fwd_panel(m, k, p->d_work + (int64_t) k * p->ts, p->d_work, s);
-    }
+    egs::launch_solve_init(p->d_work, src, n, p->npad, p->d_aux, s);
+    egs::launch_forward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, partials, s);
     prof_end(p, pi);
 }
 
-void run_backward(egs_problem_s *p) {
+// d_work = L^{-T} src, likewise.
+void run_backward(egs_problem_s *p, const double *src, int64_t n) {
     hipStream_t s = p->ctx->stream;
-    const egs::TileMap m = p->map();
-    for (int k = p->nt - 1; k >= 0; --k) {
-        egs::launch_trsv_t_partial(m, k, p->d_work, p->d_aux, s);
-        egs::launch_trsv_t_diag(m, k, p->winv(k), p->d_work, p->d_aux, s);
-    }
-}
-
-// Preconditioner solves of mixed plans with the diagonal-tile inverses:
-// d_ybuf = L^{-1} d_work (d_work is consumed), then d_ybuf = L^{-T} d_work.
-void run_forward_inv(egs_problem_s *p) {
-    hipStream_t s = p->ctx->stream;
-    const egs::TileMap m = p->map();
-    const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
-    for (int k = 0; k < p->nt; ++k) {
-        const int64_t o = (int64_t) k * p->ts;
-        egs::launch_fwd_diag_inv(p->d_tinv + o * p->ts, p->d_work + o, p->d_ybuf + o, p->ts, s);
-        egs::launch_fwd_panel(m, k, p->d_ybuf + o, p->d_work, s);
-    }
-    prof_end(p, pi);
-}
-
-void run_backward_inv(egs_problem_s *p) {
-    hipStream_t s = p->ctx->stream;
-    const egs::TileMap m = p->map();
-    const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
-    for (int k = p->nt - 1; k >= 0; --k) {
-        const int64_t o = (int64_t) k * p->ts;
-        egs::launch_bwd_diag_inv(p->d_tinv + o * p->ts, p->d_work + o, p->d_ybuf + o, p->ts, s);
-        egs::launch_bwd_row(m, k, p->d_ybuf + o, p->d_work, s);
-    }
+    const int pi = is_mixed(p) ? prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n) : -1;
+    egs::launch_solve_init(p->d_work, src, n, p->npad, p->d_aux, s);
+    egs::launch_backward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, s);
     prof_end(p, pi);
 }
 
 // out = (L L^T)^{-1} in with the current factor (both vectors npad long).
 void apply_factor_inverse(egs_problem_s *p, const double *in, double *out) {
-    hipStream_t s = p->ctx->stream;
-    const size_t bytes = sizeof(double) * (size_t) p->npad;
-    hipMemcpyAsync(p->d_work, in, bytes, hipMemcpyDeviceToDevice, s);
-    if (p->d_tinv) {
-        run_forward_inv(p);
-        hipMemcpyAsync(p->d_work, p->d_ybuf, bytes, hipMemcpyDeviceToDevice, s);
-        run_backward_inv(p);
-        hipMemcpyAsync(out, p->d_ybuf, bytes, hipMemcpyDeviceToDevice, s);
-        return;
-    }
-    run_forward(p, p->d_mv);   // partials of a preconditioner solve are not needed
-    run_backward(p);
-    hipMemcpyAsync(out, p->d_work, bytes, hipMemcpyDeviceToDevice, s);
+    run_forward(p, in, p->npad, nullptr);
+    run_backward(p, nullptr, 0);
+    hipMemcpyAsync(out, p->d_work, sizeof(double) * (size_t) p->npad, hipMemcpyDeviceToDevice, p->ctx->stream);
 }
 
 int host_dot(egs_problem_s *p, const double *x, const double *y, double &out) {
@@ -968,12 +910,13 @@ int refine_solve(egs_problem_s *p, const double *b) {
 }
 
 int read_partials(egs_problem_s *p, double &logdet, double &quad) {
-    p->h_partials.resize((size_t) 2 * p->nt);
-    EGS_HIP(hipMemcpy(p->h_partials.data(), p->d_partials, sizeof(double) * 2 * p->nt, hipMemcpyDeviceToHost));
+    const int blocks = p->nt * p->nsb;
+    p->h_partials.resize((size_t) 2 * blocks);
+    EGS_HIP(hipMemcpy(p->h_partials.data(), p->d_partials, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost));
     double ld = 0.0, q = 0.0;
-    for (int k = 0; k < p->nt; ++k) {
-        ld += p->h_partials[2 * k];
-        q += p->h_partials[2 * k + 1];
+    for (int b = 0; b < blocks; ++b) {
+        ld += p->h_partials[2 * b];
+        q += p->h_partials[2 * b + 1];
     }
     logdet = 2.0 * ld;
     quad = q;
@@ -1078,7 +1021,8 @@ int64_t footprint(const egs_problem_s &q) {
     const int64_t nb = (int64_t) sizeof(double) * q.n_loc, vb = (int64_t) sizeof(double) * npad;
     int64_t b = dev_class_bytes(nb) * (q.dim == 3 ? 3 : 2) + dev_class_bytes(8 * nt * nt) + dev_class_bytes(nt * nt) +
                 dev_class_bytes(8 * ntiles) + dev_class_bytes(8 * nt * q.nsb * egs::kBlk * egs::kBlk) +
-                dev_class_bytes(4 * q.sync_ints()) + 3 * dev_class_bytes(vb) + dev_class_bytes(16 * nt) + dev_class_bytes(4) +
+                dev_class_bytes(4 * q.sync_ints()) + 2 * dev_class_bytes(vb) + dev_class_bytes(vb + 8) +
+                dev_class_bytes(16 * nt * q.nsb) + dev_class_bytes(4) +
                 dev_class_bytes(8 * egs::kTabSlots * egs::kTabDoubles);
     int64_t arena = 0;
     for (int j = 0; j < q.nt; ++j)
@@ -1097,7 +1041,6 @@ int64_t footprint(const egs_problem_s &q) {
                         dev_class_bytes(panel) + dev_class_bytes(4 * npad) + dev_class_bytes(4 * (npad / 192)));
     b += dev_class_bytes(4 * nt) + dev_class_bytes(24) + dev_class_bytes(5 * vb) +
          dev_class_bytes(8 * (int64_t) egs::matvec_chunks(q.n) * npad) + dev_class_bytes(8 * egs::dot_blocks());
-    b += dev_class_bytes(8 * nt * ts * ts) + dev_class_bytes(vb);
     b += dev_class_bytes(8 * ntiles * ts * ts) + 2 * dev_class_bytes(8 * ntiles * ts);
     return b;
 }
@@ -1246,8 +1189,8 @@ int egs_problem_create(egs_context_t ctx, int kernel, int64_t n_loc, const doubl
               pmalloc(p, &p->d_winv, sizeof(double) * (size_t) nt * p->nsb * egs::kBlk * egs::kBlk) == hipSuccess &&
               pmalloc(p, &p->d_sync, sizeof(int) * (size_t) p->sync_ints()) == hipSuccess &&
               pmalloc(p, &p->d_obs, vb) == hipSuccess && pmalloc(p, &p->d_work, vb) == hipSuccess &&
-              pmalloc(p, &p->d_aux, vb) == hipSuccess &&
-              pmalloc(p, &p->d_partials, sizeof(double) * 2 * (size_t) nt) == hipSuccess &&
+              pmalloc(p, &p->d_aux, vb + sizeof(double)) == hipSuccess &&
+              pmalloc(p, &p->d_partials, sizeof(double) * 2 * (size_t) nt * p->nsb) == hipSuccess &&
               pmalloc(p, &p->d_info, sizeof(int)) == hipSuccess &&
               pmalloc(p, &p->d_tab, sizeof(double) * egs::kTabSlots * egs::kTabDoubles) == hipSuccess;
     if (!ok) return cleanup(fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the problem's device buffers"));
@@ -1356,10 +1299,7 @@ int egs_problem_set_precision(egs_problem_t p, int mode, int band_fp64, int band
     p->band32 = band_fp32;
     int st2 = layout_tiles(p);
     if (st2) return st2;
-    if (!is_mixed(p)) {
-        free_sigma_copy(p);
-        free_tile_inverses(p);
-    }
+    if (!is_mixed(p)) free_sigma_copy(p);
     return is_mixed(p) ? setup_mixed(p) : EGS_SUCCESS;
 }
 
@@ -1449,9 +1389,8 @@ int egs_solve_logdet_quad(egs_problem_t p, double *logdet, double *quad) {
     if (!p->has_obs) return fail(EGS_ERR_STATE, "the problem has no observations");
     if (!p->factored) return fail(EGS_ERR_STATE, "no factored matrix: call egs_potrf first");
     hipStream_t s = p->ctx->stream;
-    egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
-    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->n, p->d_partials, s);   // quad from the refinement
-    else run_forward(p);
+    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials, s);   // quad from the refinement
+    else run_forward(p, p->d_obs, p->n, p->d_partials);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipStreamSynchronize(s));
     double ld, q;
@@ -1476,9 +1415,8 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
         return fail(EGS_ERR_UNSUPPORTED, "the triangular solve with the stored factor runs under the FP64 plan");
     hipStream_t s = p->ctx->stream;
     EGS_HIP(hipMemcpyAsync(p->d_work, z, sizeof(double) * (size_t) n, hipMemcpyHostToDevice, s));
-    egs::launch_copy_pad(p->d_work, p->d_work, p->n, p->npad, s);
-    if (trans == 0) run_forward(p);
-    else run_backward(p);
+    if (trans == 0) run_forward(p, p->d_work, p->n, nullptr);
+    else run_backward(p, p->d_work, p->n);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipMemcpyAsync(z, p->d_work, sizeof(double) * (size_t) n, hipMemcpyDeviceToHost, s));
     EGS_HIP(hipStreamSynchronize(s));
@@ -1493,7 +1431,6 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
 // capturable (no host synchronization, no memset).
 int enqueue_fp64_eval(egs_problem_s *p) {
     hipStream_t s = p->ctx->stream;
-    egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
     const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
     p->h_prm.kernel = p->kernel;   // the launches are shaped by the kernel and the metric alone
     p->h_prm.metric = p->metric;
@@ -1502,7 +1439,7 @@ int enqueue_fp64_eval(egs_problem_s *p) {
                              p->d_tab, nullptr, s, p->d_prm);
     const int st = run_potrf(p);
     if (st) return st;
-    run_forward(p);
+    run_forward(p, p->d_obs, p->n, p->d_partials);
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;
 }
@@ -1587,15 +1524,14 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
         return EGS_SUCCESS;
     }
     EGS_HIP(hipEventRecord(p->ev[0], s));
-    egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
     st = run_covariance(p, theta);
     if (st) return st;
     EGS_HIP(hipEventRecord(p->ev[1], s));
     st = run_potrf(p);
     if (st) return st;
     EGS_HIP(hipEventRecord(p->ev[2], s));
-    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->n, p->d_partials, s);   // quad from the refinement
-    else run_forward(p);
+    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials, s);   // quad from the refinement
+    else run_forward(p, p->d_obs, p->n, p->d_partials);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipEventRecord(p->ev[3], s));
     EGS_HIP(hipStreamSynchronize(s));
@@ -1684,6 +1620,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             J.info = p->d_info;
             J.n = p->n;
             J.z = p->d_work;
+            J.pending = p->d_aux;
             J.partials = p->d_partials;
         }
     if (na > 0) {
@@ -1704,7 +1641,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
                                hipMemcpyHostToDevice, s));
         for (int b : run) {
             egs_problem_s *p = problems[b];
-            egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
+            egs::launch_solve_init(p->d_work, p->d_obs, p->n, p->npad, p->d_aux, s);
             const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
             egs::launch_matern_tables(p->d_tab, prm[b], nullptr, s);
             egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm[b], p->d_x, p->d_y, dz, p->n,
@@ -1720,8 +1657,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             const egs::BatchJob *J = ctx->d_jobs + first[k];
             egs::launch_step_batch(J, active[k], ts, max_nt - k - 1, active[k + 1], s);
         }
-        for (int k = 0; k < max_nt; ++k)
-            egs::launch_forward_batch(ctx->d_jobs + first[k], active[k], ts, max_nt - k - 1, s);
+        egs::launch_forward_batch(ctx->d_jobs, na, ts, max_nt, s);
         EGS_HIP(hipGetLastError());
         EGS_HIP(hipStreamSynchronize(s));
     }
@@ -2023,9 +1959,8 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
         }
         weights = p->d_cg;
     } else {
-        egs::launch_copy_pad(p->d_work, p->d_obs, p->n, p->npad, s);
-        run_forward(p);
-        run_backward(p);
+        run_forward(p, p->d_obs, p->n, nullptr);
+        run_backward(p, nullptr, 0);
     }
     double *d_out = p->d_pred, *dxm = d_out + rows, *dym = dxm + n_miss, *dzm = dym + n_miss;
     hipError_t e = hipMemcpyAsync(dxm, xm, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);

@@ -327,35 +327,6 @@ void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int
 }
 
 // ------------------------------------------------------------------------
-// Inverses of the diagonal tiles, X_k = L_kk^{-T} (upper triangular,
-// column-major, ts x ts), for the preconditioner solves of mixed plans.
-// Workgroup (rb, k) solves row block rb of X_k L_kk^T = I left-looking over
-// the 64-column blocks jb >= rb (blocks left of rb are zero), with the 64 x 64
-// inverses W of the diagonal blocks of L_kk.
-// ------------------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) tinv_kernel(TileMap map, const double *winv, double *tinv) {
-    __shared__ GemmSmem sm;
-    const int ts = map.ts;
-    const int nsb = ts / kBlk;
-    const int rb = blockIdx.x, k = blockIdx.y;
-    double *X = tinv + (int64_t) k * ts * ts + rb * kBlk;
-    for (int e = threadIdx.x; e < kBlk * ts; e += kThreads) {
-        const int r = e & 63, c = e >> 6;
-        X[r + (int64_t) c * ts] = (c == rb * kBlk + r) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    // from block column rb on: the solve of the tile's trailing part
-    const int64_t skip = (int64_t) rb * kBlk;
-    solve_rows<double, 64>(tile_f64(map, k, k) + skip + skip * ts, ts, nsb - rb, X + skip * ts,
-                           winv + ((int64_t) k * nsb + rb) * kBlk * kBlk, sm, NoWait());
-}
-
-void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream_t s) {
-    const int nsb = map.ts / kBlk;
-    hipLaunchKernelGGL(tinv_kernel, dim3(nsb, map.nt), dim3(kThreads), 0, s, map, winv, tinv);
-}
-
-// ------------------------------------------------------------------------
 // Cholesky and inverse of one 64 x 64 block, held in LDS (row stride kPv
 // doubles).  On entry the lower part of sD is the block A (its upper part is
 // never used) and sE is anything; on return the lower part of sD holds L with

@@ -12,10 +12,10 @@
 namespace egs {
 
 // One problem's share of a batched step (FP64 plan): step k of the tiled
-// Cholesky or of the forward solve on the tiles of `map`, with that problem's
-// update order (pairs), diagonal-block inverses of tile k, the tile column's
-// ticket and flags (launch_tile_column), not-SPD flag (n: its real dimension)
-// and solve vector with its partials.
+// Cholesky on the tiles of `map`, with that problem's update order (pairs),
+// diagonal-block inverses of tile k, the tile column's ticket and flags
+// (launch_tile_column), not-SPD flag (n: its real dimension); with step 0, the
+// forward solve's vector, words (launch_solve_init) and partials.
 struct BatchJob {
     TileMap map;
     int k;
@@ -25,6 +25,7 @@ struct BatchJob {
     int *info;
     int64_t n;
     double *z;
+    double *pending;
     double *partials;
 };
 
@@ -64,14 +65,15 @@ bool update192_supported(int ts);
 void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s);
 
 // ---- triangular solves and reductions (egs_solve.hip)
-// Forward solve of tile row k: y_k = L_kk^{-1} z_k in place, with per-tile
-// partials[2k] = sum log L_ii (L_ii > 0), partials[2k+1] = y_k . y_k.
-void launch_trsv_diag(const TileMap &map, int k, const double *winv_k, double *z, double *partials, hipStream_t s);
-// Backward solve with L^T of tile row k (after rows > k are solved):
-// partial sums of L_ik^T y_i into scratch, then the diagonal solve.
-void launch_trsv_t_partial(const TileMap &map, int k, const double *z, double *scratch, hipStream_t s);
-void launch_trsv_t_diag(const TileMap &map, int k, const double *winv_k, double *z, const double *scratch,
-                        hipStream_t s);
+// z = src (n values) padded with zeros to npad, or as it is when src is null;
+// pending (npad + 1 doubles) emptied for the next solve.
+void launch_solve_init(double *z, const double *src, int64_t n, int64_t npad, double *pending, hipStream_t s);
+// z = L^{-1} z and z = L^{-T} z with the factor's tiles (mixed: some may be FP32)
+// and its diagonal-block inverses.  partials (may be null): of 64-row block b,
+// partials[2b] = sum log L_ii (L_ii > 0), partials[2b+1] = y_b . y_b.
+void launch_forward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, double *partials,
+                    hipStream_t s);
+void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, hipStream_t s);
 // out = L e (lower-triangular product over the tiles).
 void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s);
 // out[r] = sum_c Sigma(l1_r, l2_c) x[c] for r < rows, c < cols (kriging mean).
@@ -95,22 +97,13 @@ void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, in
 // Batched steps over problems of tile size ts (jobs in device memory, those
 // with most tiles first): factor tile column k of each of njobs, then apply
 // panel k to tile columns k+1 .. of the first nrest, the ones that have them
-// (rest = the largest nt - k - 1; jobs with fewer tiles exit early);
-// forward-solve tile row k with its partials and subtract it from the rows
-// below.
+// (rest = the largest nt - k - 1; jobs with fewer tiles exit early).
 void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nrest, hipStream_t s);
-void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int rest, hipStream_t s);
-// X_k = L_kk^{-T} for every diagonal tile k (tinv: nt * ts * ts doubles).
-void launch_tinv(const TileMap &map, const double *winv, double *tinv, hipStream_t s);
-// Preconditioner solves with the diagonal-tile inverses (right-looking):
-// forward step k: y_k = X_k' z_k, then z_i -= L_ik y_k for i > k;
-// backward step k: y_k = X_k x_k, then x_j -= L_kj' y_k for j < k.
-void launch_fwd_diag_inv(const double *tinv_k, const double *z_k, double *y_k, int ts, hipStream_t s);
-void launch_fwd_panel(const TileMap &map, int k, const double *y_k, double *z, hipStream_t s);
-void launch_bwd_diag_inv(const double *tinv_k, const double *x_k, double *y_k, int ts, hipStream_t s);
-void launch_bwd_row(const TileMap &map, int k, const double *y_k, double *x, hipStream_t s);
-// logdet partials: partials[2k] = sum log L_ii over diagonal tile k (L_ii > 0).
-void launch_diag_logdet(const TileMap &map, int64_t n, double *partials, hipStream_t s);
+// The forward solves of the jobs of step 0, with their partials (max_nt: the
+// first job's tiles).
+void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int max_nt, hipStream_t s);
+// The log-det partials alone, of an FP64 or mixed factor (partials[2b+1] = 0).
+void launch_diag_logdet(const TileMap &map, double *partials, hipStream_t s);
 // Sigma v from the FP64 lower tiles written by launch_covgen_tiles: one
 // workgroup per tile (i, j) writes T_ij v_j to prow[t * ts ..] and, off the
 // diagonal, T_ij' v_i to pcol[t * ts ..] (t = i*(i+1)/2 + j).

@@ -1,0 +1,80 @@
+"""The triangular solves, one launch each, at the edges of their chains: one
+64-row block, two (the last one alone), an even and an odd number before it,
+tiles of one block, ragged last tiles; on an FP64 factor and, through the
+refinement, on one with FP32 tiles; and the product L e.
+
+Tolerances: the componentwise backward error of a substitution of n unknowns,
+n eps (|L| |x| + |z|), times 64 for the products with the 64 x 64 inverses; of
+the product L e, n eps |L| |e|; of a refined solve, its residual 1e-12 times
+the condition number.
+"""
+import numpy as np
+import pytest
+
+import exageostatcpp_amd as egs
+from exageostatcpp_amd import capi
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(float).eps
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = egs.Context(0)
+    yield c
+    c.close()
+
+
+def problem(ctx, n, dts, rng):
+    r = np.random.default_rng(n)
+    p = egs.Problem(ctx, 0, r.random(n), r.random(n), dts=dts)
+    z = r.standard_normal(n)
+    p.set_observations(z)
+    return p, z, [1.0, rng, 0.5]
+
+
+@pytest.mark.parametrize("n,dts", [(1, 64), (64, 64), (65, 64), (129, 64), (193, 64), (257, 64), (100, 320), (700, 192),
+                                   (1300, 320), (2000, 960), (3000, 64), (2049, 2048)])
+def test_solves_and_product(ctx, n, dts):
+    p, z, theta = problem(ctx, n, dts, 0.1)
+    llh, logdet, quad = p.loglik(theta)
+    low = p.get_matrix()
+    y = p.trsm(z)
+    assert np.all(np.abs(low @ y - z) <= 64 * n * EPS * (np.abs(low) @ np.abs(y) + np.abs(z)))
+    x = p.trsm(z, trans=True)
+    assert np.all(np.abs(low.T @ x - z) <= 64 * n * EPS * (np.abs(low).T @ np.abs(x) + np.abs(z)))
+    assert abs(quad - y @ y) <= 4 * n * EPS * quad
+    assert abs(logdet - 2 * np.log(np.diag(low)).sum()) <= 4 * n * EPS * 2 * np.abs(np.log(np.diag(low))).sum() + 4 * EPS
+    out = p.generate_observations(theta, seed=5)
+    e = np.linalg.solve(low, out)   # N(0, 1) values: of order one
+    assert np.all(np.abs(low @ e - out) <= 64 * n * EPS * (np.abs(low) @ np.abs(e) + 1))
+    other = egs.Problem(ctx, 0, *np.random.default_rng(n).random((2, n)), dts=64)
+    again = other.generate_observations(theta, seed=5)
+    other.close()
+    p.close()
+    assert np.max(np.abs(again - out)) <= 1e-10 * np.max(np.abs(out))
+
+
+@pytest.mark.parametrize("n,dts", [(1000, 192), (1345, 192), (2500, 384)])
+def test_refinement_with_fp32_tiles(ctx, n, dts):
+    p, z, theta = problem(ctx, n, dts, 0.03)
+    want = p.loglik(theta)
+    low = p.get_matrix()
+    p.set_precision(capi.PRECISION_MIXED, 1, 2)
+    got = p.loglik(theta)
+    p.close()
+    cond = np.linalg.cond(low) ** 2
+    assert abs(got[2] - want[2]) <= 1e-12 * cond * want[2]
+    assert abs(got[0] - want[0]) <= 1e-6 * abs(want[0])
+
+
+@pytest.mark.parametrize("trans", [False, True])
+def test_a_nan_of_any_pattern_passes_through(ctx, trans):
+    """All ones is the word of a value not yet solved; as an input it is a NaN."""
+    n = 400
+    p, z, theta = problem(ctx, n, 128, 0.1)
+    p.loglik(theta)
+    z[200] = np.array([0xFFFFFFFFFFFFFFFF], dtype=np.uint64).view(np.float64)[0]
+    x = p.trsm(z, trans=trans)
+    p.close()
+    assert np.isnan(x[200]) and np.all(np.isfinite(x[256:] if trans else x[:192]))
