@@ -224,6 +224,7 @@ struct egs_problem_s {
         m.store = d_store;
         m.nt = nt;
         m.ts = ts;
+        m.last_blocks = (int) ((n - (int64_t) (nt - 1) * ts + egs::kBlk - 1) / egs::kBlk);
         return m;
     }
     int ntheta() const { return kernel == 1 ? 6 : 3; }
@@ -619,25 +620,26 @@ void factor_panel(egs_problem_s *p, int k) {
     const double kb = real_rows(p, k);
     // rows within band64 of the diagonal are FP64 tiles, the rest FP32
     const int rows64 = is_mixed(p) ? std::min(nt - 1 - k, p->band64) : nt - 1 - k;
-    const int rows32 = nt - 1 - k - rows64;
+    // their 64-row blocks, without the last tile row's padding
+    const int first = (k + 1) * nsb;
+    const int below = std::max(0, m.blocks() - first);
+    const int blocks64 = std::min(rows64 * nsb, below), blocks32 = below - blocks64;
     // the FP64 rows go with the diagonal tile when they are few; the FP32 rows
     // of a bivariate plan are solved together with the FP64 ones (both on FP64
     // MFMA)
-    const bool fused = rows64 > 0 && egs::tile_column_solves_rows(p->ts, rows64) &&
-                       (rows32 == 0 || p->f32_panel_solve);
+    const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(blocks64) && (blocks32 == 0 || p->f32_panel_solve);
     int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0);
-    egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info, p->n, fused ? rows64 : 0, s);
+    egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info, p->n, fused ? blocks64 : 0, s);
     prof_end(p, pi);
     if (k + 1 < nt) {
         double rows_below = 0.0;
         for (int i = k + 1 + (fused ? rows64 : 0); i < nt; ++i) rows_below += real_rows(p, i);
         pi = prof_begin(p, EGS_PROFILE_PANEL_TRSM, rows_below * ts * ts);
-        const int64_t g64 = (int64_t) (k + 1) * nsb, g32 = g64 + (int64_t) rows64 * nsb;
-        if (rows32 > 0 && !p->f32_panel_solve) {
-            egs::launch_trsm_rows_mixed(m, k, g64, rows64 * nsb, rows32 * nsb, wk, s);
+        if (blocks32 > 0 && !p->f32_panel_solve) {
+            egs::launch_trsm_rows_mixed(m, k, first, blocks64, blocks32, wk, s);
         } else {
-            if (!fused) egs::launch_trsm_rows(m, k, g64, rows64 * nsb, wk, s);
-            egs::launch_trsm_rows(m, k, g32, rows32 * nsb, wk, s, true, p->f32_panel_solve);
+            if (!fused) egs::launch_trsm_rows(m, k, first, blocks64, wk, s);
+            egs::launch_trsm_rows(m, k, first + blocks64, blocks32, wk, s, true, p->f32_panel_solve);
         }
         prof_end(p, pi);
         if (is_mixed(p)) {
@@ -910,7 +912,7 @@ int refine_solve(egs_problem_s *p, const double *b) {
 }
 
 int read_partials(egs_problem_s *p, double &logdet, double &quad) {
-    const int blocks = p->nt * p->nsb;
+    const int blocks = p->map().blocks();
     p->h_partials.resize((size_t) 2 * blocks);
     EGS_HIP(hipMemcpy(p->h_partials.data(), p->d_partials, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost));
     double ld = 0.0, q = 0.0;

@@ -259,6 +259,7 @@ __device__ __forceinline__ void update_body(const TileMap &map, const double *p6
     const int sbm = bx % nsb;
     const int sbn = bx / nsb;
     if (ij.x == ij.y && sbm < sbn) return;
+    if (sbm >= map.blocks(ij.x) || sbn >= map.blocks(ij.y)) return;
     double *C = tile_f64(map, ij.x, ij.y) + sbm * kBlk + (int64_t) sbn * kBlk * ts;
     const int64_t tt = (int64_t) ts * ts;
     const double *A = (p64 ? p64 + (ij.x - k - 1) * tt : tile_f64(map, ij.x, k)) + sbm * kBlk;
@@ -663,8 +664,8 @@ struct BlockWait {
     __device__ __forceinline__ void inverse(int j) const { wait_block(flags + j * nsb + j); }
 };
 
-// Tasks of the diagonal tile, and the task of a ticket: r < 0 for rows.
-__host__ __device__ inline int tile_tasks(int nsb) { return nsb + (nsb - 1) * (nsb - 2) / 2; }
+// Tasks of a diagonal tile of so many 64 x 64 blocks.
+__host__ __device__ inline int tile_tasks(int blocks) { return blocks + (blocks - 1) * (blocks - 2) / 2; }
 
 }  // namespace
 
@@ -675,18 +676,19 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
     const int nsb = ts / kBlk;
     int *flags = sync + 1;
     double *T = tile_f64(map, k, k);
-    if (task >= tile_tasks(nsb)) {
-        const int h = task - tile_tasks(nsb);
+    const int live = map.blocks(k);
+    if (task >= tile_tasks(live)) {
+        const int h = task - tile_tasks(live);
         if (h >= halves) return;
         const int per = ts / kHalf;
         double *X = tile_f64(map, k + 1 + h / per, k) + (h % per) * kHalf;
         solve_rows<double, kHalf>(T, ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm), BlockWait{flags, nsb});
         return;
     }
-    // block column c holds the diagonal task and nsb - 2 - c others
+    // block column c holds the diagonal task and live - 2 - c others
     int c = 0, idx = task;
-    while (idx > max(0, nsb - 2 - c)) {
-        idx -= 1 + max(0, nsb - 2 - c);
+    while (idx > max(0, live - 2 - c)) {
+        idx -= 1 + max(0, live - 2 - c);
         ++c;
     }
     if (idx == 0)
@@ -718,7 +720,8 @@ __global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const Batch
     __shared__ PanelSmem sm;
     const int t = take_ticket(jobs[0].sync);
     const BatchJob &J = jobs[t % njobs];
-    const int halves = with_rows ? (J.map.nt - J.k - 1) * (J.map.ts / kHalf) : 0;
+    const int below = J.map.blocks() - (J.k + 1) * (J.map.ts / kBlk);   // none at or below the last tile
+    const int halves = with_rows ? 2 * max(below, 0) : 0;
     tile_column_task(J.map, J.k, J.winv_k, J.sync, J.info, J.n, halves, t / njobs, sm);
 }
 
@@ -726,7 +729,7 @@ template <int kRows>
 __global__ void __launch_bounds__(kThreads) trsm_rows_batch_kernel(const BatchJob *jobs) {
     const BatchJob &J = jobs[blockIdx.y];
     const int per = J.map.ts / kRows;
-    if ((int) blockIdx.x >= (J.map.nt - J.k - 1) * per) return;
+    if ((int) blockIdx.x * kRows >= (J.map.blocks() - (J.k + 1) * (J.map.ts / kBlk)) * kBlk) return;
     __shared__ GemmSmem sm;
     solve_row_block<double, kRows, double>(J.map, J.k, (int64_t) (J.k + 1) * per + blockIdx.x, J.winv_k, sm);
 }
@@ -763,13 +766,12 @@ void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nr
 
 int tile_column_sync_ints(int ts) { return 1 + (ts / kBlk) * (ts / kBlk); }
 
-bool tile_column_solves_rows(int ts, int rows) { return (int64_t) rows * (ts / kBlk) <= kFusedRows; }
+bool tile_column_solves_rows(int blocks) { return blocks <= kFusedRows; }
 
-void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int rows,
+void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,
                         hipStream_t s) {
-    const int halves = rows * (map.ts / kHalf);
-    hipLaunchKernelGGL(tile_column_kernel, dim3((unsigned) (tile_tasks(map.ts / kBlk) + halves)), dim3(kThreads), 0, s,
-                       map, k, winv_k, sync, info, n, halves);
+    hipLaunchKernelGGL(tile_column_kernel, dim3((unsigned) (tile_tasks(map.blocks(k)) + 2 * blocks)), dim3(kThreads), 0,
+                       s, map, k, winv_k, sync, info, n, 2 * blocks);
 }
 
 }  // namespace egs

@@ -21,13 +21,23 @@ enum StoragePrecision : uint8_t { kStoreF64 = 0, kStoreF32 = 1 };
 enum ComputeClass : uint8_t { kComputeF64 = 0, kComputeF32 = 1, kComputeBF16 = 2 };
 
 // Location of every lower tile in the arena.  off[i * nt + j] is the byte offset
-// of tile (i, j), i >= j; store[i * nt + j] its storage precision.
+// of tile (i, j), i >= j; store[i * nt + j] its storage precision.  Of the last
+// tile row only the first last_blocks 64-row blocks hold rows of the matrix; the
+// factorization and the solves leave out the blocks that are all padding (which
+// is its own factor): up to a tile's worth of work per row and column (400
+// locations in tiles of 384: 310 -> 247 us; 6,001 in tiles of 960: 4.32 -> 3.83
+// ms; 10,007 in tiles of 960: 10.7 -> 9.6 ms).
 struct TileMap {
     char *base;
     const int64_t *off;
     const uint8_t *store;
     int nt;
     int ts;
+    int last_blocks;
+
+    // 64-row blocks of tile row i, and of the whole matrix, that are not padding
+    __host__ __device__ int blocks(int i) const { return i == nt - 1 ? last_blocks : ts / kBlk; }
+    __host__ __device__ int blocks() const { return (nt - 1) * (ts / kBlk) + last_blocks; }
 };
 
 __device__ __forceinline__ double *tile_f64(const TileMap &m, int i, int j) {

@@ -86,13 +86,13 @@ void launch_cov_matvec(double *partial, const double *v, int64_t n, int64_t npad
                        const double *x, const double *y, const double *z, hipStream_t s);
 int matvec_chunks(int64_t n);
 // Cholesky of diagonal tile k in place, in 64 x 64 blocks, with the inverses of
-// its diagonal blocks in winv_k, and the panel solve of the `rows` FP64 tiles
-// below it (tile_column_solves_rows: whether that many should be; the others
-// take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
+// its diagonal blocks in winv_k, and the panel solve of the first `blocks` 64-row
+// blocks below it, FP64 ones (tile_column_solves_rows: whether that many should
+// be; the others take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
 // tile_column_sync_ints(ts) ints, zero before the launch.
 int tile_column_sync_ints(int ts);
-bool tile_column_solves_rows(int ts, int rows);
-void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int rows,
+bool tile_column_solves_rows(int blocks);
+void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,
                         hipStream_t s);
 // Batched steps over problems of tile size ts (jobs in device memory, those
 // with most tiles first): factor tile column k of each of njobs, then apply

@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob 
     const int t = solve_ticket(jobs[0].pending, (int64_t) jobs[0].map.nt * jobs[0].map.ts, sm);
     const BatchJob &J = jobs[t % njobs];
     const int b = t / njobs;
-    if (b >= J.map.nt * (J.map.ts / kBlk)) return;
+    if (b >= J.map.blocks()) return;
     forward_block<false>(J.map, J.winv_k, J.z, J.pending, J.partials, b, sm);
 }
 
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob 
 template <bool kMixed>
 __device__ __forceinline__ void backward_block(const TileMap &map, const double *winv, double *z, double *pending, int b,
                                                SolveSmem &sm) {
-    const int ts = map.ts, nsb = ts / kBlk, nb = map.nt * nsb;
+    const int ts = map.ts, nsb = ts / kBlk, nb = map.blocks();
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int tj = b / nsb, cb = b % nsb;
     const int last = b + 1;   // the block read transposed, if there is one
@@ -279,7 +279,7 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     double acc[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) acc[q] = 0.0;
-    int next = nb - 1, ti = map.nt - 1, rb = nsb - 1;   // the next fetch's block and its place
+    int next = nb - 1, ti = map.nt - 1, rb = map.last_blocks - 1;   // the next fetch's block and its place
     auto fetch = [&](Cols<kMixed> &c) {
         c.load(map, ti, tj, rb * kBlk + lane, cb * kBlk + 16 * w);
         c.y = peek(pending + (int64_t) next * kBlk + lane);
@@ -326,7 +326,7 @@ template <bool kMixed>
 __global__ void __launch_bounds__(kThreads) backward_kernel(TileMap map, const double *winv, double *z, double *pending) {
     __shared__ SolveSmem sm;
     const int t = solve_ticket(pending, (int64_t) map.nt * map.ts, sm);
-    backward_block<kMixed>(map, winv, z, pending, map.nt * (map.ts / kBlk) - 1 - t, sm);
+    backward_block<kMixed>(map, winv, z, pending, map.blocks() - 1 - t, sm);
 }
 
 // out = L e: one workgroup of 16 waves per 64 rows, the longest rows first; the
@@ -573,8 +573,8 @@ void launch_solve_init(double *z, const double *src, int64_t n, int64_t npad, do
 
 void launch_forward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, double *partials,
                     hipStream_t s) {
-    hipLaunchKernelGGL(mixed ? forward_kernel<true> : forward_kernel<false>, dim3((unsigned) (map.nt * (map.ts / kBlk))),
-                       dim3(kThreads), 0, s, map, winv, z, pending, partials);
+    hipLaunchKernelGGL(mixed ? forward_kernel<true> : forward_kernel<false>, dim3((unsigned) map.blocks()), dim3(kThreads), 0,
+                       s, map, winv, z, pending, partials);
 }
 
 void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int max_nt, hipStream_t s) {
@@ -583,12 +583,12 @@ void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int max_nt, h
 }
 
 void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, hipStream_t s) {
-    hipLaunchKernelGGL(mixed ? backward_kernel<true> : backward_kernel<false>,
-                       dim3((unsigned) (map.nt * (map.ts / kBlk))), dim3(kThreads), 0, s, map, winv, z, pending);
+    hipLaunchKernelGGL(mixed ? backward_kernel<true> : backward_kernel<false>, dim3((unsigned) map.blocks()), dim3(kThreads), 0,
+                       s, map, winv, z, pending);
 }
 
 void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(trmv_kernel, dim3((unsigned) (map.nt * (map.ts / kBlk))), dim3(kTrmvThreads), 0, s, map, e, out);
+    hipLaunchKernelGGL(trmv_kernel, dim3((unsigned) map.blocks()), dim3(kTrmvThreads), 0, s, map, e, out);
 }
 
 void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams &prm, const double *x1,
@@ -771,7 +771,7 @@ __global__ void __launch_bounds__(kBlk) diag_logdet_kernel(TileMap map, double *
 }
 
 void launch_diag_logdet(const TileMap &map, double *partials, hipStream_t s) {
-    hipLaunchKernelGGL(diag_logdet_kernel, dim3((unsigned) (map.nt * (map.ts / kBlk))), dim3(kBlk), 0, s, map, partials);
+    hipLaunchKernelGGL(diag_logdet_kernel, dim3((unsigned) map.blocks()), dim3(kBlk), 0, s, map, partials);
 }
 
 }  // namespace egs

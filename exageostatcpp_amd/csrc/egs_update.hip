@@ -59,6 +59,7 @@ __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef
     const int sbm = sub % nbr, sbn = sub / nbr;
     const int2 ij = pairs[pair];
     if (ij.x == ij.y && (sbm + 1) * kBR <= sbn * kBC) return;   // strictly upper block of a diagonal tile
+    if (sbm * kBR >= map.blocks(ij.x) * kBlk || sbn * kBC >= map.blocks(ij.y) * kBlk) return;   // padding
 
     const double *A = panel_tile(map, pr, ij.x, k) + sbm * kBR;
     const double *B = panel_tile(map, pr, ij.y, k) + sbn * kBC;

@@ -1,0 +1,71 @@
+"""The last tile's padding blocks, which the factorization and the solves leave
+out: one, 63, 64 and 65 rows in the last tile, all its blocks but one, none
+padded, and a single tile; FP64, batched, with both panel forms and both update
+forms, and mixed.  The reference is the same field in tiles of 64 (which pad
+less than a block): log-likelihood, observations and kriging to 1e-11 (n eps
+times the condition number of this field), mixed within its 1e-6.
+"""
+import numpy as np
+import pytest
+
+import exageostatcpp_amd as egs
+from exageostatcpp_amd import capi
+
+pytestmark = pytest.mark.gpu
+THETA = [1.0, 0.03, 0.5]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = egs.Context(0)
+    yield c
+    c.close()
+
+
+def field(ctx, n, dts):
+    r = np.random.default_rng(n)
+    p = egs.Problem(ctx, 0, r.random(n), r.random(n), dts=dts)
+    p.set_observations(r.standard_normal(n))
+    return p
+
+
+def close(a, b, tol):
+    a, b = np.asarray(a), np.asarray(b)
+    assert np.max(np.abs(a - b)) <= tol * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("n,dts", [(10, 384), (385, 384), (447, 384), (448, 384), (449, 384), (768, 384), (705, 384),
+                                   (2900, 960), (4801, 960), (6720, 192), (6721, 192), (9000, 128), (2049, 2048),
+                                   (3000, 2048)])
+def test_fp64(ctx, n, dts):
+    t = np.random.default_rng(1).random((2, 20))
+    out = []
+    for ts in (dts, 64):
+        p = field(ctx, n, ts)
+        llh = p.loglik(THETA)
+        out.append((llh, p.predict(THETA, t[0], t[1])[0], p.generate_observations(THETA, seed=3)))
+        p.close()
+    for a, b in zip(*out):
+        close(a, b, 1e-11)
+
+
+def test_batch(ctx):
+    sizes = [385, 1100, 447, 448, 10, 1537, 769, 1152]
+    probs = [field(ctx, n, 384) for n in sizes]
+    got = capi.loglik_batch(probs, [THETA] * len(sizes))
+    for p, n, g in zip(probs, sizes, got):
+        q = field(ctx, n, 64)
+        close(g, q.loglik(THETA), 1e-11)
+        q.close()
+        p.close()
+
+
+@pytest.mark.parametrize("n,dts,bands", [(1729, 576, (1, 2)), (2000, 384, (1, 2)), (2369, 192, (2, 4)), (3000, 960, (1, 1))])
+def test_mixed(ctx, n, dts, bands):
+    p = field(ctx, n, dts)
+    want = p.loglik(THETA)
+    p.set_precision(capi.PRECISION_MIXED, *bands)
+    got = p.loglik(THETA)
+    p.close()
+    close(got[0], want[0], 1e-6)
+    close(got[2], want[2], 1e-8)
