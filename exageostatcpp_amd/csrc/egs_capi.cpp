@@ -84,7 +84,7 @@ struct egs_context_s {
     hipStream_t bulk = nullptr;       // trailing updates that the next panel does not wait for
     std::vector<egs_problem_s *> problems;   // live problems, released by egs_finalize
     std::mutex mu;                           // guards problems (problems move between contexts)
-    egs::BatchJob *d_jobs = nullptr;         // job records of egs_loglik_batch, jobs_cap entries
+    char *d_jobs = nullptr;                  // job records of egs_loglik_batch, jobs_cap bytes
     int64_t jobs_cap = 0, dev_bytes = 0;
 };
 
@@ -226,6 +226,15 @@ struct egs_problem_s {
         m.ts = ts;
         m.last_blocks = (int) ((n - (int64_t) (nt - 1) * ts + egs::kBlk - 1) / egs::kBlk);
         return m;
+    }
+    egs::CovJob cov_job(const egs::MaternParams &prm, double *sig64, const egs::MaternParams *prm_dev) const {
+        const double *z = kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY ? d_z : nullptr;
+        return egs::CovJob{map(), d_pairs, (int) h_pairs.size(), prm, egs::Locs{d_x, d_y, z}, n, d_tab, sig64, prm_dev};
+    }
+    // A factorization's tickets and flags, and a solve of src (null: of d_work).
+    egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) const {
+        return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_info, d_work, src, count, npad,
+                            solve ? d_aux : nullptr};
     }
     int ntheta() const { return kernel == 1 ? 6 : 3; }
     int64_t sync_ints() const { return (int64_t) nt * egs::tile_column_sync_ints(ts); }
@@ -585,11 +594,9 @@ int run_covariance(egs_problem_s *p, const double *theta) {
     egs::MaternParams prm;
     int st = make_params(p->kernel, p->metric, theta, prm);
     if (st) return st;
-    const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
     const int pi = prof_begin(p, EGS_PROFILE_COVARIANCE, 0.0);
     egs::launch_matern_tables(p->d_tab, prm, nullptr, p->ctx->stream);
-    egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm, p->d_x, p->d_y, dz, p->n, p->d_tab,
-                             is_mixed(p) ? p->d_sig64 : nullptr, p->ctx->stream);
+    egs::launch_covgen_tiles(p->cov_job(prm, is_mixed(p) ? p->d_sig64 : nullptr, nullptr), p->ctx->stream);
     prof_end(p, pi);
     EGS_HIP(hipGetLastError());
     p->factored = false;
@@ -706,7 +713,9 @@ void launch_mixed_update(egs_problem_s *p, int k, int jcol_lo, int jcol_hi, hipS
 // lists tiles by descending column, so both tile sets are contiguous ranges of
 // it.  The caller checks d_info after synchronizing the critical stream, which
 // ends waiting for the bulk stream.
-int run_potrf(egs_problem_s *p) {
+// then_solve: the forward solve of the observations follows (run_forward is
+// told so), and what it starts from is prepared by the same launch.
+int run_potrf(egs_problem_s *p, bool then_solve = false) {
     // EGS_NO_LOOKAHEAD=1 runs every launch on one stream (for measuring kernels
     // without the overlap of the two streams).
     static const bool no_lookahead = [] {
@@ -725,8 +734,7 @@ int run_potrf(egs_problem_s *p) {
         p->ev_bulk.push_back(e2);
     }
     // a fill kernel, not a memset: this sequence is captured into a graph
-    egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_info), 1, s);
-    egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_sync), (int) p->sync_ints(), s);
+    egs::launch_init(p->init_job(true, then_solve, p->d_obs, p->n), s);
     if (p->mode == EGS_PRECISION_MIXED) {
         egs::launch_zero_u32(p->d_pmax, nt, s);
         egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_counts), 6, s);
@@ -792,12 +800,12 @@ int read_info(egs_problem_s *p) {
     return EGS_SUCCESS;
 }
 
-// d_work = L^{-1} src (src null: of d_work itself); the log-det and dot partials
-// of its 64-row blocks go to `partials` (may be null).
-void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partials) {
+// d_work = L^{-1} src (src null: of d_work itself; prepared: by run_potrf); the
+// log-det and dot partials of its 64-row blocks go to `partials` (may be null).
+void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partials, bool prepared = false) {
     hipStream_t s = p->ctx->stream;
     const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
-    egs::launch_solve_init(p->d_work, src, n, p->npad, p->d_aux, s);
+    if (!prepared) egs::launch_init(p->init_job(false, true, src, n), s);
     egs::launch_forward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, partials, s);
     prof_end(p, pi);
 }
@@ -806,7 +814,7 @@ void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partial
 void run_backward(egs_problem_s *p, const double *src, int64_t n) {
     hipStream_t s = p->ctx->stream;
     const int pi = is_mixed(p) ? prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n) : -1;
-    egs::launch_solve_init(p->d_work, src, n, p->npad, p->d_aux, s);
+    egs::launch_init(p->init_job(false, true, src, n), s);
     egs::launch_backward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, s);
     prof_end(p, pi);
 }
@@ -1433,15 +1441,13 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
 // capturable (no host synchronization, no memset).
 int enqueue_fp64_eval(egs_problem_s *p) {
     hipStream_t s = p->ctx->stream;
-    const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
     p->h_prm.kernel = p->kernel;   // the launches are shaped by the kernel and the metric alone
     p->h_prm.metric = p->metric;
     egs::launch_matern_tables(p->d_tab, p->h_prm, p->d_prm, s);
-    egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), p->h_prm, p->d_x, p->d_y, dz, p->n,
-                             p->d_tab, nullptr, s, p->d_prm);
-    const int st = run_potrf(p);
+    egs::launch_covgen_tiles(p->cov_job(p->h_prm, nullptr, p->d_prm), s);
+    const int st = run_potrf(p, true);
     if (st) return st;
-    run_forward(p, p->d_obs, p->n, p->d_partials);
+    run_forward(p, p->d_obs, p->n, p->d_partials, true);
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;
 }
@@ -1529,11 +1535,11 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
     st = run_covariance(p, theta);
     if (st) return st;
     EGS_HIP(hipEventRecord(p->ev[1], s));
-    st = run_potrf(p);
+    st = run_potrf(p, !is_mixed(p));
     if (st) return st;
     EGS_HIP(hipEventRecord(p->ev[2], s));
     if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials, s);   // quad from the refinement
-    else run_forward(p, p->d_obs, p->n, p->d_partials);
+    else run_forward(p, p->d_obs, p->n, p->d_partials, true);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipEventRecord(p->ev[3], s));
     EGS_HIP(hipStreamSynchronize(s));
@@ -1627,39 +1633,60 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
         }
     if (na > 0) {
         EGS_HIP(hipSetDevice(ctx->device));
-        if (njobs > ctx->jobs_cap) {
+        // the records on the device: steps, covariances (those a launch serves
+        // together side by side), initializations
+        std::vector<egs::CovJob> cov;
+        std::vector<int> group;   // first of each group, and the end
+        std::vector<char> grouped(na, 0);
+        for (int a = 0; a < na; ++a) {
+            if (grouped[a]) continue;
+            group.push_back((int) cov.size());
+            for (int c = a; c < na; ++c)
+                if (!grouped[c] && egs::covgen_same_launch(prm[run[a]], prm[run[c]])) {
+                    cov.push_back(problems[run[c]]->cov_job(prm[run[c]], nullptr, nullptr));
+                    grouped[c] = 1;
+                }
+        }
+        group.push_back(na);
+        std::vector<egs::InitJob> init;
+        int64_t extent = 0;
+        for (int b : run) {
+            egs_problem_s *p = problems[b];
+            init.push_back(p->init_job(true, true, p->d_obs, p->n));
+            extent = std::max(extent, egs::init_extent(init.back()));
+            p->has_cov = false;
+            p->factored = false;
+            invalidate_graph(p);
+        }
+        const size_t job_bytes = sizeof(egs::BatchJob) * (size_t) njobs, cov_bytes = sizeof(egs::CovJob) * (size_t) na,
+                     init_bytes = sizeof(egs::InitJob) * (size_t) na;
+        std::vector<char> records(job_bytes + cov_bytes + init_bytes);
+        std::memcpy(records.data(), jobs.data(), job_bytes);
+        std::memcpy(records.data() + job_bytes, cov.data(), cov_bytes);
+        std::memcpy(records.data() + job_bytes + cov_bytes, init.data(), init_bytes);
+        if ((int64_t) records.size() > ctx->jobs_cap) {
             EGS_HIP(hipStreamSynchronize(s));
             egs::dev_free(ctx->d_jobs, &ctx->dev_bytes);
             ctx->d_jobs = nullptr;
             ctx->jobs_cap = 0;
             void *v = nullptr;
-            if (egs::dev_alloc(&v, sizeof(egs::BatchJob) * (size_t) njobs, &ctx->dev_bytes) != hipSuccess)
+            if (egs::dev_alloc(&v, records.size(), &ctx->dev_bytes) != hipSuccess)
                 return fail(EGS_ERR_OUT_OF_MEMORY, "egs_loglik_batch: cannot allocate the job records");
-            ctx->d_jobs = static_cast<egs::BatchJob *>(v);
-            ctx->jobs_cap = njobs;
+            ctx->d_jobs = static_cast<char *>(v);
+            ctx->jobs_cap = (int64_t) records.size();
         }
         // the previous batch on this context has completed (every call returns synchronized)
-        EGS_HIP(hipMemcpyAsync(ctx->d_jobs, jobs.data(), sizeof(egs::BatchJob) * (size_t) njobs,
-                               hipMemcpyHostToDevice, s));
-        for (int b : run) {
-            egs_problem_s *p = problems[b];
-            egs::launch_solve_init(p->d_work, p->d_obs, p->n, p->npad, p->d_aux, s);
-            const double *dz = (p->kernel == EGS_KERNEL_UNIVARIATE_MATERN_STATIONARY) ? p->d_z : nullptr;
-            egs::launch_matern_tables(p->d_tab, prm[b], nullptr, s);
-            egs::launch_covgen_tiles(p->map(), p->d_pairs, (int) p->h_pairs.size(), prm[b], p->d_x, p->d_y, dz, p->n,
-                                     p->d_tab, nullptr, s);
-            egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_info), 1, s);
-            egs::launch_zero_u32(reinterpret_cast<unsigned *>(p->d_sync), (int) p->sync_ints(), s);
-            p->has_cov = false;
-            p->factored = false;
-            invalidate_graph(p);
-        }
+        EGS_HIP(hipMemcpyAsync(ctx->d_jobs, records.data(), records.size(), hipMemcpyHostToDevice, s));
+        const auto *d_steps = reinterpret_cast<const egs::BatchJob *>(ctx->d_jobs);
+        const auto *d_cov = reinterpret_cast<const egs::CovJob *>(ctx->d_jobs + job_bytes);
+        egs::launch_init_batch(reinterpret_cast<const egs::InitJob *>(ctx->d_jobs + job_bytes + cov_bytes), na, extent, s);
+        for (size_t g = 0; g + 1 < group.size(); ++g)
+            egs::launch_covgen_batch(d_cov + group[g], cov.data() + group[g], group[g + 1] - group[g], s);
         // lockstep right-looking factorization: one launch per kernel and step for all problems
         for (int k = 0; k < max_nt; ++k) {
-            const egs::BatchJob *J = ctx->d_jobs + first[k];
-            egs::launch_step_batch(J, active[k], ts, max_nt - k - 1, active[k + 1], s);
+            egs::launch_step_batch(d_steps + first[k], active[k], ts, max_nt - k - 1, active[k + 1], s);
         }
-        egs::launch_forward_batch(ctx->d_jobs, na, ts, max_nt, s);
+        egs::launch_forward_batch(d_steps, na, ts, max_nt, s);
         EGS_HIP(hipGetLastError());
         EGS_HIP(hipStreamSynchronize(s));
     }

@@ -719,7 +719,7 @@ __global__ void __launch_bounds__(kThreads) tile_column_kernel(TileMap map, int 
 __global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const BatchJob *jobs, int njobs, int with_rows) {
     __shared__ PanelSmem sm;
     const int t = take_ticket(jobs[0].sync);
-    const BatchJob &J = jobs[t % njobs];
+    const BatchJob J = scalar_load(jobs + t % njobs);
     const int below = J.map.blocks() - (J.k + 1) * (J.map.ts / kBlk);   // none at or below the last tile
     const int halves = with_rows ? 2 * max(below, 0) : 0;
     tile_column_task(J.map, J.k, J.winv_k, J.sync, J.info, J.n, halves, t / njobs, sm);
@@ -727,7 +727,7 @@ __global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const Batch
 
 template <int kRows>
 __global__ void __launch_bounds__(kThreads) trsm_rows_batch_kernel(const BatchJob *jobs) {
-    const BatchJob &J = jobs[blockIdx.y];
+    const BatchJob J = scalar_load(jobs + blockIdx.y);
     const int per = J.map.ts / kRows;
     if ((int) blockIdx.x * kRows >= (J.map.blocks() - (J.k + 1) * (J.map.ts / kBlk)) * kBlk) return;
     __shared__ GemmSmem sm;
@@ -735,7 +735,7 @@ __global__ void __launch_bounds__(kThreads) trsm_rows_batch_kernel(const BatchJo
 }
 
 __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *jobs) {
-    const BatchJob &J = jobs[blockIdx.z];
+    const BatchJob J = scalar_load(jobs + blockIdx.z);
     const int rest = J.map.nt - J.k - 1;   // tile columns k+1 .. nt-1: the first rest (rest + 1) / 2 pairs
     if ((int) blockIdx.y >= rest * (rest + 1) / 2) return;
     update_body(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y);

@@ -47,6 +47,23 @@ __device__ __forceinline__ float *tile_f32(const TileMap &m, int i, int j) {
     return reinterpret_cast<float *>(m.base + m.off[i * m.nt + j]);
 }
 
+// What a launch only reads, the same for the whole wave (the tile table, a job's
+// record), through scalar loads: it stays out of the vector registers, and
+// waiting for it does not wait for the vector loads in flight.
+template <typename T> __device__ __forceinline__ T scalar_load(const T *p) {
+    typedef const __attribute__((address_space(4))) uint32_t *Words;
+    if constexpr (sizeof(T) % 4 != 0 || alignof(T) < 4) return *p;
+    const Words q = reinterpret_cast<Words>(reinterpret_cast<uintptr_t>(p));
+    union U {
+        uint32_t w[sizeof(T) / 4];
+        T v;
+        __device__ U() {}
+    } u;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) u.w[i] = q[i];
+    return u.v;
+}
+
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin (workgroup w
 // runs on XCD w % 8), and each XCD has its own L2.  xcd_remap gives XCD x a
 // contiguous range of the logical block order, so blocks that share operand

@@ -54,12 +54,10 @@ __device__ __forceinline__ void add_product(double &sum, double &err, double a, 
     sum = t;
 }
 
-__global__ void __launch_bounds__(kThreads) matern_table_kernel(double *tabs, MaternParams prm_host,
-                                                                const MaternParams *prm_dev) {
+__device__ __forceinline__ void matern_table(double *tabs, const MaternParams &prm) {
     __shared__ double s_cos[4 * kNodes];   // cos(pi m / (2 kNodes))
     __shared__ double s_f[kRowsPerGroup][kNodes];
     __shared__ double s_c[kRowsPerGroup][kDegree + 1], s_e[kRowsPerGroup][kDegree + 1];
-    const MaternParams prm = prm_dev ? *prm_dev : prm_host;
     const int slot = blockIdx.y;
     if (slot >= prm.ntab) return;
     const int pair = prm.tab_pair[slot];
@@ -103,25 +101,24 @@ __global__ void __launch_bounds__(kThreads) matern_table_kernel(double *tabs, Ma
     }
 }
 
+__global__ void __launch_bounds__(kThreads) matern_table_kernel(double *tabs, MaternParams prm,
+                                                                const MaternParams *prm_dev) {
+    const MaternParams p = prm_dev ? *prm_dev : prm;
+    matern_table(tabs, p);
+}
+
+__global__ void __launch_bounds__(kThreads) matern_table_batch_kernel(const CovJob *jobs) {
+    const CovJob &J = jobs[blockIdx.z];   // in memory: its parameters are indexed
+    matern_table(J.tabs, J.prm);
+}
+
+constexpr int kTableGroups = (kTabRows + kRowsPerGroup - 1) / kRowsPerGroup;
+
 void launch_matern_tables(double *tabs, const MaternParams &prm, const MaternParams *prm_dev, hipStream_t s) {
     const int slots = prm_dev ? (prm.kernel == 1 ? kTabSlots : 1) : prm.ntab;
     if (slots == 0) return;
-    hipLaunchKernelGGL(matern_table_kernel, dim3((kTabRows + kRowsPerGroup - 1) / kRowsPerGroup, slots),
-                       dim3(kThreads), 0, s, tabs, prm, prm_dev);
+    hipLaunchKernelGGL(matern_table_kernel, dim3(kTableGroups, slots), dim3(kThreads), 0, s, tabs, prm, prm_dev);
 }
-
-struct CovTilesArgs {
-    TileMap map;
-    const int2 *pairs;      // lower tiles (i, j) to generate
-    MaternParams prm;
-    Locs loc;
-    int64_t n;              // true matrix dimension; rows/cols >= n are identity padding
-    int three_d;
-    int cols;               // columns per workgroup, a multiple of 64
-    const double *tabs;     // Matern tables of prm
-    double *sig64;          // optional FP64 copy of every lower tile (tile i*(i+1)/2 + j, ts*ts each)
-    const MaternParams *prm_dev;   // optional: read the parameters here instead of prm
-};
 
 // One workgroup per 64-row strip and `cols` columns of a tile: the strip's row
 // locations and the tables sit in LDS, the columns' locations pass through it
@@ -136,19 +133,17 @@ struct CovTilesArgs {
 // 1.08 ms -> 16 us each (one strip of 64 x ts per workgroup left most of the
 // GPU idle there; see the split in launch_covgen_tiles).
 template <int kTabs, bool kSphere>
-__global__ void __launch_bounds__(kThreads, 4) covgen_tiles_kernel(CovTilesArgs a) {
+__device__ __forceinline__ void covgen_strip(const CovJob &a, const MaternParams &prm, int cols, int part) {
     constexpr int kStageCols = 256;
     __shared__ double s_cx[kStageCols], s_cy[kStageCols], s_cz[kStageCols];
     __shared__ __align__(16) double s_tab[kTabs > 0 ? kTabs * kTabDoubles : 1];
-    // parameters from device memory when given (a captured graph replays with new theta)
-    const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
     const int ts = a.map.ts;
     const int2 ij = a.pairs[blockIdx.y];
     const int sbr = blockIdx.x;
     const int64_t r0 = (int64_t) ij.x * ts + sbr * kBlk;
-    const int c_beg = blockIdx.z * a.cols, c_end = min(ts, c_beg + a.cols);
+    const int c_beg = part * cols, c_end = min(ts, c_beg + cols);
     const int t = threadIdx.x;
-    const bool three_d = a.three_d != 0;
+    const bool three_d = a.loc.z != nullptr;
     if (kTabs > 0 && prm.ntab > 0)
         for (int e = t; e < kTabs * kTabDoubles; e += kThreads) s_tab[e] = a.tabs[e];
 
@@ -198,15 +193,14 @@ __global__ void __launch_bounds__(kThreads, 4) covgen_tiles_kernel(CovTilesArgs 
 constexpr int kBivThreads = 512;
 
 template <int kTabs, bool kSphere>
-__global__ void __launch_bounds__(kBivThreads, kTabs < 3 ? 4 : 2) covgen_tiles_biv_kernel(CovTilesArgs a) {
+__device__ __forceinline__ void covgen_strip_biv(const CovJob &a, const MaternParams &prm, int cols, int part) {
     constexpr int kRowLocs = kBlk / 2, kColStep = kBivThreads / kRowLocs;
     __shared__ __align__(16) double s_tab[kTabs > 0 ? kTabs * kTabDoubles : 1];
-    const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
     const int ts = a.map.ts;
     const int2 ij = a.pairs[blockIdx.y];
     const int sbr = blockIdx.x;
     const int64_t r0 = (int64_t) ij.x * ts + sbr * kBlk, c0 = (int64_t) ij.y * ts;
-    const int c_beg = blockIdx.z * a.cols, c_end = min(ts, c_beg + a.cols);
+    const int c_beg = part * cols, c_end = min(ts, c_beg + cols);
     const int t = threadIdx.x;
     if (kTabs > 0 && prm.ntab > 0) {
         for (int e = t; e < kTabs * kTabDoubles; e += kBivThreads) s_tab[e] = a.tabs[e];
@@ -251,6 +245,35 @@ __global__ void __launch_bounds__(kBivThreads, kTabs < 3 ? 4 : 2) covgen_tiles_b
     }
 }
 
+// One problem's tiles, or those of a batch (blockIdx.z: its jobs, `parts` column
+// parts each; workgroups past a job's tiles exit at once).  The parameters come
+// from device memory when prm_dev is given (a captured graph replays with new
+// theta).
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kThreads, 4) covgen_tiles_kernel(CovJob a, int cols) {
+    const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
+    covgen_strip<kTabs, kSphere>(a, prm, cols, blockIdx.z);
+}
+
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kThreads, 4) covgen_tiles_batch_kernel(const CovJob *jobs, int cols, int parts) {
+    const CovJob J = scalar_load(jobs + blockIdx.z / parts);
+    if ((int) blockIdx.y < J.npairs) covgen_strip<kTabs, kSphere>(J, J.prm, cols, blockIdx.z % parts);
+}
+
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kBivThreads, kTabs < 3 ? 4 : 2) covgen_tiles_biv_kernel(CovJob a, int cols) {
+    const MaternParams prm = a.prm_dev ? *a.prm_dev : a.prm;
+    covgen_strip_biv<kTabs, kSphere>(a, prm, cols, blockIdx.z);
+}
+
+template <int kTabs, bool kSphere>
+__global__ void __launch_bounds__(kBivThreads, kTabs < 3 ? 4 : 2)
+    covgen_tiles_biv_batch_kernel(const CovJob *jobs, int cols, int parts) {
+    const CovJob J = scalar_load(jobs + blockIdx.z / parts);
+    if ((int) blockIdx.y < J.npairs) covgen_strip_biv<kTabs, kSphere>(J, J.prm, cols, blockIdx.z % parts);
+}
+
 // A rows x cols column-major block (ld = rows) of Sigma(l1, l2) starting at
 // matrix row row_off and column col_off: the plugin interface
 // Kernel<T>::GenerateCovarianceMatrix evaluated on the device.
@@ -272,31 +295,23 @@ __global__ void __launch_bounds__(kThreads) covgen_rect_kernel(CovRectArgs a) {
     a.out[idx] = covariance_entry(a.prm, a.l1, a.l2, a.row_off + i, a.col_off + j, a.three_d != 0);
 }
 
-void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, const MaternParams &prm,
-                         const double *x, const double *y, const double *z, int64_t n, const double *tabs,
-                         double *sig64, hipStream_t s, const MaternParams *prm_dev) {
-    if (npairs <= 0) return;
-    CovTilesArgs a;
-    a.map = map;
-    a.pairs = pairs;
-    a.prm = prm;
-    a.loc = Locs{x, y, z};
-    a.n = n;
-    a.three_d = z != nullptr;
-    a.tabs = tabs;
-    a.sig64 = sig64;
-    a.prm_dev = prm_dev;
-    // a strip's columns are split over workgroups until these fill the GPU
-    // (kFill: eight per CU); whole strips stage the tables once each
+// A strip's columns are split over workgroups until `tiles` tiles fill the GPU
+// (kFill: eight per CU); whole strips stage the tables once each.  Returns the
+// 64-column blocks per workgroup.
+static int covgen_blocks(int nsb, int64_t tiles) {
     constexpr int kFill = 2048;
-    const int nsb = map.ts / kBlk;
-    const int want = (int) std::min<int64_t>(nsb, (kFill + (int64_t) nsb * npairs - 1) / ((int64_t) nsb * npairs));
-    const int per = (nsb + want - 1) / want;
-    a.cols = per * kBlk;
-    const dim3 grid(nsb, npairs, (nsb + per - 1) / per);
+    const int want = (int) std::min<int64_t>(nsb, (kFill + nsb * tiles - 1) / (nsb * tiles));
+    return (nsb + want - 1) / want;
+}
+
+void launch_covgen_tiles(const CovJob &job, hipStream_t s) {
+    if (job.npairs <= 0) return;
+    const int nsb = job.map.ts / kBlk, per = covgen_blocks(nsb, job.npairs);
+    const dim3 grid(nsb, job.npairs, (nsb + per - 1) / per);
     // a captured launch serves every theta: as many tables as the kernel may need
-    const int tables = prm_dev ? (prm.kernel == 1 ? kTabSlots : 1) : prm.ntab;
-    using Kernel = void (*)(CovTilesArgs);
+    const MaternParams &prm = job.prm;
+    const int tables = job.prm_dev ? (prm.kernel == 1 ? kTabSlots : 1) : prm.ntab;
+    using Kernel = void (*)(CovJob, int);
     static const Kernel univariate[2][2] = {{covgen_tiles_kernel<0, false>, covgen_tiles_kernel<1, false>},
                                             {covgen_tiles_kernel<0, true>, covgen_tiles_kernel<1, true>}};
     static const Kernel bivariate[2][kTabSlots + 1] = {
@@ -306,9 +321,42 @@ void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, cons
          covgen_tiles_biv_kernel<3, true>}};
     const bool sphere = prm.metric == 1;
     if (prm.kernel == 1)
-        hipLaunchKernelGGL(bivariate[sphere][tables], grid, dim3(kBivThreads), 0, s, a);
+        hipLaunchKernelGGL(bivariate[sphere][tables], grid, dim3(kBivThreads), 0, s, job, per * kBlk);
     else
-        hipLaunchKernelGGL(univariate[sphere][tables], grid, dim3(kThreads), 0, s, a);
+        hipLaunchKernelGGL(univariate[sphere][tables], grid, dim3(kThreads), 0, s, job, per * kBlk);
+}
+
+bool covgen_same_launch(const MaternParams &a, const MaternParams &b) {
+    return a.kernel == b.kernel && a.ntab == b.ntab && (a.metric == 1) == (b.metric == 1);
+}
+
+void launch_covgen_batch(const CovJob *jobs, const CovJob *h_jobs, int count, hipStream_t s) {
+    if (count <= 0) return;
+    const MaternParams &prm = h_jobs[0].prm;
+    if (prm.ntab > 0)
+        hipLaunchKernelGGL(matern_table_batch_kernel, dim3(kTableGroups, prm.ntab, count), dim3(kThreads), 0, s, jobs);
+    int64_t tiles = 0;
+    int most = 0;
+    for (int b = 0; b < count; ++b) {
+        tiles += h_jobs[b].npairs;
+        most = std::max(most, h_jobs[b].npairs);
+    }
+    const int nsb = h_jobs[0].map.ts / kBlk, per = covgen_blocks(nsb, tiles), parts = (nsb + per - 1) / per;
+    const dim3 grid(nsb, most, count * parts);
+    using Kernel = void (*)(const CovJob *, int, int);
+    static const Kernel univariate[2][2] = {
+        {covgen_tiles_batch_kernel<0, false>, covgen_tiles_batch_kernel<1, false>},
+        {covgen_tiles_batch_kernel<0, true>, covgen_tiles_batch_kernel<1, true>}};
+    static const Kernel bivariate[2][kTabSlots + 1] = {
+        {covgen_tiles_biv_batch_kernel<0, false>, covgen_tiles_biv_batch_kernel<1, false>,
+         covgen_tiles_biv_batch_kernel<2, false>, covgen_tiles_biv_batch_kernel<3, false>},
+        {covgen_tiles_biv_batch_kernel<0, true>, covgen_tiles_biv_batch_kernel<1, true>,
+         covgen_tiles_biv_batch_kernel<2, true>, covgen_tiles_biv_batch_kernel<3, true>}};
+    const bool sphere = prm.metric == 1;
+    if (prm.kernel == 1)
+        hipLaunchKernelGGL(bivariate[sphere][prm.ntab], grid, dim3(kBivThreads), 0, s, jobs, per * kBlk, parts);
+    else
+        hipLaunchKernelGGL(univariate[sphere][prm.ntab], grid, dim3(kThreads), 0, s, jobs, per * kBlk, parts);
 }
 
 void launch_covgen_rect(double *out, int rows, int cols, int64_t row_off, int64_t col_off, const MaternParams &prm,

@@ -15,7 +15,7 @@ namespace egs {
 // Cholesky on the tiles of `map`, with that problem's update order (pairs),
 // diagonal-block inverses of tile k, the tile column's ticket and flags
 // (launch_tile_column), not-SPD flag (n: its real dimension); with step 0, the
-// forward solve's vector, words (launch_solve_init) and partials.
+// forward solve's vector, words (launch_init) and partials.
 struct BatchJob {
     TileMap map;
     int k;
@@ -33,14 +33,29 @@ struct BatchJob {
 // Tables of the orders prm marks (MaternParams::tab) into tabs, kTabSlots of
 // kTabDoubles; prm_dev as in launch_covgen_tiles.
 void launch_matern_tables(double *tabs, const MaternParams &prm, const MaternParams *prm_dev, hipStream_t s);
-// tabs: the tables of prm (launch_matern_tables, earlier on the same stream).
-// sig64 (may be null): also writes every generated tile in FP64 to
-// sig64 + (i*(i+1)/2 + j) * ts * ts, column-major.
-// prm_dev, when given, holds the parameters in device memory (read instead of
-// prm, so that a captured launch can be replayed for another theta).
-void launch_covgen_tiles(const TileMap &map, const int2 *pairs, int npairs, const MaternParams &prm,
-                         const double *x, const double *y, const double *z, int64_t n, const double *tabs, double *sig64,
-                         hipStream_t s, const MaternParams *prm_dev = nullptr);
+// The lower tiles (i, j) of pairs; rows and columns >= n are identity padding.
+// loc.z may be null (2D).  tabs: the tables of prm (launch_matern_tables, earlier
+// on the same stream).  sig64 (may be null): also writes every generated tile in
+// FP64 to sig64 + (i*(i+1)/2 + j) * ts * ts, column-major.  prm_dev, when given,
+// holds the parameters in device memory (read instead of prm, so that a captured
+// launch can be replayed for another theta).
+struct CovJob {
+    TileMap map;
+    const int2 *pairs;
+    int npairs;
+    MaternParams prm;
+    Locs loc;
+    int64_t n;
+    double *tabs;
+    double *sig64;
+    const MaternParams *prm_dev;
+};
+void launch_covgen_tiles(const CovJob &job, hipStream_t s);
+// The tables and tiles of `count` jobs of one tile size, in device memory (and
+// h_jobs, the same on the host), that a launch can serve together: one table and
+// one covariance launch.  24 regions of 500-3,000, 18 with tables: 0.91 -> 0.19 ms.
+bool covgen_same_launch(const MaternParams &a, const MaternParams &b);
+void launch_covgen_batch(const CovJob *jobs, const CovJob *h_jobs, int count, hipStream_t s);
 void launch_covgen_rect(double *out, int rows, int cols, int64_t row_off, int64_t col_off, const MaternParams &prm,
                         const double *x1, const double *y1, const double *z1, const double *x2, const double *y2,
                         const double *z2, hipStream_t s);
@@ -65,9 +80,23 @@ bool update192_supported(int ts);
 void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s);
 
 // ---- triangular solves and reductions (egs_solve.hip)
-// z = src (n values) padded with zeros to npad, or as it is when src is null;
-// pending (npad + 1 doubles) emptied for the next solve.
-void launch_solve_init(double *z, const double *src, int64_t n, int64_t npad, double *pending, hipStream_t s);
+// What a factorization (sync, null for none) and a solve (pending, null for none)
+// start from: sync_ints zeros in sync, no failure in info; z = src (n values)
+// padded with zeros to npad, or as it is when src is null, and pending (npad + 1
+// doubles) emptied.
+struct InitJob {
+    int *sync;
+    int64_t sync_ints;
+    int *info;
+    double *z;
+    const double *src;
+    int64_t n, npad;
+    double *pending;
+};
+void launch_init(const InitJob &job, hipStream_t s);
+// Several jobs (device memory), `most` the largest extent of any (init_extent).
+int64_t init_extent(const InitJob &job);
+void launch_init_batch(const InitJob *jobs, int count, int64_t most, hipStream_t s);
 // z = L^{-1} z and z = L^{-T} z with the factor's tiles (mixed: some may be FP32)
 // and its diagonal-block inverses.  partials (may be null): of 64-row block b,
 // partials[2b] = sum log L_ii (L_ii > 0), partials[2b+1] = y_b . y_b.

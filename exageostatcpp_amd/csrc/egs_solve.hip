@@ -8,6 +8,8 @@
 // also writes sum(log L_ii) over L_ii > 0 and y_k . y_k for that tile.  The host
 // sums the per-tile partials in tile order, so results do not depend on
 // scheduling.  All reductions inside a workgroup use a fixed order.
+#include <algorithm>
+
 #include "egs_common.hpp"
 #include "egs_kernels.hpp"
 #include "egs_matern.hpp"
@@ -48,12 +50,6 @@ __device__ double wg_sum(double v, double *red) {
 // tile and a launch per panel, 2.8 and 7.8 ms.
 // ------------------------------------------------------------------------
 constexpr unsigned long long kPending = ~0ull;
-
-// The tile table, constant during a launch, through scalar loads: waiting for a
-// tile's address does not wait for the vector loads in flight.
-template <typename T> __device__ __forceinline__ T scalar_load(const T *p) {
-    return *reinterpret_cast<const __attribute__((address_space(4))) T *>(reinterpret_cast<uintptr_t>(p));
-}
 
 __device__ __forceinline__ double peek(const double *p) {
     return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const unsigned long long *>(p),
@@ -252,7 +248,7 @@ __global__ void __launch_bounds__(kThreads) forward_kernel(TileMap map, const do
 __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob *jobs, int njobs) {
     __shared__ SolveSmem sm;
     const int t = solve_ticket(jobs[0].pending, (int64_t) jobs[0].map.nt * jobs[0].map.ts, sm);
-    const BatchJob &J = jobs[t % njobs];
+    const BatchJob J = scalar_load(jobs + t % njobs);
     const int b = t / njobs;
     if (b >= J.map.blocks()) return;
     forward_block<false>(J.map, J.winv_k, J.z, J.pending, J.partials, b, sm);
@@ -433,13 +429,23 @@ __global__ void __launch_bounds__(kThreads) copy_pad_kernel(double *dst, const d
     if (i < npad) dst[i] = (i < n) ? src[i] : 0.0;
 }
 
-// A solve's right-hand side (src padded with zeros; z as it is when src is null)
-// and its empty words: npad of the solution and the ticket.
-__global__ void __launch_bounds__(kThreads) solve_init_kernel(double *z, const double *src, int64_t n, int64_t npad,
-                                                              double *pending) {
-    const int64_t i = (int64_t) blockIdx.x * kThreads + threadIdx.x;
-    if (src && i < npad) z[i] = (i < n) ? src[i] : 0.0;
-    if (i <= npad) reinterpret_cast<unsigned long long *>(pending)[i] = kPending;
+__device__ __forceinline__ void init_element(const InitJob &j, int64_t i) {
+    if (j.sync) {
+        if (i < j.sync_ints) j.sync[i] = 0;
+        if (i == 0) *j.info = 0;
+    }
+    if (j.pending) {
+        if (j.src && i < j.npad) j.z[i] = (i < j.n) ? j.src[i] : 0.0;
+        if (i <= j.npad) reinterpret_cast<unsigned long long *>(j.pending)[i] = kPending;
+    }
+}
+
+__global__ void __launch_bounds__(kThreads) init_kernel(InitJob job) {
+    init_element(job, (int64_t) blockIdx.x * kThreads + threadIdx.x);
+}
+
+__global__ void __launch_bounds__(kThreads) init_batch_kernel(const InitJob *jobs) {
+    init_element(jobs[blockIdx.y], (int64_t) blockIdx.x * kThreads + threadIdx.x);
 }
 
 // ------------------------------------------------------------------------
@@ -566,9 +572,18 @@ void launch_axpby(double *y, const double *x, double a, double b, int64_t n, hip
                        b, n);
 }
 
-void launch_solve_init(double *z, const double *src, int64_t n, int64_t npad, double *pending, hipStream_t s) {
-    hipLaunchKernelGGL(solve_init_kernel, dim3((unsigned) (npad / kThreads + 1)), dim3(kThreads), 0, s, z, src, n, npad,
-                       pending);
+int64_t init_extent(const InitJob &j) {
+    return std::max(j.sync ? j.sync_ints : 0, j.pending ? j.npad + 1 : 0);
+}
+
+void launch_init(const InitJob &job, hipStream_t s) {
+    const int64_t n = init_extent(job);
+    hipLaunchKernelGGL(init_kernel, dim3((unsigned) ((n + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, job);
+}
+
+void launch_init_batch(const InitJob *jobs, int count, int64_t most, hipStream_t s) {
+    hipLaunchKernelGGL(init_batch_kernel, dim3((unsigned) ((most + kThreads - 1) / kThreads), count), dim3(kThreads), 0,
+                       s, jobs);
 }
 
 void launch_forward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, double *partials,
