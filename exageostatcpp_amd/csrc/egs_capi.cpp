@@ -191,14 +191,16 @@ struct egs_problem_s {
     int2 *d_pairs = nullptr;
     double *d_winv = nullptr;
     int *d_sync = nullptr;      // tickets and flags of the tile columns' factorization (launch_tile_column)
-    double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr, *d_partials = nullptr;
-    int *d_info = nullptr;
+    double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr;
+    // Read back together: a word whose int is the failed minor (0: none), then
+    // the partials of the log-determinant and the quadratic form (launch_forward).
+    double *d_results = nullptr;
     double *d_tab = nullptr;    // Matern tables of the last covariance parameters (kTabSlots of them)
 
     std::vector<int64_t> h_off;
     std::vector<uint8_t> h_store;
     std::vector<int2> h_pairs;
-    std::vector<double> h_partials;
+    std::vector<double> h_results;
 
     bool has_obs = false;
     bool has_cov = false;    // the tiles hold Sigma(cov_theta), not yet factored
@@ -233,9 +235,12 @@ struct egs_problem_s {
     }
     // A factorization's tickets and flags, and a solve of src (null: of d_work).
     egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) const {
-        return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_info, d_work, src, count, npad,
+        return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_info(), d_work, src, count, npad,
                             solve ? d_aux : nullptr};
     }
+    int *d_info() const { return reinterpret_cast<int *>(d_results); }
+    double *d_partials() const { return d_results + 1; }
+    int result_count() const { return 1 + 2 * map().blocks(); }
     int ntheta() const { return kernel == 1 ? 6 : 3; }
     int64_t sync_ints() const { return (int64_t) nt * egs::tile_column_sync_ints(ts); }
     int *sync(int k) const { return d_sync + (int64_t) k * egs::tile_column_sync_ints(ts); }
@@ -375,8 +380,7 @@ void free_problem_buffers(egs_problem_s *p) {
     pfree(p, p->d_obs);
     pfree(p, p->d_work);
     pfree(p, p->d_aux);
-    pfree(p, p->d_partials);
-    pfree(p, p->d_info);
+    pfree(p, p->d_results);
     pfree(p, p->d_tab);
     for (auto &q : p->d_pairs_cls) {
         pfree(p, q);
@@ -427,8 +431,7 @@ void free_problem_buffers(egs_problem_s *p) {
     p->d_store = nullptr;
     p->d_pairs = nullptr;
     p->d_sync = nullptr;
-    p->d_winv = p->d_obs = p->d_work = p->d_aux = p->d_partials = nullptr;
-    p->d_info = nullptr;
+    p->d_winv = p->d_obs = p->d_work = p->d_aux = p->d_results = nullptr;
     p->d_tab = nullptr;
     for (auto &e : p->ev) e = nullptr;
 }
@@ -636,7 +639,7 @@ void factor_panel(egs_problem_s *p, int k) {
     // MFMA)
     const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(blocks64) && (blocks32 == 0 || p->f32_panel_solve);
     int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0);
-    egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info, p->n, fused ? blocks64 : 0, s);
+    egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info(), p->n, fused ? blocks64 : 0, s);
     prof_end(p, pi);
     if (k + 1 < nt) {
         double rows_below = 0.0;
@@ -711,8 +714,8 @@ void launch_mixed_update(egs_problem_s *p, int k, int jcol_lo, int jcol_hi, hipS
 // stream updates tile column k+1, factors it and solves its panel while the
 // bulk stream applies panel k to the columns beyond k+1.  The update order
 // lists tiles by descending column, so both tile sets are contiguous ranges of
-// it.  The caller checks d_info after synchronizing the critical stream, which
-// ends waiting for the bulk stream.
+// it.  The caller checks d_info after synchronizing the critical stream, whose
+// last step has waited for all of the bulk stream's work.
 // then_solve: the forward solve of the observations follows (run_forward is
 // told so), and what it starts from is prepared by the same launch.
 int run_potrf(egs_problem_s *p, bool then_solve = false) {
@@ -755,8 +758,9 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
             egs::launch_update(m, nullptr, p->d_pairs + n_beyond, n_next, k, true, s);
             prof_end(p, pi, s);
         }
-        EGS_HIP(hipEventRecord(p->ev_column[k], s));
+        if (beyond > 0) EGS_HIP(hipEventRecord(p->ev_column[k], s));
         factor_panel(p, k + 1);
+        if (beyond == 0) break;   // no bulk part; that of the step before, its last, was waited for above
         // Bulk step k: column k+2 first, then ev_bulk[k], then columns k+3 ..:
         // the critical stream's step k+1 needs only column k+2, so it overlaps
         // the rest of this step.  (The list holds columns in descending order:
@@ -778,26 +782,51 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
             prof_end(p, pi, b);
         }
     }
-    // ev_bulk[nt - 1] (unused by the steps) marks the end of the bulk stream;
-    // a one-tile matrix never uses it (and a capture must not wait on an event
-    // recorded outside it)
-    if (nt >= 2) {
-        EGS_HIP(hipEventRecord(p->ev_bulk[nt - 1], b));
-        EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[nt - 1], 0));
-    }
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;
 }
 
-int read_info(egs_problem_s *p) {
+// The first `count` words of d_results (result_count(): all), once the stream is
+// done with everything before: one copy behind the kernels, one wait (with a wait
+// first and a copy each for the failure and the partials, 400 locations took 242
+// us for 225 now; a batch of 24, read back problem by problem, 3.20 ms for 2.56).
+int read_results(egs_problem_s *p, int count) {
+    p->h_results.resize((size_t) p->result_count());
+    EGS_HIP(hipMemcpyAsync(p->h_results.data(), p->d_results, sizeof(double) * (size_t) count, hipMemcpyDeviceToHost,
+                           p->ctx->stream));
+    EGS_HIP(hipStreamSynchronize(p->ctx->stream));
+    return EGS_SUCCESS;
+}
+
+int info_of(const double *results) {
+    int info;
+    std::memcpy(&info, results, sizeof(int));
+    return info;
+}
+
+int check_info(egs_problem_s *p) {
     prof_collect(p);
-    int info = 0;
-    EGS_HIP(hipMemcpy(&info, p->d_info, sizeof(int), hipMemcpyDeviceToHost));
+    const int info = info_of(p->h_results.data());
     if (info != 0) {
         p->factored = false;
         return fail(EGS_ERR_NOT_SPD, "dpotrf failed, Matrix is not positive definite (leading minor %d)", info);
     }
     return EGS_SUCCESS;
+}
+
+int read_info(egs_problem_s *p) {
+    const int st = read_results(p, 1);
+    return st ? st : check_info(p);
+}
+
+void sum_partials(const egs_problem_s *p, const double *results, double &logdet, double &quad) {
+    double ld = 0.0, q = 0.0;
+    for (int b = 0; b < p->map().blocks(); ++b) {
+        ld += results[1 + 2 * b];
+        q += results[2 + 2 * b];
+    }
+    logdet = 2.0 * ld;
+    quad = q;
 }
 
 // d_work = L^{-1} src (src null: of d_work itself; prepared: by run_potrf); the
@@ -919,20 +948,6 @@ int refine_solve(egs_problem_s *p, const double *b) {
     return EGS_SUCCESS;
 }
 
-int read_partials(egs_problem_s *p, double &logdet, double &quad) {
-    const int blocks = p->map().blocks();
-    p->h_partials.resize((size_t) 2 * blocks);
-    EGS_HIP(hipMemcpy(p->h_partials.data(), p->d_partials, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost));
-    double ld = 0.0, q = 0.0;
-    for (int b = 0; b < blocks; ++b) {
-        ld += p->h_partials[2 * b];
-        q += p->h_partials[2 * b + 1];
-    }
-    logdet = 2.0 * ld;
-    quad = q;
-    return EGS_SUCCESS;
-}
-
 // A covariance tile request of egs_covariance_tile: only the locations the
 // tile touches are staged on the device, rows / P of the first set from
 // row_off / P on and cols / P of the second from col_off / P on.
@@ -1032,7 +1047,7 @@ int64_t footprint(const egs_problem_s &q) {
     int64_t b = dev_class_bytes(nb) * (q.dim == 3 ? 3 : 2) + dev_class_bytes(8 * nt * nt) + dev_class_bytes(nt * nt) +
                 dev_class_bytes(8 * ntiles) + dev_class_bytes(8 * nt * q.nsb * egs::kBlk * egs::kBlk) +
                 dev_class_bytes(4 * q.sync_ints()) + 2 * dev_class_bytes(vb) + dev_class_bytes(vb + 8) +
-                dev_class_bytes(16 * nt * q.nsb) + dev_class_bytes(4) +
+                dev_class_bytes(8 + 16 * nt * q.nsb) +
                 dev_class_bytes(8 * egs::kTabSlots * egs::kTabDoubles);
     int64_t arena = 0;
     for (int j = 0; j < q.nt; ++j)
@@ -1200,8 +1215,7 @@ int egs_problem_create(egs_context_t ctx, int kernel, int64_t n_loc, const doubl
               pmalloc(p, &p->d_sync, sizeof(int) * (size_t) p->sync_ints()) == hipSuccess &&
               pmalloc(p, &p->d_obs, vb) == hipSuccess && pmalloc(p, &p->d_work, vb) == hipSuccess &&
               pmalloc(p, &p->d_aux, vb + sizeof(double)) == hipSuccess &&
-              pmalloc(p, &p->d_partials, sizeof(double) * 2 * (size_t) nt * p->nsb) == hipSuccess &&
-              pmalloc(p, &p->d_info, sizeof(int)) == hipSuccess &&
+              pmalloc(p, &p->d_results, sizeof(double) * (1 + 2 * (size_t) nt * p->nsb)) == hipSuccess &&
               pmalloc(p, &p->d_tab, sizeof(double) * egs::kTabSlots * egs::kTabDoubles) == hipSuccess;
     if (!ok) return cleanup(fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the problem's device buffers"));
     for (auto &e : p->ev)
@@ -1385,7 +1399,6 @@ int egs_potrf(egs_problem_t p) {
     if (!p->has_cov) return fail(EGS_ERR_STATE, "no covariance matrix to factor: call egs_covariance first");
     st = run_potrf(p);
     if (st) return st;
-    EGS_HIP(hipStreamSynchronize(p->ctx->stream));
     st = read_info(p);
     if (st) return st;
     p->factored = true;
@@ -1399,13 +1412,12 @@ int egs_solve_logdet_quad(egs_problem_t p, double *logdet, double *quad) {
     if (!p->has_obs) return fail(EGS_ERR_STATE, "the problem has no observations");
     if (!p->factored) return fail(EGS_ERR_STATE, "no factored matrix: call egs_potrf first");
     hipStream_t s = p->ctx->stream;
-    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials, s);   // quad from the refinement
-    else run_forward(p, p->d_obs, p->n, p->d_partials);
+    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials(), s);   // quad from the refinement
+    else run_forward(p, p->d_obs, p->n, p->d_partials());
     EGS_HIP(hipGetLastError());
-    EGS_HIP(hipStreamSynchronize(s));
+    if ((st = read_results(p, p->result_count()))) return st;
     double ld, q;
-    st = read_partials(p, ld, q);
-    if (st) return st;
+    sum_partials(p, p->h_results.data(), ld, q);
     if (is_mixed(p)) {
         if ((st = refine_solve(p, p->d_obs))) return st;
         if ((st = host_dot(p, p->d_obs, p->d_cg, q))) return st;
@@ -1447,7 +1459,7 @@ int enqueue_fp64_eval(egs_problem_s *p) {
     egs::launch_covgen_tiles(p->cov_job(p->h_prm, nullptr, p->d_prm), s);
     const int st = run_potrf(p, true);
     if (st) return st;
-    run_forward(p, p->d_obs, p->n, p->d_partials, true);
+    run_forward(p, p->d_obs, p->n, p->d_partials(), true);
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;
 }
@@ -1513,10 +1525,9 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
         if (st) return st;
         p->has_cov = false;   // the replay factored the tiles
         EGS_HIP(hipEventRecord(p->ev[3], s));
-        EGS_HIP(hipStreamSynchronize(s));
+        if ((st = read_results(p, p->result_count()))) return st;
         std::memcpy(p->cov_theta, theta, sizeof(double) * p->ntheta());
-        st = read_info(p);
-        if (st) return st;
+        if ((st = check_info(p))) return st;
         p->factored = true;
         std::memcpy(p->factored_theta, theta, sizeof(double) * p->ntheta());
         float ms = 0;
@@ -1524,8 +1535,7 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
         p->t_cov = p->t_solve = 0.0;   // one graph: only the total is timed
         p->t_fact = ms;
         double ld, q;
-        st = read_partials(p, ld, q);
-        if (st) return st;
+        sum_partials(p, p->h_results.data(), ld, q);
         *loglik = -0.5 * q - 0.5 * ld - (double) p->n / 2.0 * std::log(2.0 * kPi);
         if (logdet) *logdet = ld;
         if (quad) *quad = q;
@@ -1538,13 +1548,12 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
     st = run_potrf(p, !is_mixed(p));
     if (st) return st;
     EGS_HIP(hipEventRecord(p->ev[2], s));
-    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials, s);   // quad from the refinement
-    else run_forward(p, p->d_obs, p->n, p->d_partials, true);
+    if (is_mixed(p)) egs::launch_diag_logdet(p->map(), p->d_partials(), s);   // quad from the refinement
+    else run_forward(p, p->d_obs, p->n, p->d_partials(), true);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipEventRecord(p->ev[3], s));
-    EGS_HIP(hipStreamSynchronize(s));
-    st = read_info(p);
-    if (st) return st;
+    if ((st = read_results(p, p->result_count()))) return st;
+    if ((st = check_info(p))) return st;
     p->factored = true;
     std::memcpy(p->factored_theta, theta, sizeof(double) * p->ntheta());
     float ms = 0;
@@ -1555,8 +1564,7 @@ static int loglik_once(egs_problem_s *p, const double *theta, double *loglik, do
     hipEventElapsedTime(&ms, p->ev[2], p->ev[3]);
     p->t_solve = ms;
     double ld, q;
-    st = read_partials(p, ld, q);
-    if (st) return st;
+    sum_partials(p, p->h_results.data(), ld, q);
     if (is_mixed(p)) {
         // z' Sigma^{-1} z from the refined FP64 solution instead of ||L^{-1} z||^2
         st = refine_solve(p, p->d_obs);
@@ -1616,6 +1624,7 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
     for (int k = 0; k < max_nt; ++k) first[k + 1] = first[k] + active[k];
     const int64_t njobs = first[max_nt];
     std::vector<egs::BatchJob> jobs((size_t) std::max<int64_t>(njobs, 1));
+    std::vector<double> results;
     for (int k = 0; k < max_nt; ++k)
         for (int a = 0; a < active[k]; ++a) {
             egs_problem_s *p = problems[run[a]];
@@ -1625,11 +1634,9 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             J.pairs = p->d_pairs;
             J.winv_k = p->winv(k);
             J.sync = p->sync(k);
-            J.info = p->d_info;
             J.n = p->n;
             J.z = p->d_work;
             J.pending = p->d_aux;
-            J.partials = p->d_partials;
         }
     if (na > 0) {
         EGS_HIP(hipSetDevice(ctx->device));
@@ -1658,23 +1665,36 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
             p->factored = false;
             invalidate_graph(p);
         }
+        // every problem's results side by side, read back in one copy
+        std::vector<int64_t> result_at(na + 1, 0);
+        for (int a = 0; a < na; ++a) result_at[a + 1] = result_at[a] + problems[run[a]]->result_count();
         const size_t job_bytes = sizeof(egs::BatchJob) * (size_t) njobs, cov_bytes = sizeof(egs::CovJob) * (size_t) na,
                      init_bytes = sizeof(egs::InitJob) * (size_t) na;
-        std::vector<char> records(job_bytes + cov_bytes + init_bytes);
-        std::memcpy(records.data(), jobs.data(), job_bytes);
-        std::memcpy(records.data() + job_bytes, cov.data(), cov_bytes);
-        std::memcpy(records.data() + job_bytes + cov_bytes, init.data(), init_bytes);
-        if ((int64_t) records.size() > ctx->jobs_cap) {
+        const size_t record_bytes = (job_bytes + cov_bytes + init_bytes + 7) & ~size_t(7);
+        const size_t result_bytes = sizeof(double) * (size_t) result_at[na];
+        std::vector<char> records(record_bytes);
+        if ((int64_t) (record_bytes + result_bytes) > ctx->jobs_cap) {
             EGS_HIP(hipStreamSynchronize(s));
             egs::dev_free(ctx->d_jobs, &ctx->dev_bytes);
             ctx->d_jobs = nullptr;
             ctx->jobs_cap = 0;
             void *v = nullptr;
-            if (egs::dev_alloc(&v, records.size(), &ctx->dev_bytes) != hipSuccess)
+            if (egs::dev_alloc(&v, record_bytes + result_bytes, &ctx->dev_bytes) != hipSuccess)
                 return fail(EGS_ERR_OUT_OF_MEMORY, "egs_loglik_batch: cannot allocate the job records");
             ctx->d_jobs = static_cast<char *>(v);
-            ctx->jobs_cap = (int64_t) records.size();
+            ctx->jobs_cap = (int64_t) (record_bytes + result_bytes);
         }
+        double *d_results = reinterpret_cast<double *>(ctx->d_jobs + record_bytes);
+        for (int k = 0; k < max_nt; ++k)
+            for (int a = 0; a < active[k]; ++a) {
+                egs::BatchJob &J = jobs[(size_t) (first[k] + a)];
+                J.info = reinterpret_cast<int *>(d_results + result_at[a]);
+                J.partials = d_results + result_at[a] + 1;
+            }
+        for (int a = 0; a < na; ++a) init[a].info = reinterpret_cast<int *>(d_results + result_at[a]);
+        std::memcpy(records.data(), jobs.data(), job_bytes);
+        std::memcpy(records.data() + job_bytes, cov.data(), cov_bytes);
+        std::memcpy(records.data() + job_bytes + cov_bytes, init.data(), init_bytes);
         // the previous batch on this context has completed (every call returns synchronized)
         EGS_HIP(hipMemcpyAsync(ctx->d_jobs, records.data(), records.size(), hipMemcpyHostToDevice, s));
         const auto *d_steps = reinterpret_cast<const egs::BatchJob *>(ctx->d_jobs);
@@ -1688,22 +1708,23 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
         }
         egs::launch_forward_batch(d_steps, na, ts, max_nt, s);
         EGS_HIP(hipGetLastError());
+        results.resize((size_t) result_at[na]);
+        EGS_HIP(hipMemcpyAsync(results.data(), d_results, result_bytes, hipMemcpyDeviceToHost, s));
         EGS_HIP(hipStreamSynchronize(s));
     }
+    const double *result = results.data();
     for (int b : run) {
         egs_problem_s *p = problems[b];
         prof_collect(p);
-        int info = 0;
+        const double *r = result;
+        result += p->result_count();
+        const int info = info_of(r);
         double ld = 0.0, q = 0.0;
-        if (hipMemcpy(&info, p->d_info, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
-            status[b] = fail(EGS_ERR_HIP, "egs_loglik_batch: reading the factorization status failed");
-            continue;
-        }
         if (info != 0) {
             status[b] = fail(EGS_ERR_NOT_SPD, "dpotrf failed, Matrix is not positive definite (leading minor %d)", info);
             continue;
         }
-        if ((status[b] = read_partials(p, ld, q)) != EGS_SUCCESS) continue;
+        sum_partials(p, r, ld, q);
         p->factored = true;
         std::memcpy(p->factored_theta, thetas + 6 * b, sizeof(double) * p->ntheta());
         std::memcpy(p->cov_theta, thetas + 6 * b, sizeof(double) * p->ntheta());
@@ -1928,14 +1949,15 @@ static int generate_observations_fp64(egs_problem_s *p, const double *theta, int
     if (st) return st;
     egs::launch_trmv(p->map(), p->d_aux, p->d_work, s);
     EGS_HIP(hipGetLastError());
-    EGS_HIP(hipStreamSynchronize(s));
     st = read_info(p);
     if (st) return st;
     p->factored = true;
     std::memcpy(p->factored_theta, theta, sizeof(double) * p->ntheta());
-    EGS_HIP(hipMemcpy(p->d_obs, p->d_work, sizeof(double) * (size_t) p->n, hipMemcpyDeviceToDevice));
+    const size_t bytes = sizeof(double) * (size_t) p->n;
+    EGS_HIP(hipMemcpyAsync(p->d_obs, p->d_work, bytes, hipMemcpyDeviceToDevice, s));
     p->has_obs = true;
-    if (z_out) EGS_HIP(hipMemcpy(z_out, p->d_obs, sizeof(double) * (size_t) p->n, hipMemcpyDeviceToHost));
+    if (z_out) EGS_HIP(hipMemcpyAsync(z_out, p->d_work, bytes, hipMemcpyDeviceToHost, s));
+    EGS_HIP(hipStreamSynchronize(s));
     return EGS_SUCCESS;
 }
 
