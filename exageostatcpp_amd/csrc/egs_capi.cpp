@@ -235,8 +235,8 @@ struct egs_problem_s {
     }
     // A factorization's tickets and flags, and a solve of src (null: of d_work).
     egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) const {
-        return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_info(), d_work, src, count, npad,
-                            solve ? d_aux : nullptr};
+        return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_winv, (int64_t) map().blocks() * egs::kBlk * egs::kBlk,
+                            d_info(), d_work, src, count, npad, solve ? d_aux : nullptr};
     }
     int *d_info() const { return reinterpret_cast<int *>(d_results); }
     double *d_partials() const { return d_results + 1; }

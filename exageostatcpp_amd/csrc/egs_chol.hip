@@ -106,6 +106,11 @@ __device__ __forceinline__ void lds_product(Acc<CT, kRows> &acc, const CT *a, co
     }
 }
 
+template <bool kShared> __device__ __forceinline__ double load_as(const double *p) {
+    if constexpr (kShared) return load_shared(p);
+    else return *p;
+}
+
 // acc += A (kRows x K, column-major, lda) * B (64 x K, column-major, ldb)^T; K a
 // multiple of 64.  K chunks of 32 columns go through LDS, double buffered; two
 // chunks' loads are in flight in registers while one is multiplied (these
@@ -114,7 +119,7 @@ __device__ __forceinline__ void lds_product(Acc<CT, kRows> &acc, const CT *a, co
 // products (below): the panel solve of 60 row blocks of 960 columns 268 -> 246
 // us, one evaluation of 1,600 locations 0.85 -> 0.79 ms, of 20,000 55.4 ->
 // 53.8 ms.
-template <typename CT, int kRows, typename TA>
+template <typename CT, int kRows, bool kShared = false, typename TA>
 __device__ void wg_gemm_nt(Acc<CT, kRows> &acc, const TA *__restrict__ A, int64_t lda, const double *__restrict__ B,
                            int64_t ldb, int K, Smem<CT> &sm) {
     constexpr int kA = kRows * kKc / kThreads, kB = kBlk * kKc / kThreads;   // elements per thread and chunk
@@ -130,7 +135,7 @@ __device__ void wg_gemm_nt(Acc<CT, kRows> &acc, const TA *__restrict__ A, int64_
 #pragma unroll
         for (int q = 0; q < kA; ++q) ra[set][q] = Ap[(k0 + q * (kThreads / kRows)) * lda];
 #pragma unroll
-        for (int q = 0; q < kB; ++q) rb[set][q] = Bp[(k0 + q * (kThreads / kBlk)) * ldb];
+        for (int q = 0; q < kB; ++q) rb[set][q] = load_as<kShared>(Bp + (k0 + q * (kThreads / kBlk)) * ldb);
     };
     auto stage = [&](int set) {
 #pragma unroll
@@ -191,14 +196,14 @@ __device__ __forceinline__ void solve_rows(const double *T, int ts, int nsb, TX 
             for (int q = 0; q < 16; ++q) wv[q] = W[row + (w + 4 * q) * kBlk];
         if (jb > 0) {
             wait.row(jb);
-            wg_gemm_nt<CT, kRows>(acc, X, ts, T + jb * kBlk, ts, jb * kBlk, sm);
+            wg_gemm_nt<CT, kRows, !Wait::kAhead>(acc, X, ts, T + jb * kBlk, ts, jb * kBlk, sm);
         }
         e = 0;
         acc_foreach(acc, [&](int r, int c, CT v) { sT[c * kLdsPad + r] = (CT) xv[e++] - v; });
         if (!Wait::kAhead) {
             wait.inverse(jb);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) wv[q] = W[row + (w + 4 * q) * kBlk];
+            for (int q = 0; q < 16; ++q) wv[q] = load_shared(W + row + (w + 4 * q) * kBlk);
         }
 #pragma unroll
         for (int q = 0; q < 16; ++q) sW[(w + 4 * q) * kLdsPad + row] = (CT) wv[q];
@@ -447,8 +452,10 @@ __device__ __forceinline__ void panel_tile(double *sD, double *sE, const double 
 }
 
 // s_piv: 2 * 64 + 2 * 16 doubles.  Thread 0 gets the first column without a
-// positive pivot (-1: none).
-__device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv, double *s_rs) {
+// positive pivot (-1: none).  Wave 3 calls beside(p) at the start of panel p:
+// rows 0 .. 16 p - 1 of the inverse are there by then.
+template <typename Beside>
+__device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv, double *s_rs, const Beside &beside) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave index, held in a scalar register
     const int lr = lane & 15;
@@ -477,6 +484,7 @@ __device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv
             }
         } else {
             __syncthreads();
+            if (w == 3) beside(p);
             // the columns beyond panel p, minus panel p - 1
             int idx = 0;
             if (p > 0)
@@ -514,15 +522,21 @@ __device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv
 //                        then the tasks (r, c), r >= c + 2 (one block each);
 //   after them           the 32-row blocks below the tile, all block columns.
 // A task adds up its blocks' products with the earlier block columns as those
-// are published (flags in `sync`, one per block, zero at the launch), so that
-// a diagonal task has only X = T W^T, D -= X X^T and the factorization left
-// when the inverse before it arrives.  Bound: that chain, 20 us per 64 columns
-// alone (7.8 us of it the factorization, the rest two 64 x 64 x 64 products, the
-// loads and the flag).  One launch per block column (each waiting anew for room
-// beside the trailing update), a copy, and the panel solve after the whole tile
-// took 36 us per 64 columns alone, 90 to 140 us beside the trailing update, plus
-// 40 (ts 320) to 440 us (ts 960) for the panel.  One evaluation: 400 locations
-// 0.54 -> 0.34 ms, 1,600 1.41 -> 0.83 ms, 10,007 14.8 -> 13.2 ms.
+// are published (flags in `sync`, one per block, zero at the launch).  The inverse
+// comes in four panels of 16 rows while its block is still being factored (its
+// words are their own flags, empty at the launch), and X = T W^T and D -= X X^T
+// follow panel by panel, so that a diagonal task has only a quarter of both left
+// when the last rows arrive.  What is handed over is stored and loaded past the
+// L2s, without fences: a release or acquire fence of agent scope writes back or
+// invalidates the L2 of its XCD, with everything the trailing update has there.
+// Bound: the chain of diagonal tasks, 14.4 us per 64 columns alone (7.8 us of it
+// the factorization, the rest the way of the last rows through memory, a quarter
+// of two products and the exchange through LDS); with the whole inverse published
+// at the end, between fences, 19 us.  Tile of 960 alone 284 -> 218 us, with 60
+// row blocks below 372 -> 310 us, of 384 109 -> 86 us; 400 locations 225 -> 194
+// us, 1,600 674 -> 568 us.  One launch per block column (each waiting anew for
+// room beside the trailing update), a copy, and the panel solve after the whole
+// tile took 36 us per 64 columns alone, 90 to 140 us beside the trailing update.
 // ------------------------------------------------------------------------
 namespace {
 
@@ -534,28 +548,25 @@ struct PanelSmem {
 };
 static_assert(sizeof(GemmSmem) <= sizeof(PanelSmem), "the row blocks stage through the same LDS");
 
-// Waits until another workgroup of the launch has published the block.
-__device__ __forceinline__ void wait_block(const int *flag) {
-    if (threadIdx.x == 0) {
-        while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) __builtin_amdgcn_s_sleep(1);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    __syncthreads();
+// A flag says that the stores of a wave (store_shared) are complete.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void set_flag(int *flag) {
+    __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Publishes what the workgroup has stored.
-__device__ __forceinline__ void publish_block(int *flag) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Waits, wave by wave, until the flag is set.
+__device__ __forceinline__ void wait_flag(const int *flag) {
+    while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
+        __builtin_amdgcn_s_sleep(1);
+    asm volatile("" ::: "memory");
 }
 
-// A 64 x 64 block of a column-major matrix into LDS, in flight as 16 loads per
-// thread.
+// A published 64 x 64 block of a column-major matrix into LDS, in flight as 16
+// loads per thread.
 __device__ __forceinline__ void load_block(double (&v)[16], const double *src, int64_t ld) {
     const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = src[row + (int64_t) (w + 4 * q) * ld];
+    for (int q = 0; q < 16; ++q) v[q] = load_shared(src + row + (int64_t) (w + 4 * q) * ld);
 }
 __device__ __forceinline__ void put_block(double *s, const double (&v)[16]) {
     const int row = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -589,69 +600,179 @@ __device__ __forceinline__ void acc_load(Acc64 &acc, const double *C, int64_t ld
             for (int v = 0; v < 4; ++v) acc.v[ni][mi][v] = C[r + mi * 16 + (int64_t) (c + ni * 16 + 4 * v) * ld];
 }
 
-// Block (r, c) of the tile T (ld ts), r > c: solved in place and published;
-// its columns stay in sm.a.  With acc_d, acc_d -= L_rb L_rb^T for every b <= c.
-// The products are subtracted from the block itself, one MFMA after another:
-// the residual shrinks as they go, and with it the rounding (summing them
-// first rounds at the size of the block).
-__device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, int c, const double *winv_k, int *flags,
-                                            PanelSmem &sm, Acc64 *acc_d) {
-    double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
-    double va[16], vb[16];
-    Acc64 acc;
-    acc_load(acc, X, ts);
-    for (int b = 0; b < c; ++b) {
-        wait_block(flags + r * nsb + b);
-        wait_block(flags + c * nsb + b);
-        load_block(va, T + r * kBlk + (int64_t) b * kBlk * ts, ts);
-        load_block(vb, T + c * kBlk + (int64_t) b * kBlk * ts, ts);
-        put_block(sm.a, va);
-        put_block(sm.b, vb);
-        __syncthreads();
-        subtract_block(acc, sm.a, sm.b);
-        if (acc_d) subtract_block(*acc_d, sm.a, sm.a);
-        __syncthreads();
+// The lower 16 x 16 tiles of a diagonal block, ten, dealt to the waves: tile w +
+// 4 q of the rows' order (waves 2 and 3 carry the last one along as their third,
+// of no effect: a branch around it cost as much, and the compiler then counted
+// the products' latency wrong across it, which gave wrong results).
+struct DiagAcc {
+    f64x4 v[3];
+    static __device__ __forceinline__ int tile(int w, int q) { return 4 * min(w + 4 * q, 9); }
+    static __device__ __forceinline__ int row(int w, int q) { return (int) (0x3333222110ull >> tile(w, q) & 15) * 16; }
+    static __device__ __forceinline__ int col(int w, int q) { return (int) (0x3210210100ull >> tile(w, q) & 15) * 16; }
+
+    // every element's value becomes f(row, col, value)
+    template <typename F> __device__ __forceinline__ void foreach(int w, F f) {
+        const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[q][e] = f(row(w, q) + lr, col(w, q) + lk + 4 * e, v[q][e]);
     }
-    acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
-    wait_block(flags + c * nsb + c);
-    load_block(vb, winv_k + (int64_t) c * kBlk * kBlk, kBlk);
-    put_block(sm.b, vb);
-    __syncthreads();
-    acc_zero(acc);
-    lds_product<double, 64, kBlk>(acc, sm.a, sm.b);
-    __syncthreads();
-    acc_foreach(acc, [&](int i, int j, double v) {
-        X[i + (int64_t) j * ts] = v;
-        sm.a[j * kPv + i] = v;
-    });
-    if (acc_d) {
-        __syncthreads();
-        subtract_block(*acc_d, sm.a, sm.a);
+    // minus X X^T for K columns of X in LDS
+    template <int K> __device__ __forceinline__ void subtract(int w, const double *x) {
+        const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll 4
+        for (int kk = 0; kk < K; kk += 4) {
+            const double *xk = x + (kk + lk) * kPv + lr;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v[q] = mfma_f64(xk[col(w, q)], -xk[row(w, q)], v[q]);
+        }
     }
-    publish_block(flags + r * nsb + c);
+};
+
+// Block (r, c) of the tile T (ld ts), r > c, solved in place: X = T W^T in panels
+// of 16 columns, as the inverse's rows come.  Without kDia it is published; with
+// it, dia -= L_rb L_rb^T for every b <= c, and the last panel stays in LDS
+// (last_panel) for the caller to store and publish.  The products are subtracted
+// from the block itself, one MFMA after another: the residual shrinks as they go,
+// and with it the rounding (summing them first rounds at the size of the block).
+__device__ __forceinline__ double *last_panel(PanelSmem &sm) { return sm.b + 16 * kPv; }
+
+// Columns 16 P .. 16 P + 15 of X; W, t, out: this lane's element of each.
+template <bool kDia, int P>
+__device__ __forceinline__ void solve_panel(const double *W, const double *t, double *out, int ts, int w, PanelSmem &sm,
+                                            DiagAcc &dia) {
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    constexpr int kSteps = 4 * (P + 1);
+    double wv[kSteps];
+    bool waiting;
+    do {
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) wv[q] = load_shared(W + kPan * P + 4 * q * kBlk);
+        waiting = false;
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) waiting |= is_pending(wv[q]);
+    } while (__ballot(waiting) != 0);
+    f64x4 x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < kSteps; ++q) x = mfma_f64(wv[q], t[4 * q * kPv], x);
+    if (kDia) {
+        double *s = sm.b + (P & 1) * kPan * kPv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[(lk + 4 * e) * kPv + 16 * w + lr] = x[e];
+        __syncthreads();
+        dia.subtract<kPan>(w, s);
+    }
+    if (!kDia || P < 3) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_shared(out + (int64_t) (kPan * P + 4 * e) * ts, x[e]);
+    }
 }
+
+template <bool kDia>
+__device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, int c, const double *winv_k, int *flags,
+                                            PanelSmem &sm, DiagAcc &dia) {
+    double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
+    const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    {
+        double va[16], vb[16];
+        Acc64 acc;
+        acc_load(acc, X, ts);
+        for (int b = 0; b < c; ++b) {
+            wait_flag(flags + r * nsb + b);
+            load_block(va, T + r * kBlk + (int64_t) b * kBlk * ts, ts);
+            wait_flag(flags + c * nsb + b);
+            load_block(vb, T + c * kBlk + (int64_t) b * kBlk * ts, ts);
+            put_block(sm.a, va);
+            put_block(sm.b, vb);
+            __syncthreads();
+            subtract_block(acc, sm.a, sm.b);
+            if (kDia) dia.subtract<kBlk>(w, sm.a);
+            __syncthreads();
+        }
+        acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
+        __syncthreads();
+    }
+    const double *W = winv_k + (int64_t) c * kBlk * kBlk + lr + lk * kBlk;
+    const double *t = sm.a + lk * kPv + 16 * w + lr;
+    double *out = X + 16 * w + lr + (int64_t) lk * ts;
+    solve_panel<kDia, 0>(W, t, out, ts, w, sm, dia);
+    solve_panel<kDia, 1>(W, t, out, ts, w, sm, dia);
+    solve_panel<kDia, 2>(W, t, out, ts, w, sm, dia);
+    solve_panel<kDia, 3>(W, t, out, ts, w, sm, dia);
+    if (!kDia) {
+        wait_stores();
+        __syncthreads();
+        if (threadIdx.x == 0) set_flag(flags + r * nsb + c);
+    }
+}
+
+// Rows 16 p .. 16 p + 15 of the inverse, columns lk + 4 q for q in [q0, q1), from
+// L^{-T} and the pivots in LDS.
+__device__ __forceinline__ void store_inverse_rows(double *W, const PanelSmem &sm, int p, int q0, int q1) {
+    const int i = kPan * p + (threadIdx.x & 15), lk = (threadIdx.x & 63) >> 4;
+    const double rsi = rsqrt_f64(sm.piv[2 * i + 1]);
+#pragma unroll 4
+    for (int q = q0; q < q1; ++q) {
+        const int j = lk + 4 * q;
+        store_word(W + i + j * kBlk, i >= j ? sm.b[j * kPv + i] * rsi : 0.0);
+    }
+}
+
+// What wave 3 hands out while a diagonal block is factored: the last panel of the
+// block left of it, then the inverse's rows, a panel behind.  It waits for none
+// of its stores where the factorization would wait for it.
+struct HandOut {
+    double *W, *X;   // X null for the first block
+    int ts;
+    PanelSmem &sm;
+    int *x_flag;
+    __device__ __forceinline__ void operator()(int p) const {
+        const int lane = threadIdx.x & 63;
+        if (p == 0 && X) {
+            const double *s = last_panel(sm) + lane;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) store_shared(X + lane + (int64_t) (48 + q) * ts, s[q * kPv]);
+        }
+        if (p == 1 && X) {
+            wait_stores();
+            if (lane == 0) set_flag(x_flag);
+        }
+        if (p > 0) store_inverse_rows(W, sm, p - 1, 0, 16);
+    }
+};
 
 // Diagonal task r: block (r, r - 1), then block (r, r) factored and inverted.
 __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r, double *winv_k, int *flags, int *info,
                                               int64_t col0, int64_t n, PanelSmem &sm) {
     double *D = T + r * kBlk + (int64_t) r * kBlk * ts;
-    Acc64 acc_d;
-    acc_load(acc_d, D, ts);
-    if (r > 0) solve_block(T, ts, nsb, r, r - 1, winv_k, flags, sm, &acc_d);
-    acc_foreach(acc_d, [&](int i, int j, double v) { sm.a[i * kPv + j] = v; });
-    __syncthreads();
-    const int bad = potrf64_lds(sm.a, sm.b, sm.piv, sm.rs);
-    if (threadIdx.x == 0 && bad >= 0 && col0 + r * kBlk + bad < n) atomicCAS(info, 0, (int) (col0 + r * kBlk + bad + 1));
     double *W = winv_k + (int64_t) r * kBlk * kBlk;
-    const int i = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    DiagAcc dia;
+    dia.foreach(w, [&](int i, int j, double) { return D[i + (int64_t) j * ts]; });
+    if (r > 0) {
+        solve_block<true>(T, ts, nsb, r, r - 1, winv_k, flags, sm, dia);
+        wait_stores();   // the panels before the last: long done
+    }
+    dia.foreach(w, [&](int i, int j, double v) { return sm.a[i * kPv + j] = v; });
+    __syncthreads();
+    const HandOut beside{W, r > 0 ? D - (int64_t) kBlk * ts : nullptr, ts, sm, flags + r * nsb + r - 1};
+    const int bad = potrf64_lds(sm.a, sm.b, sm.piv, sm.rs, beside);
+    store_inverse_rows(W, sm, kBlk / kPan - 1, 4 * w, 4 * w + 4);
+    wait_stores();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        set_flag(flags + r * nsb + r);
+        if (bad >= 0 && col0 + r * kBlk + bad < n) atomicCAS(info, 0, (int) (col0 + r * kBlk + bad + 1));
+    }
+    const int i = threadIdx.x & 63;
     const double rsi = sm.rs[i];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int j = w + 4 * q;
-        W[i + j * kBlk] = i >= j ? sm.b[j * kPv + i] * rsi : 0.0;
         D[i + (int64_t) j * ts] = i > j ? sm.a[i * kPv + j] * sm.rs[j] : i == j ? sm.piv[2 * j + 1] * rsi : 0.0;
     }
-    publish_block(flags + r * nsb + r);
 }
 
 // What a row block below the tile waits for (the diagonal task of block column
@@ -660,8 +781,8 @@ struct BlockWait {
     static constexpr bool kAhead = false;
     const int *flags;
     int nsb;
-    __device__ __forceinline__ void row(int j) const { wait_block(flags + j * nsb + j - 1); }
-    __device__ __forceinline__ void inverse(int j) const { wait_block(flags + j * nsb + j); }
+    __device__ __forceinline__ void row(int j) const { wait_flag(flags + j * nsb + j - 1); }
+    __device__ __forceinline__ void inverse(int j) const { wait_flag(flags + j * nsb + j); }
 };
 
 // Tasks of a diagonal tile of so many 64 x 64 blocks.
@@ -691,10 +812,12 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
         idx -= 1 + max(0, live - 2 - c);
         ++c;
     }
-    if (idx == 0)
+    if (idx == 0) {
         diagonal_task(T, ts, nsb, c, winv_k, flags, info, (int64_t) k * ts, n, sm);
-    else
-        solve_block(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, nullptr);
+    } else {
+        DiagAcc none;
+        solve_block<false>(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, none);
+    }
 }
 
 __device__ __forceinline__ int take_ticket(int *counter) {

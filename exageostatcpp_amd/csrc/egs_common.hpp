@@ -64,6 +64,25 @@ template <typename T> __device__ __forceinline__ T scalar_load(const T *p) {
     return u.v;
 }
 
+// What workgroups of one launch hand each other goes past the L2s, each of which
+// belongs to an XCD: stored and loaded at agent scope.  A word that holds ~0
+// (kPending) has not been stored yet, so that the value is its own flag; a NaN of
+// that pattern is stored as another one.
+constexpr unsigned long long kPending = ~0ull;
+
+__device__ __forceinline__ double load_shared(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool is_pending(double v) {
+    return __builtin_bit_cast(unsigned long long, v) == kPending;
+}
+__device__ __forceinline__ void store_shared(double *p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_word(double *p, double v) {
+    store_shared(p, is_pending(v) ? __builtin_bit_cast(double, 0x7ff8000000000000ull) : v);
+}
+
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin (workgroup w
 // runs on XCD w % 8), and each XCD has its own L2.  xcd_remap gives XCD x a
 // contiguous range of the logical block order, so blocks that share operand

@@ -81,12 +81,14 @@ void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, 
 
 // ---- triangular solves and reductions (egs_solve.hip)
 // What a factorization (sync, null for none) and a solve (pending, null for none)
-// start from: sync_ints zeros in sync, no failure in info; z = src (n values)
-// padded with zeros to npad, or as it is when src is null, and pending (npad + 1
-// doubles) emptied.
+// start from: sync_ints zeros in sync, winv_words empty words (kPending) of the
+// inverses, no failure in info; z = src (n values) padded with zeros to npad, or
+// as it is when src is null, and pending (npad + 1 doubles) emptied.
 struct InitJob {
     int *sync;
     int64_t sync_ints;
+    double *winv;
+    int64_t winv_words;
     int *info;
     double *z;
     const double *src;
@@ -118,7 +120,8 @@ int matvec_chunks(int64_t n);
 // its diagonal blocks in winv_k, and the panel solve of the first `blocks` 64-row
 // blocks below it, FP64 ones (tile_column_solves_rows: whether that many should
 // be; the others take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
-// tile_column_sync_ints(ts) ints, zero before the launch.
+// tile_column_sync_ints(ts) ints, zero before the launch, winv_k empty
+// (launch_init).
 int tile_column_sync_ints(int ts);
 bool tile_column_solves_rows(int blocks);
 void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,

@@ -49,27 +49,14 @@ __device__ double wg_sum(double v, double *red) {
 // 0.60 forward and 0.77 ms backward; with one workgroup solving the diagonal
 // tile and a launch per panel, 2.8 and 7.8 ms.
 // ------------------------------------------------------------------------
-constexpr unsigned long long kPending = ~0ull;
-
-__device__ __forceinline__ double peek(const double *p) {
-    return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const unsigned long long *>(p),
-                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
-// v, peeked from p earlier, once every lane's word is published.
+// v, loaded from p earlier, once every lane's word is published.
 __device__ __forceinline__ double await(const double *p, double v) {
-    auto pending = [&] { return __ballot(__builtin_bit_cast(unsigned long long, v) == kPending) != 0; };
+    auto pending = [&] { return __ballot(is_pending(v)) != 0; };
     if (pending()) {   // apart from the loop, whose wait for its own load would also be one for all in flight
-        do v = peek(p);
+        do v = load_shared(p);
         while (pending());
     }
     return v;
-}
-
-__device__ __forceinline__ void publish(double *p, double v) {
-    unsigned long long bits = __builtin_bit_cast(unsigned long long, v);
-    if (bits == kPending) bits = 0x7ff8000000000000ull;   // a NaN stays one, of another pattern
-    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // a += sum_q m[q] * x[lane q of the 16-lane row], in two interleaved sums (the
@@ -210,7 +197,7 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
     int next = 0, tj = 0, cb = 0;   // the next fetch's block, its tile column and block column there
     auto fetch = [&](Cols<kMixed> &c) {
         c.load(map, ti, tj, rb * kBlk + lane, cb * kBlk + 16 * w);
-        c.y = peek(yw + (int64_t) next * kBlk);
+        c.y = load_shared(yw + (int64_t) next * kBlk);
         if (next < b - 1) {   // the last block is fetched again (two_in_flight)
             ++next;
             if (++cb == nsb) cb = 0, ++tj;
@@ -224,7 +211,7 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
     two_in_flight<Cols<kMixed>>(b, fetch, use);
     const double y = finish_block(acc, m, w, lane, sm);
     if (w == 0) {
-        publish(pending + (int64_t) b * kBlk + lane, y);
+        store_word(pending + (int64_t) b * kBlk + lane, y);
         z[(int64_t) b * kBlk + lane] = y;
         if (partials) {
             const double q = wave_sum(y * y);
@@ -278,7 +265,7 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     int next = nb - 1, ti = map.nt - 1, rb = map.last_blocks - 1;   // the next fetch's block and its place
     auto fetch = [&](Cols<kMixed> &c) {
         c.load(map, ti, tj, rb * kBlk + lane, cb * kBlk + 16 * w);
-        c.y = peek(pending + (int64_t) next * kBlk + lane);
+        c.y = load_shared(pending + (int64_t) next * kBlk + lane);
         if (next > last + 1) {
             --next;
             if (--rb < 0) rb = nsb - 1, --ti;
@@ -309,11 +296,11 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     if (last < nb) {
         T.widen(0);
         const double *yp = pending + (int64_t) last * kBlk + 16 * w + (lane & 15);
-        x = row_product(T.v, -await(yp, peek(yp)), x);
+        x = row_product(T.v, -await(yp, load_shared(yp)), x);
     }
     const double y = finish_block(x, m, w, lane, sm);
     if (w == 0) {
-        publish(pending + (int64_t) b * kBlk + lane, y);
+        store_word(pending + (int64_t) b * kBlk + lane, y);
         z[(int64_t) b * kBlk + lane] = y;
     }
 }
@@ -433,6 +420,7 @@ __device__ __forceinline__ void init_element(const InitJob &j, int64_t i) {
     if (j.sync) {
         if (i < j.sync_ints) j.sync[i] = 0;
         if (i == 0) *j.info = 0;
+        if (i < j.winv_words) reinterpret_cast<unsigned long long *>(j.winv)[i] = kPending;
     }
     if (j.pending) {
         if (j.src && i < j.npad) j.z[i] = (i < j.n) ? j.src[i] : 0.0;
@@ -573,7 +561,7 @@ void launch_axpby(double *y, const double *x, double a, double b, int64_t n, hip
 }
 
 int64_t init_extent(const InitJob &j) {
-    return std::max(j.sync ? j.sync_ints : 0, j.pending ? j.npad + 1 : 0);
+    return std::max(j.sync ? std::max(j.sync_ints, j.winv_words) : 0, j.pending ? j.npad + 1 : 0);
 }
 
 void launch_init(const InitJob &job, hipStream_t s) {
