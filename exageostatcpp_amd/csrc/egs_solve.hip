@@ -46,15 +46,19 @@ __device__ double wg_sum(double v, double *red) {
 // wave and do not wait for the solution; the solution itself is its own flag (a
 // word that holds ~0 has not been published), which saves a hop one flag load
 // and one fence.  20,000 locations, tiles of 960 (1.6 GB of L):
-// 0.60 forward and 0.77 ms backward; with one workgroup solving the diagonal
+// 0.57 ms forward and 0.58 backward; with one workgroup solving the diagonal
 // tile and a launch per panel, 2.8 and 7.8 ms.
 // ------------------------------------------------------------------------
-// v, loaded from p earlier, once every lane's word is published.
-__device__ __forceinline__ double await(const double *p, double v) {
+// v, loaded from p earlier, once every lane's word is published.  far: other blocks
+// come before this one is waited for; it asks less often, so that the words of
+// the chain's next block are not queued behind everybody's requests.
+__device__ __forceinline__ double await(const double *p, double v, bool far) {
     auto pending = [&] { return __ballot(is_pending(v)) != 0; };
     if (pending()) {   // apart from the loop, whose wait for its own load would also be one for all in flight
-        do v = load_shared(p);
-        while (pending());
+        do {
+            if (far) __builtin_amdgcn_s_sleep(16);
+            v = load_shared(p);
+        } while (pending());
     }
     return v;
 }
@@ -204,7 +208,7 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
         }
     };
     auto use = [&](Cols<kMixed> &c, int j) {
-        const double y = await(yw + (int64_t) j * kBlk, c.y);
+        const double y = await(yw + (int64_t) j * kBlk, c.y, b - j > 2);
         c.widen(lane);
         acc = row_product(c.v, -y, acc);
     };
@@ -243,17 +247,25 @@ __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob 
 
 // Block b of L^T y = z, y in z's place and in pending.  Down the block's column
 // lanes hold rows (coalesced), so the 16 column sums of a wave stay spread over
-// its lanes and are added up before the last block, which is read transposed:
-// nothing but that block's product waits for the block solved just before.
+// its lanes and are added up before the last two blocks, which are read
+// transposed: nothing but a block's product waits for the block solved just
+// before (with the sums added up between the last two, 0.9 us more per block).
 template <bool kMixed>
 __device__ __forceinline__ void backward_block(const TileMap &map, const double *winv, double *z, double *pending, int b,
                                                SolveSmem &sm) {
     const int ts = map.ts, nsb = ts / kBlk, nb = map.blocks();
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int tj = b / nsb, cb = b % nsb;
-    const int last = b + 1;   // the block read transposed, if there is one
-    Cols<kMixed, true> T;
-    if (last < nb) T.load(map, last / nsb, tj, (last % nsb) * kBlk + 16 * w, cb * kBlk + lane);
+    // the last two blocks are read transposed
+    const int last = b + 2;
+    Cols<kMixed, true> T[2];
+    const double *y_last[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = min(last - u, nb - 1);
+        T[u].load(map, i / nsb, tj, (i % nsb) * kBlk + 16 * w, cb * kBlk + lane);
+        y_last[u] = pending + (int64_t) i * kBlk + 16 * w + (lane & 15);
+    }
     double m[16];
     const double *W = winv + (int64_t) b * kBlk * kBlk + lane * kBlk + 16 * w;
 #pragma unroll
@@ -272,12 +284,14 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
         }
     };
     auto use = [&](Cols<kMixed> &c, int m) {
-        const double y = -await(pending + (int64_t) (nb - 1 - m) * kBlk + lane, c.y);
+        const double y = -await(pending + (int64_t) (nb - 1 - m) * kBlk + lane, c.y, nb - 1 - m - b > 3);
         c.widen(lane);
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[q] = fma(c.v[q], y, acc[q]);
     };
-    two_in_flight<Cols<kMixed>>(max(nb - 1 - last, 0), fetch, use);   // none for the last two blocks
+    two_in_flight<Cols<kMixed>>(max(nb - 1 - last, 0), fetch, use);   // none for the last three blocks
+    if (last < nb) T[0].y = load_shared(y_last[0]);
+    if (last - 1 < nb) T[1].y = load_shared(y_last[1]);
     // the sums over the 64 lanes: each step halves the columns a lane keeps
 #pragma unroll
     for (int half = 8, bit = 32; half > 0; half >>= 1, bit >>= 1) {
@@ -293,11 +307,12 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     if ((lane & 3) == 0) sm.base[16 * w + (lane >> 2)] = acc[0];
     __syncthreads();
     double x = w == 0 ? zb + sm.base[lane] : 0.0;
-    if (last < nb) {
-        T.widen(0);
-        const double *yp = pending + (int64_t) last * kBlk + 16 * w + (lane & 15);
-        x = row_product(T.v, -await(yp, load_shared(yp)), x);
-    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (last - u < nb) {
+            T[u].widen(0);
+            x = row_product(T[u].v, -await(y_last[u], T[u].y, false), x);
+        }
     const double y = finish_block(x, m, w, lane, sm);
     if (w == 0) {
         store_word(pending + (int64_t) b * kBlk + lane, y);
