@@ -710,6 +710,19 @@ void launch_mixed_update(egs_problem_s *p, int k, int jcol_lo, int jcol_hi, hipS
     }
 }
 
+// Whether panel k is applied to tile column k + 2 by the critical stream, together
+// with panel k + 1, instead of by a bulk launch of its own (FP64 plans).  That
+// launch is short and ends, like every launch, in a nearly empty last wave, before
+// the rest of the bulk step may start.  The critical stream has time for it while
+// the bulk steps are longer than its own: down to eight tile columns beyond, where
+// six to 15 measured alike in either direction (launch of its own -> so: 10,007
+// locations, tiles of 384: 9.13 -> 8.73 ms; 20,000, tiles of 960: 50.2 -> 48.8;
+// 40,000: 345 -> 340).
+bool defers_column(const egs_problem_s *p, int k) {
+    constexpr int kColumnsBeyond = 8;
+    return !is_mixed(p) && p->nt - k - 3 >= kColumnsBeyond;
+}
+
 // Enqueue the tiled Cholesky with a lookahead of one panel: the critical
 // stream updates tile column k+1, factors it and solves its panel while the
 // bulk stream applies panel k to the columns beyond k+1.  The update order
@@ -750,12 +763,13 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
         // Tile column k+1 first, and alone but for what is left of bulk step
         // k-1: beside bulk step k it would take twice as long, and with it
         // everything after it.  Then its factorization beside bulk step k.
-        if (k > 0) EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[k - 1], 0));
+        const int panels = k > 0 && defers_column(p, k - 1) ? 2 : 1;
+        if (k >= panels) EGS_HIP(hipStreamWaitEvent(s, p->ev_bulk[k - panels], 0));
         if (is_mixed(p)) {
             launch_mixed_update(p, k, k + 1, k + 2, s, true);
         } else {
-            const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 1, k + 2), s);
-            egs::launch_update(m, nullptr, p->d_pairs + n_beyond, n_next, k, true, s);
+            const int pi = prof_begin(p, EGS_PROFILE_UPDATE, panels * update_flops(p, k + 1, k + 2), s);
+            egs::launch_update(m, nullptr, p->d_pairs + n_beyond, n_next, k + 1 - panels, true, s, panels);
             prof_end(p, pi, s);
         }
         if (beyond > 0) EGS_HIP(hipEventRecord(p->ev_column[k], s));
@@ -764,16 +778,18 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
         // Bulk step k: column k+2 first, then ev_bulk[k], then columns k+3 ..:
         // the critical stream's step k+1 needs only column k+2, so it overlaps
         // the rest of this step.  (The list holds columns in descending order:
-        // column k+2 is the last beyond - 1 ... entries of the prefix.)
+        // column k+2 is the last beyond - 1 ... entries of the prefix.)  Where
+        // column k+2 is left to the critical stream (defers_column), its step
+        // k+1 needs the bulk step before this one, and ev_bulk[k] ends it.
         EGS_HIP(hipStreamWaitEvent(b, p->ev_column[k], 0));
         if (is_mixed(p)) {
             if (k + 2 < nt) launch_mixed_update(p, k, k + 2, k + 3, b);
-        } else if (n_beyond > 0) {
+        } else if (!defers_column(p, k)) {
             const int pi = prof_begin(p, EGS_PROFILE_UPDATE, update_flops(p, k + 2, k + 3), b);
             egs::launch_update(m, nullptr, p->d_pairs + (n_beyond - beyond), beyond, k, false, b);
             prof_end(p, pi, b);
         }
-        EGS_HIP(hipEventRecord(p->ev_bulk[k], b));
+        if (!defers_column(p, k)) EGS_HIP(hipEventRecord(p->ev_bulk[k], b));
         if (is_mixed(p)) {
             if (k + 3 < nt) launch_mixed_update(p, k, k + 3, nt, b);
         } else if (n_beyond > beyond) {
@@ -781,6 +797,7 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
             egs::launch_update(m, nullptr, p->d_pairs, n_beyond - beyond, k, false, b);
             prof_end(p, pi, b);
         }
+        if (defers_column(p, k)) EGS_HIP(hipEventRecord(p->ev_bulk[k], b));
     }
     EGS_HIP(hipGetLastError());
     return EGS_SUCCESS;

@@ -255,8 +255,9 @@ __global__ void __launch_bounds__(kThreads) trsm_rows_mixed_kernel(TileMap map, 
 // ------------------------------------------------------------------------
 // p64 (may be null): read panel k from its contiguous FP64 copy (tile i at
 // p64 + (i - k - 1) ts^2) instead of from the tiles.
+// panels = 2 (without p64): with the panels k and k + 1.
 __device__ __forceinline__ void update_body(const TileMap &map, const double *p64, const int2 *pairs, int k, int bx,
-                                            int by) {
+                                            int by, int panels) {
     __shared__ GemmSmem sm;
     const int ts = map.ts;
     const int nsb = ts / kBlk;
@@ -276,12 +277,15 @@ __device__ __forceinline__ void update_body(const TileMap &map, const double *p6
     int q = 0;
     acc_foreach(acc, [&](int r, int c, double) { cv[q++] = C[r + (int64_t) c * ts]; });
     wg_gemm_nt(acc, A, ts, B, ts, ts, sm);
+    if (panels == 2)
+        wg_gemm_nt(acc, tile_f64(map, ij.x, k + 1) + sbm * kBlk, ts, tile_f64(map, ij.y, k + 1) + sbn * kBlk, ts, ts, sm);
     q = 0;
     acc_foreach(acc, [&](int r, int c, double v) { C[r + (int64_t) c * ts] = cv[q++] - v; });
 }
 
-__global__ void __launch_bounds__(kThreads) update_kernel(TileMap map, const double *p64, const int2 *pairs, int k) {
-    update_body(map, p64, pairs, k, blockIdx.x, blockIdx.y);
+__global__ void __launch_bounds__(kThreads) update_kernel(TileMap map, const double *p64, const int2 *pairs, int k,
+                                                          int panels) {
+    update_body(map, p64, pairs, k, blockIdx.x, blockIdx.y, panels);
 }
 
 // A panel of fewer 64-row blocks than this is solved in 32-row blocks (with
@@ -321,15 +325,15 @@ void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, 
 constexpr int kSmallBlocks = 768, kSmallBlocksCritical = 1800;
 
 void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, bool critical,
-                   hipStream_t s) {
+                   hipStream_t s, int panels) {
     if (npairs <= 0) return;
     const int nsb = map.ts / kBlk;
     if (update192_supported(map.ts) &&
         (int64_t) npairs * nsb * nsb > (critical ? kSmallBlocksCritical : kSmallBlocks)) {
-        launch_update192(map, p64, pairs, npairs, k, s);
+        launch_update192(map, p64, pairs, npairs, k, panels, s);
         return;
     }
-    hipLaunchKernelGGL(update_kernel, dim3(nsb * nsb, npairs), dim3(kThreads), 0, s, map, p64, pairs, k);
+    hipLaunchKernelGGL(update_kernel, dim3(nsb * nsb, npairs), dim3(kThreads), 0, s, map, p64, pairs, k, panels);
 }
 
 // ------------------------------------------------------------------------
@@ -861,7 +865,7 @@ __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *
     const BatchJob J = scalar_load(jobs + blockIdx.z);
     const int rest = J.map.nt - J.k - 1;   // tile columns k+1 .. nt-1: the first rest (rest + 1) / 2 pairs
     if ((int) blockIdx.y >= rest * (rest + 1) / 2) return;
-    update_body(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y);
+    update_body(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y, 1);
 }
 
 // Panels of at most this many 64-row blocks are solved by the launch that

@@ -73,11 +73,13 @@ void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, 
 // p64 (may be null): read panel k from its contiguous FP64 copy (tile i at
 // p64 + (i-k-1) ts^2) instead of from the tiles.  critical: the next panel waits
 // for these tiles.
+// panels = 2 (FP64 plans): with the panels k and k + 1.
 void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, bool critical,
-                   hipStream_t s);
+                   hipStream_t s, int panels = 1);
 // Its 96 x 192-block form (egs_update.hip), for ts % 192 == 0.
 bool update192_supported(int ts);
-void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s);
+void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, int panels,
+                      hipStream_t s);
 
 // ---- triangular solves and reductions (egs_solve.hip)
 // What a factorization (sync, null for none) and a solve (pending, null for none)

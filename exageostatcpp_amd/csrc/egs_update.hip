@@ -47,6 +47,8 @@ __device__ __forceinline__ const double *panel_tile(const TileMap &map, const Pa
     return reinterpret_cast<const double *>(map.base + map.off[i * map.nt + k]);
 }
 
+// kPanels = 2: with the panels k and k + 1 of an FP64 plan, one after the other.
+template <int kPanels>
 __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef pr, const int2 *pairs, int k) {
     __shared__ __align__(16) double sA[2][kKC * kBR];
     __shared__ __align__(16) double sB[2][kKC * kBC];
@@ -63,6 +65,9 @@ __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef
 
     const double *A = panel_tile(map, pr, ij.x, k) + sbm * kBR;
     const double *B = panel_tile(map, pr, ij.y, k) + sbn * kBC;
+    const double *A2 = kPanels == 2 ? panel_tile(map, pr, ij.x, k + 1) + sbm * kBR : nullptr;
+    const double *B2 = kPanels == 2 ? panel_tile(map, pr, ij.y, k + 1) + sbn * kBC : nullptr;
+    const int per_panel = ts / kKC;
 
     const int t = threadIdx.x;
     const int lane = t & 63, w = t >> 6;
@@ -77,8 +82,10 @@ __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef
     const int lb = 2 * (t & 31) + (t >> 5) * kBC;
     f64x2 ra[3], rb[6];
     auto issue = [&](int c) {
-        const double *Ac = A + (int64_t) c * kKC * ts;
-        const double *Bc = B + (int64_t) c * kKC * ts, *Bd = Bc + (int64_t) (kKC / 2) * ts;
+        const bool second = kPanels == 2 && c >= per_panel;
+        const int64_t at = (int64_t) (second ? c - per_panel : c) * kKC * ts;
+        const double *Ac = (second ? A2 : A) + at;
+        const double *Bc = (second ? B2 : B) + at, *Bd = Bc + (int64_t) (kKC / 2) * ts;
 #pragma unroll
         for (int q = 0; q < 3; ++q) ra[q] = *reinterpret_cast<const f64x2 *>(Ac + ga + 32 * q);
 #pragma unroll
@@ -120,7 +127,7 @@ __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef
             for (int ni = 0; ni < 3; ++ni) acc[mi][ni] = mfma_f64(b[set][ni], a[set][mi], acc[mi][ni]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    const int nchunks = ts / kKC;
+    const int nchunks = kPanels * per_panel;
     issue(0);
     stage(0);
     issue(1);
@@ -173,12 +180,14 @@ __global__ void __launch_bounds__(kNT, 2) update192_kernel(TileMap map, PanelRef
 
 bool update192_supported(int ts) { return ts % kBC == 0; }
 
-void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, hipStream_t s) {
+void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, int panels,
+                      hipStream_t s) {
     if (npairs <= 0) return;
     const unsigned blocks = (unsigned) npairs * (unsigned) ((map.ts / kBR) * (map.ts / kBC));
     const PanelRef pr{reinterpret_cast<const char *>(p64), (int64_t) map.ts * map.ts * (int64_t) sizeof(double),
                       p64 != nullptr};
-    hipLaunchKernelGGL(update192_kernel, dim3(blocks), dim3(kNT), 0, s, map, pr, pairs, k);
+    hipLaunchKernelGGL(panels == 2 ? update192_kernel<2> : update192_kernel<1>, dim3(blocks), dim3(kNT), 0, s, map, pr,
+                       pairs, k);
 }
 
 }  // namespace egs
