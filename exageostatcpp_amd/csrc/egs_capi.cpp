@@ -192,8 +192,9 @@ struct egs_problem_s {
     double *d_winv = nullptr;
     int *d_sync = nullptr;      // tickets and flags of the tile columns' factorization (launch_tile_column)
     double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr;
-    // Read back together: a word whose int is the failed minor (0: none), then
-    // the partials of the log-determinant and the quadratic form (launch_forward).
+    // Read back together: a word of two ints, the failed minor (0: none) and
+    // whether a wait was lost (launch_tile_column), then the partials of the
+    // log-determinant and the quadratic form (launch_forward).
     double *d_results = nullptr;
     double *d_tab = nullptr;    // Matern tables of the last covariance parameters (kTabSlots of them)
 
@@ -205,6 +206,7 @@ struct egs_problem_s {
     bool has_obs = false;
     bool has_cov = false;    // the tiles hold Sigma(cov_theta), not yet factored
     bool factored = false;
+    bool info_stale = false;    // the factor is a batch's, whose results are not in d_results
     double factored_theta[6] = {0, 0, 0, 0, 0, 0};
     double cov_theta[6] = {0, 0, 0, 0, 0, 0};
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -234,9 +236,11 @@ struct egs_problem_s {
         return egs::CovJob{map(), d_pairs, (int) h_pairs.size(), prm, egs::Locs{d_x, d_y, z}, n, d_tab, sig64, prm_dev};
     }
     // A factorization's tickets and flags, and a solve of src (null: of d_work).
-    egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) const {
+    egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) {
+        const bool clear = factor || info_stale;
+        info_stale = false;
         return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_winv, (int64_t) map().blocks() * egs::kBlk * egs::kBlk,
-                            d_info(), d_work, src, count, npad, solve ? d_aux : nullptr};
+                            clear ? d_info() : nullptr, d_work, src, count, npad, solve ? d_aux : nullptr};
     }
     int *d_info() const { return reinterpret_cast<int *>(d_results); }
     double *d_partials() const { return d_results + 1; }
@@ -815,20 +819,31 @@ int read_results(egs_problem_s *p, int count) {
     return EGS_SUCCESS;
 }
 
-int info_of(const double *results) {
-    int info;
-    std::memcpy(&info, results, sizeof(int));
-    return info;
+// The two ints of the first word of the results.
+int failed_minor(const double *results) {
+    int info[2];
+    std::memcpy(info, results, sizeof(info));
+    return info[0];
+}
+bool lost_wait(const double *results) {
+    int info[2];
+    std::memcpy(info, results, sizeof(info));
+    return info[1] != 0;
+}
+int lost_error() { return fail(EGS_ERR_HIP, "a workgroup waited in vain for the result of another one"); }
+
+int status_of(const double *results) {
+    if (lost_wait(results)) return lost_error();
+    if (const int minor = failed_minor(results))
+        return fail(EGS_ERR_NOT_SPD, "dpotrf failed, Matrix is not positive definite (leading minor %d)", minor);
+    return EGS_SUCCESS;
 }
 
 int check_info(egs_problem_s *p) {
     prof_collect(p);
-    const int info = info_of(p->h_results.data());
-    if (info != 0) {
-        p->factored = false;
-        return fail(EGS_ERR_NOT_SPD, "dpotrf failed, Matrix is not positive definite (leading minor %d)", info);
-    }
-    return EGS_SUCCESS;
+    const int st = status_of(p->h_results.data());
+    if (st) p->factored = false;
+    return st;
 }
 
 int read_info(egs_problem_s *p) {
@@ -852,7 +867,7 @@ void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partial
     hipStream_t s = p->ctx->stream;
     const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
     if (!prepared) egs::launch_init(p->init_job(false, true, src, n), s);
-    egs::launch_forward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, partials, s);
+    egs::launch_forward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, partials, p->d_info(), s);
     prof_end(p, pi);
 }
 
@@ -861,7 +876,7 @@ void run_backward(egs_problem_s *p, const double *src, int64_t n) {
     hipStream_t s = p->ctx->stream;
     const int pi = is_mixed(p) ? prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n) : -1;
     egs::launch_init(p->init_job(false, true, src, n), s);
-    egs::launch_backward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, s);
+    egs::launch_backward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, p->d_info(), s);
     prof_end(p, pi);
 }
 
@@ -958,6 +973,8 @@ int refine_solve(egs_problem_s *p, const double *b) {
     // true residual of the returned solution
     if ((st = sigma_times(p, X, R, b))) return st;
     if ((st = host_dot(p, R, R, rr))) return st;
+    if ((st = read_results(p, 1))) return st;
+    if (lost_wait(p->h_results.data())) return lost_error();
     prof_end(p, pi);
     p->refine_iters = it;
     p->refine_resid = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
@@ -1433,6 +1450,7 @@ int egs_solve_logdet_quad(egs_problem_t p, double *logdet, double *quad) {
     else run_forward(p, p->d_obs, p->n, p->d_partials());
     EGS_HIP(hipGetLastError());
     if ((st = read_results(p, p->result_count()))) return st;
+    if ((st = check_info(p))) return st;
     double ld, q;
     sum_partials(p, p->h_results.data(), ld, q);
     if (is_mixed(p)) {
@@ -1458,7 +1476,7 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
     else run_backward(p, p->d_work, p->n);
     EGS_HIP(hipGetLastError());
     EGS_HIP(hipMemcpyAsync(z, p->d_work, sizeof(double) * (size_t) n, hipMemcpyDeviceToHost, s));
-    EGS_HIP(hipStreamSynchronize(s));
+    if ((st = read_info(p))) return st;
     if (alpha != 1.0)
         for (int64_t i = 0; i < n; ++i) z[i] *= alpha;
     return EGS_SUCCESS;
@@ -1735,14 +1753,11 @@ int egs_loglik_batch(egs_problem_t *problems, const double *thetas, int count, d
         prof_collect(p);
         const double *r = result;
         result += p->result_count();
-        const int info = info_of(r);
         double ld = 0.0, q = 0.0;
-        if (info != 0) {
-            status[b] = fail(EGS_ERR_NOT_SPD, "dpotrf failed, Matrix is not positive definite (leading minor %d)", info);
-            continue;
-        }
+        if ((status[b] = status_of(r)) != EGS_SUCCESS) continue;
         sum_partials(p, r, ld, q);
         p->factored = true;
+        p->info_stale = true;
         std::memcpy(p->factored_theta, thetas + 6 * b, sizeof(double) * p->ntheta());
         std::memcpy(p->cov_theta, thetas + 6 * b, sizeof(double) * p->ntheta());
         loglik[b] = -0.5 * q - 0.5 * ld - (double) p->n / 2.0 * std::log(2.0 * kPi);
@@ -2041,12 +2056,12 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(zmiss, d_out, sizeof(double) * (size_t) rows, hipMemcpyDeviceToHost, s);
-    const hipError_t e2 = hipStreamSynchronize(s);
-    if (e == hipSuccess) e = e2;
-    if (e != hipSuccess) return fail(EGS_ERR_HIP, "prediction: %s", hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void) hipStreamSynchronize(s);
+        return fail(EGS_ERR_HIP, "prediction: %s", hipGetErrorString(e));
+    }
+    if ((st = read_info(p))) return st;
     if (!reuse) {
-        st = read_info(p);
-        if (st) return st;
         p->factored = true;
         std::memcpy(p->factored_theta, theta, sizeof(double) * p->ntheta());
     }

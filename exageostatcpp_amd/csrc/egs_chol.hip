@@ -559,8 +559,10 @@ __device__ __forceinline__ void set_flag(int *flag) {
 }
 
 // Waits, wave by wave, until the flag is set.
-__device__ __forceinline__ void wait_flag(const int *flag) {
-    while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
+__device__ __forceinline__ void wait_flag(const int *flag, int *lost) {
+    Patience patience{lost};
+    while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0 &&
+           !patience.over())
         __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");
 }
@@ -645,10 +647,11 @@ __device__ __forceinline__ double *last_panel(PanelSmem &sm) { return sm.b + 16 
 // Columns 16 P .. 16 P + 15 of X; W, t, out: this lane's element of each.
 template <bool kDia, int P>
 __device__ __forceinline__ void solve_panel(const double *W, const double *t, double *out, int ts, int w, PanelSmem &sm,
-                                            DiagAcc &dia) {
+                                            DiagAcc &dia, int *lost) {
     const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
     constexpr int kSteps = 4 * (P + 1);
     double wv[kSteps];
+    Patience patience{lost};
     bool waiting;
     do {
 #pragma unroll
@@ -656,7 +659,8 @@ __device__ __forceinline__ void solve_panel(const double *W, const double *t, do
         waiting = false;
 #pragma unroll
         for (int q = 0; q < kSteps; ++q) waiting |= is_pending(wv[q]);
-    } while (__ballot(waiting) != 0);
+        if (!kDia && __ballot(waiting) != 0) __builtin_amdgcn_s_sleep(4);   // off the chain: ask less often
+    } while (__ballot(waiting) != 0 && !patience.over());
     f64x4 x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int q = 0; q < kSteps; ++q) x = mfma_f64(wv[q], t[4 * q * kPv], x);
@@ -675,7 +679,7 @@ __device__ __forceinline__ void solve_panel(const double *W, const double *t, do
 
 template <bool kDia>
 __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, int c, const double *winv_k, int *flags,
-                                            PanelSmem &sm, DiagAcc &dia) {
+                                            PanelSmem &sm, DiagAcc &dia, int *lost) {
     double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
     const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -684,9 +688,9 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
         Acc64 acc;
         acc_load(acc, X, ts);
         for (int b = 0; b < c; ++b) {
-            wait_flag(flags + r * nsb + b);
+            wait_flag(flags + r * nsb + b, lost);
             load_block(va, T + r * kBlk + (int64_t) b * kBlk * ts, ts);
-            wait_flag(flags + c * nsb + b);
+            wait_flag(flags + c * nsb + b, lost);
             load_block(vb, T + c * kBlk + (int64_t) b * kBlk * ts, ts);
             put_block(sm.a, va);
             put_block(sm.b, vb);
@@ -701,10 +705,10 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
     const double *W = winv_k + (int64_t) c * kBlk * kBlk + lr + lk * kBlk;
     const double *t = sm.a + lk * kPv + 16 * w + lr;
     double *out = X + 16 * w + lr + (int64_t) lk * ts;
-    solve_panel<kDia, 0>(W, t, out, ts, w, sm, dia);
-    solve_panel<kDia, 1>(W, t, out, ts, w, sm, dia);
-    solve_panel<kDia, 2>(W, t, out, ts, w, sm, dia);
-    solve_panel<kDia, 3>(W, t, out, ts, w, sm, dia);
+    solve_panel<kDia, 0>(W, t, out, ts, w, sm, dia, lost);
+    solve_panel<kDia, 1>(W, t, out, ts, w, sm, dia, lost);
+    solve_panel<kDia, 2>(W, t, out, ts, w, sm, dia, lost);
+    solve_panel<kDia, 3>(W, t, out, ts, w, sm, dia, lost);
     if (!kDia) {
         wait_stores();
         __syncthreads();
@@ -756,7 +760,7 @@ __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r,
     DiagAcc dia;
     dia.foreach(w, [&](int i, int j, double) { return D[i + (int64_t) j * ts]; });
     if (r > 0) {
-        solve_block<true>(T, ts, nsb, r, r - 1, winv_k, flags, sm, dia);
+        solve_block<true>(T, ts, nsb, r, r - 1, winv_k, flags, sm, dia, info + 1);
         wait_stores();   // the panels before the last: long done
     }
     dia.foreach(w, [&](int i, int j, double v) { return sm.a[i * kPv + j] = v; });
@@ -785,8 +789,9 @@ struct BlockWait {
     static constexpr bool kAhead = false;
     const int *flags;
     int nsb;
-    __device__ __forceinline__ void row(int j) const { wait_flag(flags + j * nsb + j - 1); }
-    __device__ __forceinline__ void inverse(int j) const { wait_flag(flags + j * nsb + j); }
+    int *lost;
+    __device__ __forceinline__ void row(int j) const { wait_flag(flags + j * nsb + j - 1, lost); }
+    __device__ __forceinline__ void inverse(int j) const { wait_flag(flags + j * nsb + j, lost); }
 };
 
 // Tasks of a diagonal tile of so many 64 x 64 blocks.
@@ -807,7 +812,7 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
         if (h >= halves) return;
         const int per = ts / kHalf;
         double *X = tile_f64(map, k + 1 + h / per, k) + (h % per) * kHalf;
-        solve_rows<double, kHalf>(T, ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm), BlockWait{flags, nsb});
+        solve_rows<double, kHalf>(T, ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm), BlockWait{flags, nsb, info + 1});
         return;
     }
     // block column c holds the diagonal task and live - 2 - c others
@@ -820,7 +825,7 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
         diagonal_task(T, ts, nsb, c, winv_k, flags, info, (int64_t) k * ts, n, sm);
     } else {
         DiagAcc none;
-        solve_block<false>(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, none);
+        solve_block<false>(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, none, info + 1);
     }
 }
 

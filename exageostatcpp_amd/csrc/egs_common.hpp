@@ -83,6 +83,23 @@ __device__ __forceinline__ void store_word(double *p, double v) {
     store_shared(p, is_pending(v) ? __builtin_bit_cast(double, 0x7ff8000000000000ull) : v);
 }
 
+// Every wait for another workgroup of a launch ends: after kPatience requests
+// (of half a microsecond and more: several seconds, where the longest wait that
+// was measured is a few milliseconds) the wave sets *lost and goes on with what is
+// there, and every other wait of the launch follows within kLook requests.  The
+// host reads lost with the results.
+struct Patience {
+    int *lost;
+    unsigned polls = 0;
+
+    __device__ __forceinline__ bool over() {
+        constexpr unsigned kPatience = 1u << 23, kLook = 1u << 10;
+        if ((++polls & (kLook - 1)) != 0) return false;
+        if (polls >= kPatience) __hip_atomic_store(lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __builtin_amdgcn_readfirstlane(__hip_atomic_load(lost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+    }
+};
+
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin (workgroup w
 // runs on XCD w % 8), and each XCD has its own L2.  xcd_remap gives XCD x a
 // contiguous range of the logical block order, so blocks that share operand

@@ -84,8 +84,9 @@ void launch_update192(const TileMap &map, const double *p64, const int2 *pairs, 
 // ---- triangular solves and reductions (egs_solve.hip)
 // What a factorization (sync, null for none) and a solve (pending, null for none)
 // start from: sync_ints zeros in sync, winv_words empty words (kPending) of the
-// inverses, no failure in info; z = src (n values) padded with zeros to npad, or
-// as it is when src is null, and pending (npad + 1 doubles) emptied.
+// inverses; no failed minor and no lost wait in info (null: as they are); z = src
+// (n values) padded with zeros to npad, or as it is when src is null, and pending
+// (npad + 1 doubles) emptied.
 struct InitJob {
     int *sync;
     int64_t sync_ints;
@@ -104,9 +105,11 @@ void launch_init_batch(const InitJob *jobs, int count, int64_t most, hipStream_t
 // z = L^{-1} z and z = L^{-T} z with the factor's tiles (mixed: some may be FP32)
 // and its diagonal-block inverses.  partials (may be null): of 64-row block b,
 // partials[2b] = sum log L_ii (L_ii > 0), partials[2b+1] = y_b . y_b.
+// info: as for launch_tile_column.
 void launch_forward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, double *partials,
-                    hipStream_t s);
-void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, hipStream_t s);
+                    int *info, hipStream_t s);
+void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, int *info,
+                     hipStream_t s);
 // out = L e (lower-triangular product over the tiles).
 void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s);
 // out[r] = sum_c Sigma(l1_r, l2_c) x[c] for r < rows, c < cols (kriging mean).
@@ -123,7 +126,8 @@ int matvec_chunks(int64_t n);
 // blocks below it, FP64 ones (tile_column_solves_rows: whether that many should
 // be; the others take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
 // tile_column_sync_ints(ts) ints, zero before the launch, winv_k empty
-// (launch_init).
+// (launch_init).  info[0]: the first minor without a positive pivot, if it is 0;
+// info[1] becomes 1 if a wait between workgroups ends in vain (Patience).
 int tile_column_sync_ints(int ts);
 bool tile_column_solves_rows(int blocks);
 void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,

@@ -52,13 +52,14 @@ __device__ double wg_sum(double v, double *red) {
 // v, loaded from p earlier, once every lane's word is published.  far: other blocks
 // come before this one is waited for; it asks less often, so that the words of
 // the chain's next block are not queued behind everybody's requests.
-__device__ __forceinline__ double await(const double *p, double v, bool far) {
+__device__ __forceinline__ double await(const double *p, double v, bool far, int *lost) {
     auto pending = [&] { return __ballot(is_pending(v)) != 0; };
     if (pending()) {   // apart from the loop, whose wait for its own load would also be one for all in flight
+        Patience patience{lost};
         do {
             if (far) __builtin_amdgcn_s_sleep(16);
             v = load_shared(p);
-        } while (pending());
+        } while (pending() && !patience.over());
     }
     return v;
 }
@@ -186,7 +187,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 // [2b] = sum log L_ii over L_ii > 0, [2b+1] = y_b . y_b.
 template <bool kMixed>
 __device__ __forceinline__ void forward_block(const TileMap &map, const double *winv, double *z, double *pending,
-                                              double *partials, int b, SolveSmem &sm) {
+                                              double *partials, int b, SolveSmem &sm, int *lost) {
     const int ts = map.ts, nsb = ts / kBlk;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int ti = b / nsb, rb = b % nsb;
@@ -208,7 +209,7 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
         }
     };
     auto use = [&](Cols<kMixed> &c, int j) {
-        const double y = await(yw + (int64_t) j * kBlk, c.y, b - j > 2);
+        const double y = await(yw + (int64_t) j * kBlk, c.y, b - j > 2, lost);
         c.widen(lane);
         acc = row_product(c.v, -y, acc);
     };
@@ -229,10 +230,10 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
 
 template <bool kMixed>
 __global__ void __launch_bounds__(kThreads) forward_kernel(TileMap map, const double *winv, double *z, double *pending,
-                                                           double *partials) {
+                                                           double *partials, int *info) {
     __shared__ SolveSmem sm;
     const int b = solve_ticket(pending, (int64_t) map.nt * map.ts, sm);
-    forward_block<kMixed>(map, winv, z, pending, partials, b, sm);
+    forward_block<kMixed>(map, winv, z, pending, partials, b, sm, info + 1);
 }
 
 // The jobs' blocks in turn, so that a ticket's chain is in lower tickets.
@@ -242,7 +243,7 @@ __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob 
     const BatchJob J = scalar_load(jobs + t % njobs);
     const int b = t / njobs;
     if (b >= J.map.blocks()) return;
-    forward_block<false>(J.map, J.winv_k, J.z, J.pending, J.partials, b, sm);
+    forward_block<false>(J.map, J.winv_k, J.z, J.pending, J.partials, b, sm, J.info + 1);
 }
 
 // Block b of L^T y = z, y in z's place and in pending.  Down the block's column
@@ -252,7 +253,7 @@ __global__ void __launch_bounds__(kThreads) forward_batch_kernel(const BatchJob 
 // before (with the sums added up between the last two, 0.9 us more per block).
 template <bool kMixed>
 __device__ __forceinline__ void backward_block(const TileMap &map, const double *winv, double *z, double *pending, int b,
-                                               SolveSmem &sm) {
+                                               SolveSmem &sm, int *lost) {
     const int ts = map.ts, nsb = ts / kBlk, nb = map.blocks();
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int tj = b / nsb, cb = b % nsb;
@@ -284,7 +285,7 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
         }
     };
     auto use = [&](Cols<kMixed> &c, int m) {
-        const double y = -await(pending + (int64_t) (nb - 1 - m) * kBlk + lane, c.y, nb - 1 - m - b > 3);
+        const double y = -await(pending + (int64_t) (nb - 1 - m) * kBlk + lane, c.y, nb - 1 - m - b > 3, lost);
         c.widen(lane);
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[q] = fma(c.v[q], y, acc[q]);
@@ -311,7 +312,7 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     for (int u = 0; u < 2; ++u)
         if (last - u < nb) {
             T[u].widen(0);
-            x = row_product(T[u].v, -await(y_last[u], T[u].y, false), x);
+            x = row_product(T[u].v, -await(y_last[u], T[u].y, false, lost), x);
         }
     const double y = finish_block(x, m, w, lane, sm);
     if (w == 0) {
@@ -321,10 +322,11 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
 }
 
 template <bool kMixed>
-__global__ void __launch_bounds__(kThreads) backward_kernel(TileMap map, const double *winv, double *z, double *pending) {
+__global__ void __launch_bounds__(kThreads) backward_kernel(TileMap map, const double *winv, double *z, double *pending,
+                                                            int *info) {
     __shared__ SolveSmem sm;
     const int t = solve_ticket(pending, (int64_t) map.nt * map.ts, sm);
-    backward_block<kMixed>(map, winv, z, pending, map.blocks() - 1 - t, sm);
+    backward_block<kMixed>(map, winv, z, pending, map.blocks() - 1 - t, sm, info + 1);
 }
 
 // out = L e: one workgroup of 16 waves per 64 rows, the longest rows first; the
@@ -432,9 +434,9 @@ __global__ void __launch_bounds__(kThreads) copy_pad_kernel(double *dst, const d
 }
 
 __device__ __forceinline__ void init_element(const InitJob &j, int64_t i) {
+    if (j.info && i < 2) j.info[i] = 0;
     if (j.sync) {
         if (i < j.sync_ints) j.sync[i] = 0;
-        if (i == 0) *j.info = 0;
         if (i < j.winv_words) reinterpret_cast<unsigned long long *>(j.winv)[i] = kPending;
     }
     if (j.pending) {
@@ -590,9 +592,9 @@ void launch_init_batch(const InitJob *jobs, int count, int64_t most, hipStream_t
 }
 
 void launch_forward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, double *partials,
-                    hipStream_t s) {
+                    int *info, hipStream_t s) {
     hipLaunchKernelGGL(mixed ? forward_kernel<true> : forward_kernel<false>, dim3((unsigned) map.blocks()), dim3(kThreads), 0,
-                       s, map, winv, z, pending, partials);
+                       s, map, winv, z, pending, partials, info);
 }
 
 void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int max_nt, hipStream_t s) {
@@ -600,9 +602,10 @@ void launch_forward_batch(const BatchJob *jobs, int njobs, int ts, int max_nt, h
                        njobs);
 }
 
-void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, hipStream_t s) {
+void launch_backward(const TileMap &map, bool mixed, const double *winv, double *z, double *pending, int *info,
+                     hipStream_t s) {
     hipLaunchKernelGGL(mixed ? backward_kernel<true> : backward_kernel<false>, dim3((unsigned) map.blocks()), dim3(kThreads), 0,
-                       s, map, winv, z, pending);
+                       s, map, winv, z, pending, info);
 }
 
 void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s) {

@@ -39,3 +39,22 @@ def test_batch_of_forms(forms):
     for p in probs:
         p.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("failed_before", [False, True])
+def test_predict_with_the_factor_of_a_batch(failed_before):
+    """A prediction that reuses a batch's factor: nothing that an earlier
+    factorization of the problem left (or did not leave) is read for it."""
+    ctx = egs.Context(0)
+    theta, miss = [1.0, 0.1, 0.5], np.random.default_rng(3).random((2, 20))
+    p, q, fresh = (problem(ctx, 0, 300, 0, 2, s) for s in (5, 6, 5))
+    if failed_before:
+        with pytest.raises(egs.NotPositiveDefinite):
+            p.loglik([-1.0, 0.1, 0.5])   # negative variance
+    assert not any(isinstance(r, Exception) for r in capi.loglik_batch([p, q], [theta, theta]))
+    want = fresh.predict(theta, *miss)[0]
+    got = p.predict(theta, *miss)[0]
+    assert np.max(np.abs(got - want)) <= 1e-9 * np.max(np.abs(want))
+    for e in (p, q, fresh):
+        e.close()
+    ctx.close()
