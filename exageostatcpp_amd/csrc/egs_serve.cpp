@@ -16,7 +16,7 @@
 // in HBM for later requests: a kriging request at the theta of the region's
 // last evaluation reuses the factor.  Regions are admitted by their footprint
 // (egs_problem_estimate_bytes, which counts a mixed plan's panel copies, FP64
-// copy of Sigma and inverses) against the HBM budget; when a region does not
+// copy of Sigma) against the HBM budget; when a region does not
 // fit, the least recently used idle regions are released, and the request
 // waits while the regions in use leave no room.  Creation, release and upload
 // happen outside the server's lock; released blocks stay in the library's

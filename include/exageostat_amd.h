@@ -108,7 +108,7 @@ int egs_problem_set_context(egs_problem_t problem, egs_context_t ctx);
 int egs_problem_device_bytes(egs_problem_t problem, int64_t *bytes);
 /* Device bytes a problem of this shape and plan holds once evaluated (its
  * tiles, factor workspaces and vectors; under a mixed plan also the panel
- * copies, the FP64 copy of Sigma and the diagonal-tile inverses), before it
+ * copies and the FP64 copy of Sigma), before it
  * exists: the footprint the serving loop admits requests by.  dim is 2 or 3;
  * mode and bands as egs_problem_set_precision.  Prediction buffers (grown on
  * demand, 8 * n_miss * (P + 3) bytes) are not included. */
@@ -272,11 +272,11 @@ int egs_last_timings(egs_problem_t problem, double *t_covariance, double *t_fact
  * kernels below with HIP events on the library stream; egs_problem_kernel_stats
  * returns, per kernel, the number of timed launches, their summed duration and
  * their summed algorithmic flops (FP64 real rows only, padding excluded). */
-#define EGS_PROFILE_UPDATE 0        /* trailing SYRK/GEMM update, one launch per step */
+#define EGS_PROFILE_UPDATE 0        /* trailing SYRK/GEMM update */
 #define EGS_PROFILE_COVARIANCE 1    /* covariance generation of all lower tiles */
-#define EGS_PROFILE_PANEL_TRSM 2    /* panel triangular solve, one launch per step */
-#define EGS_PROFILE_DIAGONAL 3      /* diagonal-tile factorization (all its launches) */
-#define EGS_PROFILE_SOLVE 4         /* forward solve with log-det and dot product */
+#define EGS_PROFILE_PANEL_TRSM 2    /* panel triangular solve, but for rows solved with the diagonal tile */
+#define EGS_PROFILE_DIAGONAL 3      /* diagonal-tile factorization, with the FP64 rows below when they are few */
+#define EGS_PROFILE_SOLVE 4         /* forward solve with log-det and dot product; mixed plans: both solves */
 #define EGS_PROFILE_UPDATE_F32 5    /* mixed plans: FP32-band update */
 #define EGS_PROFILE_UPDATE_16 6      /* mixed plans: update with 16-bit products */
 #define EGS_PROFILE_REFINE 7        /* mixed plans: refinement of z'Sigma^{-1}z */
