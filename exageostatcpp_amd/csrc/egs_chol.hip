@@ -11,7 +11,7 @@
 //     (trsm_rows_kernel);
 //   * the trailing tiles are updated with FP64 MFMA: update192 (egs_update.hip)
 //     when ts is a multiple of 192 and the tiles are many, else update_kernel
-//     here, one workgroup per 64 x 64 output block with K = ts.
+//     here, one workgroup per 64 x 64 output block (or half of one) with K = ts.
 // Every contraction uses v_mfma_f64_16x16x4f64 through wg_gemm_nt: four waves
 // each own a 32 x 32 quadrant of the 64 x 64 output; K is staged through LDS in
 // chunks of 32 columns, double buffered, with the next chunk's global loads
@@ -256,36 +256,39 @@ __global__ void __launch_bounds__(kThreads) trsm_rows_mixed_kernel(TileMap map, 
 // p64 (may be null): read panel k from its contiguous FP64 copy (tile i at
 // p64 + (i - k - 1) ts^2) instead of from the tiles.
 // panels = 2 (without p64): with the panels k and k + 1.
+template <int kRows>
 __device__ __forceinline__ void update_body(const TileMap &map, const double *p64, const int2 *pairs, int k, int bx,
                                             int by, int panels) {
     __shared__ GemmSmem sm;
     const int ts = map.ts;
-    const int nsb = ts / kBlk;
+    const int per = ts / kRows;
     const int2 ij = pairs[by];
-    const int sbm = bx % nsb;
-    const int sbn = bx / nsb;
+    const int r0 = (bx % per) * kRows, sbm = r0 / kBlk;
+    const int sbn = bx / per;
     if (ij.x == ij.y && sbm < sbn) return;
     if (sbm >= map.blocks(ij.x) || sbn >= map.blocks(ij.y)) return;
-    double *C = tile_f64(map, ij.x, ij.y) + sbm * kBlk + (int64_t) sbn * kBlk * ts;
+    double *C = tile_f64(map, ij.x, ij.y) + r0 + (int64_t) sbn * kBlk * ts;
     const int64_t tt = (int64_t) ts * ts;
-    const double *A = (p64 ? p64 + (ij.x - k - 1) * tt : tile_f64(map, ij.x, k)) + sbm * kBlk;
+    const double *A = (p64 ? p64 + (ij.x - k - 1) * tt : tile_f64(map, ij.x, k)) + r0;
     const double *B = (p64 ? p64 + (ij.y - k - 1) * tt : tile_f64(map, ij.y, k)) + sbn * kBlk;
-    // C's 16 values are loaded ahead of the product, whose loads follow in flight
-    Acc64 acc;
+    // C's values are loaded ahead of the product, whose loads follow in flight
+    using Block = Acc<double, kRows>;
+    Block acc;
     acc_zero(acc);
-    double cv[16];
+    double cv[Block::kNi * 8];
     int q = 0;
     acc_foreach(acc, [&](int r, int c, double) { cv[q++] = C[r + (int64_t) c * ts]; });
     wg_gemm_nt(acc, A, ts, B, ts, ts, sm);
     if (panels == 2)
-        wg_gemm_nt(acc, tile_f64(map, ij.x, k + 1) + sbm * kBlk, ts, tile_f64(map, ij.y, k + 1) + sbn * kBlk, ts, ts, sm);
+        wg_gemm_nt(acc, tile_f64(map, ij.x, k + 1) + r0, ts, tile_f64(map, ij.y, k + 1) + sbn * kBlk, ts, ts, sm);
     q = 0;
     acc_foreach(acc, [&](int r, int c, double v) { C[r + (int64_t) c * ts] = cv[q++] - v; });
 }
 
+template <int kRows>
 __global__ void __launch_bounds__(kThreads) update_kernel(TileMap map, const double *p64, const int2 *pairs, int k,
                                                           int panels) {
-    update_body(map, p64, pairs, k, blockIdx.x, blockIdx.y, panels);
+    update_body<kRows>(map, p64, pairs, k, blockIdx.x, blockIdx.y, panels);
 }
 
 // A panel of fewer 64-row blocks than this is solved in 32-row blocks (with
@@ -322,7 +325,13 @@ void launch_trsm_rows_mixed(const TileMap &map, int k, int64_t g0, int count64, 
 // 166; 64 tiles of 192 39 / 46).  On the critical path, where the update shares
 // the GPU with the one before, the shorter workgroups pay up to twice as many
 // (6,001 locations, tiles of 960: 5.2 against 5.4 ms).
-constexpr int kSmallBlocks = 768, kSmallBlocksCritical = 1800;
+// Up to half a block per CU are updated in halves of 32 rows, on twice the CUs
+// with half of a chunk's products each (what bounds such a launch is one
+// workgroup's way through ts / 32 chunks): 400 locations, tiles of 320, 192.0 ->
+// 186.0 us, 1,600 552 -> 524 us; up to two per CU measured alike there and at
+// 10,007 (8.75 ms), and a mixed evaluation of 45,001, whose halves wait for room
+// beside the 16-bit updates, 0.6% slower.
+constexpr int kSmallBlocks = 768, kSmallBlocksCritical = 1800, kHalfBlocks = 128;
 
 void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int npairs, int k, bool critical,
                    hipStream_t s, int panels) {
@@ -333,7 +342,9 @@ void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int
         launch_update192(map, p64, pairs, npairs, k, panels, s);
         return;
     }
-    hipLaunchKernelGGL(update_kernel, dim3(nsb * nsb, npairs), dim3(kThreads), 0, s, map, p64, pairs, k, panels);
+    const bool half = (int64_t) npairs * nsb * nsb <= kHalfBlocks;
+    hipLaunchKernelGGL(half ? update_kernel<32> : update_kernel<64>, dim3((nsb << half) * nsb, npairs), dim3(kThreads), 0,
+                       s, map, p64, pairs, k, panels);
 }
 
 // ------------------------------------------------------------------------
@@ -870,7 +881,7 @@ __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *
     const BatchJob J = scalar_load(jobs + blockIdx.z);
     const int rest = J.map.nt - J.k - 1;   // tile columns k+1 .. nt-1: the first rest (rest + 1) / 2 pairs
     if ((int) blockIdx.y >= rest * (rest + 1) / 2) return;
-    update_body(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y, 1);
+    update_body<kBlk>(J.map, nullptr, J.pairs, J.k, blockIdx.x, blockIdx.y, 1);
 }
 
 // Panels of at most this many 64-row blocks are solved by the launch that

@@ -20,10 +20,12 @@ def ctx():
     c.close()
 
 
+# 128 blocks of 64 x 64 (32-row halves up to there): 32 tiles of 128 (33 columns), 5 of 320 (6), 14 of 192 (15)
 # 768 blocks of 64 x 64: 85 tiles of 192 (13 columns), 21 of 384 (6), 9 of 576 (4), 3 of 960 (2)
 @pytest.mark.parametrize("n,dts", [(200, 192), (500, 192), (2700, 192), (3100, 192), (900, 384), (2650, 384),
                                    (3500, 384), (1800, 576), (2900, 576), (2000, 960), (3000, 960), (1900, 1152),
-                                   (3000, 128)])
+                                   (3000, 128), (4224, 128), (4340, 128), (1900, 320), (2210, 320), (2880, 192),
+                                   (2900, 192), (65, 64), (97, 64)])
 def test_factor_and_likelihood(ctx, n, dts):
     r = np.random.default_rng(n)
     x, y, z = r.random(n), r.random(n), r.standard_normal(n)
