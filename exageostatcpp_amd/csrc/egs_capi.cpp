@@ -951,7 +951,8 @@ int refine_solve(egs_problem_s *p, const double *b) {
     int it = 0;
     if (bb > 0.0 && std::sqrt(rr / bb) > kRefineTol) {
         apply_factor_inverse(p, R, W);
-        egs::launch_axpby(P, W, 1.0, 0.0, np, s);
+        // a copy: P is not written yet, and 0 times what recycled memory holds may be NaN
+        EGS_HIP(hipMemcpyAsync(P, W, sizeof(double) * (size_t) np, hipMemcpyDeviceToDevice, s));
         if ((st = host_dot(p, R, W, rz))) return st;
         for (it = 1; it <= kRefineMaxIter; ++it) {
             if ((st = sigma_times(p, P, Q, nullptr))) return st;
