@@ -974,9 +974,13 @@ int refine_solve(egs_problem_s *p, const double *b) {
     // true residual of the returned solution
     if ((st = sigma_times(p, X, R, b))) return st;
     if ((st = host_dot(p, R, R, rr))) return st;
-    if ((st = read_results(p, 1))) return st;
-    if (lost_wait(p->h_results.data())) return lost_error();
+    st = read_results(p, 1);
     prof_end(p, pi);
+    if (st) return st;
+    if (lost_wait(p->h_results.data())) {
+        p->factored = false;   // only the next factorization clears the mark
+        return lost_error();
+    }
     p->refine_iters = it;
     p->refine_resid = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
     p->refine_converged = p->refine_resid <= kRefineAccept;
@@ -1806,6 +1810,17 @@ int egs_loglik(egs_problem_t p, const double *theta, double *loglik, double *log
     ++p->fallbacks;
     if (st_eval) g_last_error = err;
     return st_eval;
+}
+
+// Not in the header, for the tests of the error path: the mark that a kernel leaves
+// when a wait between workgroups ends in vain, as if the factorization whose
+// factor the problem holds had left it.
+int egs_test_mark_lost_wait(egs_problem_t p) {
+    int st = check_problem(p);
+    if (st) return st;
+    const int lost = 1;
+    EGS_HIP(hipMemcpy(p->d_info() + 1, &lost, sizeof(int), hipMemcpyHostToDevice));
+    return EGS_SUCCESS;
 }
 
 int egs_problem_set_fallback(egs_problem_t p, int max_iterations, double tolerance) {
