@@ -642,13 +642,14 @@ void factor_panel(egs_problem_s *p, int k) {
     // of a bivariate plan are solved together with the FP64 ones (both on FP64
     // MFMA)
     const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(blocks64) && (blocks32 == 0 || p->f32_panel_solve);
-    int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0);
+    double real64 = 0.0, real32 = 0.0;   // rows below that hold rows of the matrix, for the flops
+    for (int i = k + 1; i < nt; ++i) (i <= k + rows64 ? real64 : real32) += real_rows(p, i);
+    int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0 + (fused ? real64 * ts * ts : 0.0));
     egs::launch_tile_column(m, k, wk, p->sync(k), p->d_info(), p->n, fused ? blocks64 : 0, s);
     prof_end(p, pi);
     if (k + 1 < nt) {
-        double rows_below = 0.0;
-        for (int i = k + 1 + (fused ? rows64 : 0); i < nt; ++i) rows_below += real_rows(p, i);
-        pi = prof_begin(p, EGS_PROFILE_PANEL_TRSM, rows_below * ts * ts);
+        const bool panel = blocks32 > 0 || (blocks64 > 0 && !fused);   // a launch of its own follows
+        pi = panel ? prof_begin(p, EGS_PROFILE_PANEL_TRSM, ((fused ? 0.0 : real64) + real32) * ts * ts) : -1;
         if (blocks32 > 0 && !p->f32_panel_solve) {
             egs::launch_trsm_rows_mixed(m, k, first, blocks64, blocks32, wk, s);
         } else {
