@@ -641,7 +641,7 @@ void factor_panel(egs_problem_s *p, int k) {
     // the FP64 rows go with the diagonal tile when they are few; the FP32 rows
     // of a bivariate plan are solved together with the FP64 ones (both on FP64
     // MFMA)
-    const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(blocks64) && (blocks32 == 0 || p->f32_panel_solve);
+    const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(p->ts, blocks64) && (blocks32 == 0 || p->f32_panel_solve);
     double real64 = 0.0, real32 = 0.0;   // rows below that hold rows of the matrix, for the flops
     for (int i = k + 1; i < nt; ++i) (i <= k + rows64 ? real64 : real32) += real_rows(p, i);
     int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0 + (fused ? real64 * ts * ts : 0.0));

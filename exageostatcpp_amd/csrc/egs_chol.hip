@@ -5,7 +5,8 @@
 // Step k of the factorization:
 //   * the diagonal tile is factored in 64 x 64 blocks, which also leaves the
 //     64 x 64 inverses of its diagonal blocks, and a short panel below it is
-//     solved by the same launch (tile_column_kernel);
+//     solved by the same launch (tile_column_kernel; tiles above kOneLaunchTile:
+//     block_column_kernel);
 //   * a longer panel is solved by one workgroup per 64-row block, marching over
 //     the 64-column blocks of L_kk and applying the 64 x 64 inverses
 //     (trsm_rows_kernel);
@@ -17,6 +18,8 @@
 // chunks of 32 columns, double buffered, with the next chunk's global loads
 // issued before the current chunk's MFMAs (these kernels run on few
 // workgroups, so each one has to hide its own memory latency).
+#include <algorithm>
+
 #include "egs_common.hpp"
 #include "egs_kernels.hpp"
 
@@ -653,6 +656,8 @@ struct DiagAcc {
 // (last_panel) for the caller to store and publish.  The products are subtracted
 // from the block itself, one MFMA after another: the residual shrinks as they go,
 // and with it the rounding (summing them first rounds at the size of the block).
+// kApplied: block columns before c - 1 are already subtracted from the block, and
+// all before c from dia.
 __device__ __forceinline__ double *last_panel(PanelSmem &sm) { return sm.b + 16 * kPv; }
 
 // Columns 16 P .. 16 P + 15 of X; W, t, out: this lane's element of each.
@@ -688,7 +693,7 @@ __device__ __forceinline__ void solve_panel(const double *W, const double *t, do
     }
 }
 
-template <bool kDia>
+template <bool kDia, bool kApplied>
 __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, int c, const double *winv_k, int *flags,
                                             PanelSmem &sm, DiagAcc &dia, int *lost) {
     double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
@@ -698,7 +703,7 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
         double va[16], vb[16];
         Acc64 acc;
         acc_load(acc, X, ts);
-        for (int b = 0; b < c; ++b) {
+        for (int b = kApplied ? max(c - 1, 0) : 0; b < c; ++b) {
             wait_flag(flags + r * nsb + b, lost);
             load_block(va, T + r * kBlk + (int64_t) b * kBlk * ts, ts);
             wait_flag(flags + c * nsb + b, lost);
@@ -707,7 +712,7 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
             put_block(sm.b, vb);
             __syncthreads();
             subtract_block(acc, sm.a, sm.b);
-            if (kDia) dia.subtract<kBlk>(w, sm.a);
+            if (kDia && !kApplied) dia.subtract<kBlk>(w, sm.a);
             __syncthreads();
         }
         acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
@@ -763,6 +768,7 @@ struct HandOut {
 };
 
 // Diagonal task r: block (r, r - 1), then block (r, r) factored and inverted.
+template <bool kApplied>
 __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r, double *winv_k, int *flags, int *info,
                                               int64_t col0, int64_t n, PanelSmem &sm) {
     double *D = T + r * kBlk + (int64_t) r * kBlk * ts;
@@ -771,7 +777,7 @@ __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r,
     DiagAcc dia;
     dia.foreach(w, [&](int i, int j, double) { return D[i + (int64_t) j * ts]; });
     if (r > 0) {
-        solve_block<true>(T, ts, nsb, r, r - 1, winv_k, flags, sm, dia, info + 1);
+        solve_block<true, kApplied>(T, ts, nsb, r, r - 1, winv_k, flags, sm, dia, info + 1);
         wait_stores();   // the panels before the last: long done
     }
     dia.foreach(w, [&](int i, int j, double v) { return sm.a[i * kPv + j] = v; });
@@ -810,20 +816,34 @@ __host__ __device__ inline int tile_tasks(int blocks) { return blocks + (blocks 
 
 }  // namespace
 
+// Task idx of block column c of diagonal tile k: 0 the diagonal task, then the
+// blocks (c + 1 + idx, c).
+template <bool kApplied>
+__device__ __forceinline__ void block_column_task(const TileMap &map, int k, double *winv_k, int *sync, int *info,
+                                                  int64_t n, int c, int idx, PanelSmem &sm) {
+    const int nsb = map.ts / kBlk;
+    double *T = tile_f64(map, k, k);
+    if (idx == 0) {
+        diagonal_task<kApplied>(T, map.ts, nsb, c, winv_k, sync + 1, info, (int64_t) k * map.ts, n, sm);
+    } else {
+        DiagAcc none;
+        solve_block<false, kApplied>(T, map.ts, nsb, c + 1 + idx, c, winv_k, sync + 1, sm, none, info + 1);
+    }
+}
+
 // One task of tile column k; sync: the column's ticket (unused here) and flags.
 __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, double *winv_k, int *sync, int *info,
                                                  int64_t n, int halves, int task, PanelSmem &sm) {
     const int ts = map.ts;
     const int nsb = ts / kBlk;
-    int *flags = sync + 1;
-    double *T = tile_f64(map, k, k);
     const int live = map.blocks(k);
     if (task >= tile_tasks(live)) {
         const int h = task - tile_tasks(live);
         if (h >= halves) return;
         const int per = ts / kHalf;
         double *X = tile_f64(map, k + 1 + h / per, k) + (h % per) * kHalf;
-        solve_rows<double, kHalf>(T, ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm), BlockWait{flags, nsb, info + 1});
+        solve_rows<double, kHalf>(tile_f64(map, k, k), ts, nsb, X, winv_k, *reinterpret_cast<GemmSmem *>(&sm),
+                                  BlockWait{sync + 1, nsb, info + 1});
         return;
     }
     // block column c holds the diagonal task and live - 2 - c others
@@ -832,12 +852,7 @@ __device__ __forceinline__ void tile_column_task(const TileMap &map, int k, doub
         idx -= 1 + max(0, live - 2 - c);
         ++c;
     }
-    if (idx == 0) {
-        diagonal_task(T, ts, nsb, c, winv_k, flags, info, (int64_t) k * ts, n, sm);
-    } else {
-        DiagAcc none;
-        solve_block<false>(T, ts, nsb, c + 1 + idx, c, winv_k, flags, sm, none, info + 1);
-    }
+    block_column_task<false>(map, k, winv_k, sync, info, n, c, idx, sm);
 }
 
 __device__ __forceinline__ int take_ticket(int *counter) {
@@ -853,6 +868,49 @@ __global__ void __launch_bounds__(kThreads) tile_column_kernel(TileMap map, int 
     tile_column_task(map, k, winv_k, sync, info, n, halves, take_ticket(sync), sm);
 }
 
+// A larger diagonal tile (kOneLaunchTile), in three launches per block column
+// whose workgroups wait for earlier launches only (the flags and words they look
+// for are there): the diagonal task, the blocks below it, and their products off
+// the blocks (r, s), r >= s >= c + 2.  (Column c + 1's blocks are left to their
+// tasks: block (c + 1, c) comes with the next diagonal task.)
+enum BlockColumnPart { kDiagonalPart, kBelowPart, kUpdatePart };
+
+__device__ __forceinline__ void block_column_part(const TileMap &map, int k, double *winv_k, int *sync, int *info,
+                                                  int64_t n, int c, BlockColumnPart part, int at, PanelSmem &sm) {
+    const int live = map.blocks(k), ts = map.ts;
+    if (part == kDiagonalPart) {
+        if (c < live) block_column_task<true>(map, k, winv_k, sync, info, n, c, 0, sm);
+        return;
+    }
+    if (part == kBelowPart) {
+        if (c + 2 + at < live) block_column_task<true>(map, k, winv_k, sync, info, n, c, 1 + at, sm);
+        return;
+    }
+    int i = 0;   // row of `at` in the lower triangle
+    while (at > i) at -= ++i;
+    const int r = c + 2 + i, q = c + 2 + at;
+    if (r >= live) return;
+    double *T = tile_f64(map, k, k);
+    double *C = T + r * kBlk + (int64_t) q * kBlk * ts;
+    double va[16], vb[16];
+    Acc64 acc;
+    acc_load(acc, C, ts);
+    load_block(va, T + r * kBlk + (int64_t) c * kBlk * ts, ts);
+    load_block(vb, T + q * kBlk + (int64_t) c * kBlk * ts, ts);
+    put_block(sm.a, va);
+    put_block(sm.b, vb);
+    __syncthreads();
+    subtract_block(acc, sm.a, sm.b);
+    acc_foreach(acc, [&](int row, int col, double v) { C[row + (int64_t) col * ts] = v; });
+}
+
+template <BlockColumnPart kPart>
+__global__ void __launch_bounds__(kThreads) block_column_kernel(TileMap map, int k, double *winv_k, int *sync, int *info,
+                                                                int64_t n, int c) {
+    __shared__ PanelSmem sm;
+    block_column_part(map, k, winv_k, sync, info, n, c, kPart, blockIdx.x, sm);
+}
+
 // ------------------------------------------------------------------------
 // Batched forms: one launch applies the same step to several problems of the
 // same tile size, problem b described by jobs[b] (blockIdx.y, or blockIdx.z
@@ -866,6 +924,13 @@ __global__ void __launch_bounds__(kThreads) tile_column_batch_kernel(const Batch
     const int below = J.map.blocks() - (J.k + 1) * (J.map.ts / kBlk);   // none at or below the last tile
     const int halves = with_rows ? 2 * max(below, 0) : 0;
     tile_column_task(J.map, J.k, J.winv_k, J.sync, J.info, J.n, halves, t / njobs, sm);
+}
+
+template <BlockColumnPart kPart>
+__global__ void __launch_bounds__(kThreads) block_column_batch_kernel(const BatchJob *jobs, int c) {
+    __shared__ PanelSmem sm;
+    const BatchJob J = scalar_load(jobs + blockIdx.y);
+    block_column_part(J.map, J.k, J.winv_k, J.sync, J.info, J.n, c, kPart, blockIdx.x, sm);
 }
 
 template <int kRows>
@@ -890,13 +955,34 @@ __global__ void __launch_bounds__(kThreads) update_batch_kernel(const BatchJob *
 // and 64-row blocks load L_kk half as often per flop).
 constexpr int kFusedRows = 128;
 
+// Tiles up to this size are factored by one launch per tile column, whose
+// workgroups wait for each other.  Larger ones take three launches per block
+// column, without such waits: one call with tiles of 2,048 (or of 64: the record
+// does not say which of two) has not returned, for a reason that is not known, and
+// up to here that launch has run often.  1,500 locations in tiles of 1,216 1.5 ms,
+// 4,000 in tiles of 1,984 5.4 ms, eight of 1,500 in a batch 1.5 ms; in two launches
+// per block column, each block adding up its products in turn, 2.6, 12.2 and 3.3.
+constexpr int kOneLaunchTile = 1152;
+
 void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nrest, hipStream_t s) {
     if (njobs <= 0) return;
     const int nsb = ts / kBlk;
-    const bool fused = rest * nsb * nrest <= kFusedRows;
-    const int tasks = tile_tasks(nsb) + (fused ? rest * (ts / kHalf) : 0);
-    hipLaunchKernelGGL(tile_column_batch_kernel, dim3((unsigned) (tasks * njobs)), dim3(kThreads), 0, s, jobs, njobs,
-                       fused ? 1 : 0);
+    const bool one_launch = ts <= kOneLaunchTile;
+    const bool fused = one_launch && rest * nsb * nrest <= kFusedRows;
+    if (one_launch) {
+        const int tasks = tile_tasks(nsb) + (fused ? rest * (ts / kHalf) : 0);
+        hipLaunchKernelGGL(tile_column_batch_kernel, dim3((unsigned) (tasks * njobs)), dim3(kThreads), 0, s, jobs, njobs,
+                           fused ? 1 : 0);
+    }
+    for (int c = 0; c < nsb && !one_launch; ++c) {
+        const int below = std::max(nsb - 2 - c, 0);
+        const unsigned count = (unsigned) njobs;
+        hipLaunchKernelGGL(block_column_batch_kernel<kDiagonalPart>, dim3(1, count), dim3(kThreads), 0, s, jobs, c);
+        if (below == 0) continue;
+        hipLaunchKernelGGL(block_column_batch_kernel<kBelowPart>, dim3((unsigned) below, count), dim3(kThreads), 0, s, jobs, c);
+        hipLaunchKernelGGL(block_column_batch_kernel<kUpdatePart>, dim3((unsigned) (below * (below + 1) / 2), count),
+                           dim3(kThreads), 0, s, jobs, c);
+    }
     if (rest <= 0 || nrest <= 0) return;
     if (!fused) {
         const int half = rest * nsb * nrest < kHalfRowsBelow;
@@ -909,10 +995,21 @@ void launch_step_batch(const BatchJob *jobs, int njobs, int ts, int rest, int nr
 
 int tile_column_sync_ints(int ts) { return 1 + (ts / kBlk) * (ts / kBlk); }
 
-bool tile_column_solves_rows(int blocks) { return blocks <= kFusedRows; }
+bool tile_column_solves_rows(int ts, int blocks) { return ts <= kOneLaunchTile && blocks <= kFusedRows; }
 
 void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,
                         hipStream_t s) {
+    const int live = map.blocks(k);
+    for (int c = 0; c < live && map.ts > kOneLaunchTile; ++c) {
+        const int below = std::max(live - 2 - c, 0);
+        hipLaunchKernelGGL(block_column_kernel<kDiagonalPart>, dim3(1), dim3(kThreads), 0, s, map, k, winv_k, sync, info, n, c);
+        if (below == 0) continue;
+        hipLaunchKernelGGL(block_column_kernel<kBelowPart>, dim3((unsigned) below), dim3(kThreads), 0, s, map, k, winv_k, sync,
+                           info, n, c);
+        hipLaunchKernelGGL(block_column_kernel<kUpdatePart>, dim3((unsigned) (below * (below + 1) / 2)), dim3(kThreads), 0, s,
+                           map, k, winv_k, sync, info, n, c);
+    }
+    if (map.ts > kOneLaunchTile) return;
     hipLaunchKernelGGL(tile_column_kernel, dim3((unsigned) (tile_tasks(map.blocks(k)) + 2 * blocks)), dim3(kThreads), 0,
                        s, map, k, winv_k, sync, info, n, 2 * blocks);
 }

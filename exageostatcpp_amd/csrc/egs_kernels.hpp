@@ -127,9 +127,10 @@ int matvec_chunks(int64_t n);
 // be; the others take launch_trsm_rows afterwards).  sync: the column's ticket and flags,
 // tile_column_sync_ints(ts) ints, zero before the launch, winv_k empty
 // (launch_init).  info[0]: the first minor without a positive pivot, if it is 0;
-// info[1] becomes 1 if a wait between workgroups ends in vain (Patience).
+// info[1] becomes 1 if a wait between workgroups ends in vain (Patience).  Tiles
+// above 1,152 take several launches, none of which has such waits, and no rows below.
 int tile_column_sync_ints(int ts);
-bool tile_column_solves_rows(int blocks);
+bool tile_column_solves_rows(int ts, int blocks);
 void launch_tile_column(const TileMap &map, int k, double *winv_k, int *sync, int *info, int64_t n, int blocks,
                         hipStream_t s);
 // Batched steps over problems of tile size ts (jobs in device memory, those
