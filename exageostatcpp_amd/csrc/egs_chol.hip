@@ -353,24 +353,24 @@ void launch_update(const TileMap &map, const double *p64, const int2 *pairs, int
 // ------------------------------------------------------------------------
 // Cholesky and inverse of one 64 x 64 block, held in LDS (row stride kPv
 // doubles).  On entry the lower part of sD is the block A (its upper part is
-// never used) and sE is anything; on return the lower part of sD holds L with
-// column c still to be multiplied by s_rs[c], and the upper part of sE holds
-// L^{-T} with column c still to be multiplied by s_rs[c].  The identity is
-// stacked under A and takes the same column operations: A L^{-T} = L turns I
-// into L^{-T}.
+// never used) and sE is anything; on return the lower part of sD holds L and the
+// upper part of sE L^{-T}.  The identity is stacked under A and takes the same
+// column operations: A L^{-T} = L turns I into L^{-T}.
 //
 // Four panels of 16 columns.  Waves 0 and 1 factor a panel in registers, one
 // row per lane: wave 0 the rows of A from the panel's diagonal down and, in the
 // lanes above, the identity's rows that are no longer zero; wave 1 the
 // identity's 16 rows of the panel.  Both keep the 16 diagonal rows in every
-// 16-lane row as well, so that a column step y_c -= (y_j / piv) a_cj is one
+// 16-lane row as well, so that a column step y_c -= y_j a_cj is one
 // v_fmac_f64_dpp per register, the a_cj broadcast inside the 16 lanes (lane
-// reads into scalar registers cost three times the issue slots).  The next
-// pivot a_j+1,j+1 - a_j+1,j^2 / piv and its reciprocal (hardware estimate and
-// one third-order step) are formed ahead of the update, so that no step waits
-// for it.  The other columns are updated with FP64 MFMA: after panel p the 16
-// columns of panel p + 1 (one 16 x 16 tile per wave), the rest by waves 2 and
-// 3 while waves 0 and 1 factor panel p + 1.
+// reads into scalar registers cost three times the issue slots).  The columns
+// are scaled by 1 / sqrt(pivot) before they are subtracted (unscaled, with
+// 1 / pivot and the scale at the end, the inverse is off by 1.4 times as much).
+// The next pivot a_j+1,j+1 - a_j+1,j^2 and its reciprocal
+// root (hardware estimate and one third-order step) are formed ahead of the
+// update, so that no step waits for it.  The other columns are updated with FP64
+// MFMA: after panel p the 16 columns of panel p + 1 (one 16 x 16 tile per wave),
+// the rest by waves 2 and 3 while waves 0 and 1 factor panel p + 1.
 //
 // Bound: the issue of wave 0 (64 column steps of about 160 cycles); 7.8 us per
 // block from LDS to LDS.  The form before (the block over four waves, one LDS
@@ -380,22 +380,13 @@ constexpr int kHalf = 32;         // rows of a panel block solved beside the dia
 constexpr int kPan = 16;
 constexpr int kPv = kLdsPad;
 
-// 1 / sqrt(x): the hardware estimate and two Newton steps (each doubles the
-// correct bits)
-__device__ __forceinline__ double rsqrt_f64(double x) {
-    double r = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    r = fma(r, fma(-h * r, r, 0.5), r);
-    return fma(r, fma(-h * r, r, 0.5), r);
-}
-
-// yc += z_j[lane C of the 16-lane row] * my, zc likewise with mz
+// yc -= z_j[lane C of the 16-lane row] * y_j, zc likewise
 template <int C>
-__device__ __forceinline__ void fmac2_bcast(double &yc, double &zc, double zj, double my, double mz) {
-    asm("v_fmac_f64_dpp %0, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+__device__ __forceinline__ void fmac2_bcast(double &yc, double &zc, double zj, double yj) {
+    asm("v_fmac_f64_dpp %0, %2, -%3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %2, -%2 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
         : "+v"(yc), "+v"(zc)
-        : "v"(zj), "v"(my), "v"(mz), "n"(C));
+        : "v"(zj), "v"(yj), "n"(C));
 }
 
 // a and b of lane N of the 16-lane row (after two wait states, which a DPP
@@ -409,71 +400,74 @@ __device__ __forceinline__ void bcast2(double a, double b, double &oa, double &o
         : "v"(a), "v"(b), "n"(N));
 }
 
-// Columns J + 2 .. 15 of column step J: the G-th third of them, column J + 2
-// (the next step's pivot column) first.
+// Columns J + 2 .. 15 of column step J: the G-th of four parts of them, column
+// J + 2 (the next step's pivot column) first.
 template <int J, int G, int C = J + 2>
-__device__ __forceinline__ void panel_group(double (&y)[kPan], double (&z)[kPan], double my, double mz) {
+__device__ __forceinline__ void panel_group(double (&y)[kPan], double (&z)[kPan]) {
     if constexpr (C < kPan) {
         constexpr int rest = kPan - 3 - J;
-        constexpr int g = C == J + 2 ? 0 : (C - J - 3) * 3 / rest;
-        if constexpr (g == G) fmac2_bcast<C>(y[C], z[C], z[J], my, mz);
-        panel_group<J, G, C + 1>(y, z, my, mz);
+        constexpr int g = C == J + 2 ? 0 : (C - J - 3) * 4 / rest;
+        if constexpr (g == G) fmac2_bcast<C>(y[C], z[C], z[J], y[J]);
+        panel_group<J, G, C + 1>(y, z);
     }
 }
 
-// Column steps J .. 15 of a panel: piv is pivot J, r its reciprocal; both go
-// to s_piv (the same from every lane).  The scheduling fences keep the
-// reciprocal's dependent steps apart, with the update's FMAs between them.
+// Column steps J .. 15 of a panel: piv is pivot J (kept in s_piv, the same from
+// every lane), rs its reciprocal root.  The scheduling fences keep the dependent
+// steps of the next one apart, with the update's FMAs between them.
 template <int J>
-__device__ __forceinline__ void panel_steps(double (&y)[kPan], double (&z)[kPan], double piv, double r,
-                                            double *s_piv) {
-    s_piv[2 * J] = r;
-    s_piv[2 * J + 1] = piv;
+__device__ __forceinline__ void panel_steps(double (&y)[kPan], double (&z)[kPan], double piv, double rs, double *s_piv) {
+    s_piv[J] = piv;
+    y[J] *= rs;
     if constexpr (J + 1 < kPan) {
-        const double my = -y[J] * r, mz = -z[J] * r;
+        z[J] *= rs;
         double zb, zd;
         bcast2<J + 1>(z[J], z[J + 1], zb, zd);
-        const double next = fma(-(zb * r), zb, zd);   // rounded as the update below rounds it
-        double q = __builtin_amdgcn_rcp(next);
-        fmac2_bcast<J + 1>(y[J + 1], z[J + 1], z[J], my, mz);
+        const double next = fma(-zb, zb, zd);   // rounded as the update below rounds it
+        const double q = __builtin_amdgcn_rsq(next);
+        fmac2_bcast<J + 1>(y[J + 1], z[J + 1], z[J], y[J]);
         __builtin_amdgcn_sched_barrier(0);
-        panel_group<J, 0>(y, z, my, mz);
+        panel_group<J, 0>(y, z);
         __builtin_amdgcn_sched_barrier(0);
-        double e = fma(-next, q, 1.0);
+        const double t = next * q;
         __builtin_amdgcn_sched_barrier(0);
-        panel_group<J, 1>(y, z, my, mz);
+        panel_group<J, 1>(y, z);
         __builtin_amdgcn_sched_barrier(0);
-        e = fma(e, e, e);
+        const double e = fma(-t, q, 1.0);
         __builtin_amdgcn_sched_barrier(0);
-        panel_group<J, 2>(y, z, my, mz);
+        panel_group<J, 2>(y, z);
         __builtin_amdgcn_sched_barrier(0);
-        q = fma(e, q, q);
-        panel_steps<J + 1>(y, z, next, q, s_piv);
+        const double m = q * e, h = fma(0.375, e, 0.5);
+        __builtin_amdgcn_sched_barrier(0);
+        panel_group<J, 3>(y, z);
+        __builtin_amdgcn_sched_barrier(0);
+        panel_steps<J + 1>(y, z, next, fma(m, h, q), s_piv);
     }
 }
 
-// Tile (rb, cb) of 16 x 16 minus panel p's product: rows of A (rb > p) or of
-// the identity (rb <= p; still zero at rb == p).
-__device__ __forceinline__ void panel_tile(double *sD, double *sE, const double *s_piv, int p, int rb, int cb) {
+// Tile (rb, cb) of 16 x 16 minus panel p's product, summed in halves: rows of A
+// (rb > p) or of the identity (rb <= p; still zero at rb == p).
+__device__ __forceinline__ void panel_tile(double *sD, double *sE, int p, int rb, int cb) {
     const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
     double *S = rb <= p ? sE : sD;
-    f64x4 acc;
+    double old[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) acc[v] = rb == p ? 0.0 : S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr];
+    for (int v = 0; v < 4; ++v) old[v] = rb == p ? 0.0 : S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr];
+    f64x4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
     for (int kk = 0; kk < kPan; kk += 4) {
         const int c = kPan * p + kk + lk;
-        acc = mfma_f64(-S[(kPan * rb + lr) * kPv + c] * s_piv[2 * c], sD[(kPan * cb + lr) * kPv + c], acc);
+        acc[kk / 8] = mfma_f64(S[(kPan * rb + lr) * kPv + c], sD[(kPan * cb + lr) * kPv + c], acc[kk / 8]);
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr] = acc[v];
+    for (int v = 0; v < 4; ++v) S[(kPan * rb + lk + 4 * v) * kPv + kPan * cb + lr] = old[v] - (acc[0][v] + acc[1][v]);
 }
 
-// s_piv: 2 * 64 + 2 * 16 doubles.  Thread 0 gets the first column without a
+// s_piv: 64 + 16 doubles.  Thread 0 gets the first column without a
 // positive pivot (-1: none).  Wave 3 calls beside(p) at the start of panel p:
 // rows 0 .. 16 p - 1 of the inverse are there by then.
 template <typename Beside>
-__device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv, double *s_rs, const Beside &beside) {
+__device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv, const Beside &beside) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave index, held in a scalar register
     const int lr = lane & 15;
@@ -492,10 +486,9 @@ __device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv
             __syncthreads();   // both waves have read the diagonal rows
             double piv, unused;
             bcast2<0>(z[0], z[0], piv, unused);
-            double r = __builtin_amdgcn_rcp(piv);
-            const double e = fma(-piv, r, 1.0);
-            r = fma(fma(e, e, e), r, r);
-            panel_steps<0>(y, z, piv, r, w == 0 ? s_piv + 2 * c0 : s_piv + 2 * kBlk);
+            const double q = __builtin_amdgcn_rsq(piv);
+            const double e = fma(-(piv * q), q, 1.0);
+            panel_steps<0>(y, z, piv, fma(q * e, fma(0.375, e, 0.5), q), w == 0 ? s_piv + c0 : s_piv + kBlk);
             if (w == 0 || lane < kPan) {
 #pragma unroll
                 for (int q = 0; q < kPan; ++q) row[q] = y[q];
@@ -508,20 +501,18 @@ __device__ __forceinline__ int potrf64_lds(double *sD, double *sE, double *s_piv
             if (p > 0)
                 for (int cb = p + 1; cb < kPanels; ++cb)
                     for (int rb = 0; rb < kPanels; ++rb)
-                        if ((rb < p || rb >= cb) && (idx++ & 1) == (w & 1)) panel_tile(sD, sE, s_piv, p - 1, rb, cb);
+                        if ((rb < p || rb >= cb) && (idx++ & 1) == (w & 1)) panel_tile(sD, sE, p - 1, rb, cb);
         }
         __syncthreads();
         if (p + 1 < kPanels) {
-            panel_tile(sD, sE, s_piv, p, w, p + 1);
+            panel_tile(sD, sE, p, w, p + 1);
             __syncthreads();
         }
     }
     int bad = -1;
     if (w == 0) {
-        const double piv = s_piv[2 * lane + 1];
-        const unsigned long long m = __ballot(!(piv > 0.0));
+        const unsigned long long m = __ballot(!(s_piv[lane] > 0.0));
         if (m) bad = __ffsll((long long) m) - 1;
-        s_rs[lane] = rsqrt_f64(piv);
     }
     __syncthreads();
     return bad;
@@ -561,8 +552,7 @@ namespace {
 struct PanelSmem {
     double a[kBlk * kPv];   // operand columns: element (row, col) at col * kPv + row
     double b[kBlk * kPv];
-    double piv[2 * kBlk + 2 * kPan];
-    double rs[kBlk];
+    double piv[kBlk + kPan];
 };
 static_assert(sizeof(GemmSmem) <= sizeof(PanelSmem), "the row blocks stage through the same LDS");
 
@@ -594,17 +584,26 @@ __device__ __forceinline__ void put_block(double *s, const double (&v)[16]) {
     for (int q = 0; q < 16; ++q) s[(w + 4 * q) * kPv + row] = v[q];
 }
 
-// acc -= A B^T for 64 x 64 operands in LDS.
+// acc -= A B^T for 64 x 64 operands in LDS, 32 columns at a time (see solve_block).
 __device__ __forceinline__ void subtract_block(Acc64 &acc, const double *a, const double *b) {
     const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int half = 0; half < kBlk; half += kBlk / 2) {
+        Acc64 p;
+        acc_zero(p);
 #pragma unroll 4
-    for (int kk = 0; kk < kBlk; kk += 4) {
-        const double *x = a + (kk + lk) * kPv + Acc64::row0() + lr, *y = b + (kk + lk) * kPv + Acc64::col0() + lr;
-        const double a0 = -x[0], a1 = -x[16], b0 = y[0], b1 = y[16];
-        acc.v[0][0] = mfma_f64(b0, a0, acc.v[0][0]);
-        acc.v[0][1] = mfma_f64(b0, a1, acc.v[0][1]);
-        acc.v[1][0] = mfma_f64(b1, a0, acc.v[1][0]);
-        acc.v[1][1] = mfma_f64(b1, a1, acc.v[1][1]);
+        for (int kk = half; kk < half + kBlk / 2; kk += 4) {
+            const double *x = a + (kk + lk) * kPv + Acc64::row0() + lr, *y = b + (kk + lk) * kPv + Acc64::col0() + lr;
+            const double a0 = x[0], a1 = x[16], b0 = y[0], b1 = y[16];
+            p.v[0][0] = mfma_f64(b0, a0, p.v[0][0]);
+            p.v[0][1] = mfma_f64(b0, a1, p.v[0][1]);
+            p.v[1][0] = mfma_f64(b1, a0, p.v[1][0]);
+            p.v[1][1] = mfma_f64(b1, a1, p.v[1][1]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc.v[i][j] -= p.v[i][j];
     }
 }
 
@@ -638,14 +637,22 @@ struct DiagAcc {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[q][e] = f(row(w, q) + lr, col(w, q) + lk + 4 * e, v[q][e]);
     }
-    // minus X X^T for K columns of X in LDS
-    template <int K> __device__ __forceinline__ void subtract(int w, const double *x) {
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+    }
+    __device__ __forceinline__ void subtract(const DiagAcc &p) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v[q] -= p.v[q];
+    }
+    // plus X X^T for K columns of X in LDS
+    template <int K> __device__ __forceinline__ void add(int w, const double *x) {
         const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
 #pragma unroll 4
         for (int kk = 0; kk < K; kk += 4) {
             const double *xk = x + (kk + lk) * kPv + lr;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) v[q] = mfma_f64(xk[col(w, q)], -xk[row(w, q)], v[q]);
+            for (int q = 0; q < 3; ++q) v[q] = mfma_f64(xk[col(w, q)], xk[row(w, q)], v[q]);
         }
     }
 };
@@ -653,14 +660,20 @@ struct DiagAcc {
 // Block (r, c) of the tile T (ld ts), r > c, solved in place: X = T W^T in panels
 // of 16 columns, as the inverse's rows come.  Without kDia it is published; with
 // it, dia -= L_rb L_rb^T for every b <= c, and the last panel stays in LDS
-// (last_panel) for the caller to store and publish.  The products are subtracted
-// from the block itself, one MFMA after another: the residual shrinks as they go,
-// and with it the rounding (summing them first rounds at the size of the block).
+// (last_panel) for the caller to store and publish.  Products of 32 (for dia 64)
+// columns are summed first and subtracted then.  Subtracted one MFMA after another,
+// each rounds at the size of the block, and the error of the factor grows with the
+// tile: nine fields of 1,600 in tiles of 64 to 960, against 80-bit factors of the
+// same matrices, geometric mean of the rms errors of the log-determinant 6.1e-13 ->
+// 3.7e-13 and of z' Sigma^-1 z (relative) 8.4e-16 -> 4.7e-16; it costs an evaluation
+// of 1,600 1.5% (523 -> 531 us; 400 locations 183 -> 184).  Summed over all block columns
+// first, the sums round at that size.
 // kApplied: block columns before c - 1 are already subtracted from the block, and
 // all before c from dia.
 __device__ __forceinline__ double *last_panel(PanelSmem &sm) { return sm.b + 16 * kPv; }
 
-// Columns 16 P .. 16 P + 15 of X; W, t, out: this lane's element of each.
+// Columns 16 P .. 16 P + 15 of X, their product with themselves added to dia; W, t,
+// out: this lane's element of each.
 template <bool kDia, int P>
 __device__ __forceinline__ void solve_panel(const double *W, const double *t, double *out, int ts, int w, PanelSmem &sm,
                                             DiagAcc &dia, int *lost) {
@@ -685,7 +698,7 @@ __device__ __forceinline__ void solve_panel(const double *W, const double *t, do
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[(lk + 4 * e) * kPv + 16 * w + lr] = x[e];
         __syncthreads();
-        dia.subtract<kPan>(w, s);
+        dia.add<kPan>(w, s);
     }
     if (!kDia || P < 3) {
 #pragma unroll
@@ -699,6 +712,7 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
     double *X = T + r * kBlk + (int64_t) c * kBlk * ts;
     const int lr = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    DiagAcc part;
     {
         double va[16], vb[16];
         Acc64 acc;
@@ -712,7 +726,11 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
             put_block(sm.b, vb);
             __syncthreads();
             subtract_block(acc, sm.a, sm.b);
-            if (kDia && !kApplied) dia.subtract<kBlk>(w, sm.a);
+            if (kDia && !kApplied) {
+                part.zero();
+                part.add<kBlk>(w, sm.a);
+                dia.subtract(part);
+            }
             __syncthreads();
         }
         acc_foreach(acc, [&](int i, int j, double v) { sm.a[j * kPv + i] = v; });
@@ -721,10 +739,12 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
     const double *W = winv_k + (int64_t) c * kBlk * kBlk + lr + lk * kBlk;
     const double *t = sm.a + lk * kPv + 16 * w + lr;
     double *out = X + 16 * w + lr + (int64_t) lk * ts;
-    solve_panel<kDia, 0>(W, t, out, ts, w, sm, dia, lost);
-    solve_panel<kDia, 1>(W, t, out, ts, w, sm, dia, lost);
-    solve_panel<kDia, 2>(W, t, out, ts, w, sm, dia, lost);
-    solve_panel<kDia, 3>(W, t, out, ts, w, sm, dia, lost);
+    part.zero();
+    solve_panel<kDia, 0>(W, t, out, ts, w, sm, part, lost);
+    solve_panel<kDia, 1>(W, t, out, ts, w, sm, part, lost);
+    solve_panel<kDia, 2>(W, t, out, ts, w, sm, part, lost);
+    solve_panel<kDia, 3>(W, t, out, ts, w, sm, part, lost);
+    if (kDia) dia.subtract(part);
     if (!kDia) {
         wait_stores();
         __syncthreads();
@@ -733,14 +753,13 @@ __device__ __forceinline__ void solve_block(double *T, int ts, int nsb, int r, i
 }
 
 // Rows 16 p .. 16 p + 15 of the inverse, columns lk + 4 q for q in [q0, q1), from
-// L^{-T} and the pivots in LDS.
+// L^{-T} in LDS.
 __device__ __forceinline__ void store_inverse_rows(double *W, const PanelSmem &sm, int p, int q0, int q1) {
     const int i = kPan * p + (threadIdx.x & 15), lk = (threadIdx.x & 63) >> 4;
-    const double rsi = rsqrt_f64(sm.piv[2 * i + 1]);
 #pragma unroll 4
     for (int q = q0; q < q1; ++q) {
         const int j = lk + 4 * q;
-        store_word(W + i + j * kBlk, i >= j ? sm.b[j * kPv + i] * rsi : 0.0);
+        store_word(W + i + j * kBlk, i >= j ? sm.b[j * kPv + i] : 0.0);
     }
 }
 
@@ -783,7 +802,7 @@ __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r,
     dia.foreach(w, [&](int i, int j, double v) { return sm.a[i * kPv + j] = v; });
     __syncthreads();
     const HandOut beside{W, r > 0 ? D - (int64_t) kBlk * ts : nullptr, ts, sm, flags + r * nsb + r - 1};
-    const int bad = potrf64_lds(sm.a, sm.b, sm.piv, sm.rs, beside);
+    const int bad = potrf64_lds(sm.a, sm.b, sm.piv, beside);
     store_inverse_rows(W, sm, kBlk / kPan - 1, 4 * w, 4 * w + 4);
     wait_stores();
     __syncthreads();
@@ -792,11 +811,10 @@ __device__ __forceinline__ void diagonal_task(double *T, int ts, int nsb, int r,
         if (bad >= 0 && col0 + r * kBlk + bad < n) atomicCAS(info, 0, (int) (col0 + r * kBlk + bad + 1));
     }
     const int i = threadIdx.x & 63;
-    const double rsi = sm.rs[i];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int j = w + 4 * q;
-        D[i + (int64_t) j * ts] = i > j ? sm.a[i * kPv + j] * sm.rs[j] : i == j ? sm.piv[2 * j + 1] * rsi : 0.0;
+        D[i + (int64_t) j * ts] = i >= j ? sm.a[i * kPv + j] : 0.0;
     }
 }
 
