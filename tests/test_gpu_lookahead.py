@@ -1,8 +1,8 @@
 """The two schedules of the trailing update: tile column k + 2 updated by a launch
 of its own, or by the critical stream with two panels at once, which FP64
 factorizations of at least eleven tile columns begin with.  Ten to fourteen
-columns, 64 x 64 and 96 x 192 updates, ragged last tiles, direct and replayed
-from a graph; against the covariance matrix itself: 64 n eps on the factor's
+columns, 64 x 64 updates (these tiles are too few for the 96 x 192 form), ragged
+last tiles, direct and replayed from a graph; against the covariance matrix itself: 64 n eps on the factor's
 backward error (Higham), and the replays equal to the first to 1e-12.
 """
 import numpy as np

@@ -21,7 +21,8 @@ def ctx():
 
 
 # 128 blocks of 64 x 64 (32-row halves up to there): 32 tiles of 128 (33 columns), 5 of 320 (6), 14 of 192 (15)
-# 768 blocks of 64 x 64: 85 tiles of 192 (13 columns), 21 of 384 (6), 9 of 576 (4), 3 of 960 (2)
+# more than 768 blocks of 64 x 64 in a launch: 2,900 and 3,100 locations in tiles of 192 (91 and 105 tiles of 9
+# blocks), 3,500 in tiles of 384 (28 of 36); the other tile sizes in test_gpu_update192.py
 @pytest.mark.parametrize("n,dts", [(200, 192), (500, 192), (2700, 192), (3100, 192), (900, 384), (2650, 384),
                                    (3500, 384), (1800, 576), (2900, 576), (2000, 960), (3000, 960), (1900, 1152),
                                    (3000, 128), (4224, 128), (4340, 128), (1900, 320), (2210, 320), (2880, 192),
