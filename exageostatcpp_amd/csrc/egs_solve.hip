@@ -64,10 +64,10 @@ __device__ __forceinline__ double await(const double *p, double v, bool far, int
     return v;
 }
 
-// a += sum_q m[q] * x[lane q of the 16-lane row], in two interleaved sums (the
-// two wait states are what a DPP read of a just written register needs).
-__device__ __forceinline__ double row_product(const double (&m)[16], double x, double a) {
-    double b = 0.0;
+// sum_q m[q] * x[lane q of the 16-lane row], in two interleaved sums (the two wait
+// states are what a DPP read of a just written register needs).
+__device__ __forceinline__ double row_product(const double (&m)[16], double x) {
+    double a = 0.0, b = 0.0;
     asm("s_nop 1\n\t"
         "v_fmac_f64_dpp %0, %2, %3 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f64_dpp %1, %2, %4 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
@@ -90,6 +90,21 @@ __device__ __forceinline__ double row_product(const double (&m)[16], double x, d
           "v"(m[9]), "v"(m[10]), "v"(m[11]), "v"(m[12]), "v"(m[13]), "v"(m[14]), "v"(m[15]));
     return a + b;
 }
+
+// A sum of many terms, in groups of 16: the terms of a group round at its size, only
+// the groups at that of the whole.  With every product added to the running sum, the
+// residual of a forward solve grew with the square root of the rows: 5,700 locations
+// 1.04e-15 rms, 11,500 1.38e-15; so 1.8e-16 and 2.0e-16, for 0 to 1% of the solve.
+struct GroupedSum {
+    double sum, part = 0.0;
+    __device__ __forceinline__ void add(double v, int m) {   // the m-th
+        const bool last = (m & 15) == 15;
+        part += v;
+        sum += last ? part : 0.0;
+        part = last ? 0.0 : part;
+    }
+    __device__ __forceinline__ double total() const { return sum + part; }
+};
 
 // A lane's 16 elements of a block of L in flight, with the word of the solution
 // they multiply: a row's, ts apart, or (kAcross) a column's, one after the other.
@@ -172,7 +187,7 @@ __device__ __forceinline__ double finish_block(double x, const double (&m)[16], 
     __syncthreads();
     const int c = 16 * w + (lane & 15);
     const double t = ((sm.part[0][0][c] + sm.part[0][1][c]) + sm.part[0][2][c]) + sm.part[0][3][c];
-    sm.part[1][w][lane] = row_product(m, t, 0.0);
+    sm.part[1][w][lane] = row_product(m, t);
     __syncthreads();
     return ((sm.part[1][0][lane] + sm.part[1][1][lane]) + sm.part[1][2][lane]) + sm.part[1][3][lane];
 }
@@ -198,7 +213,7 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
     for (int q = 0; q < 16; ++q) m[q] = W[q * kBlk];
     double d = 1.0;
     if (partials && w == 3) d = tile_f64(map, ti, ti)[(int64_t) (rb * kBlk + lane) * (ts + 1)];
-    double acc = w == 0 ? z[(int64_t) b * kBlk + lane] : 0.0;
+    GroupedSum acc{w == 0 ? z[(int64_t) b * kBlk + lane] : 0.0};
     int next = 0, tj = 0, cb = 0;   // the next fetch's block, its tile column and block column there
     auto fetch = [&](Cols<kMixed> &c) {
         c.load(map, ti, tj, rb * kBlk + lane, cb * kBlk + 16 * w);
@@ -211,10 +226,10 @@ __device__ __forceinline__ void forward_block(const TileMap &map, const double *
     auto use = [&](Cols<kMixed> &c, int j) {
         const double y = await(yw + (int64_t) j * kBlk, c.y, b - j > 2, lost);
         c.widen(lane);
-        acc = row_product(c.v, -y, acc);
+        acc.add(row_product(c.v, -y), j);
     };
     two_in_flight<Cols<kMixed>>(b, fetch, use);
-    const double y = finish_block(acc, m, w, lane, sm);
+    const double y = finish_block(acc.total(), m, w, lane, sm);
     if (w == 0) {
         store_word(pending + (int64_t) b * kBlk + lane, y);
         z[(int64_t) b * kBlk + lane] = y;
@@ -312,7 +327,7 @@ __device__ __forceinline__ void backward_block(const TileMap &map, const double 
     for (int u = 0; u < 2; ++u)
         if (last - u < nb) {
             T[u].widen(0);
-            x = row_product(T[u].v, -await(y_last[u], T[u].y, false, lost), x);
+            x += row_product(T[u].v, -await(y_last[u], T[u].y, false, lost));
         }
     const double y = finish_block(x, m, w, lane, sm);
     if (w == 0) {
@@ -350,17 +365,17 @@ __global__ void __launch_bounds__(kTrmvThreads) trmv_kernel(TileMap map, const d
         c.load(map, i, k, rb * kBlk + lane, c0);
         if (next + kWaves < strips) next += kWaves;
     };
-    double acc = 0.0;
+    GroupedSum acc{0.0};
     auto use = [&](Cols<false> &c, int m) {
         const int s = w + m * kWaves;
         if (s >= 4 * b) {   // the diagonal block
 #pragma unroll
             for (int q = 0; q < 16; ++q) c.v[q] = 16 * (s - 4 * b) + q <= lane ? c.v[q] : 0.0;
         }
-        acc = row_product(c.v, c.y, acc);
+        acc.add(row_product(c.v, c.y), m);
     };
     two_in_flight<Cols<false>>((strips - w + kWaves - 1) / kWaves, fetch, use);
-    sp[w][lane] = acc;
+    sp[w][lane] = acc.total();
     __syncthreads();
     if (w == 0) {
         double a = 0.0;
