@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -194,7 +195,8 @@ struct egs_problem_s {
     double *d_obs = nullptr, *d_work = nullptr, *d_aux = nullptr;
     // Read back together: a word of two ints, the failed minor (0: none) and
     // whether a wait was lost (launch_tile_column), then the partials of the
-    // log-determinant and the quadratic form (launch_forward).
+    // log-determinant and the quadratic form (launch_forward), or a vector of up to
+    // npad values that a call returns.
     double *d_results = nullptr;
     double *d_tab = nullptr;    // Matern tables of the last covariance parameters (kTabSlots of them)
 
@@ -236,11 +238,11 @@ struct egs_problem_s {
         return egs::CovJob{map(), d_pairs, (int) h_pairs.size(), prm, egs::Locs{d_x, d_y, z}, n, d_tab, sig64, prm_dev};
     }
     // A factorization's tickets and flags, and a solve of src (null: of d_work).
-    egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count) {
+    egs::InitJob init_job(bool factor, bool solve, const double *src, int64_t count, double *z = nullptr) {
         const bool clear = factor || info_stale;
         info_stale = false;
         return egs::InitJob{factor ? d_sync : nullptr, sync_ints(), d_winv, (int64_t) map().blocks() * egs::kBlk * egs::kBlk,
-                            clear ? d_info() : nullptr, d_work, src, count, npad, solve ? d_aux : nullptr};
+                            clear ? d_info() : nullptr, z ? z : d_work, src, count, npad, solve ? d_aux : nullptr};
     }
     int *d_info() const { return reinterpret_cast<int *>(d_results); }
     double *d_partials() const { return d_results + 1; }
@@ -808,14 +810,18 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
     return EGS_SUCCESS;
 }
 
-// The first `count` words of d_results (result_count(): all), once the stream is
-// done with everything before: one copy behind the kernels, one wait (with a wait
+// The first `count` words of d_results (result_count(): with all partials), once the
+// stream is done with everything before: one copy behind the kernels, one wait (with a wait
 // first and a copy each for the failure and the partials, 400 locations took 242
 // us for 225 now; a batch of 24, read back problem by problem, 3.20 ms for 2.56).
-int read_results(egs_problem_s *p, int count) {
-    p->h_results.resize((size_t) p->result_count());
-    EGS_HIP(hipMemcpyAsync(p->h_results.data(), p->d_results, sizeof(double) * (size_t) count, hipMemcpyDeviceToHost,
-                           p->ctx->stream));
+int read_results(egs_problem_s *p, int64_t count, const double *from = nullptr) {
+    try {
+        p->h_results.resize((size_t) std::max<int64_t>(p->result_count(), count));
+    } catch (const std::bad_alloc &) {
+        return fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate %lld doubles for the results", (long long) count);
+    }
+    EGS_HIP(hipMemcpyAsync(p->h_results.data(), from ? from : p->d_results, sizeof(double) * (size_t) count,
+                           hipMemcpyDeviceToHost, p->ctx->stream));
     EGS_HIP(hipStreamSynchronize(p->ctx->stream));
     return EGS_SUCCESS;
 }
@@ -862,22 +868,34 @@ void sum_partials(const egs_problem_s *p, const double *results, double &logdet,
     quad = q;
 }
 
-// d_work = L^{-1} src (src null: of d_work itself; prepared: by run_potrf); the
+// The `count` values behind the failure word, or behind a copy of it (from), with it
+// in one copy (with a copy of its own for the word, which waits for the one before,
+// the triangular solve of 300 locations took 48.6 us for 36.9 now).
+int return_vector(egs_problem_s *p, const double *from, double *out, int64_t count) {
+    int st = read_results(p, 1 + count, from);
+    if (st) return st;
+    if ((st = check_info(p))) return st;
+    std::memcpy(out, p->h_results.data() + 1, sizeof(double) * (size_t) count);
+    return EGS_SUCCESS;
+}
+
+// z = L^{-1} src (z null: d_work; src null: of z itself; prepared: by run_potrf); the
 // log-det and dot partials of its 64-row blocks go to `partials` (may be null).
-void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partials, bool prepared = false) {
+void run_forward(egs_problem_s *p, const double *src, int64_t n, double *partials, bool prepared = false,
+                 double *z = nullptr) {
     hipStream_t s = p->ctx->stream;
     const int pi = prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n);
-    if (!prepared) egs::launch_init(p->init_job(false, true, src, n), s);
-    egs::launch_forward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, partials, p->d_info(), s);
+    if (!prepared) egs::launch_init(p->init_job(false, true, src, n, z), s);
+    egs::launch_forward(p->map(), is_mixed(p), p->d_winv, z ? z : p->d_work, p->d_aux, partials, p->d_info(), s);
     prof_end(p, pi);
 }
 
-// d_work = L^{-T} src, likewise.
-void run_backward(egs_problem_s *p, const double *src, int64_t n) {
+// z = L^{-T} src, likewise.
+void run_backward(egs_problem_s *p, const double *src, int64_t n, double *z = nullptr) {
     hipStream_t s = p->ctx->stream;
     const int pi = is_mixed(p) ? prof_begin(p, EGS_PROFILE_SOLVE, (double) p->n * (double) p->n) : -1;
-    egs::launch_init(p->init_job(false, true, src, n), s);
-    egs::launch_backward(p->map(), is_mixed(p), p->d_winv, p->d_work, p->d_aux, p->d_info(), s);
+    egs::launch_init(p->init_job(false, true, src, n, z), s);
+    egs::launch_backward(p->map(), is_mixed(p), p->d_winv, z ? z : p->d_work, p->d_aux, p->d_info(), s);
     prof_end(p, pi);
 }
 
@@ -1086,8 +1104,7 @@ int64_t footprint(const egs_problem_s &q) {
     const int64_t nb = (int64_t) sizeof(double) * q.n_loc, vb = (int64_t) sizeof(double) * npad;
     int64_t b = dev_class_bytes(nb) * (q.dim == 3 ? 3 : 2) + dev_class_bytes(8 * nt * nt) + dev_class_bytes(nt * nt) +
                 dev_class_bytes(8 * ntiles) + dev_class_bytes(8 * nt * q.nsb * egs::kBlk * egs::kBlk) +
-                dev_class_bytes(4 * q.sync_ints()) + 2 * dev_class_bytes(vb) + dev_class_bytes(vb + 8) +
-                dev_class_bytes(8 + 16 * nt * q.nsb) +
+                dev_class_bytes(4 * q.sync_ints()) + 2 * dev_class_bytes(vb) + 2 * dev_class_bytes(vb + 8) +
                 dev_class_bytes(8 * egs::kTabSlots * egs::kTabDoubles);
     int64_t arena = 0;
     for (int j = 0; j < q.nt; ++j)
@@ -1255,7 +1272,7 @@ int egs_problem_create(egs_context_t ctx, int kernel, int64_t n_loc, const doubl
               pmalloc(p, &p->d_sync, sizeof(int) * (size_t) p->sync_ints()) == hipSuccess &&
               pmalloc(p, &p->d_obs, vb) == hipSuccess && pmalloc(p, &p->d_work, vb) == hipSuccess &&
               pmalloc(p, &p->d_aux, vb + sizeof(double)) == hipSuccess &&
-              pmalloc(p, &p->d_results, sizeof(double) * (1 + 2 * (size_t) nt * p->nsb)) == hipSuccess &&
+              pmalloc(p, &p->d_results, vb + sizeof(double)) == hipSuccess &&
               pmalloc(p, &p->d_tab, sizeof(double) * egs::kTabSlots * egs::kTabDoubles) == hipSuccess;
     if (!ok) return cleanup(fail(EGS_ERR_OUT_OF_MEMORY, "cannot allocate the problem's device buffers"));
     for (auto &e : p->ev)
@@ -1478,11 +1495,10 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
         return fail(EGS_ERR_UNSUPPORTED, "the triangular solve with the stored factor runs under the FP64 plan");
     hipStream_t s = p->ctx->stream;
     EGS_HIP(hipMemcpyAsync(p->d_work, z, sizeof(double) * (size_t) n, hipMemcpyHostToDevice, s));
-    if (trans == 0) run_forward(p, p->d_work, p->n, nullptr);
-    else run_backward(p, p->d_work, p->n);
+    if (trans == 0) run_forward(p, p->d_work, p->n, nullptr, false, p->d_partials());
+    else run_backward(p, p->d_work, p->n, p->d_partials());
     EGS_HIP(hipGetLastError());
-    EGS_HIP(hipMemcpyAsync(z, p->d_work, sizeof(double) * (size_t) n, hipMemcpyDeviceToHost, s));
-    if ((st = read_info(p))) return st;
+    if ((st = return_vector(p, p->d_results, z, n))) return st;
     if (alpha != 1.0)
         for (int64_t i = 0; i < n; ++i) z[i] *= alpha;
     return EGS_SUCCESS;
@@ -2030,7 +2046,7 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
     // targets and predictions share one buffer that the problem keeps (grown
     // on demand), so repeated predictions allocate nothing
     const int64_t rows = n_miss * p->p;
-    const int64_t need = rows + 3 * n_miss;
+    const int64_t need = 1 + rows + 3 * n_miss;
     if (need > p->pred_cap) {
         EGS_HIP(hipStreamSynchronize(s));
         pfree(p, p->d_pred);
@@ -2062,22 +2078,21 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
         run_forward(p, p->d_obs, p->n, nullptr);
         run_backward(p, nullptr, 0);
     }
-    double *d_out = p->d_pred, *dxm = d_out + rows, *dym = dxm + n_miss, *dzm = dym + n_miss;
+    double *d_out = p->d_pred + 1, *dxm = d_out + rows, *dym = dxm + n_miss, *dzm = dym + n_miss;
     hipError_t e = hipMemcpyAsync(dxm, xm, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(dym, ym, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess && three_d) e = hipMemcpyAsync(dzm, zm, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         egs::launch_matern_tables(p->d_tab, prm, nullptr, s);
         egs::launch_cov_gemv(d_out, rows, p->n, prm, dxm, dym, three_d ? dzm : nullptr, p->d_x, p->d_y,
-                             three_d ? p->d_z : nullptr, weights, p->d_tab, s);
+                             three_d ? p->d_z : nullptr, weights, p->d_tab, p->d_results, s);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(zmiss, d_out, sizeof(double) * (size_t) rows, hipMemcpyDeviceToHost, s);
     if (e != hipSuccess) {
         (void) hipStreamSynchronize(s);
         return fail(EGS_ERR_HIP, "prediction: %s", hipGetErrorString(e));
     }
-    if ((st = read_info(p))) return st;
+    if ((st = return_vector(p, p->d_pred, zmiss, rows))) return st;
     if (!reuse) {
         p->factored = true;
         std::memcpy(p->factored_theta, theta, sizeof(double) * p->ntheta());

@@ -112,10 +112,11 @@ void launch_backward(const TileMap &map, bool mixed, const double *winv, double 
                      hipStream_t s);
 // out = L e (lower-triangular product over the tiles).
 void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s);
-// out[r] = sum_c Sigma(l1_r, l2_c) x[c] for r < rows, c < cols (kriging mean).
+// out[r] = sum_c Sigma(l1_r, l2_c) x[c] for r < rows, c < cols (kriging mean);
+// out[-1] = *word.
 void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams &prm, const double *x1,
                      const double *y1, const double *z1, const double *x2, const double *y2, const double *z2,
-                     const double *xv, const double *tabs, hipStream_t s);
+                     const double *xv, const double *tabs, const double *word, hipStream_t s);
 // partial[cb * npad + r] = sum over column chunk cb of Sigma(r, c) v[c] (FP64,
 // regenerated from the locations); matvec_chunks(n) chunks.
 void launch_cov_matvec(double *partial, const double *v, int64_t n, int64_t npad, const MaternParams &prm,

@@ -393,6 +393,7 @@ struct CovGemvArgs {
     Locs l1, l2;
     const double *x;
     const double *tabs;
+    const double *word;   // copied to out[-1]
     int three_d;
 };
 
@@ -417,6 +418,7 @@ __global__ void __launch_bounds__(kThreads, kTabs < 2 ? 4 : 4 - kTabs) cov_gemv_
     }
     s = wg_sum(s, red);
     if (threadIdx.x == 0) a.out[r] = s;
+    if (r == 0 && threadIdx.x == 0) a.out[-1] = *a.word;
 }
 
 // dlarnv(idist = 3): value m uses the uniforms number 2m and 2m+1 of the
@@ -629,7 +631,7 @@ void launch_trmv(const TileMap &map, const double *e, double *out, hipStream_t s
 
 void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams &prm, const double *x1,
                      const double *y1, const double *z1, const double *x2, const double *y2, const double *z2,
-                     const double *xv, const double *tabs, hipStream_t s) {
+                     const double *xv, const double *tabs, const double *word, hipStream_t s) {
     if (rows <= 0) return;
     CovGemvArgs a;
     a.out = out;
@@ -640,6 +642,7 @@ void launch_cov_gemv(double *out, int64_t rows, int64_t cols, const MaternParams
     a.l2 = Locs{x2, y2, z2};
     a.x = xv;
     a.tabs = tabs;
+    a.word = word;
     a.three_d = (z1 != nullptr && z2 != nullptr);
     static void (*const kernels[2][kTabSlots + 1])(CovGemvArgs) = {
         {cov_gemv_kernel<0, false>, cov_gemv_kernel<1, false>, cov_gemv_kernel<2, false>, cov_gemv_kernel<3, false>},
