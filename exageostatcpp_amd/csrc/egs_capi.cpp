@@ -2083,6 +2083,11 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
     if (e == hipSuccess) e = hipMemcpyAsync(dym, ym, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess && three_d) e = hipMemcpyAsync(dzm, zm, sizeof(double) * n_miss, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
+        // With one location per thread and two rows per CU a table costs more than it
+        // saves: kriging of 1 / 100 / 500 points, nu 0.83, 50 locations 103 / 104 / 110
+        // us with it, 83 / 89 / 95 without; 150 104 / 104 / 108 and 91 / 90 / 103; 300 113 / 113 / 117 and
+        // 110 / 116 / 139; 2,000 points at 50 locations 112 and 135.
+        if (p->n <= 256 && rows <= 512) prm.ntab = 0;
         egs::launch_matern_tables(p->d_tab, prm, nullptr, s);
         egs::launch_cov_gemv(d_out, rows, p->n, prm, dxm, dym, three_d ? dzm : nullptr, p->d_x, p->d_y,
                              three_d ? p->d_z : nullptr, weights, p->d_tab, p->d_results, s);
