@@ -3,7 +3,7 @@
 // Host orchestration only: shape checks, HBM layout of a problem, the order of
 // kernel launches on the context's stream.  All arithmetic on Sigma runs in the
 // HIP kernels of egs_covgen.hip, egs_chol.hip and egs_solve.hip; the host adds
-// up nt per-tile partials in tile order and evaluates the closing formula of
+// up the partials of the 64-row blocks in order and evaluates the closing formula of
 // ChameleonImplementation.cpp:257-265.
 #include <hip/hip_runtime.h>
 
@@ -643,7 +643,8 @@ void factor_panel(egs_problem_s *p, int k) {
     // the FP64 rows go with the diagonal tile when they are few; the FP32 rows
     // of a bivariate plan are solved together with the FP64 ones (both on FP64
     // MFMA)
-    const bool fused = blocks64 > 0 && egs::tile_column_solves_rows(p->ts, blocks64) && (blocks32 == 0 || p->f32_panel_solve);
+    const bool fused =
+        blocks64 > 0 && egs::tile_column_solves_rows(p->ts, blocks64) && (blocks32 == 0 || p->f32_panel_solve);
     double real64 = 0.0, real32 = 0.0;   // rows below that hold rows of the matrix, for the flops
     for (int i = k + 1; i < nt; ++i) (i <= k + rows64 ? real64 : real32) += real_rows(p, i);
     int pi = prof_begin(p, EGS_PROFILE_DIAGONAL, kb * kb * kb / 3.0 + (fused ? real64 * ts * ts : 0.0));
@@ -810,10 +811,11 @@ int run_potrf(egs_problem_s *p, bool then_solve = false) {
     return EGS_SUCCESS;
 }
 
-// The first `count` words of d_results (result_count(): with all partials), once the
-// stream is done with everything before: one copy behind the kernels, one wait (with a wait
-// first and a copy each for the failure and the partials, 400 locations took 242
-// us for 225 now; a batch of 24, read back problem by problem, 3.20 ms for 2.56).
+// The first `count` words of d_results (result_count(): with all partials) or of
+// `from`, once the stream is done with everything before: one copy behind the
+// kernels, one wait (with a wait first and a copy each for the failure and the
+// partials, 400 locations took 242 us for 225; a batch of 24, read back problem by
+// problem, 3.20 ms for 2.56).
 int read_results(egs_problem_s *p, int64_t count, const double *from = nullptr) {
     try {
         p->h_results.resize((size_t) std::max<int64_t>(p->result_count(), count));
@@ -1506,7 +1508,7 @@ int egs_trsm_vector(egs_problem_t p, int trans, double alpha, double *z, int64_t
 
 // One FP64 evaluation on the problem's streams, with the covariance parameters
 // read from d_prm: observations copied, covariance, factorization, forward solve
-// with the per-tile log-det and dot partials.  Everything it enqueues is
+// with the log-det and dot partials of its 64-row blocks.  Everything it enqueues is
 // capturable (no host synchronization, no memset).
 int enqueue_fp64_eval(egs_problem_s *p) {
     hipStream_t s = p->ctx->stream;
@@ -2085,8 +2087,8 @@ static int predict_once(egs_problem_s *p, const double *theta, int64_t n_miss, c
     if (e == hipSuccess) {
         // With one location per thread and two rows per CU a table costs more than it
         // saves: kriging of 1 / 100 / 500 points, nu 0.83, 50 locations 103 / 104 / 110
-        // us with it, 83 / 89 / 95 without; 150 104 / 104 / 108 and 91 / 90 / 103; 300 113 / 113 / 117 and
-        // 110 / 116 / 139; 2,000 points at 50 locations 112 and 135.
+        // us with it, 83 / 89 / 95 without; 150 104 / 104 / 108 and 91 / 90 / 103; 300
+        // 113 / 113 / 117 and 110 / 116 / 139; 2,000 points at 50 locations 112 and 135.
         if (p->n <= 256 && rows <= 512) prm.ntab = 0;
         egs::launch_matern_tables(p->d_tab, prm, nullptr, s);
         egs::launch_cov_gemv(d_out, rows, p->n, prm, dxm, dym, three_d ? dzm : nullptr, p->d_x, p->d_y,

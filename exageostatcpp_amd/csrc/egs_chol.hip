@@ -13,11 +13,11 @@
 //   * the trailing tiles are updated with FP64 MFMA: update192 (egs_update.hip)
 //     when ts is a multiple of 192 and the tiles are many, else update_kernel
 //     here, one workgroup per 64 x 64 output block (or half of one) with K = ts.
-// Every contraction uses v_mfma_f64_16x16x4f64 through wg_gemm_nt: four waves
-// each own a 32 x 32 quadrant of the 64 x 64 output; K is staged through LDS in
-// chunks of 32 columns, double buffered, with the next chunk's global loads
-// issued before the current chunk's MFMAs (these kernels run on few
-// workgroups, so each one has to hide its own memory latency).
+// The panel solves and update_kernel contract through wg_gemm_nt: four waves each
+// own a 32 x 32 quadrant of the 64 x 64 output (16 columns of 32 rows); K is staged
+// through LDS in chunks of 32 columns, double buffered, with the loads of the next
+// two chunks in flight during a chunk's MFMAs.  The tasks of a diagonal tile
+// multiply whole 64 x 64 blocks in LDS.
 #include <algorithm>
 
 #include "egs_common.hpp"
@@ -621,8 +621,7 @@ __device__ __forceinline__ void acc_load(Acc64 &acc, const double *C, int64_t ld
 
 // The lower 16 x 16 tiles of a diagonal block, ten, dealt to the waves: tile w +
 // 4 q of the rows' order (waves 2 and 3 carry the last one along as their third,
-// of no effect: a branch around it cost as much, and the compiler then counted
-// the products' latency wrong across it, which gave wrong results).
+// of no effect: a branch around it cost as much).
 struct DiagAcc {
     f64x4 v[3];
     static __device__ __forceinline__ int tile(int w, int q) { return 4 * min(w + 4 * q, 9); }

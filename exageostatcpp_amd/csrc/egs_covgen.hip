@@ -20,7 +20,8 @@ namespace egs {
 // row's own error is common to all entries it serves, so that the jumps
 // between rows, unlike rounding noise, add up in z'Sigma^-1 z (at 40,000
 // locations and nu = 1, 16 nodes and one double for a_0 put 1.3e-11 into the
-// log-likelihood).  Bound: the latency of one K_nu, 20 us whatever the size.
+// log-likelihood).  Bound: latency, 28 us whatever the size (K_nu, then
+// the sums over its nodes).
 // ------------------------------------------------------------------------
 constexpr int kNodes = 64;
 constexpr int kDegree = kTabDegree;

@@ -2,12 +2,12 @@
 // and the synthetic-data helpers on gfx950.
 //
 // The forward solve replaces CHAMELEON_dtrsm_Tile(Left, Lower, NoTrans) on Z
-// (ChameleonImplementation.cpp:216-217, 337-347) and fuses the per-tile
-// reductions the reference runs as dmdet (dmdet-codelet.cpp:70-80) and ddotp
-// (ddotp-codelet.cpp:62-72) tasks: the workgroup that solves diagonal tile k
-// also writes sum(log L_ii) over L_ii > 0 and y_k . y_k for that tile.  The host
-// sums the per-tile partials in tile order, so results do not depend on
-// scheduling.  All reductions inside a workgroup use a fixed order.
+// (ChameleonImplementation.cpp:216-217, 337-347) and fuses the reductions the
+// reference runs per tile as dmdet (dmdet-codelet.cpp:70-80) and ddotp
+// (ddotp-codelet.cpp:62-72) tasks: the workgroup that solves a block b of 64 rows
+// also writes sum(log L_ii) over L_ii > 0 and y_b . y_b of that block.  The host
+// sums the blocks' partials in order, so results do not depend on scheduling.  All
+// reductions inside a workgroup use a fixed order.
 #include <algorithm>
 
 #include "egs_common.hpp"
